@@ -324,6 +324,23 @@ def test_swiglu_and_combine(ops, oracle):
     assert np.array_equal(got, oracle.moe_combine(ys, wt16.float().cpu().numpy()))
 
 
+@pytest.mark.parametrize("T,k,n", [(1, 1, 4), (3, 4, 1020), (2, 5, 1024), (2, 8, 1028), (3, 9, 2048), (5, 17, 512), (3, 3, 6), (2, 8, 1022)])
+@pytest.mark.parametrize("shift", [0, 4])
+def test_combine_vector_rows_and_remainders(ops, oracle, T, k, n, shift):
+    """Rows of whole and broken groups of four, more slots than one batch of loads, and rows that are not 16-byte aligned."""
+    rng = np.random.default_rng(T * 1000 + k * 10 + n)
+    ys = rng.standard_normal((T, k, n)).astype(np.float32)
+    wt = rng.random((T, k)).astype(np.float32)
+    buf = torch.empty(T * k * n + 1, device="cuda")
+    dev = buf[shift // 4: shift // 4 + T * k * n].view(T, k, n)
+    dev.copy_(torch.from_numpy(ys))
+    want = oracle.moe_combine(ys, wt)
+    got = ops.moe_combine(dev, torch.from_numpy(wt).cuda(), torch.float32).cpu().numpy()
+    assert np.array_equal(got, want)  # the same fmaf chain in slot order
+    got16 = ops.moe_combine(dev, torch.from_numpy(wt).cuda(), torch.bfloat16)
+    assert np.array_equal(bits(got16), rne_bf16(want))
+
+
 @pytest.mark.parametrize("T,k,E", [(1, 8, 256), (9, 8, 256), (130, 8, 64), (33, 3, 7), (2048, 8, 256), (1024, 4, 32), (1025, 4, 32),
                                    (8192, 8, 256), (70001, 2, 16)])  # the last one: more than one chunk of 64 rounds
 @pytest.mark.parametrize("idt", [torch.int32, torch.int64])
