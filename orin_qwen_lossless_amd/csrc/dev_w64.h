@@ -186,6 +186,10 @@ struct w64_dec_t {
         e0 = entry(W & 0x3FFCu);
         const uint32_t W2 = W >> (e0 & 31u);
         e1 = entry(W2 & 0x3FFCu);
+        advance(e0, e1);
+    }
+    // the position moves past two pair codes
+    __device__ __forceinline__ void advance(uint32_t e0, uint32_t e1) {
         // entry bits 5 and 6 are zero: the low seven bits of the running sum are exact (the exponent fields only add
         // above them), and two pair codes are at most 24 bits, so bit 5 changes exactly when a word boundary is passed
         P = P + e0 + e1;
@@ -215,6 +219,23 @@ struct w64_dec_t {
     }
 };
 typedef w64_dec_t<-1> w64_dec;
+
+// Two pair codes of two chains (e[chain][code]; entry(chain, offset): a table entry).  The lookups of the chains are
+// issued together and the barriers keep them so: left to itself under register pressure the compiler finishes one chain
+// before it starts the other, and every LDS read is waited for with nothing beside it.
+template <int HINT, typename L>
+__device__ __forceinline__ void two_chains(w64_dec_t<HINT> & a, w64_dec_t<HINT> & b, L entry, uint32_t (&e)[2][2]) {
+    const uint32_t wa = __builtin_amdgcn_alignbit(a.w1, a.w0, a.P), wb = __builtin_amdgcn_alignbit(b.w1, b.w0, b.P);
+    e[0][0] = entry(0, wa & 0x3FFCu);
+    e[1][0] = entry(1, wb & 0x3FFCu);
+    __builtin_amdgcn_sched_barrier(0);
+    e[0][1] = entry(0, wa >> (e[0][0] & 31u) & 0x3FFCu);
+    e[1][1] = entry(1, wb >> (e[1][0] & 31u) & 0x3FFCu);
+    __builtin_amdgcn_sched_barrier(0);
+    a.advance(e[0][0], e[0][1]);
+    b.advance(e[1][0], e[1][1]);
+    __builtin_amdgcn_sched_barrier(0);
+}
 
 // Every block of a launch stages the same 16 KiB; the blocks start at different 1 KiB pieces of it so that they do not
 // all ask for the same cache lines at the same moment.

@@ -7,6 +7,7 @@
 //   * k_mm_tile: batched MoE prefill (reference mm_ids / k_hp_mm_ids, core/src/launch.cu:473-535,
 //     core/src/kernels.cuh:1162-1505).  Weights go from the decoder's registers into the matrix cores; the activations
 //     of up to 128 tokens are staged in LDS, 128 columns at a time, and shared by the eight wavefronts of a block.
+//   * k_mm_wide: the same for many tokens per expert: up to 320 tokens per decode.
 //   * k_tile_mmv: GEMV / fused gate-up GEMV at decode (reference mmv / mmv_glu, launch.cu:313-365): a lane accumulates
 //     one row over the whole tile, so a tile ends with one cross-half add instead of a reduction per row.
 //   * k_tile_dequant, k_tile_get_rows: exact BF16 rows (launch.cu:367-443).
@@ -468,6 +469,243 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_tile(const bf
     }
 }
 
+// ---------------------------------------------------------------- batched products with many tokens per expert
+//
+// A work item is (expert, slab of eight row groups: eight of the matrix, or four of gate and the same four of up) and a
+// pass up to 320 of the expert's tokens.  What bounds these products is the decode: a step of a chain is eight dependent
+// LDS reads, some 3000 cycles at two wavefronts per SIMD whatever it feeds, and k_mm_tile, which keeps two row groups
+// per wavefront, has registers for 128 tokens of them.  Here a wavefront owns one row group and ten accumulator blocks
+// of 32 tokens (160 registers), and its two decode chains are the two halves of that row group's columns, which end in
+// the same accumulators: an expert with 129 to 320 tokens is decoded once.  The two blocks of 32 columns that a step
+// needs of every token are copied from memory into LDS by the load instructions themselves (no registers, two buffers,
+// a step ahead): 128 bytes per token, the 16-byte piece c of row r at c ^ (r & 7), so that eight tokens meet all banks.
+// 256 experts of 512 x 2048, top-8, fused gate / up and down product, against k_mm_tile's 128-token passes (us):
+//   4096 tokens: 402 + 266 -> 306 + 218;  6000: 478 + 328 -> 363 + 265;  8192: 643 + 426 -> 430 + 319.
+// Measured and dropped: multiplying a half step while the next is decoded, with a second set of A operands (8192 tokens:
+// 483 + 360); nine accumulator blocks and operands read two blocks ahead (483 + 332: 288 tokens are one pass too few
+// for some experts); the flat form of the LDS copies (466 + 337), for which the compiler drains all LDS reads at each use.
+constexpr int WD_WAVES = 8, WD_NT = 10, WD_TOK = 32 * WD_NT;
+constexpr int WD_ROW = 128, WD_BUF = WD_TOK * WD_ROW;                         // bytes per staged token, per buffer
+constexpr int WD_COPIES = WD_TOK / (8 * WD_WAVES);                            // copy instructions per wavefront and step: eight tokens each
+// Routed pairs per expert from which it runs.  Below, every expert's tokens fit one 128-token pass of k_mm_tile, which
+// has half the LDS reads per matrix instruction: 3000 tokens of the layer above (94 pairs) 246 + 177 against 272 + 194 us,
+// 3300 tokens (103 pairs, where the first experts have more than 128) 321 + 205 against 277 + 204.
+constexpr int WD_MIN_PAIRS = 98;
+
+template <bool GLU>
+__global__ void __launch_bounds__(WD_WAVES * 64) k_mm_wide(const bf16n_weight w, const bf16n_weight w_up, const mm_args a) {
+    constexpr int NM = GLU ? 2 : 1, GPI = WD_WAVES / NM; // row groups per work item
+    extern __shared__ __align__(16) uint32_t shm[];
+    char * bbuf = (char *) (shm + NM * LUT_WORDS + WD_WAVES * 2 * WAVE_LDS_WORDS);
+    const int tid = threadIdx.x, lane = tid & 63, l32 = tid & 31, half = lane >> 5, wave = (int) uniform(tid >> 6);
+    const int m = GLU ? wave / GPI : 0, gw = GLU ? wave % GPI : wave; // matrix and row group inside the item
+    uint32_t * ring = shm + NM * LUT_WORDS + wave * (2 * WAVE_LDS_WORDS);
+    stage_lut(shm, (const uint32_t *) (w.aux + w.off_a));
+    if (GLU) {
+        stage_lut(shm + LUT_WORDS, (const uint32_t *) (w_up.aux + w_up.off_a));
+    }
+    const uint32_t lut_base = (uint32_t) m * (LUT_WORDS * 4);   // LDS address of this wavefront's table
+    const w64_ptrs q = w64p(GLU && m ? w_up : w);
+    const int slabs = (int) (w.K / TILE_K), chain_tiles = slabs / 2, n_steps = chain_tiles * T_STEPS;
+    const int groups = (int) (a.rows / TILE_R), spe = (groups + GPI - 1) / GPI; // work items per expert
+    // The items of an expert read the same activations: they are dealt to blocks of one XCD (block b runs on XCD b % 8)
+    const bool xcds = gridDim.x % 8 == 0 && a.n_experts % 8 == 0;
+    const int lanes_x = xcds ? 8 : 1, xcd = xcds ? (int) blockIdx.x % 8 : 0, bl = (int) blockIdx.x / lanes_x, bn = (int) gridDim.x / lanes_x;
+    // where this lane's B operands start: token l32's row, piece `half`, as the swizzle places it
+    const uint32_t b_at = (uint32_t) (l32 * WD_ROW + ((half ^ (l32 & 7)) << 4));
+    __syncthreads();
+    for (int it = bl;; it += bn) {
+        const int e = it / spe * lanes_x + xcd, sl = it % spe;
+        if (e >= a.n_experts) {
+            break;
+        }
+        const int first = a.bounds ? a.bounds[e] : 0, n = a.bounds ? a.bounds[e + 1] - first : a.n_tok;
+        if (n <= 0) {
+            continue;
+        }
+        // (a wavefront without a row group of its own decodes the last one and stores nothing)
+        const bool live = sl * GPI + gw < groups;
+        const int g = live ? sl * GPI + gw : groups - 1;
+        // passes of equal length
+        const int n_pass = (n + WD_TOK - 1) / WD_TOK, pass = ((n + n_pass - 1) / n_pass + 31) & ~31;
+        for (int tp = 0; tp < n; tp += pass) {
+            const int nn = n - tp < pass ? n - tp : pass, nt = (nn + 31) >> 5, j0 = first + tp;
+            const int n_copies = (nt + 1) >> 1;
+            // this lane's source in the copies of the wavefront: token 8 (wave + 8 i) + lane / 8, piece as swizzled
+            uint32_t src[WD_COPIES];
+            {
+                const int c = (lane & 7) ^ (lane >> 3);
+#pragma unroll
+                for (int i = 0; i < WD_COPIES; i++) {
+                    const int tok = 8 * (wave + WD_WAVES * i) + (lane >> 3), j = j0 + (tok < nn ? tok : nn - 1);
+                    src[i] = (uint32_t) (a.ids_src1 ? a.ids_src1[j] : j) * (uint32_t) (2 * a.x_row) + ((c & 3) << 4) + (c >> 2) * (uint32_t) w.K; // (K / 2 BF16)
+                }
+            }
+            const range_t xr = make_range(a.x, 0xFFFFFFFFu);
+            int xs = 0; // byte offset of the columns of the next copies
+            // (through a buffer descriptor: the compiler takes the flat form of these copies for LDS traffic of unknown
+            // order and waits for all LDS reads in flight at every use of one)
+            auto copy = [&](int buf) {
+#pragma unroll
+                for (int i = 0; i < WD_COPIES; i++) {
+                    if (i < n_copies) {
+                        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void *) (bbuf + buf * WD_BUF + (wave + WD_WAVES * i) * 1024),
+                                                                 16, (int) src[i], xs, 0, 0);
+                    }
+                }
+            };
+            tchain_t<2, false> ch[2];
+            {
+                const int64_t u0 = ((int64_t) e * groups + g) * slabs, u1 = u0 + chain_tiles;
+                const uint32_t f0 = q.ubase[u0], f1 = q.ubase[u1], e1 = q.ubase[u1 + chain_tiles];
+                ch[0].start(ring, q, u0, chain_tiles, lane, f0, f1, false, true);
+                ch[1].start(ring + WAVE_LDS_WORDS, q, u1, chain_tiles, lane, f1, e1, false, true);
+            }
+            copy(0);
+            ch[0].dec.start_finish();
+            ch[1].dec.start_finish();
+            f32x16_t acc[WD_NT];
+#pragma unroll
+            for (int t = 0; t < WD_NT; t++) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    acc[t][i] = 0.f;
+                }
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): the first copies are in LDS
+            __syncthreads();
+#pragma unroll 1
+            for (int st = 0; st < n_steps; st += 2) {
+                if (st % T_STEPS == 0) {
+                    ch[0].begin_tile();
+                    ch[1].begin_tile();
+                }
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    ch[0].dec.keep_ahead();
+                    ch[1].dec.keep_ahead();
+                    // the next step's activations (after the last step the same again, into the buffer nobody reads)
+                    xs += s == 0 || st + 2 < n_steps ? 64 : 0;
+                    copy(1 - s);
+                    const uint4 p0 = ch[0].sm[s], p1 = ch[1].sm[s];
+                    const uint32_t smw[2][4] = {{p0.x, p0.y, p0.z, p0.w}, {p1.x, p1.y, p1.z, p1.w}};
+#pragma unroll
+                    for (int kb = 0; kb < 2; kb++) {
+                        uint32_t wq[2][4];
+#pragma unroll
+                        for (int j = 0; j < 2; j++) {
+                            uint32_t en[2][2];
+                            two_chains(ch[0].dec, ch[1].dec, [lut_base](int, uint32_t off) {
+                                return *(const __attribute__((address_space(3))) uint32_t *) (uintptr_t) (GLU ? off | lut_base : off);
+                            }, en);
+#pragma unroll
+                            for (int k = 0; k < 2; k++) {
+                                wq[k][2 * j] = merge(spread_lo(smw[k][2 * kb + j]), en[k][0]);
+                                wq[k][2 * j + 1] = merge(spread_hi(smw[k][2 * kb + j]), en[k][1]);
+                            }
+                        }
+                        const char * bp0 = bbuf + s * WD_BUF + (b_at ^ (uint32_t) (kb * 32)), * bp1 = bbuf + s * WD_BUF + (b_at ^ (uint32_t) (64 + kb * 32));
+                        const u32x4_t v0 = {wq[0][0], wq[0][1], wq[0][2], wq[0][3]}, v1 = {wq[1][0], wq[1][1], wq[1][2], wq[1][3]};
+                        const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, v0), a1 = __builtin_bit_cast(bf16x8_t, v1);
+                        // the operands of the next token block travel while this one's are multiplied
+                        bf16x8_t bv[2][2]; // [block parity][chain]
+                        bv[0][0] = *(const bf16x8_t *) bp0;
+                        bv[0][1] = *(const bf16x8_t *) bp1;
+#pragma unroll
+                        for (int t = 0; t < WD_NT; t++) {
+                            if (t > 0 && t >= nt) { // (an exit, not a condition per block: the waits for LDS stay exact)
+                                break;
+                            }
+                            if (t + 1 < WD_NT) {
+                                bv[(t + 1) & 1][0] = *(const bf16x8_t *) (bp0 + (t + 1) * 32 * WD_ROW);
+                                bv[(t + 1) & 1][1] = *(const bf16x8_t *) (bp1 + (t + 1) * 32 * WD_ROW);
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
+                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, bv[t & 1][0], acc[t], 0, 0, 0);
+                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, bv[t & 1][1], acc[t], 0, 0, 0);
+                        }
+                    }
+                    // The copies of this step have to be in LDS before the barrier; the two plane loads behind them
+                    // (which the fences keep there) stay in flight.
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    ch[0].reload(s, lane);
+                    ch[1].reload(s, lane);
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    __builtin_amdgcn_s_waitcnt(0x0072); // vmcnt(2) lgkmcnt(0)
+                    __builtin_amdgcn_s_barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" ::: "memory");
+                }
+            }
+            // accumulator element i of a lane: row 8 (i / 4) + 4 (lane / 32) + i % 4 of the group, token lane % 32
+            auto store = [&](int t, const float (&v)[16]) {
+                const int tk = 32 * t + l32;
+                if (live && tk < nn) {
+                    const int64_t o = (int64_t) (a.ids_dst ? a.ids_dst[j0 + tk] : tp + tk) * a.dst_col + (int64_t) g * TILE_R + 4 * half;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        if (a.dst_bf16) {
+                            *(uint2 *) ((uint16_t *) a.dst + o + 8 * k) =
+                                make_uint2(f32_to_bf16_rne(v[4 * k]) | ((uint32_t) f32_to_bf16_rne(v[4 * k + 1]) << 16),
+                                           f32_to_bf16_rne(v[4 * k + 2]) | ((uint32_t) f32_to_bf16_rne(v[4 * k + 3]) << 16));
+                        } else {
+                            *(float4 *) ((float *) a.dst + o + 8 * k) = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+                        }
+                    }
+                }
+            };
+            if constexpr (GLU) {
+                // the gate and the up wavefront of a row group swap token blocks through their idle rings: gate finishes
+                // the even blocks, up the odd ones
+                float4 * mine = (float4 *) ring + lane;
+                const float4 * other = (const float4 *) (m ? ring - GPI * 2 * WAVE_LDS_WORDS : ring + GPI * 2 * WAVE_LDS_WORDS) + lane;
+#pragma unroll
+                for (int r = 0; r < WD_NT / 2; r++) {
+                    if (2 * r < nt) {
+                        float v[16];
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                v[i] = m ? acc[2 * r][4 * k + i] : acc[2 * r + 1][4 * k + i];
+                            }
+                            mine[64 * k] = make_float4(v[0], v[1], v[2], v[3]);
+                        }
+                        __syncthreads();
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const float4 o4 = other[64 * k];
+                            const float o[4] = {o4.x, o4.y, o4.z, o4.w};
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                v[4 * k + i] = m ? acc[2 * r + 1][4 * k + i] * silu(o[i]) : o[i] * silu(acc[2 * r][4 * k + i]);
+                            }
+                        }
+                        store(2 * r + m, v);
+                        __syncthreads();
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < WD_NT; t++) {
+                    if (t < nt) {
+                        float v[16];
+#pragma unroll
+                        for (int i = 0; i < 16; i++) {
+                            v[i] = acc[t][i];
+                        }
+                        store(t, v);
+                    }
+                }
+            }
+        }
+    }
+}
+
+size_t wd_shm(bool glu) { return (size_t) (glu ? 2 : 1) * LUT_WORDS * 4 + (size_t) WD_WAVES * 2 * WAVE_LDS_WORDS * 4 + 2 * (size_t) WD_BUF; }
+
 // ---------------------------------------------------------------- batched MoE prefill in two phases (many tokens per expert)
 //
 // With a few hundred tokens per expert the fused kernel above decodes every expert once per pass of 128 tokens, at
@@ -584,20 +822,22 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uin
             const int left = n - tp, nt = left >= S::TOK ? NT : (left + 31) >> 5;
             const int btk = tp + b_tok;
             const int bj = j0 + (btk < n ? btk : 0);
-            const uint16_t * xsrc = a.x + ((int64_t) (a.ids_src1 ? a.ids_src1[bj] : bj) * a.x_row + S::CPT * b_part);
+            // (staged together: 64 columns of either half of the row, the order in which k_mm_wide adds them up)
+            const uint16_t * xsrc = a.x + ((int64_t) (a.ids_src1 ? a.ids_src1[bj] : bj) * a.x_row + (S::CPT * b_part) / (MT_HK / 2) * (TILE_K / 2 * slabs) +
+                                           (S::CPT * b_part) % (MT_HK / 2));
             uint16_t * bdst = bbuf + b_tok * MT_BSTRIDE + S::CPT * b_part;
             uint4 f0, f1, f2, f3;
             if (stager) {
                 MT_STAGE_LOAD(S::VPT, f0, f1, f2, f3, (const uint4 *) xsrc);
             }
-            // A operands of the first D steps: [step][chain][16-column block]
+            // A operands of the first D steps: [step][chain][half of the columns].  A step is 16 columns of either half
             uint4 av[D][2][2];
 #pragma unroll
             for (int s = 0; s < D; s++) {
-                av[s][0][0] = pa0[(s * 2) * 64];
-                av[s][0][1] = pa0[(s * 2 + 1) * 64];
-                av[s][1][0] = pa1[(s * 2) * 64];
-                av[s][1][1] = pa1[(s * 2 + 1) * 64];
+                av[s][0][0] = pa0[s * 64];
+                av[s][0][1] = pa0[(s + n_steps) * 64];
+                av[s][1][0] = pa1[s * 64];
+                av[s][1][1] = pa1[(s + n_steps) * 64];
             }
             f32x16_t acc[2][NT];
 #pragma unroll
@@ -620,25 +860,25 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uin
                 const int nxt = hs + 1 < halves ? hs + 1 : hs;
                 uint4 b0, b1, b2, b3;
                 if (stager) {
-                    MT_STAGE_LOAD(S::VPT, b0, b1, b2, b3, (const uint4 *) (xsrc + nxt * MT_HK));
+                    MT_STAGE_LOAD(S::VPT, b0, b1, b2, b3, (const uint4 *) (xsrc + nxt * (MT_HK / 2)));
                 }
 #pragma unroll
                 for (int s = 0; s < 4; s++) {
-                    const uint16_t * bp = bcur + l32 * MT_BSTRIDE + 32 * s + 8 * half;
+                    const uint16_t * bp = bcur + l32 * MT_BSTRIDE + 16 * s + 8 * half;
                     const int sd = s % D;
                     const bf16x8_t a00 = __builtin_bit_cast(bf16x8_t, av[sd][0][0]), a01 = __builtin_bit_cast(bf16x8_t, av[sd][0][1]);
                     const bf16x8_t a10 = __builtin_bit_cast(bf16x8_t, av[sd][1][0]), a11 = __builtin_bit_cast(bf16x8_t, av[sd][1][1]);
                     // the same slot's operands D steps on (the last steps of a pass ask for the pass's last step again)
                     const int st = 4 * hs + s + D, sn = st < n_steps ? st : n_steps - 1;
-                    av[sd][0][0] = pa0[(sn * 2) * 64];
-                    av[sd][0][1] = pa0[(sn * 2 + 1) * 64];
-                    av[sd][1][0] = pa1[(sn * 2) * 64];
-                    av[sd][1][1] = pa1[(sn * 2 + 1) * 64];
+                    av[sd][0][0] = pa0[sn * 64];
+                    av[sd][0][1] = pa0[(sn + n_steps) * 64];
+                    av[sd][1][0] = pa1[sn * 64];
+                    av[sd][1][1] = pa1[(sn + n_steps) * 64];
 #pragma unroll
                     for (int t = 0; t < NT; t++) {
                         if (t == 0 || t < nt) {
                             const bf16x8_t bv0 = *(const bf16x8_t *) (bp + t * 32 * MT_BSTRIDE);
-                            const bf16x8_t bv1 = *(const bf16x8_t *) (bp + t * 32 * MT_BSTRIDE + 16);
+                            const bf16x8_t bv1 = *(const bf16x8_t *) (bp + t * 32 * MT_BSTRIDE + MT_HK / 2);
                             acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a00, bv0, acc[0][t], 0, 0, 0);
                             acc[1][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a10, bv0, acc[1][t], 0, 0, 0);
                             acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a01, bv1, acc[0][t], 0, 0, 0);
@@ -1400,6 +1640,8 @@ void tile_init() {
     nb_attr<true, 1>(); nb_attr<false, 1>(); nb_attr<true, 2>(); nb_attr<false, 2>(); nb_attr<true, 4>(); nb_attr<false, 4>();
     mt_attr<true, 4, 8>();
     mt_attr<false, 4, 8>();
+    lds_attr((const void *) k_mm_wide<true>, wd_shm(true));
+    lds_attr((const void *) k_mm_wide<false>, wd_shm(false));
     mt_attr<true, 1, 16>();
     mt_attr<false, 1, 16>();
     lds_attr((const void *) k_mm_tile<false, 1, 16, true>, mt_shm<1, 16>(false));
@@ -1424,6 +1666,17 @@ void mt_launch(const bf16n_weight & w, const bf16n_weight * up, const mm_args & 
         hipLaunchKernelGGL((k_mm_tile<true, NT, W>), grid, dim3(S::THREADS), (mt_shm<NT, W>(true)), stream, w, *up, a);
     } else {
         hipLaunchKernelGGL((k_mm_tile<false, NT, W>), grid, dim3(S::THREADS), (mt_shm<NT, W>(false)), stream, w, w, a);
+    }
+}
+
+void wd_launch(const bf16n_weight & w, const bf16n_weight * up, const mm_args & a, int cus, hipStream_t stream) {
+    const int groups = (int) (a.rows / TILE_R), gpi = up ? WD_WAVES / 2 : WD_WAVES;
+    const int64_t items = (int64_t) a.n_experts * ((groups + gpi - 1) / gpi);
+    const dim3 grid((unsigned) (items < cus ? items : cus)); // the LDS of a CU holds one block
+    if (up) {
+        hipLaunchKernelGGL((k_mm_wide<true>), grid, dim3(WD_WAVES * 64), wd_shm(true), stream, w, *up, a);
+    } else {
+        hipLaunchKernelGGL((k_mm_wide<false>), grid, dim3(WD_WAVES * 64), wd_shm(false), stream, w, w, a);
     }
 }
 
@@ -1469,6 +1722,8 @@ void launch_tile_mm_ids(const bf16n_weight & w, const bf16n_weight * up, const v
     // passes of 32 tokens while few experts can hold more than 32 (every further pass decodes the expert again)
     if (n_pairs <= (int64_t) MT_SMALL_PAIRS * n_experts) {
         mt_launch_small(w, up, a, n_pairs, cus, stream);
+    } else if (n_pairs > (int64_t) WD_MIN_PAIRS * n_experts && n_pairs * x_row * 2 < ((int64_t) 1 << 32)) {
+        wd_launch(w, up, a, cus, stream); // (a has at most n_pairs rows of activations)
     } else {
         mt_launch<4, 8>(w, up, a, cus, stream);
     }

@@ -437,3 +437,31 @@ def test_two_phase_batched_product_equals_the_fused_kernel(ops, E, N, K, T, k, s
         assert torch.equal(ops.moe_mm_ids(want16, ids, down, E, routes=r3, scratch=buf), want_d)
     with pytest.raises(ValueError, match="scratch"):
         ops.moe_mm_ids(x, ids, gate, E, up=up, routes=routes, scratch=buf[: per // 2])
+
+
+@pytest.mark.parametrize("E,N,K,per_slot,counts", [
+    (5, 32, 512, False, {0: 320, 1: 321, 2: 0}),      # one row group for eight wavefronts; a full pass, one token more, none
+    (8, 288, 512, True, {0: 1, 1: 33, 2: 641, 7: 0}),  # a ninth row group; experts dealt by XCD
+    (4, 128, 1536, False, {0: 64, 1: 289}),            # an odd number of tiles per chain
+    (5, 96, 2048, True, {0: 0, 1: 479}),
+])
+def test_mm_ids_many_tokens_per_expert(ops, E, N, K, per_slot, counts):
+    """More than 98 routed pairs per expert: passes of up to 320 tokens, the two halves of the columns side by side."""
+    k, T = 2, (98 * E) // 2 + 300
+    wb, ub = synth.weights(E * N, K, 61 + N), synth.weights(E * N, K, 62 + N)
+    w, u = enc(ops, wb, HP, 32, False, True), enc(ops, ub, HP, 32, False, True)
+    wf, uf = synth.bf16_bits_to_f32(wb), synth.bf16_bits_to_f32(ub)
+    ids = routing(T, k, E, counts, 5)
+    it = torch.from_numpy(ids).cuda()
+    xb = synth.activations(T * (k if per_slot else 1), K, 3).reshape((T, k, K) if per_slot else (T, K))
+    xf = synth.bf16_bits_to_f32(xb)
+    got = ops.moe_mm_ids(tbf16(xb), it, w, E).cpu().numpy()
+    y, s = reference(wf, xf, ids, N, per_slot)
+    assert np.all(np.abs(got - y) <= GEMV_REL * s + 1e-30)
+    got16 = ops.moe_mm_ids(tbf16(xb), it, w, E, out_dtype=torch.bfloat16)
+    assert np.array_equal(bits(got16), rne_bf16(got))
+    yu = ops.moe_mm_ids(tbf16(xb), it, u, E).cpu().numpy().astype(np.float64)
+    fused = ops.moe_mm_ids(tbf16(xb), it, w, E, up=u).cpu().numpy()
+    want = yu * (got.astype(np.float64) / (1.0 + np.exp(-got.astype(np.float64))))  # the same sums: only silu's rounding differs
+    assert np.all(np.abs(fused - want) <= 2e-6 * np.abs(want) + 1e-12)
+    assert np.array_equal(bits(ops.moe_mm_ids(tbf16(xb), it, w, E, up=u, out_dtype=torch.bfloat16)), rne_bf16(fused))
