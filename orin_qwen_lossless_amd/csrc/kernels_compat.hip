@@ -2,9 +2,9 @@
 // dequant, row gather).  Buffers made by the reference encoder decode here unchanged.
 //
 // A wave64 carries two units (HUFPAIR / HUFFMAN) or two rows (NIBBLE): lanes 0..31 the even one, lanes 32..63 the odd
-// one; each half reads its 512-byte plane chunk with one 16-byte load per lane.  Lane streams are per-lane sequential
-// reads through the vector cache.  These kernels favour generality (any K, R, layout, expert ids, FP32 or BF16
-// activations) over speed; the wave64 layout (kernels_w64.hip) is the fast path.
+// one; each half reads its 512-byte plane chunk with one 16-byte load per lane, four chunks ahead.  Lane streams pass
+// through rings in LDS (lane_ring).  These kernels take any K, R, layout, expert ids and FP32 or BF16 activations; the
+// wave64 layout (kernels_w64.hip), which has twice the chains per unit, is the fast path.
 #include "dev_common.h"
 #include "dev_compat.h"
 #include "launchers.h"
@@ -18,20 +18,147 @@ constexpr int NT = 256;          // threads per block
 constexpr int NIB_MM_MIN_COLS = 5; // dense NIBBLE batches of BF16 columns go through the matrix cores from this many on at the earliest
 constexpr int HALVES = NT / 32;  // units (rows) per block
 
+// One lane's MSB-first bit stream, read through a ring of 16 words in LDS.  What bounds these kernels is the chain of
+// one unit (two dependent table lookups per two codes, all lanes of a half-wave in step), so nothing else may be waited
+// for in it: 64 lanes read 64 cache lines, and with the next word loaded where it is needed nearly every pair of codes
+// waited for some lane's cache miss (one column of 8192 x 2048, R = 16: 74 us then, 59 us with the ring; 65536 x 4096:
+// 266 and 162; dequant of the first 88 and 49).  Here a lane loads whole 16-byte
+// blocks, one per four code pairs (96 bits at most, less than a block), LOOK blocks beyond the one it reads, and stores
+// what it loaded DEEP rounds ago; the same block again while it has not moved on.  The stream buffers end with padding
+// words (32 of HUFPAIR, 16 of HUFFMAN): the last lane reads at most 17 (13) words past its end.
+constexpr int LR_WORDS = 16;                     // ring words per lane
+constexpr int LR_BYTES = LR_WORDS * 64 * 4;      // per wavefront: word i of a lane at [i % 16][lane]
+template <int FORMAT> struct lane_ring {
+    static constexpr int BITS = FORMAT == FMT_HUFPAIR ? HP_LP : HUF_LMAX;
+    static constexpr int DEEP = FORMAT == FMT_HUFPAIR ? 2 : 1, LOOK = DEEP + 1;
+    const uint4 * src;    // the block that holds the lane's first word
+    uint32_t * ring;      // this lane's column of the ring
+    uint32_t w0, w1, nw;  // the next 32 bits are bits s.. of w0:w1; nw: the word after w1
+    int s;                // unread bits of w0 (0: it is used up)
+    uint32_t p;           // index of nw, counted from src
+    uint4 f[DEEP];        // blocks in flight
+    uint32_t fb[DEEP];    // their indices
+    __device__ __forceinline__ void put(uint32_t b, const uint4 v) {
+        uint32_t * r = ring + (b & 3) * 256;
+        r[0] = v.x; r[64] = v.y; r[128] = v.z; r[192] = v.w;
+    }
+    __device__ __forceinline__ uint32_t word(uint32_t i) const { return ring[(i & (LR_WORDS - 1)) * 64]; }
+    __device__ __forceinline__ void begin(const uint32_t * sp, uint32_t * ring_) {
+        src = (const uint4 *) ((uintptr_t) sp & ~(uintptr_t) 15);
+        ring = ring_;
+        uint4 b[LOOK + 1];
+#pragma unroll
+        for (int i = 0; i <= LOOK; i++) {
+            b[i] = src[i];
+        }
+#pragma unroll
+        for (int i = 0; i <= LOOK; i++) {
+            put(i, b[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < DEEP; i++) {
+            f[i] = b[LOOK];
+            fb[i] = LOOK;
+        }
+        p = ((uint32_t) ((uintptr_t) sp & 15) >> 2) + 1;
+        w0 = 0;
+        w1 = word(p - 1);
+        nw = word(p);
+        s = 0;
+    }
+    __device__ __forceinline__ void round(int i) { // before every four code pairs; i: a compile-time counter
+        put(fb[i % DEEP], f[i % DEEP]);
+        fb[i % DEEP] = (p >> 2) + LOOK;
+        f[i % DEEP] = src[fb[i % DEEP]];
+    }
+    __device__ __forceinline__ void two(const uint32_t * lut, uint32_t & e0, uint32_t & e1) {
+        const uint32_t W = __builtin_amdgcn_alignbit(w0, w1, (uint32_t) s);
+        e0 = lut[W >> (32 - BITS)];
+        e1 = lut[(W << (e0 & 31u)) >> (32 - BITS)];
+        s -= (int) ((e0 + e1) & 31u); // (bits 5 and 6 of an entry are zero, two codes at most 24 bits)
+        const bool m = s < 0;
+        s += m ? 32 : 0;
+        w0 = m ? w1 : w0;
+        w1 = m ? nw : w1;
+        p += m ? 1 : 0;
+        nw = word(p);
+    }
+    // the 16 weights of the lane in one chunk as 8 BF16 pairs, columns 128 j + 4 l + {0, 1}, {2, 3}; i: chunk counter
+    __device__ __forceinline__ void chunk(int i, const uint32_t * lut, const uint4 sm, uint32_t (&wp)[8]) {
+        const uint32_t smw[4] = {sm.x, sm.y, sm.z, sm.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (FORMAT == FMT_HUFPAIR) {
+                uint32_t e0, e1;
+                if (j == 0) {
+                    round(i);
+                }
+                two(lut, e0, e1);
+                wp[2 * j] = merge(spread_lo(smw[j]), e0);
+                wp[2 * j + 1] = merge(spread_hi(smw[j]), e1);
+            } else { // single exponents, entry = len | exponent << 7
+                uint32_t a, b, c, d;
+                if (j % 2 == 0) {
+                    round(0);
+                }
+                two(lut, a, b);
+                two(lut, c, d);
+                wp[2 * j] = merge(spread_lo(smw[j]), (a & 0x7F80u) | ((b & 0x7F80u) << 16));
+                wp[2 * j + 1] = merge(spread_hi(smw[j]), (c & 0x7F80u) | ((d & 0x7F80u) << 16));
+            }
+        }
+    }
+};
+
+// the chunks [0, n) of a half-wave's unit in stream order, four plane chunks in flight: f(chunk, weights), and before a
+// chunk is decoded pre()
+template <int FORMAT, typename P, typename F>
+__device__ __forceinline__ void for_chunks(const uint8_t * plane, const uint32_t * sp, uint32_t * ring, const uint32_t * lut, int n, int l32, P pre, F f) {
+    constexpr int D = 4;
+    const uint4 * pl = (const uint4 *) plane + l32;
+    uint4 sm[D];
+#pragma unroll
+    for (int i = 0; i < D; i++) {
+        sm[i] = pl[(i < n ? i : n - 1) * 32];
+    }
+    lane_ring<FORMAT> bits;
+    bits.begin(sp, ring);
+    auto one = [&](int o, int i) {
+        uint32_t wp[8];
+        pre();
+        bits.chunk(i, lut, sm[i], wp);
+        sm[i] = pl[(o + i + D < n ? o + i + D : n - 1) * 32]; // (past the end the last chunk again, unused)
+        f(o + i, wp);
+    };
+    int o = 0;
+#pragma unroll 1
+    for (; o + D <= n; o += D) { // (no exit inside: the waits for loads in flight stay exact)
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            one(o, i);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < D - 1; i++) {
+        if (o + i < n) {
+            one(o, i);
+        }
+    }
+}
+
 template <typename TX>
 __device__ __forceinline__ float x_at(const char * x, int i);
 template <> __device__ __forceinline__ float x_at<float>(const char * x, int i) { return ((const float *) x)[i]; }
 template <> __device__ __forceinline__ float x_at<bf16_t>(const char * x, int i) { return bf16_bits_to_f32(((const uint16_t *) x)[i]); }
 
-__device__ __forceinline__ float dot_chunk(const uint32_t (&wp)[8], const float * xs, int l32) {
+__device__ __forceinline__ float dot_chunk(const uint32_t (&wp)[8], const float4 (&x)[4]) {
     float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const float4 xv = *(const float4 *) (xs + 128 * j + 4 * l32);
-        a0 = fmaf(bf16_bits_to_f32(wp[2 * j] & 0xFFFFu), xv.x, a0);
-        a1 = fmaf(__uint_as_float(wp[2 * j] & 0xFFFF0000u), xv.y, a1);
-        a2 = fmaf(bf16_bits_to_f32(wp[2 * j + 1] & 0xFFFFu), xv.z, a2);
-        a3 = fmaf(__uint_as_float(wp[2 * j + 1] & 0xFFFF0000u), xv.w, a3);
+        a0 = fmaf(bf16_bits_to_f32(wp[2 * j] & 0xFFFFu), x[j].x, a0);
+        a1 = fmaf(__uint_as_float(wp[2 * j] & 0xFFFF0000u), x[j].y, a1);
+        a2 = fmaf(bf16_bits_to_f32(wp[2 * j + 1] & 0xFFFFu), x[j].z, a2);
+        a3 = fmaf(__uint_as_float(wp[2 * j + 1] & 0xFFFF0000u), x[j].w, a3);
     }
     return (a0 + a1) + (a2 + a3);
 }
@@ -39,33 +166,41 @@ __device__ __forceinline__ float dot_chunk(const uint32_t (&wp)[8], const float 
 // One unit of R rows: y[rr] (rr < R) ends up in lane rr of the half-wave.  Row-major streams finish a row every C
 // chunks; chunk-major streams add one partial sum per (chunk, row).
 template <int FORMAT>
-__device__ __forceinline__ float unit_dot(const uint8_t * plane, const uint32_t * lut, const uint32_t * sp, int64_t gu, int R,
+__device__ __forceinline__ float unit_dot(const uint8_t * plane, const uint32_t * lut, const uint32_t * sp, uint32_t * ring, int64_t gu, int R,
                                           int C, bool cm, const float * xs, int l32) {
-    lane_bits bits;
-    bits.begin(sp);
-    const uint8_t * up = plane + gu * R * (int64_t) C * CHUNK;
-    float mine = 0.f;
-    if (cm) {
-        for (int c = 0; c < C; c++) {
-            for (int rr = 0; rr < R; rr++) {
-                uint32_t wp[8];
-                decode_chunk<FORMAT>(bits, lut, *((const uint4 *) (up + ((int64_t) c * R + rr) * CHUNK) + l32), wp);
-                const float s = half_wave_sum(dot_chunk(wp, xs + c * CHUNK, l32));
-                mine += l32 == rr ? s : 0.f;
+    const bool upper = (threadIdx.x & 32) != 0;
+    auto sum = [&](float v) { // over the half-wave, on the VALU (lanes 31 and 63 get the sums)
+        const int t = __builtin_bit_cast(int, half_wave_sum_dpp(v));
+        const int lo = __builtin_amdgcn_readlane(t, 31), hi = __builtin_amdgcn_readlane(t, 63);
+        return __builtin_bit_cast(float, upper ? hi : lo);
+    };
+    float mine = 0.f, acc = 0.f;
+    int rr = 0, c = 0;
+    float4 x[4]; // the chunk's activations, requested before its chain of lookups (8192 x 2048: 3 us of 66)
+    for_chunks<FORMAT>(plane + gu * R * (int64_t) C * CHUNK, sp, ring, lut, R * C, l32, [&] {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            x[j] = *(const float4 *) (xs + c * CHUNK + 128 * j + 4 * l32);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }, [&](int, const uint32_t (&wp)[8]) {
+        const float d = dot_chunk(wp, x);
+        if (cm) {
+            const float v = sum(d);
+            mine += l32 == rr ? v : 0.f;
+            rr = rr + 1 < R ? rr + 1 : 0;
+            c += rr == 0;
+        } else {
+            acc += d;
+            c = c + 1 < C ? c + 1 : 0;
+            if (c == 0) {
+                const float v = sum(acc);
+                mine = l32 == rr ? v : mine;
+                acc = 0.f;
+                rr++;
             }
         }
-    } else {
-        for (int rr = 0; rr < R; rr++) {
-            float acc = 0.f;
-            for (int c = 0; c < C; c++) {
-                uint32_t wp[8];
-                decode_chunk<FORMAT>(bits, lut, *((const uint4 *) (up + ((int64_t) rr * C + c) * CHUNK) + l32), wp);
-                acc += dot_chunk(wp, xs + c * CHUNK, l32);
-            }
-            const float s = half_wave_sum(acc);
-            mine = l32 == rr ? s : mine;
-        }
-    }
+    });
     return mine;
 }
 
@@ -80,7 +215,7 @@ __device__ __forceinline__ const uint32_t * lane_stream(const bf16n_weight & w, 
 }
 
 // y = W x (GLU: y = silu(gate x) * up x) for HUFPAIR / HUFFMAN in the 32-lane layouts; one half-wave per unit,
-// blockIdx.y = column.  Shared memory: x as FP32 [K], then one table per matrix.
+// blockIdx.y = column.  Shared memory: x as FP32 [K], then one table per matrix, then a ring per wavefront.
 template <int FORMAT, typename TX, bool GLU>
 __global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16n_weight w_up, const cols p) {
     constexpr int LUT_N = FORMAT == FMT_HUFPAIR ? (1 << HP_LP) : (1 << HUF_LMAX);
@@ -89,32 +224,38 @@ __global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16
     float * xs = (float *) shm_raw;
     uint32_t * lut = (uint32_t *) (xs + K);
     uint32_t * lut_up = lut + LUT_N;
+    uint32_t * ring = lut + (GLU ? 2 : 1) * LUT_N + (threadIdx.x >> 6) * (LR_BYTES / 4) + (threadIdx.x & 63);
+    const int nt = (int) blockDim.x;
     const col_view cv = col_setup(p, blockIdx.y);
-    for (int i = threadIdx.x; i < K; i += NT) {
-        xs[i] = x_at<TX>(cv.x, i);
-    }
-    const uint32_t * lut_g = (const uint32_t *) (w.aux + w.off_a);
-    for (int i = threadIdx.x; i < LUT_N; i += NT) {
-        lut[i] = lut_g[i];
+    // (many loads in flight: the smallest blocks are one wavefront)
+#pragma unroll 16
+    for (int i = threadIdx.x; i < LUT_N; i += nt) {
+        lut[i] = ((const uint32_t *) (w.aux + w.off_a))[i];
     }
     if (GLU) {
-        const uint32_t * lut_ug = (const uint32_t *) (w_up.aux + w_up.off_a);
-        for (int i = threadIdx.x; i < LUT_N; i += NT) {
-            lut_up[i] = lut_ug[i];
+#pragma unroll 16
+        for (int i = threadIdx.x; i < LUT_N; i += nt) {
+            lut_up[i] = ((const uint32_t *) (w_up.aux + w_up.off_a))[i];
         }
     }
+#pragma unroll 8
+    for (int i = threadIdx.x; i < K; i += nt) {
+        xs[i] = x_at<TX>(cv.x, i);
+    }
     __syncthreads();
-    const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5;
+    const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5, halves = nt >> 5;
     const bool cm = (w.flags & FLAG_CHUNK_MAJOR) != 0;
     const int64_t units = p.nrows / R;
-    for (int64_t u = (int64_t) blockIdx.x * HALVES + half; u < units; u += (int64_t) gridDim.x * HALVES) {
+    for (int64_t u0 = (int64_t) blockIdx.x * halves + (half & ~1); u0 < units; u0 += (int64_t) gridDim.x * halves) {
+        // (both halves of a wavefront stay together: a missing last unit is decoded twice and stored once)
+        const int64_t u = u0 + (half & 1) < units ? u0 + (half & 1) : u0;
         const int64_t gu = cv.rbase / R + u;
-        float v = unit_dot<FORMAT>(w.plane, lut, lane_stream<FORMAT>(w, gu, l32), gu, R, C, cm, xs, l32);
+        float v = unit_dot<FORMAT>(w.plane, lut, lane_stream<FORMAT>(w, gu, l32), ring, gu, R, C, cm, xs, l32);
         if (GLU) {
-            const float uv = unit_dot<FORMAT>(w_up.plane, lut_up, lane_stream<FORMAT>(w_up, gu, l32), gu, R, C, false, xs, l32);
+            const float uv = unit_dot<FORMAT>(w_up.plane, lut_up, lane_stream<FORMAT>(w_up, gu, l32), ring, gu, R, C, false, xs, l32);
             v = uv * silu(v);
         }
-        if (l32 < R) {
+        if (l32 < R && u == u0 + (half & 1)) {
             store_y(cv.y, p.y_bf16, u * R + l32, v);
         }
     }
@@ -125,29 +266,34 @@ template <int FORMAT>
 __global__ void __launch_bounds__(NT) k_huf_dequant(const bf16n_weight w, int64_t row0, int64_t nrows, uint16_t * __restrict__ out) {
     constexpr int LUT_N = FORMAT == FMT_HUFPAIR ? (1 << HP_LP) : (1 << HUF_LMAX);
     __shared__ uint32_t lut[LUT_N];
-    const uint32_t * lut_g = (const uint32_t *) (w.aux + w.off_a);
-    for (int i = threadIdx.x; i < LUT_N; i += NT) {
-        lut[i] = lut_g[i];
+    __shared__ uint32_t rings[NT / 64 * LR_BYTES / 4];
+    const int nt = (int) blockDim.x;
+#pragma unroll 16
+    for (int i = threadIdx.x; i < LUT_N; i += nt) {
+        lut[i] = ((const uint32_t *) (w.aux + w.off_a))[i];
     }
     __syncthreads();
     const int K = (int) w.K, C = K / CHUNK, R = w.R;
     const bool cm = (w.flags & FLAG_CHUNK_MAJOR) != 0;
-    const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5;
-    for (int64_t u = (int64_t) blockIdx.x * HALVES + half; u < nrows / R; u += (int64_t) gridDim.x * HALVES) {
+    const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5, halves = nt >> 5;
+    uint32_t * ring = rings + (threadIdx.x >> 6) * (LR_BYTES / 4) + (threadIdx.x & 63);
+    for (int64_t u = (int64_t) blockIdx.x * halves + half; u < nrows / R; u += (int64_t) gridDim.x * halves) {
         const int64_t gu = row0 / R + u;
-        lane_bits bits;
-        bits.begin(lane_stream<FORMAT>(w, gu, l32));
-        const uint8_t * up = w.plane + gu * R * (int64_t) K;
-        for (int o = 0; o < R * C; o++) {
-            const int rr = cm ? o % R : o / C, c = cm ? o / R : o % C;
-            uint32_t wp[8];
-            decode_chunk<FORMAT>(bits, lut, *((const uint4 *) (up + (int64_t) o * CHUNK) + l32), wp);
+        int rr = 0, c = 0;
+        for_chunks<FORMAT>(w.plane + gu * R * (int64_t) K, lane_stream<FORMAT>(w, gu, l32), ring, lut, R * C, l32, [] {}, [&](int, const uint32_t (&wp)[8]) {
             uint16_t * dst = out + (u * R + rr) * K + c * CHUNK;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 *(uint2 *) (dst + 128 * j + 4 * l32) = make_uint2(wp[2 * j], wp[2 * j + 1]);
             }
-        }
+            if (cm) {
+                rr = rr + 1 < R ? rr + 1 : 0;
+                c += rr == 0;
+            } else {
+                c = c + 1 < C ? c + 1 : 0;
+                rr += c == 0;
+            }
+        });
     }
 }
 
@@ -157,40 +303,38 @@ template <bool BF>
 __global__ void __launch_bounds__(NT) k_hp_get_rows(const bf16n_weight w, const char * __restrict__ ids, int64_t ids_s0, int64_t n,
                                                     int64_t row0, char * __restrict__ dst, int64_t dst_s1) {
     __shared__ uint32_t lut[1 << HP_LP];
-    const uint32_t * lut_g = (const uint32_t *) (w.aux + w.off_a);
+    __shared__ uint32_t rings[NT / 64 * LR_BYTES / 4];
+#pragma unroll 16
     for (int i = threadIdx.x; i < (1 << HP_LP); i += NT) {
-        lut[i] = lut_g[i];
+        lut[i] = ((const uint32_t *) (w.aux + w.off_a))[i];
     }
     __syncthreads();
     const int K = (int) w.K, C = K / CHUNK, R = w.R;
     const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5;
+    uint32_t * ring = rings + (threadIdx.x >> 6) * (LR_BYTES / 4) + (threadIdx.x & 63);
     const int64_t i = (int64_t) blockIdx.x * HALVES + half;
     if (i >= n) {
         return;
     }
     const int64_t gr = row0 + *(const int32_t *) (ids + i * ids_s0);
     const int64_t gu = gr / R;
-    lane_bits bits;
-    bits.begin(lane_stream<FMT_HUFPAIR>(w, gu, l32));
     char * o = dst + i * dst_s1;
-    for (int64_t r = gu * R; r <= gr; r++) {
-        for (int c = 0; c < C; c++) {
-            uint32_t wp[8];
-            decode_chunk<FMT_HUFPAIR>(bits, lut, *((const uint4 *) (w.plane + r * K + c * CHUNK) + l32), wp);
-            if (r == gr) {
+    const int chunks = (int) (gr - gu * R + 1) * C; // of the unit, up to the end of the row
+    for_chunks<FMT_HUFPAIR>(w.plane + gu * R * (int64_t) K, lane_stream<FMT_HUFPAIR>(w, gu, l32), ring, lut, chunks, l32, [] {},
+                            [&](int k, const uint32_t (&wp)[8]) {
+        if (k >= chunks - C) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int col = c * CHUNK + 128 * j + 4 * l32;
-                    if (BF) {
-                        *(uint2 *) (o + 2 * col) = make_uint2(wp[2 * j], wp[2 * j + 1]);
-                    } else {
-                        *(float4 *) (o + 4 * col) = make_float4(bf16_bits_to_f32(wp[2 * j] & 0xFFFFu), __uint_as_float(wp[2 * j] & 0xFFFF0000u),
-                                                                bf16_bits_to_f32(wp[2 * j + 1] & 0xFFFFu), __uint_as_float(wp[2 * j + 1] & 0xFFFF0000u));
-                    }
+            for (int j = 0; j < 4; j++) {
+                const int col = (k - (chunks - C)) * CHUNK + 128 * j + 4 * l32;
+                if (BF) {
+                    *(uint2 *) (o + 2 * col) = make_uint2(wp[2 * j], wp[2 * j + 1]);
+                } else {
+                    *(float4 *) (o + 4 * col) = make_float4(bf16_bits_to_f32(wp[2 * j] & 0xFFFFu), __uint_as_float(wp[2 * j] & 0xFFFF0000u),
+                                                            bf16_bits_to_f32(wp[2 * j + 1] & 0xFFFFu), __uint_as_float(wp[2 * j + 1] & 0xFFFF0000u));
                 }
             }
         }
-    }
+    });
 }
 
 // ---------------------------------------------------------------- NIBBLE
@@ -578,10 +722,20 @@ __global__ void __launch_bounds__(NT) k_nib_rows(const bf16n_weight w, const cha
 }
 
 // blocks of HALVES units (rows) each, capped so that a launch of several columns stays within a few blocks per CU
-int grid_for(int64_t work, int ncols, int cus) {
-    const int64_t blocks = (work + HALVES - 1) / HALVES;
+int grid_for(int64_t work, int ncols, int cus, int per_block = HALVES) {
+    const int64_t blocks = (work + per_block - 1) / per_block;
     const int64_t cap = (int64_t) cus * 8 / (ncols < 1 ? 1 : ncols > 4 ? 4 : ncols);
     return (int) (blocks < 1 ? 1 : blocks > cap ? cap : blocks);
+}
+
+// Wavefronts per block of the HUFPAIR / HUFFMAN kernels, two units each: four, fewer where that leaves CUs without a
+// block (the units' chains set the time: alone on a CU they share its LDS with nobody)
+int huf_waves(int64_t units, int ncols, int cus) {
+    int waves = NT / 64;
+    while (waves > 1 && (units + 2 * waves - 1) / (2 * waves) * ncols < cus) {
+        waves /= 2;
+    }
+    return waves;
 }
 
 } // namespace
@@ -623,8 +777,6 @@ bool nib_mm_pays(const bf16n_weight & w, int64_t nrows, int ncols, int cus) {
 void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu, const cols & p, int ncols, bool x_bf16,
                        int cus, hipStream_t stream, bool matrix_cores) {
     const bf16n_weight & wu = up ? *up : w;
-    const int64_t work = w.format == FMT_NIBBLE ? p.nrows : p.nrows / w.R;
-    const dim3 grid(grid_for(work, ncols, cus), ncols);
     // the matrix cores where the row groups of 32 give enough CUs a block: from five BF16 columns on with blocks for half
     // of the CUs, from nine with a quarter, from 25 with an eighth (5120 x 2048, 160 blocks: 11.0-13.0 us for 5-32
     // columns against 9.6 / 17.9 us for 4 / 8 GEMV columns and 20 us for dequant + GEMM; 2048 x 4096, 64 blocks: 16.7-20.7
@@ -679,8 +831,11 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
         return;
     }
     const bool hp = w.format == FMT_HUFPAIR;
-    const size_t shm = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX));
-#define HUF(F, TX, G) hipLaunchKernelGGL((k_huf_mmv<F, TX, G>), grid, dim3(NT), shm, stream, w, wu, p)
+    const int64_t work = p.nrows / w.R;
+    const int waves = huf_waves(work, ncols, cus);
+    const size_t shm = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX)) + (size_t) waves * LR_BYTES;
+    const dim3 grid(grid_for(work, ncols, cus, 2 * waves), ncols);
+#define HUF(F, TX, G) hipLaunchKernelGGL((k_huf_mmv<F, TX, G>), grid, dim3(waves * 64), shm, stream, w, wu, p)
     if (hp) {
         if (x_bf16) { if (glu) HUF(FMT_HUFPAIR, bf16_t, true); else HUF(FMT_HUFPAIR, bf16_t, false); }
         else        { if (glu) HUF(FMT_HUFPAIR, float, true);  else HUF(FMT_HUFPAIR, float, false); }
@@ -693,15 +848,16 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
 
 void launch_compat_dequant(const bf16n_weight & w, int64_t row0, int64_t nrows, uint16_t * out, int cus, hipStream_t stream) {
     const int64_t work = w.format == FMT_NIBBLE ? nrows : nrows / w.R;
-    const int64_t blocks = (work + HALVES - 1) / HALVES;
+    const int waves = w.format == FMT_NIBBLE ? NT / 64 : huf_waves(work, 1, cus);
+    const int64_t blocks = (work + 2 * waves - 1) / (2 * waves);
     const dim3 grid((unsigned) (blocks < (int64_t) cus * 16 ? blocks : (int64_t) cus * 16));
     if (w.format == FMT_NIBBLE) {
         hipLaunchKernelGGL((k_nib_rows<true>), grid, dim3(NT), 0, stream, w, (const char *) nullptr, (int64_t) 0, nrows, row0,
                            (char *) out, (int64_t) w.K * 2);
     } else if (w.format == FMT_HUFPAIR) {
-        hipLaunchKernelGGL((k_huf_dequant<FMT_HUFPAIR>), grid, dim3(NT), 0, stream, w, row0, nrows, out);
+        hipLaunchKernelGGL((k_huf_dequant<FMT_HUFPAIR>), grid, dim3(waves * 64), 0, stream, w, row0, nrows, out);
     } else {
-        hipLaunchKernelGGL((k_huf_dequant<FMT_HUFFMAN>), grid, dim3(NT), 0, stream, w, row0, nrows, out);
+        hipLaunchKernelGGL((k_huf_dequant<FMT_HUFFMAN>), grid, dim3(waves * 64), 0, stream, w, row0, nrows, out);
     }
 }
 

@@ -133,3 +133,27 @@ def test_get_rows(ops):
     w = enc(ops, src, HUF, 8)
     with pytest.raises(ValueError, match="Huffman"):
         ops.get_rows(ids, w)
+
+
+@pytest.mark.parametrize("fmt,R,K,cm", [(HP, 1, 512, False), (HP, 1, 1536, False), (HP, 2, 2560, False), (HP, 16, 1024, False),
+                                        (HP, 4, 1024, True), (HUF, 1, 512, False), (HUF, 2, 1536, False), (HUF, 16, 2048, False)])
+def test_lane_streams_of_very_different_speed(ops, fmt, R, K, cm):
+    """32-lane layouts: half of the lanes read the longest codes (a word per two or three code pairs), the others the
+    shortest (a word per many chunks); an odd number of units, chunk counts that leave remainders of the loop of four."""
+    rng = np.random.default_rng(K + R)
+    rows = 3 * R if R > 1 else 7
+    common = np.full((rows, K), 120, dtype=np.uint16)
+    rare = (60 + rng.integers(0, 40, (rows, K))).astype(np.uint16)
+    slow = (np.arange(K) // 4 % 32) % 2 == 1  # a lane owns four adjacent columns of every 128
+    lone = rng.random((rows, K)) < (0.02 if fmt == HP else 0.002)  # the rare exponents stay rare enough for the longest codes
+    exps = np.where(slow & (rng.random((rows, 1)) < 0.3), rare, np.where(lone, rare, common))
+    src = (exps << 7 | rng.integers(0, 128, (rows, K)).astype(np.uint16) | rng.integers(0, 2, (rows, K)).astype(np.uint16) << 15).astype(np.uint16)
+    w = enc(ops, src, fmt, R, cm)
+    assert np.array_equal(bits(ops.dequant(w)), src)
+    if w.meta.format == HP and not cm:
+        ids = torch.arange(rows - 1, -1, -1, device="cuda")
+        assert np.array_equal(bits(ops.get_rows(ids, w)), src[::-1])
+    x = torch.zeros((2, K), device="cuda")
+    x[0, K - 1], x[1, 5] = 1.0, 1.0
+    y = ops.mmv(x, w).cpu().numpy()
+    assert np.array_equal(y, synth.bf16_bits_to_f32(src[:, [K - 1, 5]]).T)
