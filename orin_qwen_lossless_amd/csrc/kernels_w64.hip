@@ -327,83 +327,140 @@ __global__ void __launch_bounds__(1024) k_w64_glu(const bf16n_weight wg, const b
 
 // ---------------------------------------------------------------- dequant / row gather
 
-// exact BF16 bits of rows [row0, row0 + nrows) (whole units) into out (row-major); one wave per range of units.
-// only_row >= 0: store just that row (relative to row0) — the row gather decodes its unit from the start.
-__device__ __forceinline__ void w64_unit_rows(w64_dec & dec, const uint32_t * lut, const uint8_t * unit_plane, int R, int C,
-                                              int lane, int64_t only_row, char * out, int64_t out_row_bytes, bool f32) {
-    const int l32 = lane & 31, half = lane >> 5;
-    const uint4 * pp = (const uint4 *) unit_plane + lane;
-    for (int st = 0; st < R * C / 2; st++) {
-        dec.keep_ahead();
-        uint32_t wp[8];
-        dec.step(lut, pp[64 * st], wp);
-        const int o = 2 * st + half, rr = o / C, c = o % C;
-        if (only_row >= 0 && (2 * st) / C > only_row) { // same decision in both half-waves
-            break;
-        }
-        if (only_row >= 0 && rr != only_row) {
-            continue;
-        }
-        char * dst = out + (only_row >= 0 ? 0 : rr) * out_row_bytes;
+// Both kernels are bound by the chain of a unit (a step is eight dependent table lookups), so a step must not wait for
+// its plane bytes as well: loaded where they were needed, every step paid a miss that reached HBM.  R = 16, K = 2048:
+// 64 / 513 / 2048 rows gathered 20.7 / 24.0 / 26.2 -> 14.9 / 15.9 / 18.1 us; 65536 rows dequantised 97 -> 92 us.  All
+// 248320 rows stay at 356 us (1.7 GB read and written, 4.8 TB/s: many wavefronts hide the misses there).
+
+// the 16 weights of a lane in one step, to its four places in the 512 columns at dst
+__device__ __forceinline__ void w64_store_step(const uint32_t (&wp)[8], char * dst, int l32, bool f32) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int col = c * CHUNK + 128 * j + 4 * l32;
-            if (f32) {
-                *(float4 *) (dst + 4 * col) = make_float4(__uint_as_float(wp[2 * j] << 16), __uint_as_float(wp[2 * j] & 0xFFFF0000u),
-                                                          __uint_as_float(wp[2 * j + 1] << 16), __uint_as_float(wp[2 * j + 1] & 0xFFFF0000u));
-            } else {
-                *(uint2 *) (dst + 2 * col) = make_uint2(wp[2 * j], wp[2 * j + 1]);
-            }
+    for (int j = 0; j < 4; j++) {
+        const int col = 128 * j + 4 * l32;
+        if (f32) {
+            *(float4 *) (dst + 4 * col) = make_float4(__uint_as_float(wp[2 * j] << 16), __uint_as_float(wp[2 * j] & 0xFFFF0000u),
+                                                      __uint_as_float(wp[2 * j + 1] << 16), __uint_as_float(wp[2 * j + 1] & 0xFFFF0000u));
+        } else {
+            *(uint2 *) (dst + 2 * col) = make_uint2(wp[2 * j], wp[2 * j + 1]);
         }
     }
 }
 
+// Exact BF16 bits of rows [row0, row0 + nrows) (whole units) into out (row-major); one wave per range of units.  The 512
+// columns of a half-wave's step lie at the same place in the plane and in the output, unit after unit, so a wave's units
+// are one sequence of steps, with the plane bytes of four of them in flight.
 __global__ void __launch_bounds__(256) k_w64_dequant(const bf16n_weight w, int64_t row0, int64_t nrows, uint16_t * __restrict__ out,
                                                      int units_per_wave) {
+    constexpr int D = 4;
     __shared__ __align__(16) uint32_t lut[LUT_WORDS];
     extern __shared__ __align__(16) uint32_t rings[];
     const w64_ptrs q = w64p(w);
-    stage_lut(lut, q.lut);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = (int) uniform(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
-    const int R = w.R, K = (int) w.K, C = K / CHUNK;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5, wave = (int) uniform(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
+    const int R = w.R, K = (int) w.K, C = K / CHUNK, unit_steps = R * C / 2;
     const int64_t units = nrows / R;
     const int64_t u_begin = ((int64_t) blockIdx.x * nwaves + wave) * units_per_wave;
-    if (u_begin >= units) {
+    const int n_units = u_begin >= units ? 0 : u_begin + units_per_wave < units ? units_per_wave : (int) (units - u_begin);
+    const int n = n_units * unit_steps;
+    const int64_t gu0 = row0 / R + u_begin;
+    const uint4 * pp = (const uint4 *) (q.plane + gu0 * R * (int64_t) K) + lane;
+    char * dst = (char *) (out + u_begin * R * K + half * CHUNK);
+    w64_dec dec;
+    uint4 sm[D];
+    if (n > 0) { // (in flight while the block stages the table)
+        dec.start(rings + wave * WAVE_LDS_WORDS, q.stream, q.ubase[gu0], q.ubase[gu0 + n_units], lane, false, true);
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            sm[i] = pp[64 * (int64_t) (i < n ? i : n - 1)];
+        }
+    }
+    stage_lut(lut, q.lut);
+    __syncthreads();
+    if (n == 0) {
         return;
     }
-    const int64_t u_end = u_begin + units_per_wave < units ? u_begin + units_per_wave : units;
-    const int64_t gu0 = row0 / R + u_begin;
-    w64_dec dec;
-    dec.start(rings + wave * WAVE_LDS_WORDS, q.stream, q.ubase[gu0], q.ubase[gu0 + (u_end - u_begin)], lane);
-    for (int64_t u = u_begin; u < u_end; u++) {
+    dec.start_finish();
+    int left = 0; // steps of the current unit
+    auto one = [&](int st, int i) {
+        if (left == 0) {
+            dec.keep_ahead();
+            dec.begin_unit();
+            left = unit_steps;
+        }
+        left--;
         dec.keep_ahead();
-        dec.begin_unit();
-        w64_unit_rows(dec, lut, q.plane + (row0 / R + u) * R * (int64_t) K, R, C, lane, -1, (char *) (out + u * R * (int64_t) K),
-                      (int64_t) K * 2, false);
+        uint32_t wp[8];
+        dec.step(lut, sm[i], wp);
+        sm[i] = pp[64 * (int64_t) (st + D < n ? st + D : n - 1)]; // (past the end the last step's again, unused)
+        w64_store_step(wp, dst + (int64_t) st * (2 * CHUNK * 2), l32, false);
+    };
+    int st = 0;
+#pragma unroll 1
+    for (; st + D <= n; st += D) {
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            one(st + i, i);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < D - 1; i++) {
+        if (st + i < n) {
+            one(st + i, i);
+        }
     }
 }
 
+// One wave per row: it decodes the row's unit from the start, the codes alone up to the row, whose plane bytes (four
+// steps at most, K <= 4096) are requested before the chain begins.  The row's id, its unit's bases and the first stream
+// blocks, three misses in a row, are on their way while the block stages the table.
 __global__ void __launch_bounds__(256) k_w64_get_rows(const bf16n_weight w, const char * __restrict__ ids, int64_t ids_s0, int64_t n,
                                                       int64_t row0, char * __restrict__ dst, int64_t dst_s1, bool f32) {
     __shared__ __align__(16) uint32_t lut[LUT_WORDS];
     extern __shared__ __align__(16) uint32_t rings[];
     const w64_ptrs q = w64p(w);
-    stage_lut(lut, q.lut);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = (int) uniform(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5, wave = (int) uniform(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
     const int R = w.R, K = (int) w.K, C = K / CHUNK;
     const int64_t i = (int64_t) blockIdx.x * nwaves + wave;
+    const int64_t gr = i < n ? row0 + *(const int32_t *) (ids + i * ids_s0) : 0; // (a wave without a row only stages)
+    const int64_t gu = gr / R;
+    const int row = (int) (gr - gu * R), first = (int) uniform(row * C / 2), last = (int) uniform(((row + 1) * C - 1) / 2);
+    const uint4 * pp = (const uint4 *) (q.plane + gu * R * (int64_t) K) + lane;
+    w64_dec dec;
+    uint4 sm[4];
+    if (i < n) {
+        dec.start(rings + wave * WAVE_LDS_WORDS, q.stream, q.ubase[gu], q.ubase[gu + 1], lane, false, true);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            sm[s] = pp[64 * (first + s <= last ? first + s : last)];
+        }
+    }
+    stage_lut(lut, q.lut);
+    __syncthreads();
     if (i >= n) {
         return;
     }
-    const int64_t gr = row0 + *(const int32_t *) (ids + i * ids_s0);
-    const int64_t gu = gr / R;
-    w64_dec dec;
-    dec.start(rings + wave * WAVE_LDS_WORDS, q.stream, q.ubase[gu], q.ubase[gu + 1], lane);
+    dec.start_finish();
     dec.keep_ahead();
     dec.begin_unit();
-    w64_unit_rows(dec, lut, q.plane + gu * R * (int64_t) K, R, C, lane, gr - gu * R, dst + i * dst_s1, 0, f32);
+    for (int st = 0; st < first; st++) {
+        dec.keep_ahead();
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t e0, e1;
+            dec.two(lut, e0, e1);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        if (first + s <= last) {
+            dec.keep_ahead();
+            uint32_t wp[8];
+            dec.step(lut, sm[s], wp);
+            const int c = 2 * (first + s) + half - row * C; // a step at the row's ends may hold a neighbour's 512 columns
+            if (c >= 0 && c < C) {
+                w64_store_step(wp, dst + i * dst_s1 + (int64_t) c * CHUNK * (f32 ? 4 : 2), l32, f32);
+            }
+        }
+    }
 }
 
 size_t w64_shm(int waves) { return (size_t) waves * WAVE_LDS_WORDS * 4; } // dynamic part; the table is static

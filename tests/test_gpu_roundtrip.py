@@ -157,3 +157,17 @@ def test_lane_streams_of_very_different_speed(ops, fmt, R, K, cm):
     x[0, K - 1], x[1, 5] = 1.0, 1.0
     y = ops.mmv(x, w).cpu().numpy()
     assert np.array_equal(y, synth.bf16_bits_to_f32(src[:, [K - 1, 5]]).T)
+
+
+@pytest.mark.parametrize("R,K,units", [(2, 512, 3), (2, 512, 8195), (2, 1536, 5), (4, 2560, 2), (2, 3584, 4101), (16, 3584, 2), (8, 4096, 9)])
+def test_wave64_steps_across_units_and_rows(ops, R, K, units):
+    """Units of one step and of odd numbers of steps, rows that begin in the middle of a step, wavefronts with several
+    units and with fewer steps than are kept in flight; every row gathered alone."""
+    src = synth.weights(units * R, K, 7 * R + units)
+    w = enc(ops, src, HP, R, False, True)
+    assert w.meta.wave64
+    assert np.array_equal(bits(ops.dequant(w)), src)
+    ids = torch.arange(min(units * R, 99) - 1, -1, -1, device="cuda")  # (blocks of four rows and a remainder)
+    want = src[ids.cpu().numpy()]
+    assert np.array_equal(bits(ops.get_rows(ids, w, torch.bfloat16)), want)
+    assert np.array_equal(ops.get_rows(ids, w, torch.float32).cpu().numpy().view(np.uint32), synth.bf16_bits_to_f32(want).view(np.uint32))
