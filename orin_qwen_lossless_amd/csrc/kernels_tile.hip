@@ -531,26 +531,48 @@ __global__ void __launch_bounds__(WD_WAVES * 64) k_mm_wide(const bf16n_weight w,
         for (int tp = 0; tp < n; tp += pass) {
             const int nn = n - tp < pass ? n - tp : pass, nt = (nn + 31) >> 5, j0 = first + tp;
             const int n_copies = (nt + 1) >> 1;
-            // this lane's source in the copies of the wavefront: token 8 (wave + 8 i) + lane / 8, piece as swizzled
+            // this lane's source in copy i of the wavefront, in bytes from x: token 8 (wave + 8 i) + lane / 8, piece as swizzled
+            auto source = [&](int i) {
+                const int c = (lane & 7) ^ (lane >> 3), tok = 8 * (wave + WD_WAVES * i) + (lane >> 3), j = j0 + (tok < nn ? tok : nn - 1);
+                return (int64_t) a.ids_src1[j] * (2 * a.x_row) + ((c & 3) << 4) + (c >> 2) * w.K; // (K / 2 BF16)
+            };
+            // The lists may name rows anywhere (the row stride and the token stride are the caller's), a descriptor covers
+            // 4 GiB: a wavefront with a row beyond them copies by windows of 2 GiB, looking its rows up again in every step
             uint32_t src[WD_COPIES];
-            {
-                const int c = (lane & 7) ^ (lane >> 3);
+            uint64_t beyond = 0;
 #pragma unroll
-                for (int i = 0; i < WD_COPIES; i++) {
-                    const int tok = 8 * (wave + WD_WAVES * i) + (lane >> 3), j = j0 + (tok < nn ? tok : nn - 1);
-                    src[i] = (uint32_t) (a.ids_src1 ? a.ids_src1[j] : j) * (uint32_t) (2 * a.x_row) + ((c & 3) << 4) + (c >> 2) * (uint32_t) w.K; // (K / 2 BF16)
-                }
+            for (int i = 0; i < WD_COPIES; i++) {
+                const int64_t at = source(i);
+                src[i] = (uint32_t) at;
+                beyond |= __ballot((uint64_t) at + 2 * (uint64_t) w.K > 0xFFFFFFFFu);
             }
             const range_t xr = make_range(a.x, 0xFFFFFFFFu);
             int xs = 0; // byte offset of the columns of the next copies
             // (through a buffer descriptor: the compiler takes the flat form of these copies for LDS traffic of unknown
             // order and waits for all LDS reads in flight at every use of one)
             auto copy = [&](int buf) {
+                char * to = bbuf + buf * WD_BUF + wave * 1024;
+                if (beyond) {
+#pragma unroll 1
+                    for (int i = 0; i < n_copies; i++) {
+                        const int64_t at = source(i) + xs;
+                        const int window = (int) (at >> 31);
+                        for (bool todo = true; todo;) {
+                            const int now = (int) uniform((uint32_t) window); // (that of the first lane still here)
+                            if (window == now) {
+                                __builtin_amdgcn_raw_ptr_buffer_load_lds(make_range((const char *) a.x + ((int64_t) now << 31), 0xFFFFFFFFu),
+                                                                         (__attribute__((address_space(3))) void *) (to + i * (WD_WAVES * 1024)), 16,
+                                                                         (int) at & 0x7FFFFFFF, 0, 0, 0);
+                                todo = false;
+                            }
+                        }
+                    }
+                    return;
+                }
 #pragma unroll
                 for (int i = 0; i < WD_COPIES; i++) {
                     if (i < n_copies) {
-                        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void *) (bbuf + buf * WD_BUF + (wave + WD_WAVES * i) * 1024),
-                                                                 16, (int) src[i], xs, 0, 0);
+                        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void *) (to + i * (WD_WAVES * 1024)), 16, (int) src[i], xs, 0, 0);
                     }
                 }
             };
@@ -1722,8 +1744,8 @@ void launch_tile_mm_ids(const bf16n_weight & w, const bf16n_weight * up, const v
     // passes of 32 tokens while few experts can hold more than 32 (every further pass decodes the expert again)
     if (n_pairs <= (int64_t) MT_SMALL_PAIRS * n_experts) {
         mt_launch_small(w, up, a, n_pairs, cus, stream);
-    } else if (n_pairs > (int64_t) WD_MIN_PAIRS * n_experts && n_pairs * x_row * 2 < ((int64_t) 1 << 32)) {
-        wd_launch(w, up, a, cus, stream); // (a has at most n_pairs rows of activations)
+    } else if (n_pairs > (int64_t) WD_MIN_PAIRS * n_experts) {
+        wd_launch(w, up, a, cus, stream);
     } else {
         mt_launch<4, 8>(w, up, a, cus, stream);
     }

@@ -4,13 +4,15 @@ oracle (1e-3 relative, 1e-5 absolute floor; FP64 bound 1e-5 * sum|w x|), one-hot
 MoE kernel against FP64 products with the exact weights (reference tests/core/test_kernels.py:248-360)."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 from conftest import GEMV_REL
 from moe_exact import moe_layer_exact
-from orin_qwen_lossless_amd import synth
+from orin_qwen_lossless_amd import _lib, synth
 from test_gpu_kernels import check_gemv, rne_bf16, tbf16
 from test_gpu_mm_ids import reference, routing
 from test_gpu_roundtrip import bits, enc
@@ -465,3 +467,34 @@ def test_mm_ids_many_tokens_per_expert(ops, E, N, K, per_slot, counts):
     want = yu * (got.astype(np.float64) / (1.0 + np.exp(-got.astype(np.float64))))  # the same sums: only silu's rounding differs
     assert np.all(np.abs(fused - want) <= 2e-6 * np.abs(want) + 1e-12)
     assert np.array_equal(bits(ops.moe_mm_ids(tbf16(xb), it, w, E, up=u, out_dtype=torch.bfloat16)), rne_bf16(fused))
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_mm_ids_many_tokens_of_rows_beyond_4_gib(ops, shuffled):
+    """The lists may name any rows of x: with a token stride of 16384 rows of 1 KiB the later tokens lie beyond 4 GiB, in
+    token order (bf16n_mm_ids_route's sis1) or in any other, so that the tokens copied by one instruction are far apart.
+    The products are those of the same rows side by side."""
+    E, N, K, T, k, stride = 5, 64, 512, 300, 2, 16384
+    w, u = enc(ops, synth.weights(E * N, K, 71), HP, 32, False, True), enc(ops, synth.weights(E * N, K, 72), HP, 32, False, True)
+    x = tbf16(synth.activations(T, K, 73))
+    ids = torch.from_numpy(routing(T, k, E, {0: 33}, 7)).cuda()
+    src1, dst, bounds = ops.mm_ids_route(ids, E, False)
+    far = torch.empty(T * stride * K, dtype=torch.bfloat16, device="cuda")  # 4.7 GiB, of which 300 rows are written
+    L, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    if shuffled:
+        at = torch.randperm(T, generator=torch.Generator().manual_seed(1)).cuda()
+        far_src1 = (at[src1.long()] * stride).to(torch.int32)
+    else:
+        at = torch.arange(T, device="cuda")
+        far_src1 = torch.empty_like(src1)
+        _lib.check(L.bf16n_mm_ids_route(ids.data_ptr(), 0, k, far_src1.data_ptr(), dst.data_ptr(), bounds.data_ptr(), E, T, k, 1, stride, st))
+        assert torch.equal(far_src1, src1 * stride)
+    far.view(T, stride * K)[at, :K] = x
+    cw, cu = ops._cweight(w), ops._cweight(u)
+    for up in (None, cu):
+        want, got = (torch.full((T, k, N), float("nan"), device="cuda") for _ in range(2))
+        for xp, s, y in ((x, src1, want), (far, far_src1, got)):
+            _lib.check(L.bf16n_mm_ids(C.byref(cw), C.byref(up) if up is not None else None, xp.data_ptr(), K, s.data_ptr(), dst.data_ptr(),
+                                      bounds.data_ptr(), y.data_ptr(), 0, N, E, T, k, st))
+        assert not want.isnan().any()
+        assert torch.equal(got, want)
