@@ -120,9 +120,12 @@ int bf16n_mm_ids(const bf16n_weight * w, const bf16n_weight * up, const void * x
 /* No counterpart in the reference.  bf16n_mm_ids for calls with many tokens per expert (prefill), in two phases through
  * a scratch buffer of the caller's: groups of experts are decoded once into the scratch (BF16, matrix-core operand
  * order) by a kernel with the GEMV's decode rate and multiplied from there by a kernel without a decoder; the fused
- * kernel of bf16n_mm_ids decodes an expert once per pass of 128 of its tokens.  Tile layout only.  scratch: 16-byte
- * aligned device memory of at least *per_expert bytes (bf16n_mm_ids_scratch_bytes; *advised is the size whose groups
- * stay in the last-level cache between the two kernels).  Same arguments and results as bf16n_mm_ids otherwise. */
+ * kernels of bf16n_mm_ids decode an expert once per pass of 128 of its tokens, 320 above 98 routed pairs per expert.
+ * Tile layout only.  scratch: 16-byte aligned device memory of at least *per_expert bytes (bf16n_mm_ids_scratch_bytes;
+ * *advised is the size whose groups stay in the last-level cache between the two kernels).  Same arguments and results
+ * as bf16n_mm_ids otherwise: the same bits where that call has more than 16 routed pairs per expert (with fewer it may
+ * add up parts of a row).  The order of the sums follows the pairs in the lists here and n_tok * n_used there: ids
+ * outside [0, n_experts), which are in no list, can put a call on different sides of the 98 (up to the order, then). */
 int bf16n_mm_ids_scratch_bytes(const bf16n_weight * w, const bf16n_weight * up, int n_experts, uint64_t * per_expert, uint64_t * advised);
 int bf16n_mm_ids_scratch(const bf16n_weight * w, const bf16n_weight * up, const void * x_bf16, int64_t x_row,
                          const int32_t * ids_src1, const int32_t * ids_dst, const int32_t * bounds, void * dst, int dst_bf16,

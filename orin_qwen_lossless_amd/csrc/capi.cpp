@@ -491,8 +491,8 @@ int bf16n_mm_ids(const bf16n_weight * w, const bf16n_weight * up, const void * x
 
 // No counterpart in the reference.  bf16n_mm_ids for calls with many tokens per expert, in two phases through a scratch
 // buffer of the caller's: groups of experts are decoded once into the scratch (as BF16, in matrix-core operand order)
-// and multiplied from there.  The result is the one of bf16n_mm_ids up to the order of the FP32 sums, which is the same
-// here (the same instruction sequence per output element).
+// and multiplied from there.  The result is the one of bf16n_mm_ids, bit for bit from 17 routed pairs per expert on: the
+// same instruction sequence per output element, chosen by the same rule (here from the number of pairs in the lists).
 int bf16n_mm_ids_scratch_bytes(const bf16n_weight * w, const bf16n_weight * up, int n_experts, uint64_t * per_expert, uint64_t * advised) {
     return guarded([&] {
         ensure_init();

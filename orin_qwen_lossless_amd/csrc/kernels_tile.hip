@@ -491,6 +491,7 @@ constexpr int WD_COPIES = WD_TOK / (8 * WD_WAVES);                            //
 // has half the LDS reads per matrix instruction: 3000 tokens of the layer above (94 pairs) 246 + 177 against 272 + 194 us,
 // 3300 tokens (103 pairs, where the first experts have more than 128) 321 + 205 against 277 + 204.
 constexpr int WD_MIN_PAIRS = 98;
+__host__ __device__ __forceinline__ bool many_pairs(int64_t n_pairs, int n_experts) { return n_pairs > (int64_t) WD_MIN_PAIRS * n_experts; }
 
 template <bool GLU>
 __global__ void __launch_bounds__(WD_WAVES * 64) k_mm_wide(const bf16n_weight w, const bf16n_weight w_up, const mm_args a) {
@@ -815,10 +816,10 @@ __global__ void __launch_bounds__(EXPAND_WAVES * 64) k_tile_expand(const bf16n_w
 
 // The product from expanded tiles.  Work items, passes, staging of the activations and the stores are those of
 // k_mm_tile's 128-token shape; the A operands are loaded, two steps ahead, from the scratch (t0: tiles of w for the
-// experts [e0, e0 + n_e), t1: of w_up, or t0 again).
-template <bool GLU, int NT, int W>
-__global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uint4 * __restrict__ t0, const uint4 * __restrict__ t1, const mm_args a,
-                                                                       int e0, int n_e, int slabs) {
+// experts [e0, e0 + n_e), t1: of w_up, or t0 again).  HALVES: a step is 16 columns of either half of the row instead of
+// 32 adjacent ones, the order in which k_mm_wide adds them up.
+template <bool GLU, int NT, int W, bool HALVES>
+__device__ __forceinline__ void mm_raw(const uint4 * __restrict__ t0, const uint4 * __restrict__ t1, const mm_args & a, int e0, int n_e, int slabs) {
     using S = mt_shape<NT, W>;
     constexpr int D = 2; // steps of A operands in flight (four take 64 registers and spill)
     extern __shared__ __align__(16) uint32_t shm[];
@@ -831,6 +832,11 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uin
     const bool stager = S::STAGERS == S::THREADS || wave < S::STAGERS / 64;
     const int b_tok = stager ? tid / S::TPT : 0, b_part = tid % S::TPT;
     constexpr int TU = TILE_RAW_BYTES / 16; // uint4 per tile
+    const int n_steps = T_STEPS * slabs;
+    // the 16-column blocks of step s: A1 s and A2 behind it; in the staged row columns B1 s and B2 behind; BK columns of
+    // the row from one staged block to the next
+    constexpr int A1 = HALVES ? 1 : 2, B1 = 16 * A1, B2 = HALVES ? MT_HK / 2 : 16, BK = HALVES ? MT_HK / 2 : MT_HK;
+    const int A2 = HALVES ? n_steps : 1;
     for (int item = blockIdx.x; item < n_e * slabs_per_expert; item += gridDim.x) {
         const int el = item / slabs_per_expert, e = e0 + el, sl = item % slabs_per_expert;
         const int j0 = a.bounds[e], n = a.bounds[e + 1] - j0;
@@ -839,27 +845,26 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uin
         const int g1 = GLU ? g0 : (has1 ? g0 + 1 : g0);
         const uint4 * pa0 = t0 + ((int64_t) el * groups + (live ? g0 : 0)) * slabs * TU + lane;
         const uint4 * pa1 = t1 + ((int64_t) el * groups + (live ? g1 : 0)) * slabs * TU + lane;
-        const int n_steps = T_STEPS * slabs;
         for (int tp = 0; tp < n; tp += S::TOK) {
             const int left = n - tp, nt = left >= S::TOK ? NT : (left + 31) >> 5;
             const int btk = tp + b_tok;
             const int bj = j0 + (btk < n ? btk : 0);
-            // (staged together: 64 columns of either half of the row, the order in which k_mm_wide adds them up)
-            const uint16_t * xsrc = a.x + ((int64_t) (a.ids_src1 ? a.ids_src1[bj] : bj) * a.x_row + (S::CPT * b_part) / (MT_HK / 2) * (TILE_K / 2 * slabs) +
-                                           (S::CPT * b_part) % (MT_HK / 2));
+            // (HALVES: 64 columns of either half of the row are staged together)
+            const int col = HALVES ? (S::CPT * b_part) / BK * (TILE_K / 2 * slabs) + (S::CPT * b_part) % BK : S::CPT * b_part;
+            const uint16_t * xsrc = a.x + ((int64_t) (a.ids_src1 ? a.ids_src1[bj] : bj) * a.x_row + col);
             uint16_t * bdst = bbuf + b_tok * MT_BSTRIDE + S::CPT * b_part;
             uint4 f0, f1, f2, f3;
             if (stager) {
                 MT_STAGE_LOAD(S::VPT, f0, f1, f2, f3, (const uint4 *) xsrc);
             }
-            // A operands of the first D steps: [step][chain][half of the columns].  A step is 16 columns of either half
+            // A operands of the first D steps: [step][chain][16-column block]
             uint4 av[D][2][2];
 #pragma unroll
             for (int s = 0; s < D; s++) {
-                av[s][0][0] = pa0[s * 64];
-                av[s][0][1] = pa0[(s + n_steps) * 64];
-                av[s][1][0] = pa1[s * 64];
-                av[s][1][1] = pa1[(s + n_steps) * 64];
+                av[s][0][0] = pa0[(A1 * s) * 64];
+                av[s][0][1] = pa0[(A1 * s + A2) * 64];
+                av[s][1][0] = pa1[(A1 * s) * 64];
+                av[s][1][1] = pa1[(A1 * s + A2) * 64];
             }
             f32x16_t acc[2][NT];
 #pragma unroll
@@ -882,25 +887,25 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uin
                 const int nxt = hs + 1 < halves ? hs + 1 : hs;
                 uint4 b0, b1, b2, b3;
                 if (stager) {
-                    MT_STAGE_LOAD(S::VPT, b0, b1, b2, b3, (const uint4 *) (xsrc + nxt * (MT_HK / 2)));
+                    MT_STAGE_LOAD(S::VPT, b0, b1, b2, b3, (const uint4 *) (xsrc + nxt * BK));
                 }
 #pragma unroll
                 for (int s = 0; s < 4; s++) {
-                    const uint16_t * bp = bcur + l32 * MT_BSTRIDE + 16 * s + 8 * half;
+                    const uint16_t * bp = bcur + l32 * MT_BSTRIDE + B1 * s + 8 * half;
                     const int sd = s % D;
                     const bf16x8_t a00 = __builtin_bit_cast(bf16x8_t, av[sd][0][0]), a01 = __builtin_bit_cast(bf16x8_t, av[sd][0][1]);
                     const bf16x8_t a10 = __builtin_bit_cast(bf16x8_t, av[sd][1][0]), a11 = __builtin_bit_cast(bf16x8_t, av[sd][1][1]);
                     // the same slot's operands D steps on (the last steps of a pass ask for the pass's last step again)
                     const int st = 4 * hs + s + D, sn = st < n_steps ? st : n_steps - 1;
-                    av[sd][0][0] = pa0[sn * 64];
-                    av[sd][0][1] = pa0[(sn + n_steps) * 64];
-                    av[sd][1][0] = pa1[sn * 64];
-                    av[sd][1][1] = pa1[(sn + n_steps) * 64];
+                    av[sd][0][0] = pa0[(A1 * sn) * 64];
+                    av[sd][0][1] = pa0[(A1 * sn + A2) * 64];
+                    av[sd][1][0] = pa1[(A1 * sn) * 64];
+                    av[sd][1][1] = pa1[(A1 * sn + A2) * 64];
 #pragma unroll
                     for (int t = 0; t < NT; t++) {
                         if (t == 0 || t < nt) {
                             const bf16x8_t bv0 = *(const bf16x8_t *) (bp + t * 32 * MT_BSTRIDE);
-                            const bf16x8_t bv1 = *(const bf16x8_t *) (bp + t * 32 * MT_BSTRIDE + MT_HK / 2);
+                            const bf16x8_t bv1 = *(const bf16x8_t *) (bp + t * 32 * MT_BSTRIDE + B2);
                             acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a00, bv0, acc[0][t], 0, 0, 0);
                             acc[1][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a10, bv0, acc[1][t], 0, 0, 0);
                             acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a01, bv1, acc[0][t], 0, 0, 0);
@@ -947,6 +952,18 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uin
                 }
             }
         }
+    }
+}
+
+// The order of the sums is the one bf16n_mm_ids takes for as many routed pairs (launch_tile_mm_ids): the two forms give
+// the same bits.  (bounds[n_experts]: the pairs listed, which are all of the call's unless it names experts out of range.)
+template <bool GLU, int NT, int W>
+__global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_raw(const uint4 * __restrict__ t0, const uint4 * __restrict__ t1, const mm_args a,
+                                                                       int e0, int n_e, int slabs) {
+    if (many_pairs(a.bounds[a.n_experts], a.n_experts)) {
+        mm_raw<GLU, NT, W, true>(t0, t1, a, e0, n_e, slabs);
+    } else {
+        mm_raw<GLU, NT, W, false>(t0, t1, a, e0, n_e, slabs);
     }
 }
 
@@ -1744,7 +1761,7 @@ void launch_tile_mm_ids(const bf16n_weight & w, const bf16n_weight * up, const v
     // passes of 32 tokens while few experts can hold more than 32 (every further pass decodes the expert again)
     if (n_pairs <= (int64_t) MT_SMALL_PAIRS * n_experts) {
         mt_launch_small(w, up, a, n_pairs, cus, stream);
-    } else if (n_pairs > (int64_t) WD_MIN_PAIRS * n_experts) {
+    } else if (many_pairs(n_pairs, n_experts)) {
         wd_launch(w, up, a, cus, stream);
     } else {
         mt_launch<4, 8>(w, up, a, cus, stream);

@@ -405,12 +405,14 @@ def test_gate_up_gemv_that_selects_its_experts(ops, T, E, k, extra, N, K):
 
 
 @pytest.mark.parametrize("E,N,K,T,k,scratch_experts", [(8, 512, 2048, 300, 4, 8), (8, 512, 2048, 300, 4, 3), (6, 96, 512, 700, 2, 1),
-                                                        (16, 64, 1024, 2100, 1, 5)])
+                                                        (16, 64, 1024, 2100, 1, 5), (8, 512, 2048, 196, 4, 3), (8, 512, 2048, 197, 4, 3),
+                                                        (5, 96, 512, 45, 2, 2)])
 def test_two_phase_batched_product_equals_the_fused_kernel(ops, E, N, K, T, k, scratch_experts, monkeypatch):
     """bf16n_mm_ids_scratch (experts decoded once into a scratch buffer in matrix-core operand order, multiplied from
     there) writes the bits of bf16n_mm_ids (the same matrix instructions in the same order per output element): fused
     gate / up + SwiGLU, BF16 and FP32 out, the plain product and the down product, with scratch for all experts, for
-    some (several groups, the last smaller) and for one; an expert without tokens is skipped."""
+    some (several groups, the last smaller) and for one; an expert without tokens is skipped.  18 to 262 routed pairs per
+    expert: both sides of 98, where the order of the sums changes."""
     gate = enc(ops, synth.weights(E * N, K, 811), HP, 32, False, True)
     up = enc(ops, synth.weights(E * N, K, 812), HP, 32, False, True)
     down = enc(ops, synth.weights(E * K, N, 813), HP, 32, False, True) if N % 512 == 0 else None
