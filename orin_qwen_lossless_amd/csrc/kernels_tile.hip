@@ -1712,6 +1712,7 @@ void wd_launch(const bf16n_weight & w, const bf16n_weight * up, const mm_args & 
     const int groups = (int) (a.rows / TILE_R), gpi = up ? WD_WAVES / 2 : WD_WAVES;
     const int64_t items = (int64_t) a.n_experts * ((groups + gpi - 1) / gpi);
     const dim3 grid((unsigned) (items < cus ? items : cus)); // the LDS of a CU holds one block
+    note_kernel("k_mm_wide", up ? "true" : "false", 0);
     if (up) {
         hipLaunchKernelGGL((k_mm_wide<true>), grid, dim3(WD_WAVES * 64), wd_shm(true), stream, w, *up, a);
     } else {

@@ -500,3 +500,15 @@ def test_mm_ids_many_tokens_of_rows_beyond_4_gib(ops, shuffled):
                                       bounds.data_ptr(), y.data_ptr(), 0, N, E, T, k, st))
         assert not want.isnan().any()
         assert torch.equal(got, want)
+
+
+def test_last_kernel_names_the_batched_product(ops):
+    """Both kernels for more than 16 routed pairs per expert leave their name: 98 pairs per expert and one more."""
+    E, N, K = 4, 64, 512
+    w = enc(ops, synth.weights(E * N, K, 75), HP, 32, False, True)
+    x = tbf16(synth.activations(98 * E + 1, K, 76))
+    ids = torch.zeros((98 * E + 1, 1), dtype=torch.int32, device="cuda")
+    for T, up, want in ((98 * E, None, "k_mm_tile<false, 4, 8>"), (98 * E + 1, None, "k_mm_wide<false>"), (98 * E, w, "k_mm_tile<true, 4, 8>"),
+                        (98 * E + 1, w, "k_mm_wide<true>")):
+        ops.moe_mm_ids(x[:T], ids[:T], w, E, up=up)
+        assert ops.last_kernel() == want
