@@ -1,5 +1,5 @@
-// Decoders of the reference's 32-lane layouts: the bit reader of the batched MoE kernel (the GEMV / dequant kernels have
-// their own, lane_ring) and what both share.
+// Decoders of the reference's 32-lane layouts: the bit reader of the batched MoE kernel and of GEMVs that keep every CU
+// full (the other GEMVs, dequant and row gather have their own, lane_ring) and what both share.
 #pragma once
 
 #include "bf16n_c.h"
@@ -59,15 +59,28 @@ struct lane_bits {
 };
 
 // the 16 weights of one lane in one chunk as 8 BF16 pairs: wp[2j], wp[2j+1] = columns 128j + 4l + {0,1}, {2,3}
+template <int FORMAT>
 __device__ __forceinline__ void decode_chunk(lane_bits & bits, const uint32_t * lut, const uint4 sm, uint32_t (&wp)[8]) {
     const uint32_t smw[4] = {sm.x, sm.y, sm.z, sm.w};
+    if (FORMAT == FMT_HUFPAIR) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t e0 = bits.take<HP_LP>(lut);
-        const uint32_t e1 = bits.take<HP_LP>(lut);
-        bits.refill();
-        wp[2 * j] = merge(spread_lo(smw[j]), e0);
-        wp[2 * j + 1] = merge(spread_hi(smw[j]), e1);
+        for (int j = 0; j < 4; j++) {
+            const uint32_t e0 = bits.take<HP_LP>(lut);
+            const uint32_t e1 = bits.take<HP_LP>(lut);
+            bits.refill();
+            wp[2 * j] = merge(spread_lo(smw[j]), e0);
+            wp[2 * j + 1] = merge(spread_hi(smw[j]), e1);
+        }
+    } else { // single exponents, entry = len | exponent << 7
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t a = bits.take<HUF_LMAX>(lut), b = bits.take<HUF_LMAX>(lut);
+            bits.refill();
+            const uint32_t c = bits.take<HUF_LMAX>(lut), d = bits.take<HUF_LMAX>(lut);
+            bits.refill();
+            wp[2 * j] = merge(spread_lo(smw[j]), (a & 0x7F80u) | ((b & 0x7F80u) << 16));
+            wp[2 * j + 1] = merge(spread_hi(smw[j]), (c & 0x7F80u) | ((d & 0x7F80u) << 16));
+        }
     }
 }
 

@@ -3,11 +3,14 @@
 //
 // A wave64 carries two units (HUFPAIR / HUFFMAN) or two rows (NIBBLE): lanes 0..31 the even one, lanes 32..63 the odd
 // one; each half reads its 512-byte plane chunk with one 16-byte load per lane, four chunks ahead.  Lane streams pass
-// through rings in LDS (lane_ring).  These kernels take any K, R, layout, expert ids and FP32 or BF16 activations; the
-// wave64 layout (kernels_w64.hip), which has twice the chains per unit, is the fast path.
+// through rings in LDS (lane_ring), except in products with enough wavefronts to cover each other's misses (huf_direct).
+// These kernels take any K, R, layout, expert ids and FP32 or BF16 activations; the wave64 layout (kernels_w64.hip),
+// which has twice the chains per unit, is the fast path.
 #include "dev_common.h"
 #include "dev_compat.h"
 #include "launchers.h"
+
+#include <algorithm>
 
 namespace bf16n {
 namespace dev {
@@ -27,6 +30,7 @@ constexpr int HALVES = NT / 32;  // units (rows) per block
 // what it loaded DEEP rounds ago; the same block again while it has not moved on.  The stream buffers end with padding
 // words (32 of HUFPAIR, 16 of HUFFMAN): the last lane reads at most 17 (13) words past its end.
 constexpr int LR_WORDS = 16;                     // ring words per lane
+constexpr size_t LDS_BYTES = 160 * 1024;         // of a CU
 constexpr int LR_BYTES = LR_WORDS * 64 * 4;      // per wavefront: word i of a lane at [i % 16][lane]
 template <int FORMAT> struct lane_ring {
     static constexpr int BITS = FORMAT == FMT_HUFPAIR ? HP_LP : HUF_LMAX;
@@ -111,11 +115,23 @@ template <int FORMAT> struct lane_ring {
 };
 
 // the chunks [0, n) of a half-wave's unit in stream order, four plane chunks in flight: f(chunk, weights), and before a
-// chunk is decoded pre()
-template <int FORMAT, typename P, typename F>
+// chunk is decoded pre().  RING = false: the lanes read their streams and the plane where they need them (lane_bits),
+// for launches with enough wavefronts to wait beside each other (huf_direct)
+template <int FORMAT, bool RING = true, typename P, typename F>
 __device__ __forceinline__ void for_chunks(const uint8_t * plane, const uint32_t * sp, uint32_t * ring, const uint32_t * lut, int n, int l32, P pre, F f) {
     constexpr int D = 4;
     const uint4 * pl = (const uint4 *) plane + l32;
+    if constexpr (!RING) {
+        lane_bits bits;
+        bits.begin(sp);
+        for (int o = 0; o < n; o++) {
+            uint32_t wp[8];
+            decode_chunk<FORMAT>(bits, lut, pl[o * 32], wp);
+            pre();
+            f(o, wp);
+        }
+        return;
+    }
     uint4 sm[D];
 #pragma unroll
     for (int i = 0; i < D; i++) {
@@ -165,7 +181,7 @@ __device__ __forceinline__ float dot_chunk(const uint32_t (&wp)[8], const float4
 
 // One unit of R rows: y[rr] (rr < R) ends up in lane rr of the half-wave.  Row-major streams finish a row every C
 // chunks; chunk-major streams add one partial sum per (chunk, row).
-template <int FORMAT>
+template <int FORMAT, bool RING>
 __device__ __forceinline__ float unit_dot(const uint8_t * plane, const uint32_t * lut, const uint32_t * sp, uint32_t * ring, int64_t gu, int R,
                                           int C, bool cm, const float * xs, int l32) {
     const bool upper = (threadIdx.x & 32) != 0;
@@ -177,7 +193,7 @@ __device__ __forceinline__ float unit_dot(const uint8_t * plane, const uint32_t 
     float mine = 0.f, acc = 0.f;
     int rr = 0, c = 0;
     float4 x[4]; // the chunk's activations, requested before its chain of lookups (8192 x 2048: 3 us of 66)
-    for_chunks<FORMAT>(plane + gu * R * (int64_t) C * CHUNK, sp, ring, lut, R * C, l32, [&] {
+    for_chunks<FORMAT, RING>(plane + gu * R * (int64_t) C * CHUNK, sp, ring, lut, R * C, l32, [&] {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             x[j] = *(const float4 *) (xs + c * CHUNK + 128 * j + 4 * l32);
@@ -215,8 +231,8 @@ __device__ __forceinline__ const uint32_t * lane_stream(const bf16n_weight & w, 
 }
 
 // y = W x (GLU: y = silu(gate x) * up x) for HUFPAIR / HUFFMAN in the 32-lane layouts; one half-wave per unit,
-// blockIdx.y = column.  Shared memory: x as FP32 [K], then one table per matrix, then a ring per wavefront.
-template <int FORMAT, typename TX, bool GLU>
+// blockIdx.y = column.  Shared memory: x as FP32 [K], then one table per matrix, then (RING) a ring per wavefront.
+template <int FORMAT, typename TX, bool GLU, bool RING>
 __global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16n_weight w_up, const cols p) {
     constexpr int LUT_N = FORMAT == FMT_HUFPAIR ? (1 << HP_LP) : (1 << HUF_LMAX);
     extern __shared__ __align__(16) unsigned char shm_raw[];
@@ -250,9 +266,9 @@ __global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16
         // (both halves of a wavefront stay together: a missing last unit is decoded twice and stored once)
         const int64_t u = u0 + (half & 1) < units ? u0 + (half & 1) : u0;
         const int64_t gu = cv.rbase / R + u;
-        float v = unit_dot<FORMAT>(w.plane, lut, lane_stream<FORMAT>(w, gu, l32), ring, gu, R, C, cm, xs, l32);
+        float v = unit_dot<FORMAT, RING>(w.plane, lut, lane_stream<FORMAT>(w, gu, l32), ring, gu, R, C, cm, xs, l32);
         if (GLU) {
-            const float uv = unit_dot<FORMAT>(w_up.plane, lut_up, lane_stream<FORMAT>(w_up, gu, l32), ring, gu, R, C, false, xs, l32);
+            const float uv = unit_dot<FORMAT, RING>(w_up.plane, lut_up, lane_stream<FORMAT>(w_up, gu, l32), ring, gu, R, C, false, xs, l32);
             v = uv * silu(v);
         }
         if (l32 < R && u == u0 + (half & 1)) {
@@ -729,13 +745,36 @@ int grid_for(int64_t work, int ncols, int cus, int per_block = HALVES) {
 }
 
 // Wavefronts per block of the HUFPAIR / HUFFMAN kernels, two units each: four, fewer where that leaves CUs without a
-// block (the units' chains set the time: alone on a CU they share its LDS with nobody)
-int huf_waves(int64_t units, int ncols, int cus) {
+// block (the units' chains set the time: alone on a CU they share its LDS with nobody).  Units of a chunk or two are done
+// sooner than a smaller block stages its table: 1024 rows of 512, R = 1, one column 8.4 us with two wavefronts, 7.2 with four.
+int huf_waves(int64_t units, int ncols, int cus, int chunks) {
     int waves = NT / 64;
-    while (waves > 1 && (units + 2 * waves - 1) / (2 * waves) * ncols < cus) {
+    while (waves > 1 && chunks > 2 && (units + 2 * waves - 1) / (2 * waves) * ncols < cus) {
         waves /= 2;
     }
     return waves;
+}
+
+// Dense products whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers per
+// wavefront, so that 16 of them (12 at K = 4096) fit a CU instead of 20 (16), and a lane that has not moved on loads its
+// block again; with that many wavefronts there the misses of one are covered by the others.  Without against with rings:
+//  * Several columns whose wavefronts fit the CUs at once this way and not with rings: 32768 x 2048, R = 16, five columns
+//    109 us against 126 (four: 102 against 90; six: 195 against 129); 2048 x 4096, R = 4, sixteen 43 against 51; 8192 x 1024,
+//    R = 4, five 16.7 against 19.8.
+//  * HUFPAIR in short units that the caches hold, from 64 wavefronts per CU on: 16384 x 512, R = 1, eight columns 27
+//    against 40 us (32768 x 2048, four chunks: 202 against 174).
+//  * HUFFMAN, which loads a block per eight codes where HUFPAIR has one per sixteen, from 16 wavefronts per CU on unless
+//    the matrix comes from memory in short units: 8192 x 1024, R = 4, eight columns 31 against 34 us; 32768 x 1024,
+//    R = 16, sixteen 211 against 267; 32768 x 4096, R = 4, one 142 against 208; but R = 4 at 32768 x 1024, eight chunks,
+//    sixteen 242 against 223.
+bool huf_direct(const bf16n_weight & w, int64_t units, int ncols, int cus, size_t shared) {
+    const int ring = (int) std::min<size_t>(4, LDS_BYTES / (shared + 4 * LR_BYTES)), direct = std::min(5, (int) ((LDS_BYTES - 1) / shared));
+    const int64_t per_cu = units * ncols / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
+    const int chunks = w.R * (int) (w.K / CHUNK);
+    if (ncols > 1 && units * ncols > (int64_t) 8 * ring * cus && units * ncols <= (int64_t) 8 * direct * cus) {
+        return true;
+    }
+    return w.format == FMT_HUFPAIR ? chunks <= 8 && per_cu >= 64 && weights <= (16 << 20) : per_cu >= 16 && (weights <= (16 << 20) || chunks >= 32);
 }
 
 } // namespace
@@ -832,23 +871,25 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
     }
     const bool hp = w.format == FMT_HUFPAIR;
     const int64_t work = p.nrows / w.R;
-    const int waves = huf_waves(work, ncols, cus);
-    const size_t shm = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX)) + (size_t) waves * LR_BYTES;
+    const size_t shared = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX));
+    const bool direct = !glu && !p.ids && huf_direct(w, work, ncols, cus, shared);
+    const int waves = direct ? NT / 64 : huf_waves(work, ncols, cus, w.R * (int) (w.K / CHUNK));
+    const size_t shm = shared + (direct ? 0 : (size_t) waves * LR_BYTES);
     const dim3 grid(grid_for(work, ncols, cus, 2 * waves), ncols);
-#define HUF(F, TX, G) hipLaunchKernelGGL((k_huf_mmv<F, TX, G>), grid, dim3(waves * 64), shm, stream, w, wu, p)
+#define HUF(F, TX, G, RING) hipLaunchKernelGGL((k_huf_mmv<F, TX, G, RING>), grid, dim3(waves * 64), shm, stream, w, wu, p)
+#define HUFX(F, TX) do { if (glu) HUF(F, TX, true, true); else if (direct) HUF(F, TX, false, false); else HUF(F, TX, false, true); } while (0)
     if (hp) {
-        if (x_bf16) { if (glu) HUF(FMT_HUFPAIR, bf16_t, true); else HUF(FMT_HUFPAIR, bf16_t, false); }
-        else        { if (glu) HUF(FMT_HUFPAIR, float, true);  else HUF(FMT_HUFPAIR, float, false); }
+        if (x_bf16) HUFX(FMT_HUFPAIR, bf16_t); else HUFX(FMT_HUFPAIR, float);
     } else {
-        if (x_bf16) { if (glu) HUF(FMT_HUFFMAN, bf16_t, true); else HUF(FMT_HUFFMAN, bf16_t, false); }
-        else        { if (glu) HUF(FMT_HUFFMAN, float, true);  else HUF(FMT_HUFFMAN, float, false); }
+        if (x_bf16) HUFX(FMT_HUFFMAN, bf16_t); else HUFX(FMT_HUFFMAN, float);
     }
+#undef HUFX
 #undef HUF
 }
 
 void launch_compat_dequant(const bf16n_weight & w, int64_t row0, int64_t nrows, uint16_t * out, int cus, hipStream_t stream) {
     const int64_t work = w.format == FMT_NIBBLE ? nrows : nrows / w.R;
-    const int waves = w.format == FMT_NIBBLE ? NT / 64 : huf_waves(work, 1, cus);
+    const int waves = w.format == FMT_NIBBLE ? NT / 64 : huf_waves(work, 1, cus, w.R * (int) (w.K / CHUNK));
     const int64_t blocks = (work + 2 * waves - 1) / (2 * waves);
     const dim3 grid((unsigned) (blocks < (int64_t) cus * 16 ? blocks : (int64_t) cus * 16));
     if (w.format == FMT_NIBBLE) {

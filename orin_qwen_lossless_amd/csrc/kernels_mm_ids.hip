@@ -123,7 +123,7 @@ struct slab_dec {
 #pragma unroll
             for (int i = 0; i < L::ROWS_PER_PHASE; i++) {
                 uint32_t wp[8];
-                decode_chunk(bits, lut, sm[i], wp);
+                decode_chunk<FMT_HUFPAIR>(bits, lut, sm[i], wp);
                 tile_put(tile, u * L::ROWS_PER_PHASE + i, l32, wp);
             }
         }

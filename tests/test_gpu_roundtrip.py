@@ -171,3 +171,17 @@ def test_wave64_steps_across_units_and_rows(ops, R, K, units):
     want = src[ids.cpu().numpy()]
     assert np.array_equal(bits(ops.get_rows(ids, w, torch.bfloat16)), want)
     assert np.array_equal(ops.get_rows(ids, w, torch.float32).cpu().numpy().view(np.uint32), synth.bf16_bits_to_f32(want).view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt,R,rows,K,cm,T", [(HP, 4, 2048, 4096, False, 16), (HP, 8, 2048, 4096, True, 32), (HP, 1, 16381, 512, False, 8),
+                                               (HP, 1, 4093, 1024, False, 8), (HUF, 4, 8188, 1536, False, 8), (HUF, 16, 8208, 4096, False, 20),
+                                               (HUF, 1, 8191, 512, False, 3)])
+def test_columns_that_fill_the_gpu_have_the_bits_of_a_single_one(ops, fmt, R, rows, K, cm, T):
+    """32-lane layouts with many columns read their streams without the rings: the sums are those of one column, which
+    goes through them; odd numbers of units."""
+    w = enc(ops, synth.weights(rows, K, rows + T), fmt, R, cm)
+    x = torch.from_numpy(synth.bf16_bits_to_f32(synth.activations(T, K, 5))).cuda()
+    for xt in (x, x.to(torch.bfloat16)):
+        y = ops.mmv(xt, w)
+        for t in range(T):
+            assert torch.equal(y[t], ops.mmv(xt[t: t + 1], w)[0]), t
