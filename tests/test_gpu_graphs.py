@@ -93,11 +93,12 @@ def test_moe_layer_graph(ops, T):
     assert float((out.float() - ref.float()).abs().max()) <= 2e-2 * scale
 
 
-@pytest.mark.parametrize("layout,E,T", [("units", 8, 64), ("tiles", 8, 300), ("tiles", 8, 64), ("tiles", 40, 12)])
+@pytest.mark.parametrize("layout,E,T", [("units", 8, 64), ("tiles", 8, 400), ("tiles", 8, 300), ("tiles", 8, 64), ("tiles", 40, 12)])
 def test_batched_moe_graph(ops, layout, E, T):
     # routing lists, fused gate/up + SwiGLU and down run as batched kernels inside the graph: 4- and 16-row wave64 units
-    # (decode -> LDS tile -> MFMA) and the tile layout in its three shapes (128-token passes at 300 tokens, 32-token
-    # passes at 64, K split over wavefronts at 12 tokens of 40 experts); the routing changes from replay to replay
+    # (decode -> LDS tile -> MFMA) and the tile layout in its four shapes (passes of up to 320 tokens at 400 tokens,
+    # 128-token passes at 300, 32-token passes at 64, K split over wavefronts at 12 tokens of 40 experts); the routing
+    # changes from replay to replay
     k, K, N = 2, 2048, 512
     r_gu, r_dn = (4, 16) if layout == "units" else (32, 32)
     gate = enc(ops, synth.weights(E * N, K, 101), HP, r_gu, False, True)
