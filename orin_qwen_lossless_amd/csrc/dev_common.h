@@ -67,14 +67,6 @@ __device__ __forceinline__ void store_y(char * y, bool y_bf16, int64_t i, float 
 
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + __expf(-x)); }
 
-// sum over the 32 lanes of each half-wave; every lane of the half gets the result
-__device__ __forceinline__ float half_wave_sum(float v) {
-#pragma unroll
-    for (int o = 16; o; o >>= 1) {
-        v += __shfl_xor(v, o, 64);
-    }
-    return v;
-}
 // sum over the 64 lanes of the wave; every lane gets the result
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

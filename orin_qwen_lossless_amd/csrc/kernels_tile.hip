@@ -520,7 +520,7 @@ __global__ void __launch_bounds__(WD_WAVES * 64) k_mm_wide(const bf16n_weight w,
         if (e >= a.n_experts) {
             break;
         }
-        const int first = a.bounds ? a.bounds[e] : 0, n = a.bounds ? a.bounds[e + 1] - first : a.n_tok;
+        const int first = a.bounds[e], n = a.bounds[e + 1] - first;
         if (n <= 0) {
             continue;
         }
@@ -666,7 +666,7 @@ __global__ void __launch_bounds__(WD_WAVES * 64) k_mm_wide(const bf16n_weight w,
             auto store = [&](int t, const float (&v)[16]) {
                 const int tk = 32 * t + l32;
                 if (live && tk < nn) {
-                    const int64_t o = (int64_t) (a.ids_dst ? a.ids_dst[j0 + tk] : tp + tk) * a.dst_col + (int64_t) g * TILE_R + 4 * half;
+                    const int64_t o = (int64_t) a.ids_dst[j0 + tk] * a.dst_col + (int64_t) g * TILE_R + 4 * half;
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
                         if (a.dst_bf16) {
