@@ -243,6 +243,7 @@ int bf16n_cu_count(int * out) {
 int bf16n_mmv(const bf16n_weight * w, const bf16n_mmv_args * a, void * stream, int multi_col) {
     return guarded([&] {
         ensure_init();
+        dev::g_last_kernel.name = nullptr;
         check_weight(*w);
         require(a->ncols > 0 && a->ncols <= 65535, "ncols out of range");
         require(w->format == FMT_NIBBLE || (a->nrows % w->R == 0 && a->row0 % w->R == 0 && a->rows_per_matrix % w->R == 0),
@@ -273,9 +274,8 @@ int bf16n_mmv(const bf16n_weight * w, const bf16n_mmv_args * a, void * stream, i
     });
 }
 
-// The kernel instance that the calling thread's last bf16n_mmv / bf16n_mmv_glu2 launch chose, as the profiler prints it
-// ("k_w64_mmv<bf16_t, 4, 1, 2, 1>"); an empty string before the first launch or after a launch on a path that leaves
-// no note.  The pointer stays valid until the thread's next call of this function.
+// The kernel instance that the calling thread's last product (bf16n_mmv*, bf16n_mm_ids*) chose, as the profiler prints it
+// ("k_w64_mmv<bf16_t, 4, 1, 2, 1>"); an empty string before the first one or after one on a path that leaves no note.  The pointer stays valid until the thread's next call of this function.
 const char * bf16n_last_kernel(void) {
     const dev::kernel_note & k = dev::g_last_kernel;
     g_kernel_text.clear();
@@ -327,6 +327,7 @@ int bf16n_gemv_max_tokens(const bf16n_weight * w, int * out) {
 int bf16n_mmv_glu(const bf16n_weight * w, const bf16n_mmv_args * a, void * stream) {
     return guarded([&] {
         ensure_init();
+        dev::g_last_kernel.name = nullptr;
         check_weight(*w);
         require(w->format == FMT_NIBBLE, "mmv_glu supports NIBBLE matrices only");
         require(a->rows_per_matrix == 2 * a->nrows, "mmv_glu: rows per matrix must be [gate; up] of nrows each");
@@ -343,6 +344,7 @@ int bf16n_mmv_glu(const bf16n_weight * w, const bf16n_mmv_args * a, void * strea
 int bf16n_mmv_glu2(const bf16n_weight * gate, const bf16n_weight * up, const bf16n_mmv_args * a, void * stream) {
     return guarded([&] {
         ensure_init();
+        dev::g_last_kernel.name = nullptr;
         check_weight(*gate);
         check_weight(*up);
         require(gate->format == up->format && gate->K == up->K, "mmv_glu: gate/up format and K must match");
@@ -378,6 +380,7 @@ int bf16n_mmv_glu2_topk(const bf16n_weight * gate, const bf16n_weight * up, cons
                         int64_t logits_stride, int n_experts, int k, int renorm, float * weights, int64_t weights_stride, void * stream) {
     return guarded([&] {
         ensure_init();
+        dev::g_last_kernel.name = nullptr;
         check_weight(*gate);
         check_weight(*up);
         require(dev::is_tile_layout(*gate) && dev::is_tile_layout(*up) && gate->K == up->K && gate->rows == up->rows,
@@ -466,6 +469,7 @@ int bf16n_mm_ids(const bf16n_weight * w, const bf16n_weight * up, const void * x
                  int64_t dst_col, int n_experts, int n_tok, int n_used, void * stream) {
     return guarded([&] {
         ensure_init();
+        dev::g_last_kernel.name = nullptr;
         check_weight(*w);
         require(dev::mm_ids_shape_ok(*w, up), "no batched kernel for this matrix");
         require(n_experts > 0 && w->rows % n_experts == 0, "rows must split evenly into experts");
@@ -514,6 +518,7 @@ int bf16n_mm_ids_scratch(const bf16n_weight * w, const bf16n_weight * up, const 
                          int64_t dst_col, int n_experts, void * scratch, uint64_t scratch_bytes, void * stream) {
     return guarded([&] {
         ensure_init();
+        dev::g_last_kernel.name = nullptr;
         check_weight(*w);
         if (up) {
             check_weight(*up);
@@ -537,6 +542,7 @@ int bf16n_moe_mm_ids_static(const bf16n_weight * w, const bf16n_weight * up, con
                             int n_experts, int n_tok, int n_used, void * stream) {
     return guarded([&] {
         ensure_init();
+        dev::g_last_kernel.name = nullptr;
         check_weight(*w);
         require(dev::mm_ids_shape_ok(*w, up), "no batched kernel for this matrix");
         require(n_experts > 0 && w->rows % n_experts == 0, "rows must split evenly into experts");

@@ -503,7 +503,8 @@ def test_mm_ids_many_tokens_of_rows_beyond_4_gib(ops, shuffled):
 
 
 def test_last_kernel_names_the_batched_product(ops):
-    """Both kernels for more than 16 routed pairs per expert leave their name: 98 pairs per expert and one more."""
+    """Both kernels for more than 16 routed pairs per expert leave their name: 98 pairs per expert and one more; a path
+    that leaves none does not leave that of the product before."""
     E, N, K = 4, 64, 512
     w = enc(ops, synth.weights(E * N, K, 75), HP, 32, False, True)
     x = tbf16(synth.activations(98 * E + 1, K, 76))
@@ -512,3 +513,5 @@ def test_last_kernel_names_the_batched_product(ops):
                         (98 * E + 1, w, "k_mm_wide<true>")):
         ops.moe_mm_ids(x[:T], ids[:T], w, E, up=up)
         assert ops.last_kernel() == want
+    ops.moe_mm_ids(x[:2], ids[:2], w, E)
+    assert ops.last_kernel() == ""
