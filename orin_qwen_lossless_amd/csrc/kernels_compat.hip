@@ -24,9 +24,9 @@ constexpr int HALVES = NT / 32;  // units (rows) per block
 // One lane's MSB-first bit stream, read through a ring of 16 words in LDS.  What bounds these kernels is the chain of
 // one unit (two dependent table lookups per two codes, all lanes of a half-wave in step), so nothing else may be waited
 // for in it: 64 lanes read 64 cache lines, and with the next word loaded where it is needed nearly every pair of codes
-// waited for some lane's cache miss (one column of 8192 x 2048, R = 16: 74 us then, 59 us with the ring; 65536 x 4096:
-// 266 and 162; dequant of the first 88 and 49).  Here a lane loads whole 16-byte
-// blocks, one per four code pairs (96 bits at most, less than a block), LOOK blocks beyond the one it reads, and stores
+// waited for some lane's cache miss (one column of 8192 x 2048, R = 16: 77.7 us then, 42.3 now, about 15 of them by the
+// ring, the rest by plane chunks ahead, small blocks and sums on the VALU; 65536 x 4096: 266 and 162; dequant of the first
+// 88 and 49).  Here a lane loads whole 16-byte blocks, one per four code pairs (96 bits at most, less than a block), LOOK blocks beyond the one it reads, and stores
 // what it loaded DEEP rounds ago; the same block again while it has not moved on.  The stream buffers end with padding
 // words (32 of HUFPAIR, 16 of HUFFMAN): the last lane reads at most 17 (13) words past its end.
 constexpr int LR_WORDS = 16;                     // ring words per lane
@@ -192,7 +192,7 @@ __device__ __forceinline__ float unit_dot(const uint8_t * plane, const uint32_t 
     };
     float mine = 0.f, acc = 0.f;
     int rr = 0, c = 0;
-    float4 x[4]; // the chunk's activations, requested before its chain of lookups (8192 x 2048: 3 us of 66)
+    float4 x[4]; // the chunk's activations, requested before its chain of lookups (8192 x 2048, one column: 3 us)
     for_chunks<FORMAT, RING>(plane + gu * R * (int64_t) C * CHUNK, sp, ring, lut, R * C, l32, [&] {
 #pragma unroll
         for (int j = 0; j < 4; j++) {

@@ -35,8 +35,8 @@ __global__ void __launch_bounds__(256) k_moe_combine(const float * __restrict__ 
 // The same sum, four adjacent columns per thread and SLOTS rows requested before the first is waited for (16-byte rows;
 // further slots follow SLOTS at a time in order, so every element keeps the fmaf chain above bit for bit).  The kernel
 // reads n_used FP32 rows per token and is bound by that: with one 4-byte load in flight per thread 8192 tokens x top-8 of
-// 2048 columns (537 MB) took 174 us, this way 125, and 93 with the rows, which nothing reads again, loaded non-temporally
-// (5.8 TB/s); 2048 tokens 45 -> 20 us.
+// 2048 columns (537 MB) took 174 us, this way 125, and 91 with the rows, which nothing reads again, loaded non-temporally
+// (5.9 TB/s); 2048 tokens 45 -> 20 us.
 typedef float f32x4_nt __attribute__((ext_vector_type(4)));
 template <int SLOTS>
 __global__ void __launch_bounds__(256) k_moe_combine4(const float * __restrict__ ys, const char * __restrict__ w, bool w_bf16,

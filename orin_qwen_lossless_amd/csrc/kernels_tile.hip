@@ -487,9 +487,14 @@ __global__ void __launch_bounds__((mt_shape<NT, W>::THREADS)) k_mm_tile(const bf
 constexpr int WD_WAVES = 8, WD_NT = 10, WD_TOK = 32 * WD_NT;
 constexpr int WD_ROW = 128, WD_BUF = WD_TOK * WD_ROW;                         // bytes per staged token, per buffer
 constexpr int WD_COPIES = WD_TOK / (8 * WD_WAVES);                            // copy instructions per wavefront and step: eight tokens each
-// Routed pairs per expert from which it runs.  Below, every expert's tokens fit one 128-token pass of k_mm_tile, which
-// has half the LDS reads per matrix instruction: 3000 tokens of the layer above (94 pairs) 246 + 177 against 272 + 194 us,
-// 3300 tokens (103 pairs, where the first experts have more than 128) 321 + 205 against 277 + 204.
+// Routed pairs per expert, on average (the host knows no more), from which it runs.  Near-uniform routing below it gives
+// hardly an expert more than one 128-token pass of k_mm_tile, which has half the LDS reads per matrix instruction: 3000
+// tokens of the layer above (94 pairs) 246 + 177 against 272 + 194 us, 3300 tokens (103 pairs, where the first experts
+// have more than 128) 321 + 205 against 277 + 204.  Up to some 115 pairs the down product alone is 2 to 5 % behind there,
+// the two together level or ahead; 48 experts of 512 x 1024 at 104 pairs: 61 + 40 against 42 + 29.  Skewed routing (an
+// expert named by three quarters of the tokens) crosses earlier, but the host cannot tell: at 60 pairs on average it stays
+// with 1213 + 479 us of 128-token passes; at 112 it is 2174 + 822 against 914 + 437, the hot expert's passes one after the
+// other in the few blocks that its slabs were dealt to.  The order of a product's sums changes here too.
 constexpr int WD_MIN_PAIRS = 98;
 __host__ __device__ __forceinline__ bool many_pairs(int64_t n_pairs, int n_experts) { return n_pairs > (int64_t) WD_MIN_PAIRS * n_experts; }
 
@@ -539,6 +544,7 @@ __global__ void __launch_bounds__(WD_WAVES * 64) k_mm_wide(const bf16n_weight w,
             };
             // The lists may name rows anywhere (the row stride and the token stride are the caller's), a descriptor covers
             // 4 GiB: a wavefront with a row beyond them copies by windows of 2 GiB, looking its rows up again in every step
+            // (98304 tokens x 8 rows of 4096 over 128 experts of 256 rows, 6 GiB: 4.7 ms; k_mm_tile's 128-token passes 8.6)
             uint32_t src[WD_COPIES];
             uint64_t beyond = 0;
 #pragma unroll
@@ -731,9 +737,8 @@ size_t wd_shm(bool glu) { return (size_t) (glu ? 2 : 1) * LUT_WORDS * 4 + (size_
 
 // ---------------------------------------------------------------- batched MoE prefill in two phases (many tokens per expert)
 //
-// With a few hundred tokens per expert the fused kernel above decodes every expert once per pass of 128 tokens, at
-// half the decode chains per CU of the GEMV (its accumulators take the registers), and the decode is what it waits
-// for.  The two-phase form decodes a group of experts once, at the GEMV's chain count, into a scratch buffer of the
+// The fused kernels above decode an expert once per pass of its tokens, at half the decode chains per CU of the GEMV
+// (their accumulators take the registers), and the decode is what they wait for.  The two-phase form decodes a group of experts once, at the GEMV's chain count, into a scratch buffer of the
 // caller's (k_tile_expand), and multiplies from there with a kernel that has no decoder in its registers (k_mm_raw).
 // The scratch keeps the tiles in the decoder's own order, the A-operand order of the matrix instruction: tile u of
 // the group, step s, 16-column block kb, lane l -> 16 bytes at ((u * 8 + s) * 2 + kb) * 1024 + 16 l, so that both

@@ -329,7 +329,8 @@ __global__ void __launch_bounds__(1024) k_w64_glu(const bf16n_weight wg, const b
 
 // Both kernels are bound by the chain of a unit (a step is eight dependent table lookups), so a step must not wait for
 // its plane bytes as well: loaded where they were needed, every step paid a miss that reached HBM.  R = 16, K = 2048:
-// 64 / 513 / 2048 rows gathered 20.7 / 24.0 / 26.2 -> 14.9 / 15.9 / 18.1 us; 65536 rows dequantised 97 -> 92 us.  All
+// 64 / 513 / 2048 rows gathered 20.7 / 24.0 / 26.2 -> 14.9 / 15.9 / 18.1 us (the same rows again and again: a first pass
+// over a new matrix and new ids is 186 -> 173 us of cold calls and misses); 65536 rows dequantised 97 -> 92 us.  All
 // 248320 rows stay at 356 us (1.7 GB read and written, 4.8 TB/s: many wavefronts hide the misses there).
 
 // the 16 weights of a lane in one step, to its four places in the 512 columns at dst

@@ -514,10 +514,10 @@ def mm_ids_route(topk_ids: torch.Tensor, n_experts: int, per_slot: bool):
 
 
 # moe_mm_ids: routed pairs per expert from which the tile layout's two-phase form (decode a group of experts into
-# scratch once, multiply from there) replaces the fused kernel, which decodes an expert once per 128 of its tokens.
-# Off by default: measured on a 256-expert layer it is behind the fused kernel at every token count (1.86 against 1.09
-# ms at 8192 tokens, 1.03 against 0.40 ms at 2048): writing and re-reading the experts as BF16 (1.6 GB a layer) costs
-# more than the second decode it saves.  Callers that pass `scratch` and lower this value get it.
+# scratch once, multiply from there) replaces the fused kernels, which decode an expert once per 128 of its tokens, 320
+# above 98 pairs per expert.  Off by default: measured on a 256-expert layer it is behind the fused kernels at every token
+# count (1.69 against 0.81 ms at 8192 tokens, 0.95 against 0.42 ms at 2048): writing and re-reading the experts as BF16
+# (1.6 GB a layer) costs more than any second decode.  Callers that pass `scratch` and lower this value get it.
 MM_IDS_TWO_PHASE_PAIRS_PER_EXPERT = 1 << 30
 _mm_scratch: dict = {}
 
@@ -696,7 +696,7 @@ def router_topk_routes(logits: torch.Tensor, k: int, n_listed: int, renorm: bool
 
 
 def last_kernel() -> str:
-    """The kernel instance the calling thread's last dense product launch chose, as a profiler prints it
+    """The kernel instance the calling thread's last product launch chose, as a profiler prints it
     (bf16n_last_kernel; "" where the path leaves no note)."""
     return _lib.lib().bf16n_last_kernel().decode()
 
