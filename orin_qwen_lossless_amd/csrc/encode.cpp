@@ -1,9 +1,10 @@
 // Host-side BF16N encoder (C++17, std::thread).  Produces the byte layout of the reference encoder
 // (core/src/encode.cpp) for NIBBLE, HUFFMAN and HUFPAIR row-/chunk-major, and this build's wave64 stream layout.
 //
-// Structure: every format is written in two parallel passes straight into the final aux buffer — pass 1 sizes each
-// row / unit, a prefix sum places it, pass 2 writes it — so no per-unit buffers are kept and the passes scale over
-// all host cores.
+// Structure: the reference's formats are written in two parallel passes straight into the final aux buffer — pass 1 sizes
+// each row / unit, a prefix sum places it, pass 2 writes it — so no per-unit buffers are kept and the passes scale over
+// all host cores.  The wave64 stream, whose words are placed by a simulation of the decoder, is written in one pass into
+// buffers of eight units that are copied into place (encode_hufpair_w64).
 #include "encode_impl.h"
 
 #include <algorithm>
@@ -187,18 +188,55 @@ struct pair_code {
     std::vector<uint32_t> lut;  // [4096], entry = e_odd << 23 | e_even << 7 | len
 };
 
-// false: more than HP_MAX_PAIRS distinct pairs
-bool build_pair_code(const uint16_t * w, int64_t rows, int64_t K, pair_code & pc) {
+// four adjacent weights in one word: the two pair symbols (exponent of the first | exponent of the second << 8), and the
+// four sign|mantissa bytes
+inline uint64_t load4(const uint16_t * w) {
+    uint64_t v;
+    std::memcpy(&v, w, sizeof(v));
+    return v;
+}
+inline void syms_of4(uint64_t v, uint32_t & s0, uint32_t & s1) {
+    const uint64_t e = v >> 7 & 0x00FF00FF00FF00FFull, x = e | e >> 8;
+    s0 = (uint32_t) x & 0xFFFFu;
+    s1 = (uint32_t) (x >> 32) & 0xFFFFu;
+}
+inline uint32_t sm_of4(uint64_t v) {
+    uint64_t x = (v & 0x007F007F007F007Full) | (v >> 8 & 0x0080008000800080ull);
+    x = (x | x >> 8) & 0x0000FFFF0000FFFFull;
+    return (uint32_t) (x | x >> 16);
+}
+
+// the plane bytes of one 512-column chunk: byte 16 l + s = sign|mantissa of column pos_of(l, s) (encode.cpp:48-62)
+inline void write_chunk(const uint16_t * src, uint8_t * dst) {
+    for (int j = 0; j < 4; j++) {
+        for (int l = 0; l < 32; l++) {
+            const uint32_t b = sm_of4(load4(src + 128 * j + 4 * l));
+            std::memcpy(dst + 16 * l + 4 * j, &b, sizeof(b));
+        }
+    }
+}
+
+// false: more than HP_MAX_PAIRS distinct pairs.  plane (optional): the rows' plane bytes, chunk after chunk, written while
+// the rows are in the cache.
+bool build_pair_code(const uint16_t * w, int64_t rows, int64_t K, pair_code & pc, uint8_t * plane = nullptr) {
     std::vector<uint64_t> freq(65536, 0);
     {
         std::mutex mu;
-        // at most 64 blocks: every block zeroes and merges a 65536-entry histogram of its own (a block holds fewer
-        // than 2^32 pairs: rows * K < 2^37 / 64)
-        const int64_t per_block = std::max<int64_t>(256, (rows + 63) / 64);
+        // at most 32 blocks: every block zeroes and merges a 65536-entry histogram of its own (a block holds fewer
+        // than 2^32 pairs: rows * K < 2^37 / 32)
+        const int64_t per_block = std::max<int64_t>(256, (rows + 31) / 32);
         parallel_blocks(rows, per_block, [&](int64_t r0, int64_t r1) {
             std::vector<uint32_t> h(65536, 0);
-            for (int64_t i = r0 * K; i < r1 * K; i += 2) {
-                h[exp_of(w[i]) | exp_of(w[i + 1]) << 8]++;
+            for (int64_t i = r0 * K; i < r1 * K; i += CHUNK) {
+                for (int k = 0; k < CHUNK; k += 4) {
+                    uint32_t s0, s1;
+                    syms_of4(load4(w + i + k), s0, s1);
+                    h[s0]++;
+                    h[s1]++;
+                }
+                if (plane) {
+                    write_chunk(w + i, plane + i);
+                }
             }
             std::lock_guard<std::mutex> lk(mu);
             for (int s = 0; s < 65536; s++) {
@@ -248,22 +286,13 @@ void set_threads(int n) { g_threads.store(n); }
 
 // ---------------------------------------------------------------------------------------------- plane
 
-// byte 16*l + s of a chunk = sign|mantissa of column pos_of(l, s) (encode.cpp:48-62); chunk-major units keep chunk c
-// of unit row r at (c*R + r)*512 (encode.cpp:511-524)
+// row-major chunks; chunk-major units keep chunk c of unit row r at (c*R + r)*512 (encode.cpp:511-524)
 void write_plane(const uint16_t * w, int64_t rows, int64_t K, int R, bool cm, uint8_t * plane) {
     const int64_t C = K / CHUNK;
     parallel_blocks(rows, 64, [&](int64_t r0, int64_t r1) {
         for (int64_t r = r0; r < r1; r++) {
             for (int64_t c = 0; c < C; c++) {
-                const uint16_t * src = w + r * K + c * CHUNK;
-                uint8_t * dst = cm ? plane + (r / R) * R * K + (c * R + r % R) * CHUNK : plane + r * K + c * CHUNK;
-                for (int j = 0; j < 4; j++) {
-                    for (int l = 0; l < 32; l++) {
-                        const uint16_t * q = src + 128 * j + 4 * l;
-                        uint8_t * o = dst + 16 * l + 4 * j;
-                        o[0] = sm_of(q[0]); o[1] = sm_of(q[1]); o[2] = sm_of(q[2]); o[3] = sm_of(q[3]);
-                    }
-                }
+                write_chunk(w + r * K + c * CHUNK, cm ? plane + (r / R) * R * K + (c * R + r % R) * CHUNK : plane + r * K + c * CHUNK);
             }
         }
     });
@@ -556,51 +585,90 @@ bytes encode_hufpair(const uint16_t * w, int64_t rows, int64_t K, int R, bool cm
 // coalesced loads, and the lane of a refill word is its rank among the refilling lanes.  The table at off_a is
 // indexed by those 12 bits as they sit in the word (first code bit = index bit 0), i.e. the canonical table with
 // bit-reversed index.  unit_base has units + 1 entries (word index of each unit's first word and the end).
-bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, bool cm) {
+//
+// One walk over the weights writes the units' words block by block into memory of their own, and when every unit's size
+// is known the blocks are copied into place (sizing the units in a walk of its own took longer than the copy).  The codes
+// of the four weights of a check go into the lane's words as one, and neither a full word nor a refill is a branch: both
+// are taken a third of the time, unpredictably.  With the plane written in the walk that counts the pairs: 16384 x 2048 on
+// eight cores 58.5 -> 32.5 ms; a load of that matrix with upload and verification, on sixteen, 15.0 -> 11.5.
+bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, bool cm, uint8_t * plane) {
     pair_code pc;
-    if (!build_pair_code(w, rows, K, pc)) {
+    if (!build_pair_code(w, rows, K, pc, plane)) {
         return {};
     }
     const int64_t C = K / CHUNK, units = rows / R, steps = R * C / 2;
-    auto sym_at = [&](int64_t i) { return exp_of(w[i]) | exp_of(w[i + 1]) << 8; };
     // first element of the chunk that half-wave `half` decodes in step st of unit u
     auto chunk_base = [&](int64_t u, int64_t st, int half) {
         int rr; int64_t c;
         chunk_of(2 * st + half, R, C, cm, rr, c);
         return (u * R + rr) * K + c * CHUNK;
     };
-    // the two pairs of lane l at check t (pairs 2t, 2t+1) of a chunk
-    auto pair_syms = [&](int64_t base, int l, int t, int & s0, int & s1) {
-        s0 = sym_at(base + pos_of(l & 31, 4 * t));
-        s1 = sym_at(base + pos_of(l & 31, 4 * t + 2));
-    };
-    std::vector<uint16_t> rcode(65536, 0); // codes with their first bit lowest, as the stream holds them
+    std::vector<uint32_t> code(65536, 0); // code with its first bit lowest, as the stream holds it | length << 16
     for (int sidx = 0; sidx < 65536; sidx++) {
         if (pc.len[sidx]) {
-            rcode[sidx] = (uint16_t) bitrev(pc.code[sidx], pc.len[sidx]);
+            code[sidx] = bitrev(pc.code[sidx], pc.len[sidx]) | (uint32_t) pc.len[sidx] << 16;
         }
     }
-    // pass 1: words per unit = 192 + number of refills
     std::vector<uint64_t> ubase(units + 1, 0);
-    parallel_blocks(units, 8, [&](int64_t u0, int64_t u1) {
+    constexpr int64_t UNITS = 8; // per block
+    std::vector<std::vector<uint32_t, uninit_allocator<uint32_t>>> words((size_t) ((units + UNITS - 1) / UNITS));
+    // a lane takes at most 24 bits per pair of codes: steps * 4 * 24 bits and the two leading ones, + the zero words behind
+    const int64_t maxw = (steps * 4 * 24 + 2 + 31) / 32 + 5;
+    auto encode_block = [&](int64_t u0, int64_t u1, std::vector<uint32_t> & lane_words, std::vector<uint8_t> & order) {
+        auto & out = words[(size_t) (u0 / UNITS)];
         for (int64_t u = u0; u < u1; u++) {
-            uint32_t P[64] = {0};
-            uint64_t refills = 0;
+            uint64_t acc[64];
+            uint32_t nb[64], P[64];
+            uint32_t * at[64];
+            for (int l = 0; l < 64; l++) {
+                acc[l] = 0; nb[l] = 2; P[l] = 0; at[l] = lane_words.data() + l * maxw; // two leading zero bits
+            }
+            uint8_t * refill = order.data(); // the lane of every refill, in decoder order
             for (int64_t st = 0; st < steps; st++) {
-                const int64_t base[2] = {chunk_base(u, st, 0), chunk_base(u, st, 1)};
+                const uint16_t * const half[2] = {w + chunk_base(u, st, 0), w + chunk_base(u, st, 1)};
                 for (int t = 0; t < 4; t++) {
-                    for (int l = 0; l < 64; l++) {
-                        int s0, s1;
-                        pair_syms(base[l >> 5], l, t, s0, s1);
-                        P[l] += pc.len[s0] + pc.len[s1];
-                        if (P[l] >= 32) {
-                            P[l] -= 32;
-                            refills++;
-                        }
+                    for (int l = 0; l < 64; l++) { // (pos_of(l % 32, 4 t): four adjacent columns)
+                        uint32_t s0, s1;
+                        syms_of4(load4(half[l >> 5] + 128 * t + 4 * (l & 31)), s0, s1);
+                        const uint32_t c0 = code[s0], c1 = code[s1], len0 = c0 >> 16, len = len0 + (c1 >> 16);
+                        acc[l] |= (uint64_t) ((c0 & 0xFFFFu) | (c1 & 0xFFFFu) << len0) << nb[l];
+                        nb[l] += len;
+                        *at[l] = (uint32_t) acc[l]; // stays where it is once 32 bits are there
+                        const uint32_t full = nb[l] >> 5;
+                        at[l] += full;
+                        acc[l] >>= 32 * full;
+                        nb[l] &= 31;
+                        P[l] += len;
+                        *refill = (uint8_t) l;
+                        refill += P[l] >> 5;
+                        P[l] &= 31;
                     }
                 }
             }
-            ubase[u + 1] = 192 + refills;
+            const size_t n = 192 + (size_t) (refill - order.data()), first = out.size();
+            ubase[u + 1] = n;
+            out.resize(first + n);
+            uint32_t * o = out.data() + first;
+            for (int l = 0; l < 64; l++) {
+                *at[l]++ = (uint32_t) acc[l]; // partial last word, zero-filled
+                for (int z = 0; z < 4; z++) {
+                    *at[l]++ = 0;             // the words a lane requests past its last code
+                }
+                at[l] = lane_words.data() + l * maxw;
+                *o++ = *at[l]++;
+                *o++ = *at[l]++;
+                *o++ = *at[l]++;
+            }
+            for (const uint8_t * r = order.data(); r != refill; r++) {
+                *o++ = *at[*r]++;
+            }
+        }
+    };
+    parallel_blocks(units, UNITS, [&](int64_t u0, int64_t u1) {
+        std::vector<uint32_t> lane_words((size_t) (64 * maxw));
+        std::vector<uint8_t> order((size_t) (steps * 4 * 64 + 1));
+        for (int64_t u = u0; u < u1; u += UNITS) { // (one thread gets all units in one call)
+            encode_block(u, std::min(u1, u + UNITS), lane_words, order);
         }
     });
     for (int64_t u = 0; u < units; u++) {
@@ -618,7 +686,7 @@ bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, boo
     h.off_c = h.off_d;
     h.n_a = (uint64_t) units; h.n_b = n_words; h.flags = FLAG_WAVE64 | (cm ? FLAG_CHUNK_MAJOR : 0);
     // 1024 words of padding: a wave prefetches its stream in 1 KiB blocks and may run up to three blocks ahead
-    // not zeroed as a whole: pass 2 writes every stream word; zero what it does not write (header padding, the gap
+    // not zeroed as a whole: the copy writes every stream word; zero what it does not write (header padding, the gap
     // before the stream, the padding behind it)
     bytes aux(h.off_d + (n_words + 1024) * 4);
     std::memset(aux.data(), 0, h.off_d);
@@ -633,65 +701,9 @@ bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, boo
         unit_base[u] = (uint32_t) ubase[u];
     }
     uint32_t * stream = (uint32_t *) (aux.data() + h.off_d);
-    // pass 2: build each lane's words, then lay them out in the order the decoder takes them
-    // a lane takes at most 24 bits per pair of codes: steps * 4 * 24 bits and the two leading ones, + the zero words behind
-    const int64_t maxw = (steps * 4 * 24 + 2 + 31) / 32 + 5;
-    parallel_blocks(units, 8, [&](int64_t u0, int64_t u1) {
-        std::vector<uint32_t> lane_words((size_t) (64 * maxw));
-        std::vector<uint8_t> order; // lane of every refill, in decoder order
-        order.reserve((size_t) (steps * 4 * 64));
-        for (int64_t u = u0; u < u1; u++) {
-            order.clear();
-            uint64_t acc[64];
-            int nb[64], nw[64];
-            uint32_t P[64];
-            for (int l = 0; l < 64; l++) {
-                acc[l] = 0; nb[l] = 2; nw[l] = 0; P[l] = 0; // two leading zero bits
-            }
-            auto put = [&](int l, uint32_t code, int len) { // code: first bit lowest
-                acc[l] |= (uint64_t) code << nb[l];
-                nb[l] += len;
-                if (nb[l] >= 32) {
-                    lane_words[(size_t) (l * maxw + nw[l]++)] = (uint32_t) acc[l];
-                    acc[l] >>= 32;
-                    nb[l] -= 32;
-                }
-            };
-            for (int64_t st = 0; st < steps; st++) {
-                const int64_t base[2] = {chunk_base(u, st, 0), chunk_base(u, st, 1)};
-                for (int t = 0; t < 4; t++) {
-                    for (int l = 0; l < 64; l++) {
-                        int s0, s1;
-                        pair_syms(base[l >> 5], l, t, s0, s1);
-                        put(l, rcode[s0], pc.len[s0]);
-                        put(l, rcode[s1], pc.len[s1]);
-                        P[l] += pc.len[s0] + pc.len[s1];
-                        if (P[l] >= 32) {
-                            P[l] -= 32;
-                            order.push_back((uint8_t) l);
-                        }
-                    }
-                }
-            }
-            uint32_t taken[64];
-            uint32_t * out = stream + ubase[u];
-            for (int l = 0; l < 64; l++) {
-                uint32_t * lw = lane_words.data() + l * maxw;
-                lw[nw[l]++] = (uint32_t) acc[l]; // partial last word, zero-filled
-                for (int z = 0; z < 4; z++) {
-                    lw[nw[l]++] = 0;             // the words a lane requests past its last code
-                }
-                *out++ = lw[0];
-                *out++ = lw[1];
-                *out++ = lw[2];
-                taken[l] = 3;
-            }
-            for (uint8_t l : order) {
-                *out++ = lane_words[(size_t) (l * maxw + taken[l]++)];
-            }
-            if ((uint64_t) (out - stream) != ubase[u + 1]) {
-                invariant("wave64 unit size");
-            }
+    parallel_blocks((int64_t) words.size(), 8, [&](int64_t b0, int64_t b1) {
+        for (int64_t b = b0; b < b1; b++) {
+            std::memcpy(stream + ubase[b * UNITS], words[(size_t) b].data(), words[(size_t) b].size() * 4);
         }
     });
     return aux;
@@ -733,7 +745,7 @@ bool encode_tile32(const uint16_t * w, int64_t rows, int64_t K, encoded_buffers 
             }
         }
     });
-    out.aux = encode_hufpair_w64(v, vrows, CHUNK, 16, false);
+    out.aux = encode_hufpair_w64(v, vrows, CHUNK, 16, false, out.plane.data());
     if (out.aux.empty()) {
         return false;
     }
@@ -741,7 +753,6 @@ bool encode_tile32(const uint16_t * w, int64_t rows, int64_t K, encoded_buffers 
     std::memcpy(&h, out.aux.data(), sizeof(h));
     h.K = (uint32_t) K; h.R = TILE_R; h.rows = (uint64_t) rows;
     std::memcpy(out.aux.data(), &h, sizeof(h));
-    write_plane(v, vrows, CHUNK, 16, false, out.plane.data());
     out.format = FMT_HUFPAIR;
     out.R = TILE_R;
     return true;
@@ -812,11 +823,13 @@ encoded_buffers encode(const uint16_t * w, int64_t rows, int64_t K, int format, 
         R = 16; // more than 4096 distinct pairs: single-symbol fallback below, which has no special layouts
         out.R = R;
     } else if (format == FMT_HUFPAIR) {
-        out.aux = w64 ? encode_hufpair_w64(w, rows, K, R, cm) : encode_hufpair(w, rows, K, R, cm);
+        out.aux = w64 ? encode_hufpair_w64(w, rows, K, R, cm, out.plane.data()) : encode_hufpair(w, rows, K, R, cm);
     }
     if (!out.aux.empty()) {
         out.format = FMT_HUFPAIR;
-        write_plane(w, rows, K, R, cm, out.plane.data());
+        if (!w64) { // (that encoder has written it)
+            write_plane(w, rows, K, R, cm, out.plane.data());
+        }
     } else { // too many distinct pairs (or HUFFMAN requested): the single-symbol format has no special layouts
         out.aux = encode_huffman(w, rows, K, R);
         out.format = FMT_HUFFMAN;
