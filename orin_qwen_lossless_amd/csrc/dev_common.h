@@ -10,6 +10,8 @@
 namespace bf16n {
 namespace dev {
 
+constexpr size_t LDS_BYTES = 160 * 1024; // of a CU
+
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 struct bf16_t { uint16_t bits; }; // activation / output element type tag for BF16

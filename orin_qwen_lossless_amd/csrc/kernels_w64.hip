@@ -285,6 +285,140 @@ __global__ void __launch_bounds__(wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2
     }
 }
 
+// Several BF16 columns of 2048 or 4096 with the activations in LDS (C = 4, 8: a loop body is a row).  In registers
+// (k_w64_mmv) four columns of 2048 take 64 per lane, which leaves room for one chain per wavefront, and more columns for
+// fewer wavefronts too; the launch then waits for the chains' lookups.  Here an instance takes 49 to 107 registers at any
+// column count: two chains per wavefront (NCH), which are at the same columns, so that one read of the activations (uint2
+// per lane, column and plane word) serves both.  What bounds it is the vector ALU: a column adds eight products and three
+// and a half steps of a reduction to the 86 instructions of a step.  us, before and after:
+//   248320 x 2048, 2 / 3 / 4 / 5 / 6 / 7 / 8 columns: 131 / 141 / 151 / 208 / 224 / 238 / 303 -> 123 / 135 / 145 / 157 / 171 / 183 / 197
+//   131072 x 4096, 1 / 2 / 4 / 6 / 7: 120 / 164 / 188 / 353 / 366 -> 116 / 122 / 143 / 162 / 193 (eight columns of 4096 are one pass now)
+//   one unit per wavefront: 65536 x 2048, 5 / 8: 67 / 81 -> 50 / 63; 65536 x 4096, 2 / 4 / 5 / 8: 90 / 99 / 171 / 197 -> 73 / 83 / 89 / 112
+// Shorter rows stay with registers (131072 x 512 and 131072 x 1024, 2 to 8 columns: within 2.5 % either way).  Every column
+// gets the bits of its single-column launch: the same products in the same order.
+typedef uint32_t uint2_v __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(3))) uint2_v * lds_u2;
+template <int C, int NC> constexpr size_t xl_bytes() { return (size_t) geom<C>::XS * NC * 4 * 64 * sizeof(uint2); }
+
+template <int C, int NC, int N, int HINT>
+__device__ __forceinline__ void unit_pass_lds(chain<geom<C>::NB, HINT> (&ch)[2], const uint32_t * lut, lds_u2 xl, const cols & p,
+                                              const col_view & cv, int R, int lane) {
+    using G = geom<C>;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        ch[k].dec.keep_ahead();
+        ch[k].dec.begin_unit();
+        ch[k].dec.keep_ahead();
+    }
+    const int bodies = R * C / 2 / G::NB;
+    for (int b = 0; b < bodies; b++) {
+        switch (b & 3) { // issue priority by progress, as in unit_pass
+            case 0: __builtin_amdgcn_s_setprio(3); break;
+            case 1: __builtin_amdgcn_s_setprio(2); break;
+            case 2: __builtin_amdgcn_s_setprio(1); break;
+            default: __builtin_amdgcn_s_setprio(0); break;
+        }
+        float acc[N][NC];
+#pragma unroll
+        for (int s = 0; s < G::NB; s++) {
+            uint32_t smw[N][4];
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                smw[k][0] = ch[k].sm[s].x; smw[k][1] = ch[k].sm[s].y; smw[k][2] = ch[k].sm[s].z; smw[k][3] = ch[k].sm[s].w;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                // (the address is opaque per word: the compiler would otherwise keep the activations in registers after all)
+                asm volatile("" : "+v"(xl));
+                uint2_v xv[NC];
+#pragma unroll
+                for (int n = 0; n < NC; n++) {
+                    xv[n] = xl[((s * NC + n) * 4 + j) * 64];
+                }
+                uint32_t w0[N], w1[N];
+#pragma unroll
+                for (int k = 0; k < N; k++) {
+                    uint32_t e0, e1;
+                    ch[k].dec.two(lut, e0, e1);
+                    w0[k] = merge(spread_lo(smw[k][j]), e0);
+                    w1[k] = merge(spread_hi(smw[k][j]), e1);
+                }
+#pragma unroll
+                for (int n = 0; n < NC; n++) {
+#pragma unroll
+                    for (int k = 0; k < N; k++) {
+                        acc[k][n] = dot2_bf16(w1[k], xv[n].y, dot2_bf16(w0[k], xv[n].x, s == 0 && j == 0 ? 0.f : acc[k][n]));
+                        // (pinned here: left alone the products of all words sink to the row's end, with their operands)
+                        asm volatile("" : "+v"(acc[k][n]));
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                ch[k].dec.keep_ahead();
+            }
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                ch[k].reload(s, lane);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+#pragma unroll
+            for (int n = 0; n < NC; n++) {
+                const float v = wave_sum_dpp(acc[k][n]);
+                if (lane == 63) {
+                    store_y(cv.y + n * p.y_tok, p.y_bf16, ch[k].row, v);
+                }
+            }
+            ch[k].row += G::ROWS;
+        }
+    }
+}
+
+template <int C, int NC, int NCH, int HINT>
+__global__ void __launch_bounds__(1024) k_w64_mmv_lds(const bf16n_weight w, const cols p, int units_per_wave) {
+    using G = geom<C>;
+    constexpr int K = C * CHUNK;
+    __shared__ __align__(16) uint32_t lut[LUT_WORDS];   // static: sits at LDS address 0
+    extern __shared__ __align__(16) uint32_t dyn[];     // activations [set][column][plane word][lane], then two rings per wave
+    const w64_ptrs q = w64p(w);
+    const int lane = threadIdx.x & 63, wave = (int) uniform(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
+    const int R = w.R;
+    const col_view cv = col_setup(p, 0);
+    const int64_t units = p.nrows / R;
+    const int64_t u_begin = ((int64_t) blockIdx.x * nwaves + wave) * units_per_wave;
+    const bool live = u_begin < units;
+    const int64_t u_end = u_begin + units_per_wave < units ? u_begin + units_per_wave : units;
+    const int64_t n = live ? u_end - u_begin : 0, nA = NCH == 2 ? (n + 1) / 2 : n, nB = n - nA;
+    const int64_t gu0 = cv.rbase / R + (live ? u_begin : 0);
+    const uint32_t b0 = q.ubase[gu0], b1 = q.ubase[gu0 + nA], b2 = q.ubase[gu0 + n];
+    stage_lut(lut, q.lut);
+    for (int i = wave; i < G::XS * NC * 4; i += nwaves) { // (set, column, plane word) i of every lane
+        const int j = i & 3, c = (i >> 2) % NC, set = (i >> 2) / NC;
+        const int col0 = (2 * set + (lane >> 5)) * CHUNK + 128 * j + 4 * (lane & 31);
+        ((uint2 *) dyn)[i * 64 + lane] = *(const uint2 *) (cv.x + c * p.x_tok + 2 * col0);
+    }
+    __syncthreads();
+    if (!live) {
+        return;
+    }
+    const lds_u2 xl = (lds_u2) dyn + lane;
+    chain<G::NB, HINT> ch[2];
+    uint32_t * ring = dyn + xl_bytes<C, NC>() / 4 + wave * (NCH * WAVE_LDS_WORDS);
+    ch[0].start(ring, q, gu0, nA, u_begin * R, R, K, lane, b0, b1);
+    if (NCH == 2 && nB > 0) {
+        ch[1].start(ring + WAVE_LDS_WORDS, q, gu0 + nA, nB, (u_begin + nA) * R, R, K, lane, b1, b2);
+    }
+    for (int64_t i = 0; i < nA; i++) {
+        if (NCH == 2 && i < nB) {
+            unit_pass_lds<C, NC, 2, HINT>(ch, lut, xl, p, cv, R, lane);
+        } else {
+            unit_pass_lds<C, NC, 1, HINT>(ch, lut, xl, p, cv, R, lane);
+        }
+    }
+}
+
 // Fused gate / up + SwiGLU for two matrices of the same shape and unit size: every wave decodes its units of both
 // matrices side by side (the two chains) and writes silu(gate x) * (up x).
 template <typename TX, int C>
@@ -498,6 +632,51 @@ constexpr int max_group() {
 template <typename TX, int C, int NC>
 constexpr bool two_chains() { return x_regs<TX, C, NC>() <= 16; }
 
+// Instances with the activations in LDS (the figures stand at k_w64_mmv_lds).  Two chains per wavefront where the form with
+// registers has one (from two units per wavefront on); one chain where that form has registers for fewer than sixteen
+// wavefronts per CU (with sixteen of them either way the two measure the same: 65536 x 2048, 3 / 4 columns 46 us).
+template <int C, int NC, int NCH> constexpr bool lds_columns() {
+    return NCH == 2 ? C >= 4 && !two_chains<bf16_t, C, NC>() : wide_regs(x_regs<bf16_t, C, NC>(), true, C);
+}
+template <int C, int NC, int NCH> constexpr size_t lds_shm(int wpb) { return xl_bytes<C, NC>() + (size_t) wpb * NCH * WAVE_LDS_WORDS * 4; }
+// wavefronts per block: eight, two blocks to a CU, where two copies of the activations fit beside the rings
+template <int C, int NC, int NCH> constexpr int lds_wpb() { return 2 * (lds_shm<C, NC, NCH>(8) + LUT_WORDS * 4) <= LDS_BYTES ? 8 : 16; }
+// f(NC as a type) for the instance of nc columns; false: there is none
+template <int C, int NCH, int NC = 1, typename F> bool with_lds(int nc, F f) {
+    if constexpr (NC <= 8) {
+        if (nc != NC) {
+            return with_lds<C, NCH, NC + 1>(nc, f);
+        }
+        if constexpr (lds_columns<C, NC, NCH>() && lds_shm<C, NC, NCH>(16) + LUT_WORDS * 4 <= LDS_BYTES) {
+            f(std::integral_constant<int, NC>{});
+            return true;
+        }
+    }
+    return false;
+}
+template <int C, int NCH> bool mmv_lds_launch(int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
+    return with_lds<C, NCH>(nc, [&](auto n) {
+        constexpr int NC = decltype(n)::value, wpb = lds_wpb<C, NC, NCH>();
+        const dim3 grid((unsigned) ((waves + wpb - 1) / wpb));
+        note_kernel("k_w64_mmv_lds", nullptr, 4, C, NC, NCH, (int) p.plane_once);
+        if (p.plane_once) hipLaunchKernelGGL((k_w64_mmv_lds<C, NC, NCH, 1>), grid, dim3(wpb * 64), (lds_shm<C, NC, NCH>(wpb)), stream, w, p, upw);
+        else              hipLaunchKernelGGL((k_w64_mmv_lds<C, NC, NCH, 0>), grid, dim3(wpb * 64), (lds_shm<C, NC, NCH>(wpb)), stream, w, p, upw);
+    });
+}
+template <int NCH> bool mmv_lds(int C, int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
+    return C == 4 ? mmv_lds_launch<4, NCH>(nc, waves, upw, stream, w, p) : C == 8 && mmv_lds_launch<8, NCH>(nc, waves, upw, stream, w, p);
+}
+template <int C, int NCH> void set_attr_lds() {
+    for (int nc = 1; nc <= 8; nc++) {
+        with_lds<C, NCH>(nc, [](auto n) {
+            constexpr int NC = decltype(n)::value;
+            const int shm = (int) lds_shm<C, NC, NCH>(lds_wpb<C, NC, NCH>());
+            (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<C, NC, NCH, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+            (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<C, NC, NCH, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        });
+    }
+}
+
 // the load policy of plane and stream as a compile-time choice of the instance
 template <typename TX, int C, int NC, int HINT>
 void mmv_launch_hint(dim3 grid, int nt, int wpb, hipStream_t stream, const bf16n_weight & w, const cols & p, int upw) {
@@ -593,6 +772,8 @@ void w64_init() {
     set_attr_c<float>();
     set_attr_glu<bf16_t>();
     set_attr_glu<float>();
+    set_attr_lds<4, 2>(); set_attr_lds<8, 2>();
+    set_attr_lds<4, 1>(); set_attr_lds<8, 1>();
 }
 
 // shapes with a fused wave64 GEMV: K in {512, 1024, 2048, 4096} and units that hold whole loop bodies
@@ -609,7 +790,7 @@ void launch_w64_mmv(const bf16n_weight & w, const cols & p, int ncols, bool x_bf
     const int C = (int) (w.K / CHUNK);
     const int64_t units = p.nrows / w.R;
     // dense batches: groups of columns share one decode (max_group)
-    const int group_max = !multi_col || p.ids ? 1 : x_bf16 ? group_for<bf16_t>(C) : group_for<float>(C);
+    const int group_max = !multi_col || p.ids ? 1 : x_bf16 ? C == 8 ? 8 : group_for<bf16_t>(C) : group_for<float>(C);
     for (int c0 = 0; c0 < (group_max == 1 ? 1 : ncols); c0 += group_max) {
         const int nc = group_max == 1 ? 1 : (ncols - c0 < group_max ? ncols - c0 : group_max);
         const int ny = group_max == 1 ? ncols : 1;
@@ -626,6 +807,14 @@ void launch_w64_mmv(const bf16n_weight & w, const cols & p, int ncols, bool x_bf
             q.y += c0 * p.y_tok;
         }
         int wpb, blocks, upw;
+        if (x_bf16 && group_max > 1) {
+            w64_dims(units, ny, cus, wpb, blocks, upw);
+            const int waves = (int) ((units + upw - 1) / upw);
+            // (K = 4096: the rings of seven or eight columns leave room for one chain per wavefront)
+            if ((upw >= 2 && mmv_lds<2>(C, nc, waves, upw, stream, w, q)) || mmv_lds<1>(C, nc, waves, upw, stream, w, q)) {
+                continue;
+            }
+        }
         // wavefronts per CU the instance is sized for, by its activation registers (x_regs): 16 up to 64 registers,
         // then three per SIMD in blocks of four, two per SIMD beyond 112
         const int xr = nc * (C >= 2 ? C / 2 : 1) * (x_bf16 ? 8 : 16);
