@@ -7,6 +7,7 @@ torch is used for device memory and streams only; every product runs in libbf16n
 explicitly as plane + aux uint8 tensors with metadata parsed once from the aux header on the host."""
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import struct
 from dataclasses import dataclass
@@ -60,10 +61,7 @@ class Meta:
 
     @property
     def flags(self) -> int:
-        bits = 0
-        for on, bit in ((self.chunk_major, FLAG_CHUNK_MAJOR), (self.frag_order, FLAG_FRAG_ORDER), (self.wave64, FLAG_WAVE64)):
-            bits |= bit if on else 0
-        return bits
+        return (FLAG_CHUNK_MAJOR if self.chunk_major else 0) | (FLAG_FRAG_ORDER if self.frag_order else 0) | (FLAG_WAVE64 if self.wave64 else 0)
 
     def as_list(self) -> list[int]:
         """The nine integers of the torch.ops.bf16n `meta` argument: format, K, rows, R, flags, off_a .. off_d."""
@@ -109,26 +107,38 @@ class Weight:
         return int(self.plane.numel()) + int(self.aux.numel())
 
 
-def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+# A small product is bound by the host's call (512 x 2048, one token: 14.9 us with torch's Python-level device guard and
+# stream objects and a view in and out, 9.3 without; the kernel takes 3.2), so the calls below stay off both when the
+# tensor's device is the current one anyway.
+_HERE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """A guard that makes `device` current."""
+    return _HERE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+
+
+def _stream() -> int:
+    """The current stream of the current device."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _cweight(w: Weight) -> _lib.Weight:
-    m = w.meta
-    if not (w.plane.is_cuda and w.aux.is_cuda):
+    m, plane, aux = w.meta, w.plane, w.aux
+    if not (plane.is_cuda and aux.is_cuda):
         raise ValueError("bf16n: plane and aux must be device tensors")
-    if w.plane.dtype != torch.uint8 or w.aux.dtype != torch.uint8:
+    if plane.dtype is not torch.uint8 or aux.dtype is not torch.uint8:
         raise ValueError("bf16n: plane and aux must be uint8")
-    if not (w.plane.is_contiguous() and w.aux.is_contiguous()):
+    if not (plane.is_contiguous() and aux.is_contiguous()):
         raise ValueError("bf16n: plane and aux must be contiguous")
-    if w.plane.numel() != m.rows * m.K:
-        raise ValueError(f"bf16n: plane has {w.plane.numel()} bytes, meta says {m.rows} x {m.K}")
-    if max(m.off_a, m.off_b, m.off_c, m.off_d) >= w.aux.numel():
-        raise ValueError(f"bf16n: aux ({w.aux.numel()} bytes) shorter than its offsets")
-    if w.plane.data_ptr() % 16 or w.aux.data_ptr() % 16:
+    n_aux, plane_at, aux_at = aux.numel(), plane.data_ptr(), aux.data_ptr()
+    if plane.numel() != m.rows * m.K:
+        raise ValueError(f"bf16n: plane has {plane.numel()} bytes, meta says {m.rows} x {m.K}")
+    if max(m.off_a, m.off_b, m.off_c, m.off_d) >= n_aux:
+        raise ValueError(f"bf16n: aux ({n_aux} bytes) shorter than its offsets")
+    if plane_at % 16 or aux_at % 16:
         raise ValueError("bf16n: plane/aux must be 16-byte aligned")
-    return _lib.Weight(w.plane.data_ptr(), w.aux.data_ptr(), m.format, m.R, m.K, m.rows, m.flags, 0, m.off_a, m.off_b,
-                       m.off_c, m.off_d)
+    return _lib.Weight(plane_at, aux_at, m.format, m.R, m.K, m.rows, m.flags, 0, m.off_a, m.off_b, m.off_c, m.off_d)
 
 
 def _check_x(x: torch.Tensor, K: int, what: str) -> None:
@@ -243,7 +253,7 @@ def dequant(w: Weight, row0: int = 0, nrows: int | None = None) -> torch.Tensor:
     if row0 < 0 or nrows < 0 or row0 + nrows > w.meta.rows:
         raise ValueError("bf16n.dequant: rows out of range")
     out = torch.empty((nrows, w.meta.K), dtype=torch.bfloat16, device=w.plane.device)
-    with torch.cuda.device(w.plane.device):
+    with _on(w.plane.device):
         _lib.check(_lib.lib().bf16n_dequant(C.byref(cw), row0, nrows, out.data_ptr(), _stream()))
     return out
 
@@ -280,13 +290,9 @@ def _mmv_common(x: torch.Tensor, w: Weight, ids: torch.Tensor | None, rows_per_m
     cu = _cweight(up) if up is not None else None
     K, rows = w.meta.K, w.meta.rows
     _check_x(x, K, "x")
-    a = _lib.MmvArgs()
-    a.x = x.data_ptr()
-    a.x_bf16 = int(x.dtype == torch.bfloat16)
-    a.y_bf16 = int(out_bf16)
+    x_bf16 = x.dtype is torch.bfloat16
     odt = torch.bfloat16 if out_bf16 else torch.float32
     osz = 2 if out_bf16 else 4
-    a.n_used, a.x_per_slot = 1, 1
     if ids is None:
         if x.dim() != 2:
             raise ValueError("bf16n.mmv: dense x must be [tokens, K]")
@@ -300,12 +306,8 @@ def _mmv_common(x: torch.Tensor, w: Weight, ids: torch.Tensor | None, rows_per_m
         y = torch.empty((T, n_out), dtype=odt, device=x.device)
         if T == 0:
             return y
-        a.y = y.data_ptr()
-        a.ncols = T
-        a.x_tok = x.stride(0) * x.element_size()
-        a.y_tok = n_out * osz
-        a.rows_per_matrix = rpm
-        a.nrows = n_out
+        a = _lib.MmvArgs(x.data_ptr(), y.data_ptr(), None, x.stride(0) * (2 if x_bf16 else 4), n_out * osz, 0, 0, 0, 0, rpm, 0, n_out, T, 1, 1,
+                         x_bf16, out_bf16)
     else:
         _check_ids(ids)
         if ids.device != w.plane.device:
@@ -321,7 +323,7 @@ def _mmv_common(x: torch.Tensor, w: Weight, ids: torch.Tensor | None, rows_per_m
         y = torch.empty((T, n_used, n_out), dtype=odt, device=x.device)
         if T == 0 or n_used == 0:
             return y
-        a.y = y.data_ptr()
+        a = _lib.MmvArgs(x=x.data_ptr(), y=y.data_ptr(), x_bf16=x_bf16, y_bf16=out_bf16)
         a.ncols = T * n_used
         a.ids = ids.data_ptr()
         a.ids_s0 = ids.element_size()
@@ -335,7 +337,7 @@ def _mmv_common(x: torch.Tensor, w: Weight, ids: torch.Tensor | None, rows_per_m
         a.rows_per_matrix = rows_per_matrix
         a.nrows = n_out
     L = _lib.lib()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         if topk is not None:
             logits, k, renorm, wts = topk
             _lib.check(L.bf16n_mmv_glu2_topk(C.byref(cw), C.byref(cu), C.byref(a), logits.data_ptr(), logits.stride(0), logits.shape[1],
@@ -415,8 +417,7 @@ def linear(x: torch.Tensor, w: Weight, bias: torch.Tensor | None = None) -> torc
     K, rows = w.meta.K, w.meta.rows
     if x.shape[-1] != K:
         raise ValueError(f"bf16n.linear: x last dim must be K = {K}")
-    oshape = list(x.shape[:-1]) + [rows]
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     T = x2.shape[0]
     if T <= GEMV_MAX_TOKENS or T <= gemv_max_tokens(w):
         ok = x2.stride(1) == 1 and (x2.stride(0) * 2) % 16 == 0 and x2.data_ptr() % 16 == 0
@@ -441,7 +442,7 @@ def linear(x: torch.Tensor, w: Weight, bias: torch.Tensor | None = None) -> torc
                     torch.mm(x2, wc.t(), out=ys)
                 else:
                     torch.addmm(bias.narrow(0, r0, nr), x2, wc.t(), out=ys)
-    return y.view(oshape)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], rows)
 
 
 def linear_dense(x: torch.Tensor, w: Weight, scratch: torch.Tensor | None = None, gemm_workspace: torch.Tensor | None = None
@@ -464,7 +465,7 @@ def linear_dense(x: torch.Tensor, w: Weight, scratch: torch.Tensor | None = None
     y = torch.empty((T, w.meta.rows), dtype=torch.bfloat16, device=x.device)
     if T == 0:
         return y
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.check(L.bf16n_linear_dense(C.byref(cw), x.data_ptr(), x.stride(0), T, y.data_ptr(), y.stride(0), scratch.data_ptr(),
                                         scratch.numel(), gemm_workspace.data_ptr(), gemm_workspace.numel(), _stream()))
     return y
@@ -478,7 +479,7 @@ def get_rows(ids: torch.Tensor, w: Weight, out_dtype: torch.dtype = torch.bfloat
         raise ValueError("bf16n.get_rows: ids must be int32 or int64")
     n = ids.shape[0]
     out = torch.empty((n, w.meta.K), dtype=out_dtype, device=w.plane.device)
-    with torch.cuda.device(w.plane.device):
+    with _on(w.plane.device):
         _lib.check(_lib.lib().bf16n_get_rows(C.byref(cw), ids.data_ptr(), ids.stride(0) * ids.element_size(), n,
                                              out.data_ptr(), int(out_dtype == torch.bfloat16),
                                              w.meta.K * out.element_size(), _stream(), row0))
@@ -506,7 +507,7 @@ def mm_ids_route(topk_ids: torch.Tensor, n_experts: int, per_slot: bool):
     dst = torch.empty(T * n_used, dtype=torch.int32, device=dev)
     bounds = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
     nch = n_used if per_slot else 1
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(_lib.lib().bf16n_mm_ids_route(topk_ids.data_ptr(), int(topk_ids.dtype == torch.int64), topk_ids.stride(0),
                                                  src1.data_ptr(), dst.data_ptr(), bounds.data_ptr(), n_experts, T, n_used,
                                                  nch, nch, _stream()))
@@ -564,12 +565,12 @@ def moe_mm_ids(x: torch.Tensor, topk_ids: torch.Tensor, w: Weight, n_experts: in
     tiles = w.meta.wave64 and w.meta.R == 32 and w.meta.format == FMT_HUFPAIR and (up is None or (up.meta.wave64 and up.meta.R == 32))
     if tiles and T * n_used >= MM_IDS_TWO_PHASE_PAIRS_PER_EXPERT * n_experts:
         buf = scratch if scratch is not None else mm_ids_scratch(w, up, n_experts)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             _lib.check(L.bf16n_mm_ids_scratch(C.byref(cw), C.byref(cu) if cu is not None else None, x.data_ptr(), w.meta.K,
                                               src1.data_ptr(), dst.data_ptr(), bounds.data_ptr(), y.data_ptr(),
                                               int(out_dtype == torch.bfloat16), N, n_experts, buf.data_ptr(), buf.numel(), _stream()))
         return y
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.check(L.bf16n_mm_ids(C.byref(cw), C.byref(cu) if cu is not None else None, x.data_ptr(), w.meta.K,
                                   src1.data_ptr(), dst.data_ptr(), bounds.data_ptr(), y.data_ptr(),
                                   int(out_dtype == torch.bfloat16), N, n_experts, T, n_used, _stream()))
@@ -586,7 +587,7 @@ def moe_combine(ys: torch.Tensor, topk_weights: torch.Tensor, out_dtype: torch.d
     if tuple(topk_weights.shape) != (T, n_used):
         raise ValueError("bf16n.moe_combine: shape mismatch")
     y = torch.empty((T, N), dtype=out_dtype, device=ys.device)
-    with torch.cuda.device(ys.device):
+    with _on(ys.device):
         _lib.check(_lib.lib().bf16n_moe_combine(ys.data_ptr(), topk_weights.data_ptr(), int(topk_weights.dtype == torch.bfloat16),
                                                 y.data_ptr(), int(out_dtype == torch.bfloat16), T, n_used, N, _stream()))
     return y
@@ -615,7 +616,7 @@ def add_rmsnorm(a: torch.Tensor, b: torch.Tensor | None = None, c: torch.Tensor 
     y = torch.empty_like(a)
     ysum = torch.empty_like(a) if want_sum else None
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
-    with torch.cuda.device(a.device):
+    with _on(a.device):
         _lib.check(_lib.lib().bf16n_add_rmsnorm(
             a.data_ptr(), ptr(b), ptr(c), ptr(ys), ptr(topk_weights) if ys is not None else None,
             int(ys is not None and topk_weights.dtype == torch.bfloat16), n_used, ptr(gamma), ptr(ysum), y.data_ptr(), T, n,
@@ -628,7 +629,7 @@ def swiglu(g: torch.Tensor, u: torch.Tensor) -> torch.Tensor:
             and u.dtype == torch.float32 and u.is_contiguous()):
         raise ValueError("bf16n.swiglu: g and u must be contiguous f32 of one shape")
     y = torch.empty_like(g)
-    with torch.cuda.device(g.device):
+    with _on(g.device):
         _lib.check(_lib.lib().bf16n_swiglu(g.data_ptr(), u.data_ptr(), y.data_ptr(), g.numel(), _stream()))
     return y
 
@@ -650,7 +651,7 @@ def router_topk(logits: torch.Tensor, k: int, renorm: bool = True, out: tuple[to
                 and wts.shape[0] == T and wts.shape[1] >= k and wts.is_contiguous() and ids.is_contiguous()
                 and wts.device == logits.device and ids.device == logits.device):
             raise ValueError("bf16n.router_topk: out must be contiguous (f32, int32) [tokens, m >= k] tensors on the logits' device")
-    with torch.cuda.device(logits.device):
+    with _on(logits.device):
         _lib.check(_lib.lib().bf16n_router_topk_strided(logits.data_ptr(), logits.stride(0), T, E, k, int(renorm), ids.data_ptr(),
                                                         wts.data_ptr(), ids.shape[1], _stream()))
     return wts, ids
@@ -688,7 +689,7 @@ def router_topk_routes(logits: torch.Tensor, k: int, n_listed: int, renorm: bool
     src1 = torch.empty(T * n_slots, dtype=torch.int32, device=dev)
     dst = torch.empty(T * n_slots, dtype=torch.int32, device=dev)
     bounds = torch.empty(n_listed + 1, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(L.bf16n_router_topk_route(logits.data_ptr(), logits.stride(0), T, logits.shape[1], k, int(renorm), ids.data_ptr(),
                                              wts.data_ptr(), n_slots, n_slots, n_listed, src1.data_ptr(), dst.data_ptr(),
                                              bounds.data_ptr(), 1, 1, _stream()))
