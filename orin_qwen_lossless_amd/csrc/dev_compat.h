@@ -86,25 +86,44 @@ __device__ __forceinline__ void decode_chunk(lane_bits & bits, const uint32_t * 
 
 // ---------------------------------------------------------------- NIBBLE (shared by the GEMV / dequant kernels and the batched kernels)
 
-// 4 exponents of 4 adjacent columns from 4 nibble codes (16 bits) and the row's 16-byte table, as bytes e0..e3
-__device__ __forceinline__ uint32_t nib_lookup4(const uint4 T, uint32_t codes16) {
-    uint32_t s = (codes16 | (codes16 << 8)) & 0x00FF00FFu;
-    s = (s | (s << 4)) & 0x0F0F0F0Fu; // one code per byte
-    const uint32_t lo = __builtin_amdgcn_perm(T.y, T.x, s & 0x07070707u);
-    const uint32_t hi = __builtin_amdgcn_perm(T.w, T.z, s & 0x07070707u);
-    const uint32_t pick_hi = ((s >> 3) & 0x01010101u) * 0xFFu;
-    return (hi & pick_hi) | (lo & ~pick_hi);
+// The exponents of 8 adjacent columns from their 8 nibble codes and the row's 16-byte table: even has those of columns
+// 0, 2, 4, 6 as bytes, odd those of columns 1, 3, 5, 7.  The even and the odd nibbles of the word are selectors of a byte
+// permute as they stand (masked to the 8 bytes of half a table); bit 3 of a code picks between the two halves' answers
+// in a third permute.  13 instructions for 8 codes.
+__device__ __forceinline__ uint32_t nib_pick4(const uint4 T, uint32_t c, uint32_t c_shr1) {
+    const uint32_t s = c & 0x07070707u;
+    const uint32_t lo = __builtin_amdgcn_perm(T.y, T.x, s), hi = __builtin_amdgcn_perm(T.w, T.z, s);
+    return __builtin_amdgcn_perm(hi, lo, (c_shr1 & 0x04040404u) | 0x03020100u);
+}
+__device__ __forceinline__ void nib_lookup8(const uint4 T, uint32_t codes, uint32_t & even, uint32_t & odd) {
+    even = nib_pick4(T, codes, codes >> 1);
+    odd = nib_pick4(T, codes >> 4, codes >> 5);
 }
 
-// the 16 weights of one lane in one NIBBLE chunk
+// a row's table with every byte rotated right by one: bit 7 of a byte is the exponent's lowest bit
+__device__ __forceinline__ uint32_t nib_rotate4(uint32_t t) { return ((t >> 1) & 0x7F7F7F7Fu) | ((t << 7) & 0x80808080u); }
+__device__ __forceinline__ uint4 nib_rotated(const uint4 T) {
+    return make_uint4(nib_rotate4(T.x), nib_rotate4(T.y), nib_rotate4(T.z), nib_rotate4(T.w));
+}
+
+// the 16 weights of one lane in one NIBBLE chunk.  ROT: T is the row's rotated table: an exponent duplicated into both
+// bytes of its half then has every bit where merge() wants it, which saves the shift of each pair; for rows of which a
+// lane decodes several chunks (rotating the table costs as much as one and a half chunks save).  50 instructions (58
+// without ROT) where a shift, a widening and a multiply per four codes took 84; by itself that moved no launch by more
+// than 0.5 % (they wait for their loads).
+template <bool ROT = false>
 __device__ __forceinline__ void nib_chunk(const uint4 sm, const uint2 cd, const uint4 T, uint32_t (&wp)[8]) {
-    const uint32_t smw[4] = {sm.x, sm.y, sm.z, sm.w};
+    const uint32_t smw[4] = {sm.x, sm.y, sm.z, sm.w}, cw[2] = {cd.x, cd.y};
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t c16 = ((j & 2) ? cd.y : cd.x) >> ((j & 1) * 16) & 0xFFFFu;
-        const uint32_t e4 = nib_lookup4(T, c16);
-        wp[2 * j] = merge(spread_lo(smw[j]), __builtin_amdgcn_perm(0, e4, 0x0c010c00u) << 7);
-        wp[2 * j + 1] = merge(spread_hi(smw[j]), __builtin_amdgcn_perm(0, e4, 0x0c030c02u) << 7);
+    for (int i = 0; i < 2; i++) {
+        uint32_t even, odd;
+        nib_lookup8(T, cw[i], even, odd);
+#pragma unroll
+        for (int p = 0; p < 4; p++) { // columns 2 p and 2 p + 1 of the eight
+            const uint32_t sel = ROT ? 0x04040000u + 0x01010101u * p : 0x0c040c00u + 0x00010001u * p;
+            const uint32_t e = __builtin_amdgcn_perm(odd, even, sel), s = smw[2 * i + (p >> 1)];
+            wp[4 * i + p] = merge(p & 1 ? spread_hi(s) : spread_lo(s), ROT ? e : e << 7);
+        }
     }
 }
 

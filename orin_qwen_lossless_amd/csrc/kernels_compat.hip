@@ -30,7 +30,6 @@ constexpr int HALVES = NT / 32;  // units (rows) per block
 // what it loaded DEEP rounds ago; the same block again while it has not moved on.  The stream buffers end with padding
 // words (32 of HUFPAIR, 16 of HUFFMAN): the last lane reads at most 17 (13) words past its end.
 constexpr int LR_WORDS = 16;                     // ring words per lane
-constexpr size_t LDS_BYTES = 160 * 1024;         // of a CU
 constexpr int LR_BYTES = LR_WORDS * 64 * 4;      // per wavefront: word i of a lane at [i % 16][lane]
 template <int FORMAT> struct lane_ring {
     static constexpr int BITS = FORMAT == FMT_HUFPAIR ? HP_LP : HUF_LMAX;
@@ -541,7 +540,7 @@ __global__ void __launch_bounds__(NM_WAVES * 64) k_nib_mm(const bf16n_weight w, 
     const int64_t row = p.row0 + (g0 + r < p.nrows ? g0 + r : p.nrows - 1);
     const int t0 = (int) blockIdx.y * 32;
     const char * x = p.x + (int64_t) (t0 + r < ncols ? t0 + r : ncols - 1) * p.x_tok;
-    const uint4 T = *(const uint4 *) (q.table + row * 16);
+    const uint4 T = nib_rotated(*(const uint4 *) (q.table + row * 16));
     // the sums this thread finishes at the end are (token, row) = (e / 32, e % 32) for e = thread, thread + block size:
     // one row (the block size is a multiple of 32), whose escape range is requested now
     const int64_t my_row = g0 + (threadIdx.x & 31);
@@ -578,8 +577,8 @@ __global__ void __launch_bounds__(NM_WAVES * 64) k_nib_mm(const bf16n_weight w, 
 #pragma unroll
             for (int n = 0; n < 4; n++) {
                 uint32_t w0[8], w1[8];
-                nib_chunk(sm0[turn][n], make_uint2(cdv[turn][n].x, cdv[turn][n].y), T, w0);
-                nib_chunk(sm1[turn][n], make_uint2(cdv[turn][n].z, cdv[turn][n].w), T, w1);
+                nib_chunk<true>(sm0[turn][n], make_uint2(cdv[turn][n].x, cdv[turn][n].y), T, w0);
+                nib_chunk<true>(sm1[turn][n], make_uint2(cdv[turn][n].z, cdv[turn][n].w), T, w1);
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const nm_u32x4_t a = {w0[2 * j], w0[2 * j + 1], w1[2 * j], w1[2 * j + 1]};
@@ -634,7 +633,7 @@ __global__ void __launch_bounds__(NM_WAVES * 64) k_nib_mm16(const bf16n_weight w
     const int64_t row = p.row0 + (g0 + r < p.nrows ? g0 + r : p.nrows - 1);
     const int t0 = (int) blockIdx.y * 16;
     const char * x = p.x + (int64_t) (t0 + r < ncols ? t0 + r : ncols - 1) * p.x_tok;
-    const uint4 T = *(const uint4 *) (q.table + row * 16);
+    const uint4 T = nib_rotated(*(const uint4 *) (q.table + row * 16));
     // the sums this thread finishes at the end are (token, row) = (e / 16, e % 16) for e = thread, thread + block size
     const int64_t my_row = g0 + (threadIdx.x & 15);
     const int64_t my_gr = p.row0 + (my_row < p.nrows ? my_row : p.nrows - 1);
@@ -658,8 +657,8 @@ __global__ void __launch_bounds__(NM_WAVES * 64) k_nib_mm16(const bf16n_weight w
 #pragma unroll
     for (int n = 0; n < STEPS; n++) {
         uint32_t w0[8], w1[8];
-        nib_chunk(sm0[n], make_uint2(cdv[n].x, cdv[n].y), T, w0);
-        nib_chunk(sm1[n], make_uint2(cdv[n].z, cdv[n].w), T, w1);
+        nib_chunk<true>(sm0[n], make_uint2(cdv[n].x, cdv[n].y), T, w0);
+        nib_chunk<true>(sm1[n], make_uint2(cdv[n].z, cdv[n].w), T, w1);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const nm_u32x4_t a = {w0[2 * j], w0[2 * j + 1], w1[2 * j], w1[2 * j + 1]};
@@ -701,13 +700,13 @@ __global__ void __launch_bounds__(NT) k_nib_rows(const bf16n_weight w, const cha
     for (int64_t i = (int64_t) blockIdx.x * HALVES + half; i < n; i += (int64_t) gridDim.x * HALVES) {
         const int64_t gr = row0 + (ids ? (int64_t) * (const int32_t *) (ids + i * ids_s0) : i);
         char * o = dst + i * dst_s1;
-        const uint4 T = *(const uint4 *) (q.table + gr * 16);
+        const uint4 T = nib_rotated(*(const uint4 *) (q.table + gr * 16));
         const uint32_t e0 = q.esc_off[gr], e1 = q.esc_off[gr + 1];
         for (int c = 0; c < C; c++) {
             const uint4 sm = *((const uint4 *) (q.plane + gr * K + c * CHUNK) + l32);
             const uint2 cd = *((const uint2 *) (q.codes + gr * (K / 2) + c * 256) + l32);
             uint32_t wp[8];
-            nib_chunk(sm, cd, T, wp);
+            nib_chunk<true>(sm, cd, T, wp);
             // the row's escapes go into the registers of the lane that holds their column: every element is stored once
             for (uint32_t e = e0; e < e1; e++) {
                 const uint32_t rec = q.esc[e];

@@ -1191,13 +1191,16 @@ __global__ void __launch_bounds__(KS_WAVES * 64) k_mm_tile_ks(const bf16n_weight
 // chunk) in a token-major layout padded so that sixteen tokens meet all banks.  No table and no ring in LDS, so the
 // staged activations may take it all.  Escaped weights (decoded as +0) add their exact products before the SwiGLU.
 constexpr int NB_WAVES = 8;
-constexpr int NB_PAIRS_32 = 12, NB_PAIRS_64 = 40; // routed pairs per expert up to which passes are 32 / 64 tokens long
+// Routed pairs per expert up to which passes are 32 tokens long (k_nib_mm_few), and 64.  At 28 pairs on average a fifth of
+// the experts have a second pass of 32, and that is still ahead of 64-token passes: 256 experts of 512 x 2048, 890 tokens
+// x top-8 317 against 359 us (640: 290 / 340), 48 of 512 x 1536 62 / 100.
+constexpr int NB_PAIRS_32 = 28, NB_PAIRS_64 = 40;
 constexpr int NB_TOK_BYTES = 4 * 128 + 16; // a staged token: four runs of 64 columns, padded
 template <int NT> constexpr int nb_stage_bytes() { return 32 * NT * NB_TOK_BYTES; }
 template <int NT> size_t nb_shm() { return (size_t) 2 * nb_stage_bytes<NT>() + (size_t) 32 * NT * 4 + (MT_MAX_UNITS + 16) * 4; }
 
 template <bool GLU, int NT>
-__global__ void __launch_bounds__(NB_WAVES * 64, NT == 1 ? 2 : 1) k_nib_mm_ids(const bf16n_weight w, const bf16n_weight w_up, const mm_args a) {
+__global__ void __launch_bounds__(NB_WAVES * 64) k_nib_mm_ids(const bf16n_weight w, const bf16n_weight w_up, const mm_args a) {
     constexpr int TOK = 32 * NT, STAGE = nb_stage_bytes<NT>();
     constexpr int GPI = GLU ? NB_WAVES : 2 * NB_WAVES; // row groups per work item
     constexpr int SV = TOK * 32 / (NB_WAVES * 64);      // uint4 a thread stages per half chunk: 32 per token
@@ -1224,7 +1227,7 @@ __global__ void __launch_bounds__(NB_WAVES * 64, NT == 1 ? 2 : 1) k_nib_mm_ids(c
         const bool live = g0 < groups, has1 = GLU || g0 + 1 < groups;
         const int g1 = GLU || !has1 ? g0 : g0 + 1;
         const int64_t row0 = (int64_t) e * a.rows + (live ? g0 : 0) * 32 + r, row1 = (int64_t) e * a.rows + (live ? g1 : 0) * 32 + r;
-        const uint4 T0 = *(const uint4 *) (q0.table + row0 * 16), T1 = *(const uint4 *) (q1.table + row1 * 16);
+        const uint4 T0 = nib_rotated(*(const uint4 *) (q0.table + row0 * 16)), T1 = nib_rotated(*(const uint4 *) (q1.table + row1 * 16));
         // a lane takes four adjacent slots of its row at a time, 64 plane bytes and 32 code bytes, the two halves of a
         // row's 128-byte line in the same load instructions: taken 32 bytes at a time, a step apart, every line came from
         // HBM twice at 2,048 tokens (FETCH_SIZE 1.92 GB for 0.83 GB of weights: neither L1 nor L2 kept it that long)
@@ -1323,8 +1326,8 @@ __global__ void __launch_bounds__(NB_WAVES * 64, NT == 1 ? 2 : 1) k_nib_mm_ids(c
 #pragma unroll
                         for (int m = 0; m < 2; m++) {
                             const uint4 ck = cur[6 * m + 4 + st];
-                            nib_chunk(cur[6 * m + 2 * st], make_uint2(ck.x, ck.y), m ? T1 : T0, wa[m]);
-                            nib_chunk(cur[6 * m + 2 * st + 1], make_uint2(ck.z, ck.w), m ? T1 : T0, wb[m]);
+                            nib_chunk<true>(cur[6 * m + 2 * st], make_uint2(ck.x, ck.y), m ? T1 : T0, wa[m]);
+                            nib_chunk<true>(cur[6 * m + 2 * st + 1], make_uint2(ck.z, ck.w), m ? T1 : T0, wb[m]);
                         }
 #pragma unroll
                         for (int jb = 0; jb < 4; jb++) {
@@ -1404,6 +1407,180 @@ __global__ void __launch_bounds__(NB_WAVES * 64, NT == 1 ? 2 : 1) k_nib_mm_ids(c
                             *(float4 *) ((float *) a.dst + o) = make_float4(v[0], v[1], v[2], v[3]);
                         }
                     }
+                }
+            }
+        }
+    }
+}
+
+// The same product in passes of 32 tokens, where what counts is how the weights arrive.  A lane of a matrix operand is a
+// row, so lanes that load their own rows' bytes touch 64 lines per load instruction, and the L1 takes one line a cycle:
+// 113 us for the 740 M weights of 77 tokens x top-8 over 256 experts of 512 x 2048, where memory needs 165.  Here eight
+// adjacent lanes load a whole 128-byte line, and the wavefront turns lines into rows through 4 KiB of LDS of its own (no
+// barrier): 16-byte piece c of row r lies at c ^ (r / 2 % 8), so that sixteen lanes that read one piece of sixteen rows
+// meet all banks.  An operand is 32 rows: of the matrix, or sixteen of gate and the same sixteen of up, which end in the
+// same lanes.  A step is 128 columns: a line of plane bytes per row, and every second step a line of code bytes (taken 64
+// bytes at a time they came from HBM twice: FETCH_SIZE 1.2 times the weights).  Loads are one step (two steps) ahead in
+// registers, over the end of an item too: 4 KiB per wavefront, sixteen wavefronts per CU.  77 tokens, fused gate / up and down:
+// 182 + 106 us with lanes that load their own rows, 138 + 79 here (5.4 TB/s of weights).  48 experts of 512 x 1536, 150 tokens,
+// whole call: 92 and 59.  In passes of 64 tokens this form measures as much as k_nib_mm_ids, in passes of 128 a third more
+// (2048 tokens 588 against 433 us): an operand of activations serves one row group here and two there.
+constexpr int NF_TOK_BYTES = 4 * 64 + 16; // a staged token: four runs of 32 columns, padded: sixteen tokens meet all banks
+constexpr int NF_TURN = 32 * 128;         // a wavefront's lines: one of each row
+constexpr int NF_STAGE = 32 * NF_TOK_BYTES;
+constexpr size_t NF_SHM = (size_t) NB_WAVES * NF_TURN + 2 * NF_STAGE + 32 * 4 + (MT_MAX_UNITS + 16) * 4;
+
+template <bool GLU, bool ONCE>
+__global__ void __launch_bounds__(NB_WAVES * 64, 4) k_nib_mm_few(const bf16n_weight w, const bf16n_weight w_up, const mm_args a) {
+    constexpr int TOK = 32, GROUP = GLU ? 16 : 32; // rows of a matrix in an operand
+    extern __shared__ __align__(16) char nb_lds[];
+    char * stage = nb_lds + NB_WAVES * NF_TURN;         // [2][TOK][NF_TOK_BYTES]
+    int * tok_row = (int *) (stage + 2 * NF_STAGE);     // [TOK]: the activation row of every token of the pass
+    uint32_t * unit = (uint32_t *) (tok_row + TOK);
+    const nib_ptrs q0 = nibp(w, 0), q1 = GLU ? nibp(w_up, 0) : nibp(w, 16); // rows 0..15 and 16..31 of an operand
+    const int K = (int) w.K, steps = K / 128;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5, wave = (int) uniform(tid >> 6);
+    const int groups = (int) (a.rows / GROUP), slabs = (groups + NB_WAVES - 1) / NB_WAVES;
+    const int n_units = list_units<TOK>(unit, a, wave, lane, NB_WAVES), n_items = n_units * slabs;
+    // where this lane finds its row's pieces 4 h + k (plane) and 4 d + 2 h + k (codes of step d of two): at those ^ 16 k
+    char * turn = nb_lds + wave * NF_TURN;
+    const uint32_t rp = (uint32_t) (r * 128 + ((4 * h ^ (r >> 1 & 7)) << 4)), rc = (uint32_t) (r * 128 + ((2 * h ^ (r >> 1 & 7)) << 4));
+    // what it loads: 16 bytes of row 8 i + lane / 8, the piece that the swizzle places there (odd i: the line's other half)
+    const uint32_t piece = (uint32_t) (((lane & 7) ^ (lane >> 4)) << 4);
+    const uint32_t gp = (uint32_t) ((lane >> 3) * K) + piece, gc = (uint32_t) ((lane >> 3) * (K / 2)) + piece;
+    uint4 ld[4], lc[4]; // the next step's plane lines, the next two steps' code lines
+    // the first row of an item's operand (of this wavefront; a wavefront without rows of its own takes the first ones)
+    auto rows_of = [&](int item) {
+        const int e = (int) (uniform(unit[item / slabs]) & 0xFFFFu), g = item % slabs * NB_WAVES + wave;
+        return (int64_t) e * a.rows + (g < groups ? g : 0) * GROUP;
+    };
+    auto load_plane = [&](int64_t row, int p) {
+        const range_t pl[2] = {make_range(q0.plane + uniform64(row * K), (uint32_t) (16 * K)), make_range(q1.plane + uniform64(row * K), (uint32_t) (16 * K))};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const u32x4_nt v = __builtin_amdgcn_raw_buffer_load_b128(pl[i >> 1], (int) ((gp + (uint32_t) (128 * p)) ^ (64u * (i & 1))), 8 * (i & 1) * K, ONCE ? 2 : 0);
+            ld[i] = make_uint4(v.x, v.y, v.z, v.w);
+        }
+    };
+    auto load_codes = [&](int64_t row, int p) { // of steps p and p + 1
+        const range_t cd[2] = {make_range(q0.codes + uniform64(row * (K / 2)), (uint32_t) (8 * K)), make_range(q1.codes + uniform64(row * (K / 2)), (uint32_t) (8 * K))};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const u32x4_nt v = __builtin_amdgcn_raw_buffer_load_b128(cd[i >> 1], (int) ((gc + (uint32_t) (64 * p)) ^ (64u * (i & 1))), 4 * (i & 1) * K, ONCE ? 2 : 0);
+            lc[i] = make_uint4(v.x, v.y, v.z, v.w);
+        }
+    };
+    auto turn_in = [&](const uint4 (&v)[4]) { // (a wavefront's LDS accesses are served in order)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            *(uint4 *) (turn + 1024 * i + 16 * lane) = v[i];
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    int item = blockIdx.x;
+    if (item < n_items) {
+        const int64_t row = rows_of(item);
+        load_codes(row, 0);
+        load_plane(row, 0);
+    }
+    for (; item < n_items; item += gridDim.x) {
+        const uint32_t un = uniform(unit[item / slabs]);
+        const int e = (int) (un & 0xFFFFu), g = item % slabs * NB_WAVES + wave;
+        const bool live = g < groups;
+        const int64_t row = rows_of(item), next = item + (int) gridDim.x < n_items ? rows_of(item + (int) gridDim.x) : row;
+        const uint4 T = nib_rotated(*(const uint4 *) ((r < 16 ? q0.table : q1.table) + (row + (r & 15)) * 16));
+        const int j0 = a.bounds[e] + TOK * (int) (un >> 16);
+        const int left = a.bounds[e + 1] - j0, n = left < TOK ? left : TOK;
+        __syncthreads(); // the item before is done with tok_row and the staging buffers
+        if (tid < TOK) {
+            tok_row[tid] = a.ids_src1[j0 + (tid < n ? tid : n - 1)];
+        }
+        __syncthreads();
+        // staging: this thread takes part (index % 4) of column block (index / 4 % 4) of token index / 16
+        const int tok = tid >> 4, blk = (tid >> 2) & 3, part = tid & 3;
+        const char * sx = (const char *) (a.x + (int64_t) tok_row[tok] * a.x_row) + 256 * blk + 16 * part;
+        const int so = tok * NF_TOK_BYTES + 64 * blk + 16 * part;
+        f32x16_t acc;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            acc[i] = 0.f;
+        }
+        uint4 f = *(const uint4 *) sx; // the next step's activations
+#pragma unroll 1
+        for (int p = 0; p < steps; p += 2) {
+            turn_in(lc);
+            load_codes(p + 2 < steps ? row : next, p + 2 < steps ? p + 2 : 0);
+            uint4 cc[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                cc[k] = *(const uint4 *) (turn + (rc ^ (uint32_t) (16 * (4 * (k >> 1) + (k & 1)))));
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                const int q = p + d, nx = q + 1 < steps ? q + 1 : q;
+                char * bcur = stage + d * NF_STAGE;
+                *(uint4 *) (bcur + so) = f;
+                f = *(const uint4 *) (sx + 2 * ((nx >> 2) * 512 + 32 * (nx & 3)));
+                turn_in(ld);
+                load_plane(q + 1 < steps ? row : next, q + 1 < steps ? q + 1 : 0);
+                uint4 cur[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    cur[k] = *(const uint4 *) (turn + (rp ^ (uint32_t) (16 * k)));
+                }
+                __syncthreads(); // (the buffer written two steps on is the one read here: every wavefront is past it at the next barrier)
+#pragma unroll
+                for (int st = 0; st < 2; st++) { // slots 2 st, 2 st + 1 of the lane's four
+                    uint32_t wa[8], wb[8];
+                    const uint4 ck = cc[2 * d + st];
+                    nib_chunk<true>(cur[2 * st], make_uint2(ck.x, ck.y), T, wa);
+                    nib_chunk<true>(cur[2 * st + 1], make_uint2(ck.z, ck.w), T, wb);
+#pragma unroll
+                    for (int jb = 0; jb < 4; jb++) {
+                        const u32x4_t av = {wa[2 * jb], wa[2 * jb + 1], wb[2 * jb], wb[2 * jb + 1]};
+                        const bf16x8_t bv = *(const bf16x8_t *) (bcur + r * NF_TOK_BYTES + 64 * jb + 32 * h + 16 * st);
+                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, av), bv, acc, 0, 0, 0);
+                    }
+                }
+            }
+        }
+        if (!live) {
+            continue;
+        }
+        // the exact products of escaped weights; accumulator element i of a lane: row 8 (i / 4) + 4 h + i % 4, token r
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const nib_ptrs & q = m ? q1 : q0;
+            if (uniform(q.esc_off[row + 16] - q.esc_off[row]) == 0) {
+                continue;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int64_t gr = row + 8 * (i >> 2) + 4 * h + (i & 3);
+                for (uint32_t k = q.esc_off[gr]; k < q.esc_off[gr + 1]; k++) {
+                    const uint32_t rec = q.esc[k];
+                    const uint16_t xv = a.x[(int64_t) tok_row[r] * a.x_row + (rec & 0xFFFu)];
+                    acc[8 * m + i] = fmaf(bf16_bits_to_f32(esc_bits(rec)), bf16_bits_to_f32(xv), acc[8 * m + i]);
+                }
+            }
+        }
+        if (r < n) {
+            const int64_t at = (int64_t) a.ids_dst[j0 + r] * a.dst_col + (int64_t) g * GROUP + 4 * h;
+#pragma unroll
+            for (int k = 0; k < GROUP / 8; k++) {
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    v[i] = GLU ? acc[(8 + 4 * k + i) & 15] * silu(acc[4 * k + i]) : acc[4 * k + i];
+                }
+                const int64_t o = at + 8 * k;
+                if (a.dst_bf16) {
+                    *(uint2 *) ((uint16_t *) a.dst + o) =
+                        make_uint2(f32_to_bf16_rne(v[0]) | ((uint32_t) f32_to_bf16_rne(v[1]) << 16),
+                                   f32_to_bf16_rne(v[2]) | ((uint32_t) f32_to_bf16_rne(v[3]) << 16));
+                } else {
+                    *(float4 *) ((float *) a.dst + o) = make_float4(v[0], v[1], v[2], v[3]);
                 }
             }
         }
@@ -1677,7 +1854,12 @@ template <bool GLU, int NT, int W> void mt_attr() { lds_attr((const void *) k_mm
 template <bool GLU> void ks_attr() { lds_attr((const void *) k_mm_tile_ks<GLU>, ks_shm(GLU)); }
 
 template <bool GLU, int NT> void nb_attr() {
-    (void) hipFuncSetAttribute((const void *) k_nib_mm_ids<GLU, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) nb_shm<NT>());
+    if constexpr (NT == 1) {
+        lds_attr((const void *) k_nib_mm_few<GLU, false>, NF_SHM);
+        lds_attr((const void *) k_nib_mm_few<GLU, true>, NF_SHM);
+    } else {
+        lds_attr((const void *) k_nib_mm_ids<GLU, NT>, nb_shm<NT>());
+    }
 }
 
 void tile_init() {
@@ -1836,12 +2018,21 @@ int64_t nib_mm_ids_units_bound(int n_experts, int64_t n_pairs, int pass_tokens) 
 
 template <int NT>
 void nb_launch(const bf16n_weight & w, const bf16n_weight * up, const mm_args & a, int cus, hipStream_t stream) {
-    const int per_cu = (int) (160 * 1024 / nb_shm<NT>()) < 3 ? (int) (160 * 1024 / nb_shm<NT>()) : 3;
-    const dim3 grid((unsigned) (cus * (per_cu < 1 ? 1 : per_cu)));
-    if (up) {
-        hipLaunchKernelGGL((k_nib_mm_ids<true, NT>), grid, dim3(NB_WAVES * 64), nb_shm<NT>(), stream, w, *up, a);
+    const size_t shm = NT == 1 ? NF_SHM : nb_shm<NT>();
+    const dim3 grid((unsigned) (cus * std::max(1, (int) (160 * 1024 / shm))));
+    if constexpr (NT == 1) {
+        // a stack of 2^27 weights outlasts the caches between two launches: its lines stay out of the way of the activations
+        const bool once = w.rows * w.K >= ((int64_t) 1 << 27);
+        auto go = [&](auto glu, const bf16n_weight & w1) {
+            constexpr bool G = decltype(glu)::value;
+            if (once) hipLaunchKernelGGL((k_nib_mm_few<G, true>), grid, dim3(NB_WAVES * 64), shm, stream, w, w1, a);
+            else      hipLaunchKernelGGL((k_nib_mm_few<G, false>), grid, dim3(NB_WAVES * 64), shm, stream, w, w1, a);
+        };
+        if (up) go(std::true_type{}, *up);
+        else    go(std::false_type{}, w);
     } else {
-        hipLaunchKernelGGL((k_nib_mm_ids<false, NT>), grid, dim3(NB_WAVES * 64), nb_shm<NT>(), stream, w, w, a);
+        if (up) hipLaunchKernelGGL((k_nib_mm_ids<true, NT>), grid, dim3(NB_WAVES * 64), shm, stream, w, *up, a);
+        else    hipLaunchKernelGGL((k_nib_mm_ids<false, NT>), grid, dim3(NB_WAVES * 64), shm, stream, w, w, a);
     }
 }
 

@@ -1,5 +1,5 @@
-"""Experts in the 4-bit code (NIBBLE, rows of all experts stacked) through the batched matrix-core kernel
-(bf16n_mm_ids -> k_nib_mm_ids): the fused gate / up + SwiGLU product and the down product against FP64 products of the
+"""Experts in the 4-bit code (NIBBLE, rows of all experts stacked) through the batched matrix-core kernels
+(bf16n_mm_ids -> k_nib_mm_few, k_nib_mm_ids): the fused gate / up + SwiGLU product and the down product against FP64 products of the
 exact weights, at every pass length (32 / 64 / 128 tokens), with ragged passes, an expert that every token uses,
 experts without tokens, escaped weights, and row groups that do not fill the last slab.  The reference's batched kernel
 (core/src/kernels.cuh:1162-1505) does not take this format; the operator's contract is the same."""
@@ -33,6 +33,8 @@ def silu64(v):
     (32, 160, 512, 600, 2, False),   # 37 pairs per expert: passes of 64; 5 row groups: the last slab is not full
     (16, 512, 512, 9, 4, False),     # gate / up and down, 32-token passes
     (64, 64, 512, 3, 2, False),      # most experts without tokens
+    (24, 160, 1024, 120, 4, False),  # 20 pairs per expert, 32-token passes up to a few second ones; 10 operands of 16 rows
+    (256, 512, 1024, 200, 4, False), # 2^27 weights (read with the non-temporal hint), more items than blocks
 ])
 def test_batched_products_of_experts_in_the_4_bit_code(ops, E, N, K, T, topk, popular):
     g = torch.Generator(device="cuda").manual_seed(E * 1000 + T)
