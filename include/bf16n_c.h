@@ -154,6 +154,11 @@ int bf16n_swiglu(const float * g, const float * u, float * y, int64_t n, void * 
 int bf16n_add_rmsnorm(const uint16_t * a, const uint16_t * b, const uint16_t * c, const float * ys, const void * wts, int wts_bf16,
                       int n_used, const uint16_t * gamma, uint16_t * y_sum, uint16_t * y_norm, int n_tok, int64_t n, float eps,
                       void * stream);
+/* The same without ys for n = 2048, and the product of a 4-bit-code matrix of K = 2048 (a router) with y_norm in the same
+ * launch: y[t] = W y_norm[t] in FP32, rows y_tok elements apart; bit for bit what bf16n_add_rmsnorm and bf16n_mmv give one
+ * token at a time.  The results must not overlap the inputs. */
+int bf16n_add_rmsnorm_mmv(const uint16_t * a, const uint16_t * b, const uint16_t * c, const uint16_t * gamma, uint16_t * y_sum, uint16_t * y_norm,
+                          int n_tok, int64_t n, float eps, const bf16n_weight * w, float * y, int64_t y_tok, void * stream);
 
 /* Router softmax + top-k on the device, so that a whole MoE decode step can be captured into one HIP graph.  The
  * reference leaves this to the engines (vllm_bf16n/moe.py:62-67 receives topk_weights/topk_ids); it has no core

@@ -58,6 +58,7 @@ SYMBOLS = {
     "bf16n_moe_mm_ids_static": (_i, [_WP, _WP, _vp, _i64, _vp, _i, _i64, _i, _vp, _i, _i64, _i, _i, _i, _vp]),
     "bf16n_moe_combine": (_i, [_vp, _vp, _i, _vp, _i, _i, _i, _i64, _vp]),
     "bf16n_add_rmsnorm": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _i, _i64, C.c_float, _vp]),
+    "bf16n_add_rmsnorm_mmv": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i64, C.c_float, _WP, _vp, _i64, _vp]),
     "bf16n_swiglu": (_i, [_vp, _vp, _vp, _i64, _vp]),
     "bf16n_router_topk": (_i, [_vp, _i64, _i, _i, _i, _i, _vp, _vp, _vp]),
     "bf16n_router_topk_strided": (_i, [_vp, _i64, _i, _i, _i, _i, _vp, _vp, _i64, _vp]),

@@ -607,6 +607,27 @@ int bf16n_add_rmsnorm(const uint16_t * a, const uint16_t * b, const uint16_t * c
     });
 }
 
+int bf16n_add_rmsnorm_mmv(const uint16_t * a, const uint16_t * b, const uint16_t * c, const uint16_t * gamma, uint16_t * y_sum, uint16_t * y_norm,
+                          int n_tok, int64_t n, float eps, const bf16n_weight * w, float * y, int64_t y_tok, void * stream) {
+    return guarded([&] {
+        ensure_init();
+        require(a && y_norm && y && n_tok > 0 && n_tok <= 65535, "add_rmsnorm_mmv: null pointer or empty input");
+        check_weight(*w);
+        dev::add_norm_args p{};
+        p.a = a; p.b = b; p.c = c; p.gamma = gamma; p.y_sum = y_sum; p.y_norm = y_norm; p.n = n; p.eps = eps;
+        require(dev::norm_nib_mmv_ok(*w, p) && y_tok >= w->rows,
+                "add_rmsnorm_mmv: rows of 2048 elements, 16-byte aligned, and a 4-bit-code matrix of that K with at most 65536 rows");
+        // (every block reads the token's inputs, one of them writes the results)
+        const auto apart = [&](const uint16_t * o) {
+            const auto clear = [&](const uint16_t * in, int64_t len) { return !o || !in || o + n_tok * n <= in || in + len <= o; };
+            return clear(a, n_tok * n) && clear(b, n_tok * n) && clear(c, n_tok * n) && clear(gamma, n);
+        };
+        require(apart(y_sum) && apart(y_norm), "add_rmsnorm_mmv: the results must not overlap the inputs");
+        dev::launch_norm_nib_mmv(*w, p, y, y_tok, n_tok, (hipStream_t) stream);
+        launch_check("add_rmsnorm_mmv");
+    });
+}
+
 // launch.cu:574-582
 int bf16n_swiglu(const float * g, const float * u, float * y, int64_t n, void * stream) {
     return guarded([&] {

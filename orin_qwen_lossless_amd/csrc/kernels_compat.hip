@@ -8,6 +8,7 @@
 // which has twice the chains per unit, is the fast path.
 #include "dev_common.h"
 #include "dev_compat.h"
+#include "dev_norm.h"
 #include "launchers.h"
 
 #include <algorithm>
@@ -501,6 +502,71 @@ __global__ void __launch_bounds__(NT) k_nib_mmv(const bf16n_weight w, const bf16
     }
 }
 
+// The router of a decode step with the glue before it: y = W bf16(norm(a + b + c)) in FP32 for a 4-bit-code matrix of
+// K = 2048, one token per blockIdx.y.  Both are a few kilobytes whose time is a launch's latency; here every block forms
+// the token's row itself (12 KB at most, while its weights are on their way) and takes its two rows of the matrix from
+// there, and the first block stores the row.  The bits are those of k_add_rmsnorm8 and k_nib_mmv<bf16_t, 0, 1>.  256 rows,
+// one token: 3.9 us against 3.7 + 3.0 and the gap between two launches (three layers of the decode step 158 -> 150 us,
+// half a microsecond a layer of it by the faster selection); 16 tokens, two layers: 330 -> 325.
+__global__ void __launch_bounds__(NT) k_norm_nib_mmv(const bf16n_weight w, const add_norm_args p, float * __restrict__ y, int64_t y_tok) {
+    constexpr int C = NORM8_N / CHUNK, RPB = HALVES / C;
+    static_assert(NT == NORM8_THREADS, "a thread per eight elements of the row");
+    __shared__ __align__(16) uint16_t xs[NORM8_N];
+    __shared__ float wave_sq[NT / 64], part[HALVES];
+    const nib_ptrs q = nibp(w, 0);
+    const int tid = threadIdx.x, l32 = tid & 31, half = tid >> 5, lr = half / C, c = half % C;
+    const int64_t tok = blockIdx.y, at = tok * NORM8_N + 8 * tid;
+    const int64_t base = (int64_t) blockIdx.x * RPB, row = base + lr < w.rows ? base + lr : w.rows - 1;
+    const uint4 va = *(const uint4 *) (p.a + at);
+    const uint4 vb = p.b ? *(const uint4 *) (p.b + at) : make_uint4(0, 0, 0, 0);
+    const uint4 vc = p.c ? *(const uint4 *) (p.c + at) : make_uint4(0, 0, 0, 0);
+    const uint4 sm = *((const uint4 *) (q.plane + row * NORM8_N + c * CHUNK) + l32);
+    const uint2 cd = *((const uint2 *) (q.codes + row * (NORM8_N / 2) + c * (CHUNK / 2)) + l32);
+    const uint4 T = *(const uint4 *) (q.table + row * 16);
+    const uint32_t e0 = q.esc_off[row], e1 = q.esc_off[row + 1];
+    float v[8], fb[8], fc[8];
+    unpack8(va, v);
+    unpack8(vb, fb);
+    unpack8(vc, fc);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        if (p.b) {
+            v[i] += fb[i];
+        }
+        if (p.c) {
+            v[i] += fc[i];
+        }
+    }
+    const uint4 o = norm8_row(v, p.gamma, p.eps, wave_sq);
+    *(uint4 *) (xs + 8 * tid) = o;
+    if (blockIdx.x == 0) {
+        if (p.y_sum) {
+            *(uint4 *) (p.y_sum + at) = pack8(v);
+        }
+        *(uint4 *) (p.y_norm + at) = o;
+    }
+    uint32_t wp[8], xp[8];
+    nib_chunk(sm, cd, T, wp);
+    __syncthreads();
+    x_pairs16((const char *) xs, c * CHUNK + 4 * l32, xp);
+    float s = nib_dot_pairs(wp, xp);
+    if (c == 0) {
+        s += nib_escapes<bf16_t>(q, e0, e1, (const char *) xs, l32);
+    }
+    if (l32 == 31) {
+        part[half] = s;
+    }
+    __syncthreads();
+    if (c == 0 && l32 == 0 && base + lr < w.rows) {
+        float sum = part[half];
+#pragma unroll
+        for (int i = 1; i < C; i++) {
+            sum += part[half + i];
+        }
+        y[tok * y_tok + base + lr] = sum;
+    }
+}
+
 // Dense NIBBLE products through the matrix cores: y[t] = W x[t] for BF16 token columns, 32 per block (gridDim.y blocks
 // of tokens; columns past the last repeat it and are not stored).  The 4-bit code has no decode chain, so one decode of
 // the matrix serves 32 tokens at the cost of one.  A block is one group of 32 rows with K / 256 wavefronts; wavefront v
@@ -884,6 +950,18 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
     }
 #undef HUFX
 #undef HUF
+}
+
+bool norm_nib_mmv_ok(const bf16n_weight & w, const add_norm_args & a) {
+    const auto al = [](const void * q) { return ((uintptr_t) q & 15) == 0; };
+    return w.format == FMT_NIBBLE && w.K == NORM8_N && a.n == NORM8_N && w.rows <= 65536 && !a.ys && al(a.a) && al(a.b) && al(a.c) && al(a.gamma) &&
+           al(a.y_sum) && al(a.y_norm);
+}
+
+void launch_norm_nib_mmv(const bf16n_weight & w, const add_norm_args & a, float * y, int64_t y_tok, int n_tok, hipStream_t stream) {
+    constexpr int RPB = HALVES * CHUNK / NORM8_N;
+    note_kernel("k_norm_nib_mmv", nullptr, 0);
+    hipLaunchKernelGGL(k_norm_nib_mmv, dim3((unsigned) ((w.rows + RPB - 1) / RPB), n_tok), dim3(NT), 0, stream, w, a, y, y_tok);
 }
 
 void launch_compat_dequant(const bf16n_weight & w, int64_t row0, int64_t nrows, uint16_t * out, int cus, hipStream_t stream) {

@@ -2,6 +2,7 @@
 // and the router's softmax + top-k (on the device so that a decode step has no host round trip and can be captured
 // into a HIP graph).  All reductions run in a fixed order: results are bitwise reproducible.
 #include "dev_common.h"
+#include "dev_norm.h"
 #include "dev_topk.h"
 #include "launchers.h"
 
@@ -389,28 +390,11 @@ __global__ void __launch_bounds__(NORM_THREADS) k_add_rmsnorm(const add_norm_arg
 // consecutive elements through 16-byte loads (a quarter of the wavefronts to start and to meet at the barrier, an
 // eighth of the load instructions).  The slot-ordered fmaf chain per element is k_add_rmsnorm's; the mean of squares
 // is summed in another (fixed) order.
-constexpr int NORM8_THREADS = 256, NORM8_N = 8 * NORM8_THREADS;
-__device__ __forceinline__ void unpack8(const uint4 v, float (&f)[8]) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        f[2 * i] = __uint_as_float(w[i] << 16);
-        f[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-    }
-}
-__device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        w[i] = f32_to_bf16_rne(f[2 * i]) | ((uint32_t) f32_to_bf16_rne(f[2 * i + 1]) << 16);
-    }
-    return make_uint4(w[0], w[1], w[2], w[3]);
-}
 __global__ void __launch_bounds__(NORM8_THREADS) k_add_rmsnorm8(const add_norm_args p) {
     __shared__ float wave_sq[NORM8_THREADS / 64];
     __shared__ float wsm[16];
     const int64_t tok = blockIdx.x, base = tok * NORM8_N;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i0 = 8 * tid;
+    const int tid = threadIdx.x, i0 = 8 * tid;
     // every load of the thread is requested before anything is waited for
     const uint4 va = *(const uint4 *) (p.a + base + i0);
     const uint4 vb = p.b ? *(const uint4 *) (p.b + base + i0) : make_uint4(0, 0, 0, 0);
@@ -435,7 +419,6 @@ __global__ void __launch_bounds__(NORM8_THREADS) k_add_rmsnorm8(const add_norm_a
     unpack8(va, v);
     unpack8(vb, fb);
     unpack8(vc, fc);
-    float sq = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         if (p.b) {
@@ -462,30 +445,11 @@ __global__ void __launch_bounds__(NORM8_THREADS) k_add_rmsnorm8(const add_norm_a
             v[i] += acc[i];
         }
     }
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        sq = fmaf(v[i], v[i], sq);
-    }
-    sq = wave_sum(sq);
-    if (lane == 0) {
-        wave_sq[wave] = sq;
-    }
-    __syncthreads();
-    const float total = ((wave_sq[0] + wave_sq[1]) + wave_sq[2]) + wave_sq[3];
-    const float scale = 1.0f / sqrtf(total / (float) NORM8_N + p.eps);
+    const uint4 o = norm8_row(v, p.gamma, p.eps, wave_sq);
     if (p.y_sum) {
         *(uint4 *) (p.y_sum + base + i0) = pack8(v);
     }
-    float g[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
-    if (p.gamma) {
-        unpack8(*(const uint4 *) (p.gamma + i0), g);
-    }
-    float o[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        o[i] = v[i] * scale * g[i];
-    }
-    *(uint4 *) (p.y_norm + base + i0) = pack8(o);
+    *(uint4 *) (p.y_norm + base + i0) = o;
 }
 
 } // namespace

@@ -83,6 +83,9 @@ struct add_norm_args {
     int64_t n; float eps;
 };
 void launch_add_rmsnorm(const add_norm_args & a, int n_tok, hipStream_t stream);
+// the same for rows of 2048 without ys, and y = W y_norm (FP32, rows y_tok apart) for a 4-bit-code matrix in the same launch
+bool norm_nib_mmv_ok(const bf16n_weight & w, const add_norm_args & a);
+void launch_norm_nib_mmv(const bf16n_weight & w, const add_norm_args & a, float * y, int64_t y_tok, int n_tok, hipStream_t stream);
 void launch_router_topk_strided(const float * logits, int64_t stride, int n_tok, int n_experts, int k, bool renorm, int32_t * ids,
                                 float * weights, int64_t out_stride, hipStream_t stream);
 // top-k and the routing lists of launch_route over the first n_slots columns of the id rows in one launch (few tokens)

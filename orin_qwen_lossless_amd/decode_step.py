@@ -7,16 +7,16 @@ replaced by a slice of the qkv output.
 Per layer (pre-norm, residual stream h in BF16):
     x1 = rmsnorm(h)                         | comes out of the previous layer's glue launch
     q  = qkv x1;  o = W_o q[:, :4096]       | 5120 x 2048 and 2048 x 4096
-    x2 = rmsnorm(h2), h2 = h + o            | one glue launch (add_rmsnorm)
+    x2 = rmsnorm(h2), h2 = h + o            | formed by the router's launch (add_rmsnorm_mmv; a launch of its own beyond 16 tokens)
     ids, wts = top-8(softmax(router x2))    | 256 x 2048, on the device
     ys_k = down_k(silu(gate_k x2) * (up_k x2)) for the 8 routed experts and the shared one
     h' = h2 + sum_k wts_k ys_k, x1' = rmsnorm(h')             | one glue launch (weighted sum, residual, norm)
 256 experts x (gate 512 x 2048, up 512 x 2048, down 2048 x 512) and one shared expert of the same shape.  The shared
 expert is stacked behind the routed ones as expert 256 and runs as a ninth slot of every token with weight 1: its two
 products ride in the routed experts' launches instead of two launches of their own (run on a second stream beside the
-routed ones they cost more than in line: the fork and join of the graph outweighed them).  7 launches per layer while
-the experts run as GEMV columns (the gate / up launch selects them itself), 8 with the batched kernels up to 8 tokens
-(selection and routing lists in one launch), 9 beyond."""
+routed ones they cost more than in line: the fork and join of the graph outweighed them).  6 launches per layer while
+the experts run as GEMV columns (the gate / up launch selects them itself), 7 with the batched kernels up to 8 tokens
+(selection and routing lists in one launch), 8 up to 16, 9 beyond."""
 from __future__ import annotations
 
 import numpy as np
@@ -67,10 +67,11 @@ def layer_bytes(nbytes: dict, tokens: int, expected: bool = False) -> int:
 
 
 def launches_per_layer(ops, tokens: int, gemv_path: bool) -> int:
-    """Kernel launches of one layer of Bf16nStep: qkv, o, glue, router, (top-k,) gate / up, down, glue."""
+    """Kernel launches of one layer of Bf16nStep: qkv, o, (glue,) router, (top-k,) gate / up, down, glue."""
+    glue = 0 if tokens <= ops.NORM_MMV_TOKENS else 1
     if gemv_path:
-        return 7 if getattr(ops, "TOPK_IN_EXPERT_GEMV", False) else 8
-    return 8 if tokens <= ops.TOPK_ROUTE_ONE_LAUNCH_TOKENS else 9
+        return glue + (6 if getattr(ops, "TOPK_IN_EXPERT_GEMV", False) else 7)
+    return glue + (7 if tokens <= ops.TOPK_ROUTE_ONE_LAUNCH_TOKENS else 8)
 
 
 def routing_buffers(n_tok: int, device) -> tuple[torch.Tensor, torch.Tensor]:
@@ -88,10 +89,10 @@ class Bf16nStep:
         self.ops, self.sets, self.head, self.n_layers = ops, sets, head, n_layers
         self.routing = routing_buffers(n_tok, sets[0]["qkv"].plane.device)
 
-    def experts(self, w, x2):
-        """(ys [T, 9, K] FP32 per-slot outputs, wts [T, 9], ids [T, 9])."""
-        ops = self.ops
-        logits, routes = ops.mmv(x2, w["router"]), None
+    def experts(self, w, x2, logits=None):
+        """(ys [T, 9, K] FP32 per-slot outputs, wts [T, 9], ids [T, 9]).  logits: the router's, if the caller has them."""
+        ops, routes = self.ops, None
+        logits = ops.mmv(x2, w["router"]) if logits is None else logits
         batched = ops.moe_experts_batched(x2.shape[0], TOPK + 1, w["gate"], w["up"], w["down"], EA)
         if not batched and ops.topk_in_gemv_supported(w["gate"], w["up"], E, TOPK):
             # the gate / up GEMV selects the experts itself: no top-k launch
@@ -108,8 +109,11 @@ class Bf16nStep:
         ops = self.ops
         q = ops.linear(x1, w["qkv"])
         o = ops.linear(q[:, :ATT], w["o"])
-        x2, h2 = ops.add_rmsnorm(h, o, want_sum=True)
-        ys, wts, _ = self.experts(w, x2)
+        if ops.add_rmsnorm_mmv_supported(w["router"], h.shape[0]):
+            x2, h2, logits = ops.add_rmsnorm_mmv(h, w["router"], o)  # the router forms its own input
+        else:
+            (x2, h2), logits = ops.add_rmsnorm(h, o, want_sum=True), None
+        ys, wts, _ = self.experts(w, x2, logits)
         return ops.add_rmsnorm(h2, ys=ys, topk_weights=wts, want_sum=True)  # (x1', h')
 
     def __call__(self, h):

@@ -624,6 +624,36 @@ def add_rmsnorm(a: torch.Tensor, b: torch.Tensor | None = None, c: torch.Tensor 
     return (y, ysum) if want_sum else y
 
 
+# tokens up to which add_rmsnorm_mmv (every block forms its token's row) beats the two launches
+NORM_MMV_TOKENS = 16
+
+
+def add_rmsnorm_mmv_supported(w: Weight, n_tok: int) -> bool:
+    """Whether add_rmsnorm_mmv takes this matrix and is the faster way for n_tok tokens."""
+    return w.meta.format == FMT_NIBBLE and w.meta.K == 2048 and w.meta.rows <= 1024 and 0 < n_tok <= NORM_MMV_TOKENS
+
+
+def add_rmsnorm_mmv(a: torch.Tensor, w: Weight, b: torch.Tensor | None = None, c: torch.Tensor | None = None,
+                    gamma: torch.Tensor | None = None, eps: float = 1e-6) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """y_norm, y_sum = add_rmsnorm(a, b, c, gamma=gamma, eps=eps, want_sum=True) and mmv(y_norm, w) in FP32, one launch
+    (bf16n_add_rmsnorm_mmv): a decode step's router forms its own input.  a, b, c: [T, 2048] BF16 contiguous; w: a 4-bit-code
+    matrix of K = 2048.  Returns (y_norm, y_sum, product)."""
+    for t in (a, b, c):
+        if t is not None and not (t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous() and t.shape == a.shape and t.dim() == 2):
+            raise ValueError("bf16n.add_rmsnorm_mmv: inputs must be contiguous bf16 [tokens, n] of one shape")
+    if gamma is not None and not (gamma.is_cuda and gamma.dtype == torch.bfloat16 and gamma.is_contiguous() and gamma.numel() == a.shape[1]):
+        raise ValueError("bf16n.add_rmsnorm_mmv: gamma must be contiguous bf16 [n]")
+    cw = _cweight(w)
+    T, n = a.shape
+    y, ysum = torch.empty_like(a), torch.empty_like(a)
+    prod = torch.empty((T, w.meta.rows), dtype=torch.float32, device=a.device)
+    ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
+    with _on(a.device):
+        _lib.check(_lib.lib().bf16n_add_rmsnorm_mmv(a.data_ptr(), ptr(b), ptr(c), ptr(gamma), ysum.data_ptr(), y.data_ptr(), T, n,
+                                                    C.c_float(eps), C.byref(cw), prod.data_ptr(), w.meta.rows, _stream()))
+    return y, ysum, prod
+
+
 def swiglu(g: torch.Tensor, u: torch.Tensor) -> torch.Tensor:
     if not (g.is_cuda and g.dtype == torch.float32 and g.is_contiguous() and u.shape == g.shape
             and u.dtype == torch.float32 and u.is_contiguous()):
