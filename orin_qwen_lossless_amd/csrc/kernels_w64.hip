@@ -285,23 +285,40 @@ __global__ void __launch_bounds__(wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2
     }
 }
 
-// Several BF16 columns of 2048 or 4096 with the activations in LDS (C = 4, 8: a loop body is a row).  In registers
-// (k_w64_mmv) four columns of 2048 take 64 per lane, which leaves room for one chain per wavefront, and more columns for
+// Several columns of 2048 or 4096 with the activations in LDS (C = 4, 8: a loop body is a row).  In registers
+// (k_w64_mmv) four BF16 columns of 2048 take 64 per lane, which leaves room for one chain per wavefront, and more columns for
 // fewer wavefronts too; the launch then waits for the chains' lookups.  Here an instance takes 49 to 107 registers at any
-// column count: two chains per wavefront (NCH), which are at the same columns, so that one read of the activations (uint2
-// per lane, column and plane word) serves both.  What bounds it is the vector ALU: a column adds eight products and three
+// column count: two chains per wavefront (NCH), which are at the same columns, so that one read of the activations (8 or
+// 16 bytes per lane, column and plane word) serves both.  What bounds it is the vector ALU: a column adds eight products and three
 // and a half steps of a reduction to the 86 instructions of a step.  us, before and after:
 //   248320 x 2048, 2 / 3 / 4 / 5 / 6 / 7 / 8 columns: 131 / 141 / 151 / 208 / 224 / 238 / 303 -> 123 / 135 / 145 / 157 / 171 / 183 / 197
 //   131072 x 4096, 1 / 2 / 4 / 6 / 7: 120 / 164 / 188 / 353 / 366 -> 116 / 122 / 143 / 162 / 193 (eight columns of 4096 are one pass now)
 //   one unit per wavefront: 65536 x 2048, 5 / 8: 67 / 81 -> 50 / 63; 65536 x 4096, 2 / 4 / 5 / 8: 90 / 99 / 171 / 197 -> 73 / 83 / 89 / 112
-// Shorter rows stay with registers (131072 x 512 and 131072 x 1024, 2 to 8 columns: within 2.5 % either way).  Every column
+//   FP32 columns, 248320 x 2048, 1 / 2 / 3 / 4 / 5 / 6 / 8: 136 / 174 / 323 / 241 / 360 / 413 / 480 -> 130 / 139 / 151 / 163 / 179 / 195 / 245
+//   (five to eight are one pass now); 131072 x 4096, 1 / 2 / 3 / 4: 176 / 186 / 348 / 358 -> 130 / 143 / 148 / 175; 65536 x 2048, 1 / 2 / 4:
+//   43 / 58 / 66 -> 43 / 43 / 52; 65536 x 4096, 1 / 2 / 4: 93 / 97 / 193 -> 72 / 74 / 96
+// Shorter rows stay with registers (131072 x 512 and 131072 x 1024, 2 to 8 BF16 columns: within 2.5 % either way).  Every column
 // gets the bits of its single-column launch: the same products in the same order.
-typedef uint32_t uint2_v __attribute__((ext_vector_type(2)));
-typedef const __attribute__((address_space(3))) uint2_v * lds_u2;
-template <int C, int NC> constexpr size_t xl_bytes() { return (size_t) geom<C>::XS * NC * 4 * 64 * sizeof(uint2); }
+// a lane's four activations of a plane word, as they lie in LDS
+template <typename TX> struct xword;
+template <> struct xword<bf16_t> {
+    typedef uint32_t v __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ float dot(uint32_t w0, uint32_t w1, v x, float acc) { return dot2_bf16(w1, x.y, dot2_bf16(w0, x.x, acc)); }
+};
+template <> struct xword<float> {
+    typedef float v __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ float dot(uint32_t w0, uint32_t w1, v x, float acc) {
+        acc = fmaf(__uint_as_float(w0 << 16), x.x, acc);
+        acc = fmaf(__uint_as_float(w0 & 0xFFFF0000u), x.y, acc);
+        acc = fmaf(__uint_as_float(w1 << 16), x.z, acc);
+        return fmaf(__uint_as_float(w1 & 0xFFFF0000u), x.w, acc);
+    }
+};
+template <typename TX> using lds_x = const __attribute__((address_space(3))) typename xword<TX>::v *;
+template <typename TX, int C, int NC> constexpr size_t xl_bytes() { return (size_t) geom<C>::XS * NC * 4 * 64 * sizeof(typename xword<TX>::v); }
 
-template <int C, int NC, int N, int HINT>
-__device__ __forceinline__ void unit_pass_lds(chain<geom<C>::NB, HINT> (&ch)[2], const uint32_t * lut, lds_u2 xl, const cols & p,
+template <typename TX, int C, int NC, int N, int HINT>
+__device__ __forceinline__ void unit_pass_lds(chain<geom<C>::NB, HINT> (&ch)[2], const uint32_t * lut, lds_x<TX> xl, const cols & p,
                                               const col_view & cv, int R, int lane) {
     using G = geom<C>;
 #pragma unroll
@@ -330,7 +347,7 @@ __device__ __forceinline__ void unit_pass_lds(chain<geom<C>::NB, HINT> (&ch)[2],
             for (int j = 0; j < 4; j++) {
                 // (the address is opaque per word: the compiler would otherwise keep the activations in registers after all)
                 asm volatile("" : "+v"(xl));
-                uint2_v xv[NC];
+                typename xword<TX>::v xv[NC];
 #pragma unroll
                 for (int n = 0; n < NC; n++) {
                     xv[n] = xl[((s * NC + n) * 4 + j) * 64];
@@ -347,7 +364,7 @@ __device__ __forceinline__ void unit_pass_lds(chain<geom<C>::NB, HINT> (&ch)[2],
                 for (int n = 0; n < NC; n++) {
 #pragma unroll
                     for (int k = 0; k < N; k++) {
-                        acc[k][n] = dot2_bf16(w1[k], xv[n].y, dot2_bf16(w0[k], xv[n].x, s == 0 && j == 0 ? 0.f : acc[k][n]));
+                        acc[k][n] = xword<TX>::dot(w0[k], w1[k], xv[n], s == 0 && j == 0 ? 0.f : acc[k][n]);
                         // (pinned here: left alone the products of all words sink to the row's end, with their operands)
                         asm volatile("" : "+v"(acc[k][n]));
                     }
@@ -376,7 +393,7 @@ __device__ __forceinline__ void unit_pass_lds(chain<geom<C>::NB, HINT> (&ch)[2],
     }
 }
 
-template <int C, int NC, int NCH, int HINT>
+template <typename TX, int C, int NC, int NCH, int HINT>
 __global__ void __launch_bounds__(1024) k_w64_mmv_lds(const bf16n_weight w, const cols p, int units_per_wave) {
     using G = geom<C>;
     constexpr int K = C * CHUNK;
@@ -397,24 +414,25 @@ __global__ void __launch_bounds__(1024) k_w64_mmv_lds(const bf16n_weight w, cons
     for (int i = wave; i < G::XS * NC * 4; i += nwaves) { // (set, column, plane word) i of every lane
         const int j = i & 3, c = (i >> 2) % NC, set = (i >> 2) / NC;
         const int col0 = (2 * set + (lane >> 5)) * CHUNK + 128 * j + 4 * (lane & 31);
-        ((uint2 *) dyn)[i * 64 + lane] = *(const uint2 *) (cv.x + c * p.x_tok + 2 * col0);
+        typedef typename xword<TX>::v v;
+        ((v *) dyn)[i * 64 + lane] = *(const v *) (cv.x + c * p.x_tok + sizeof(TX) * col0);
     }
     __syncthreads();
     if (!live) {
         return;
     }
-    const lds_u2 xl = (lds_u2) dyn + lane;
+    const lds_x<TX> xl = (lds_x<TX>) dyn + lane;
     chain<G::NB, HINT> ch[2];
-    uint32_t * ring = dyn + xl_bytes<C, NC>() / 4 + wave * (NCH * WAVE_LDS_WORDS);
+    uint32_t * ring = dyn + xl_bytes<TX, C, NC>() / 4 + wave * (NCH * WAVE_LDS_WORDS);
     ch[0].start(ring, q, gu0, nA, u_begin * R, R, K, lane, b0, b1);
     if (NCH == 2 && nB > 0) {
         ch[1].start(ring + WAVE_LDS_WORDS, q, gu0 + nA, nB, (u_begin + nA) * R, R, K, lane, b1, b2);
     }
     for (int64_t i = 0; i < nA; i++) {
         if (NCH == 2 && i < nB) {
-            unit_pass_lds<C, NC, 2, HINT>(ch, lut, xl, p, cv, R, lane);
+            unit_pass_lds<TX, C, NC, 2, HINT>(ch, lut, xl, p, cv, R, lane);
         } else {
-            unit_pass_lds<C, NC, 1, HINT>(ch, lut, xl, p, cv, R, lane);
+            unit_pass_lds<TX, C, NC, 1, HINT>(ch, lut, xl, p, cv, R, lane);
         }
     }
 }
@@ -635,44 +653,44 @@ constexpr bool two_chains() { return x_regs<TX, C, NC>() <= 16; }
 // Instances with the activations in LDS (the figures stand at k_w64_mmv_lds).  Two chains per wavefront where the form with
 // registers has one (from two units per wavefront on); one chain where that form has registers for fewer than sixteen
 // wavefronts per CU (with sixteen of them either way the two measure the same: 65536 x 2048, 3 / 4 columns 46 us).
-template <int C, int NC, int NCH> constexpr bool lds_columns() {
-    return NCH == 2 ? C >= 4 && !two_chains<bf16_t, C, NC>() : wide_regs(x_regs<bf16_t, C, NC>(), true, C);
+template <typename TX, int C, int NC, int NCH> constexpr bool lds_columns() {
+    return NCH == 2 ? C >= 4 && !two_chains<TX, C, NC>() : wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2, C);
 }
-template <int C, int NC, int NCH> constexpr size_t lds_shm(int wpb) { return xl_bytes<C, NC>() + (size_t) wpb * NCH * WAVE_LDS_WORDS * 4; }
+template <typename TX, int C, int NC, int NCH> constexpr size_t lds_shm(int wpb) { return xl_bytes<TX, C, NC>() + (size_t) wpb * NCH * WAVE_LDS_WORDS * 4; }
 // wavefronts per block: eight, two blocks to a CU, where two copies of the activations fit beside the rings
-template <int C, int NC, int NCH> constexpr int lds_wpb() { return 2 * (lds_shm<C, NC, NCH>(8) + LUT_WORDS * 4) <= LDS_BYTES ? 8 : 16; }
+template <typename TX, int C, int NC, int NCH> constexpr int lds_wpb() { return 2 * (lds_shm<TX, C, NC, NCH>(8) + LUT_WORDS * 4) <= LDS_BYTES ? 8 : 16; }
 // f(NC as a type) for the instance of nc columns; false: there is none
-template <int C, int NCH, int NC = 1, typename F> bool with_lds(int nc, F f) {
+template <typename TX, int C, int NCH, int NC = 1, typename F> bool with_lds(int nc, F f) {
     if constexpr (NC <= 8) {
         if (nc != NC) {
-            return with_lds<C, NCH, NC + 1>(nc, f);
+            return with_lds<TX, C, NCH, NC + 1>(nc, f);
         }
-        if constexpr (lds_columns<C, NC, NCH>() && lds_shm<C, NC, NCH>(16) + LUT_WORDS * 4 <= LDS_BYTES) {
+        if constexpr (lds_columns<TX, C, NC, NCH>() && lds_shm<TX, C, NC, NCH>(16) + LUT_WORDS * 4 <= LDS_BYTES) {
             f(std::integral_constant<int, NC>{});
             return true;
         }
     }
     return false;
 }
-template <int C, int NCH> bool mmv_lds_launch(int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
-    return with_lds<C, NCH>(nc, [&](auto n) {
-        constexpr int NC = decltype(n)::value, wpb = lds_wpb<C, NC, NCH>();
+template <typename TX, int C, int NCH> bool mmv_lds_launch(int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
+    return with_lds<TX, C, NCH>(nc, [&](auto n) {
+        constexpr int NC = decltype(n)::value, wpb = lds_wpb<TX, C, NC, NCH>();
         const dim3 grid((unsigned) ((waves + wpb - 1) / wpb));
-        note_kernel("k_w64_mmv_lds", nullptr, 4, C, NC, NCH, (int) p.plane_once);
-        if (p.plane_once) hipLaunchKernelGGL((k_w64_mmv_lds<C, NC, NCH, 1>), grid, dim3(wpb * 64), (lds_shm<C, NC, NCH>(wpb)), stream, w, p, upw);
-        else              hipLaunchKernelGGL((k_w64_mmv_lds<C, NC, NCH, 0>), grid, dim3(wpb * 64), (lds_shm<C, NC, NCH>(wpb)), stream, w, p, upw);
+        note_kernel("k_w64_mmv_lds", tx_name<TX>(), 4, C, NC, NCH, (int) p.plane_once);
+        if (p.plane_once) hipLaunchKernelGGL((k_w64_mmv_lds<TX, C, NC, NCH, 1>), grid, dim3(wpb * 64), (lds_shm<TX, C, NC, NCH>(wpb)), stream, w, p, upw);
+        else              hipLaunchKernelGGL((k_w64_mmv_lds<TX, C, NC, NCH, 0>), grid, dim3(wpb * 64), (lds_shm<TX, C, NC, NCH>(wpb)), stream, w, p, upw);
     });
 }
-template <int NCH> bool mmv_lds(int C, int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
-    return C == 4 ? mmv_lds_launch<4, NCH>(nc, waves, upw, stream, w, p) : C == 8 && mmv_lds_launch<8, NCH>(nc, waves, upw, stream, w, p);
+template <typename TX, int NCH> bool mmv_lds(int C, int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
+    return C == 4 ? mmv_lds_launch<TX, 4, NCH>(nc, waves, upw, stream, w, p) : C == 8 && mmv_lds_launch<TX, 8, NCH>(nc, waves, upw, stream, w, p);
 }
-template <int C, int NCH> void set_attr_lds() {
+template <typename TX, int C, int NCH> void set_attr_lds() {
     for (int nc = 1; nc <= 8; nc++) {
-        with_lds<C, NCH>(nc, [](auto n) {
+        with_lds<TX, C, NCH>(nc, [](auto n) {
             constexpr int NC = decltype(n)::value;
-            const int shm = (int) lds_shm<C, NC, NCH>(lds_wpb<C, NC, NCH>());
-            (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<C, NC, NCH, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-            (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<C, NC, NCH, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+            const int shm = (int) lds_shm<TX, C, NC, NCH>(lds_wpb<TX, C, NC, NCH>());
+            (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<TX, C, NC, NCH, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+            (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<TX, C, NC, NCH, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
         });
     }
 }
@@ -690,17 +708,19 @@ void mmv_launch_hint(dim3 grid, int nt, int wpb, hipStream_t stream, const bf16n
     note_kernel("k_w64_mmv", tx_name<TX>(), 4, C, NC, 1, HINT);
     hipLaunchKernelGGL((k_w64_mmv<TX, C, NC, 1, HINT>), grid, dim3(nt), w64_shm(wpb), stream, w, p, upw);
 }
+// instances of k_w64_mmv that a launch can reach: not those of several columns of 2048 or more that fill the registers
+template <typename TX, int C, int NC> constexpr bool in_registers() { return NC == 1 || C < 4 || !wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2, C); }
 template <typename TX, int C, int NC>
 void mmv_launch(dim3 grid, int nt, int wpb, hipStream_t stream, const bf16n_weight & w, const cols & p, int upw) {
-    if (p.plane_once == p.stream_once) { // (what launch_w64_mmv sets; the run-time form stays for other callers)
-        if (p.plane_once) {
+    if constexpr (in_registers<TX, C, NC>()) {
+        if (p.plane_once != p.stream_once) { // (launch_w64_mmv sets both alike; the run-time form stays for other callers)
+            mmv_launch_hint<TX, C, NC, -1>(grid, nt, wpb, stream, w, p, upw);
+        } else if (p.plane_once) {
             mmv_launch_hint<TX, C, NC, 1>(grid, nt, wpb, stream, w, p, upw);
         } else {
             mmv_launch_hint<TX, C, NC, 0>(grid, nt, wpb, stream, w, p, upw);
         }
-        return;
     }
-    mmv_launch_hint<TX, C, NC, -1>(grid, nt, wpb, stream, w, p, upw);
 }
 
 template <typename TX, int C>
@@ -742,7 +762,7 @@ int group_for(int C) {
 
 template <typename TX, int C, int NC>
 void set_attr() {
-    if constexpr (NC <= max_group<TX, C>()) {
+    if constexpr (NC <= max_group<TX, C>() && in_registers<TX, C, NC>()) {
         (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(16));
         if constexpr (two_chains<TX, C, NC>()) {
             (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(32));
@@ -772,8 +792,8 @@ void w64_init() {
     set_attr_c<float>();
     set_attr_glu<bf16_t>();
     set_attr_glu<float>();
-    set_attr_lds<4, 2>(); set_attr_lds<8, 2>();
-    set_attr_lds<4, 1>(); set_attr_lds<8, 1>();
+    set_attr_lds<bf16_t, 4, 2>(); set_attr_lds<bf16_t, 8, 2>(); set_attr_lds<bf16_t, 4, 1>(); set_attr_lds<bf16_t, 8, 1>();
+    set_attr_lds<float, 4, 2>(); set_attr_lds<float, 8, 2>(); set_attr_lds<float, 4, 1>(); set_attr_lds<float, 8, 1>();
 }
 
 // shapes with a fused wave64 GEMV: K in {512, 1024, 2048, 4096} and units that hold whole loop bodies
@@ -790,7 +810,8 @@ void launch_w64_mmv(const bf16n_weight & w, const cols & p, int ncols, bool x_bf
     const int C = (int) (w.K / CHUNK);
     const int64_t units = p.nrows / w.R;
     // dense batches: groups of columns share one decode (max_group)
-    const int group_max = !multi_col || p.ids ? 1 : x_bf16 ? C == 8 ? 8 : group_for<bf16_t>(C) : group_for<float>(C);
+    const int in_lds = C == 4 || (C == 8 && x_bf16) ? 8 : C == 8 ? 4 : 0; // (k_w64_mmv_lds; FP32 columns of 4096: 64 KiB at four)
+    const int group_max = !multi_col || p.ids ? 1 : in_lds ? in_lds : x_bf16 ? group_for<bf16_t>(C) : group_for<float>(C);
     for (int c0 = 0; c0 < (group_max == 1 ? 1 : ncols); c0 += group_max) {
         const int nc = group_max == 1 ? 1 : (ncols - c0 < group_max ? ncols - c0 : group_max);
         const int ny = group_max == 1 ? ncols : 1;
@@ -807,11 +828,12 @@ void launch_w64_mmv(const bf16n_weight & w, const cols & p, int ncols, bool x_bf
             q.y += c0 * p.y_tok;
         }
         int wpb, blocks, upw;
-        if (x_bf16 && group_max > 1) {
+        if (group_max > 1) {
             w64_dims(units, ny, cus, wpb, blocks, upw);
             const int waves = (int) ((units + upw - 1) / upw);
             // (K = 4096: the rings of seven or eight columns leave room for one chain per wavefront)
-            if ((upw >= 2 && mmv_lds<2>(C, nc, waves, upw, stream, w, q)) || mmv_lds<1>(C, nc, waves, upw, stream, w, q)) {
+            if (x_bf16 ? (upw >= 2 && mmv_lds<bf16_t, 2>(C, nc, waves, upw, stream, w, q)) || mmv_lds<bf16_t, 1>(C, nc, waves, upw, stream, w, q)
+                       : (upw >= 2 && mmv_lds<float, 2>(C, nc, waves, upw, stream, w, q)) || mmv_lds<float, 1>(C, nc, waves, upw, stream, w, q)) {
                 continue;
             }
         }

@@ -1,4 +1,4 @@
-"""k_w64_mmv_lds (several BF16 columns of 2048 or 4096, activations in LDS): every column has the bits of its single-column
+"""k_w64_mmv_lds (several columns of 2048 or 4096, activations in LDS): every column has the bits of its single-column
 launch."""
 from __future__ import annotations
 
@@ -12,11 +12,12 @@ pytestmark = pytest.mark.gpu
 
 
 # one unit per wavefront (a single chain), two and a ragged end of three units (two chains, the second ends first)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("K,R,units", [(2048, 1, 64), (2048, 1, 8199), (4096, 1, 33), (4096, 1, 8199)])
-def test_columns_in_lds_equal_single_columns(ops, K, R, units):
+def test_columns_in_lds_equal_single_columns(ops, K, R, units, dtype):
     rows = units * R
     w = enc(ops, synth.weights(rows, K, K + units), 3, R, False, True)
-    x = synth.weights_torch(9, K, 5, "cuda")
+    x = synth.weights_torch(9, K, 5, "cuda").to(dtype)
     one = ops.mmv(x, w, multi_col=False)
     names = set()
     for t in range(1, 10):
