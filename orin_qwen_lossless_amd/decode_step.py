@@ -15,7 +15,7 @@ Per layer (pre-norm, residual stream h in BF16):
 expert is stacked behind the routed ones as expert 256 and runs as a ninth slot of every token with weight 1: its two
 products ride in the routed experts' launches instead of two launches of their own (run on a second stream beside the
 routed ones they cost more than in line: the fork and join of the graph outweighed them).  6 launches per layer while
-the experts run as GEMV columns (the gate / up launch selects them itself), 7 with the batched kernels up to 8 tokens
+the experts run as GEMV columns (the gate / up launch selects them itself), 7 with the batched kernels up to 12 tokens
 (selection and routing lists in one launch), 8 up to 16, 9 beyond."""
 from __future__ import annotations
 

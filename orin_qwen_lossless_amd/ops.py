@@ -688,8 +688,8 @@ def router_topk(logits: torch.Tensor, k: int, renorm: bool = True, out: tuple[to
 
 
 # router_topk_routes: tokens up to which one block that selects and sorts beats the two launches (its one CU runs a
-# wavefront per token: 7.7 / 8.6 / 12.4 us at 4 / 8 / 16 tokens against 4.6 + 5.4 us and the gap between two launches)
-TOPK_ROUTE_ONE_LAUNCH_TOKENS = 8
+# wavefront per token: 6.8 / 7.8 / 8.9 / 9.7 / 10.1 us at 4 / 8 / 12 / 14 / 16 tokens against 9.2 to 9.4 for the two in a graph)
+TOPK_ROUTE_ONE_LAUNCH_TOKENS = 12
 
 
 def router_topk_routes(logits: torch.Tensor, k: int, n_listed: int, renorm: bool = True,
