@@ -1420,7 +1420,7 @@ __global__ void __launch_bounds__(NB_WAVES * 64) k_nib_mm_ids(const bf16n_weight
 // barrier): 16-byte piece c of row r lies at c ^ (r / 2 % 8), so that sixteen lanes that read one piece of sixteen rows
 // meet all banks.  An operand is 32 rows: of the matrix, or sixteen of gate and the same sixteen of up, which end in the
 // same lanes.  A step is 128 columns: a line of plane bytes per row, and every second step a line of code bytes (taken 64
-// bytes at a time they came from HBM twice: FETCH_SIZE 1.2 times the weights).  Loads are one step (two steps) ahead in
+// bytes at a time they came from HBM twice: fetched 1.25 times the weights' bytes, now 1.04).  Loads are one step (two steps) ahead in
 // registers, over the end of an item too: 4 KiB per wavefront, sixteen wavefronts per CU.  77 tokens, fused gate / up and down:
 // 182 + 106 us with lanes that load their own rows, 138 + 79 here (5.4 TB/s of weights).  48 experts of 512 x 1536, 150 tokens,
 // whole call: 92 and 59.  In passes of 64 tokens this form measures as much as k_nib_mm_ids, in passes of 128 a third more
