@@ -109,7 +109,7 @@ class Bf16nStep:
         ops = self.ops
         q = ops.linear(x1, w["qkv"])
         o = ops.linear(q[:, :ATT], w["o"])
-        if ops.add_rmsnorm_mmv_supported(w["router"], h.shape[0]):
+        if ops.add_rmsnorm_mmv_supported(w["router"], h.shape[0], h, o):
             x2, h2, logits = ops.add_rmsnorm_mmv(h, w["router"], o)  # the router forms its own input
         else:
             (x2, h2), logits = ops.add_rmsnorm(h, o, want_sum=True), None

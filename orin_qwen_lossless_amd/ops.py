@@ -628,9 +628,11 @@ def add_rmsnorm(a: torch.Tensor, b: torch.Tensor | None = None, c: torch.Tensor 
 NORM_MMV_TOKENS = 16
 
 
-def add_rmsnorm_mmv_supported(w: Weight, n_tok: int) -> bool:
-    """Whether add_rmsnorm_mmv takes this matrix and is the faster way for n_tok tokens."""
-    return w.meta.format == FMT_NIBBLE and w.meta.K == 2048 and w.meta.rows <= 1024 and 0 < n_tok <= NORM_MMV_TOKENS
+def add_rmsnorm_mmv_supported(w: Weight, n_tok: int, *inputs: torch.Tensor) -> bool:
+    """Whether add_rmsnorm_mmv takes this matrix and these inputs (their 16-byte alignment, which add_rmsnorm does without)
+    and is the faster way for n_tok tokens."""
+    return (w.meta.format == FMT_NIBBLE and w.meta.K == 2048 and w.meta.rows <= 1024 and 0 < n_tok <= NORM_MMV_TOKENS
+            and all(t.data_ptr() % 16 == 0 for t in inputs))
 
 
 def add_rmsnorm_mmv(a: torch.Tensor, w: Weight, b: torch.Tensor | None = None, c: torch.Tensor | None = None,

@@ -110,3 +110,19 @@ def test_forty_layer_decode_step_as_one_graph(ops, sets40, T):
     assert float(err) <= 0.02, float(err)
     errx = (x1.double() - x1_ref).norm() / x1_ref.norm()
     assert float(errx) <= 0.02, float(errx)
+
+
+@pytest.mark.parametrize("T", [1, 16])
+def test_step_on_hidden_states_that_are_not_16_byte_aligned(ops, sets40, T, monkeypatch):
+    """A contiguous h at any storage offset: the router's launch, whose loads are 16 bytes, gives way to the two launches
+    it stands for."""
+    from orin_qwen_lossless_amd import decode_step as D, synth
+
+    sets, _ = sets40
+    step = D.Bf16nStep(ops, sets, None, 1, T)
+    h = torch.empty(T * D.K_MODEL + 1, dtype=torch.bfloat16, device="cuda")[1:].view(T, D.K_MODEL)
+    h.copy_(synth.activations_torch(T, D.K_MODEL, 5200, "cuda"))
+    assert h.is_contiguous() and h.data_ptr() % 16
+    got = step(h)
+    monkeypatch.setattr(ops, "NORM_MMV_TOKENS", 0)  # the two launches
+    assert torch.equal(got, step(h))
