@@ -156,7 +156,7 @@ int bf16n_add_rmsnorm(const uint16_t * a, const uint16_t * b, const uint16_t * c
                       void * stream);
 /* The same without ys for n = 2048, and the product of a 4-bit-code matrix of K = 2048 (a router) with y_norm in the same
  * launch: y[t] = W y_norm[t] in FP32, rows y_tok elements apart; bit for bit what bf16n_add_rmsnorm and bf16n_mmv give one
- * token at a time.  The results must not overlap the inputs. */
+ * token at a time.  The results must not overlap a, b, c, gamma or each other. */
 int bf16n_add_rmsnorm_mmv(const uint16_t * a, const uint16_t * b, const uint16_t * c, const uint16_t * gamma, uint16_t * y_sum, uint16_t * y_norm,
                           int n_tok, int64_t n, float eps, const bf16n_weight * w, float * y, int64_t y_tok, void * stream);
 

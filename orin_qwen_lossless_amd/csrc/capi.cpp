@@ -617,12 +617,22 @@ int bf16n_add_rmsnorm_mmv(const uint16_t * a, const uint16_t * b, const uint16_t
         p.a = a; p.b = b; p.c = c; p.gamma = gamma; p.y_sum = y_sum; p.y_norm = y_norm; p.n = n; p.eps = eps;
         require(dev::norm_nib_mmv_ok(*w, p) && y_tok >= w->rows,
                 "add_rmsnorm_mmv: rows of 2048 elements, 16-byte aligned, and a 4-bit-code matrix of that K with at most 65536 rows");
-        // (every block reads the token's inputs, one of them writes the results)
-        const auto apart = [&](const uint16_t * o) {
-            const auto clear = [&](const uint16_t * in, int64_t len) { return !o || !in || o + n_tok * n <= in || in + len <= o; };
-            return clear(a, n_tok * n) && clear(b, n_tok * n) && clear(c, n_tok * n) && clear(gamma, n);
+        // (every block reads the token's inputs; one block writes y_sum and y_norm and each its rows of y, in no order)
+        struct span { const void * at; int64_t len; };
+        const auto clear = [](const span & u, const span & v) {
+            return !u.at || !v.at || (uintptr_t) u.at + u.len <= (uintptr_t) v.at || (uintptr_t) v.at + v.len <= (uintptr_t) u.at;
         };
-        require(apart(y_sum) && apart(y_norm), "add_rmsnorm_mmv: the results must not overlap the inputs");
+        const int64_t row_bytes = n_tok * n * 2;
+        const span in[] = {{a, row_bytes}, {b, row_bytes}, {c, row_bytes}, {gamma, n * 2}};
+        const span out[] = {{y_sum, row_bytes}, {y_norm, row_bytes}, {y, ((n_tok - 1) * y_tok + w->rows) * 4}};
+        for (int i = 0; i < 3; i++) {
+            for (const span & s : in) {
+                require(clear(out[i], s), "add_rmsnorm_mmv: the results must not overlap the inputs");
+            }
+            for (int j = 0; j < i; j++) {
+                require(clear(out[i], out[j]), "add_rmsnorm_mmv: the results must not overlap each other");
+            }
+        }
         dev::launch_norm_nib_mmv(*w, p, y, y_tok, n_tok, (hipStream_t) stream);
         launch_check("add_rmsnorm_mmv");
     });

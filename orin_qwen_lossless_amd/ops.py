@@ -645,6 +645,8 @@ def add_rmsnorm_mmv(a: torch.Tensor, w: Weight, b: torch.Tensor | None = None, c
             raise ValueError("bf16n.add_rmsnorm_mmv: inputs must be contiguous bf16 [tokens, n] of one shape")
     if gamma is not None and not (gamma.is_cuda and gamma.dtype == torch.bfloat16 and gamma.is_contiguous() and gamma.numel() == a.shape[1]):
         raise ValueError("bf16n.add_rmsnorm_mmv: gamma must be contiguous bf16 [n]")
+    if any(t is not None and t.device != a.device for t in (b, c, gamma, w.plane, w.aux)):
+        raise ValueError("bf16n.add_rmsnorm_mmv: inputs on different devices")
     cw = _cweight(w)
     T, n = a.shape
     y, ysum = torch.empty_like(a), torch.empty_like(a)

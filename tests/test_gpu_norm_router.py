@@ -30,3 +30,36 @@ def test_router_that_forms_its_own_input_refuses_other_shapes(ops):
     w = enc(ops, synth.weights(16, 1024, 1), NIB, 0, False, False)
     with pytest.raises(ValueError):
         ops.add_rmsnorm_mmv(x, w)
+
+
+def test_router_that_forms_its_own_input_refuses_results_that_overlap(ops):
+    """Every block reads the token's inputs while others write: a result over an input or over another result is refused on
+    the host; results that touch end to end are not."""
+    import ctypes as C
+
+    from orin_qwen_lossless_amd import _lib
+
+    T, n, rows, y_tok = 3, 2048, 32, 40
+    row, prod = T * n * 2, (2 * y_tok + rows) * 4  # bytes
+    w = enc(ops, synth.weights(rows, n, 4), NIB, 0, False, False)
+    cw = ops._cweight(w)
+    buf = synth.activations_torch(1, 8 * T * n, 5, "cuda").view(torch.uint8).view(-1)
+    base = buf.data_ptr()
+    assert base % 16 == 0 and prod < row
+    at = {k: base + i * row for i, k in enumerate(("a", "b", "c", "gamma", "y_sum", "y_norm", "y"))}
+
+    def call(**moved):
+        p = dict(at, **moved)
+        return _lib.lib().bf16n_add_rmsnorm_mmv(p["a"], p["b"], p["c"], p["gamma"], p["y_sum"], p["y_norm"], T, n, C.c_float(1e-6), C.byref(cw),
+                                                p["y"], y_tok, ops._stream())
+
+    assert call() == 0
+    assert call(y=at["y_norm"] - prod, y_sum=at["y"]) == 0  # y ends where y_norm begins
+    torch.cuda.synchronize()
+    for k in ("a", "b", "c", "y_sum", "y_norm"):
+        assert call(y=at[k]) != 0 and call(y=at[k] + row - 4) != 0 and call(y=at[k] - prod + 4) != 0, k
+    assert call(y=at["gamma"] + 2 * n - 4) != 0 and call(y_sum=at["gamma"]) != 0
+    assert call(y_sum=at["y_norm"]) != 0 and call(y_norm=at["y_sum"] + row - 16) != 0
+    for k in ("a", "b", "c"):
+        assert call(y_norm=at[k]) != 0 and call(y_sum=at[k] + 16) != 0, k
+    torch.cuda.synchronize()
