@@ -17,6 +17,8 @@
 #include "dev_w64.h"
 #include "launchers.h"
 
+#include <stdexcept>
+
 namespace bf16n {
 namespace dev {
 
@@ -636,10 +638,10 @@ void w64_dims(int64_t units, int ncols, int cus, int & waves_per_block, int & bl
     units_per_wave = (int) upw;
 }
 
-// columns that share one decode (reference launch.cu:174-193 groups four; its eight-column kernels are
-// kernels.cuh:2002-2104).  Up to 64 activation registers per lane an instance runs sixteen wavefronts per CU; up to 128
-// (five to eight BF16 columns at K <= 2048, three or four at K = 4096, ...) eight to twelve wavefronts of up to 256
-// registers: a lower decode rate, but one pass over the matrix instead of two.
+// columns that share one decode in k_w64_mmv (reference launch.cu:174-193 groups four; its eight-column kernels are
+// kernels.cuh:2002-2104): what 128 activation registers per lane hold.  Up to 64 of them an instance runs sixteen
+// wavefronts per CU, beyond that (five to eight BF16 columns of 1024, ...) eight to twelve of up to 256 registers: a
+// lower decode rate, but one pass over the matrix instead of two.
 template <typename TX, int C>
 constexpr int max_group() {
     constexpr int per_col = x_regs<TX, C, 1>();
@@ -659,13 +661,14 @@ template <typename TX, int C, int NC, int NCH> constexpr bool lds_columns() {
 template <typename TX, int C, int NC, int NCH> constexpr size_t lds_shm(int wpb) { return xl_bytes<TX, C, NC>() + (size_t) wpb * NCH * WAVE_LDS_WORDS * 4; }
 // wavefronts per block: eight, two blocks to a CU, where two copies of the activations fit beside the rings
 template <typename TX, int C, int NC, int NCH> constexpr int lds_wpb() { return 2 * (lds_shm<TX, C, NC, NCH>(8) + LUT_WORDS * 4) <= LDS_BYTES ? 8 : 16; }
+template <typename TX, int C, int NC, int NCH> constexpr bool has_lds() { return lds_columns<TX, C, NC, NCH>() && lds_shm<TX, C, NC, NCH>(16) + LUT_WORDS * 4 <= LDS_BYTES; }
 // f(NC as a type) for the instance of nc columns; false: there is none
 template <typename TX, int C, int NCH, int NC = 1, typename F> bool with_lds(int nc, F f) {
     if constexpr (NC <= 8) {
         if (nc != NC) {
             return with_lds<TX, C, NCH, NC + 1>(nc, f);
         }
-        if constexpr (lds_columns<TX, C, NC, NCH>() && lds_shm<TX, C, NC, NCH>(16) + LUT_WORDS * 4 <= LDS_BYTES) {
+        if constexpr (has_lds<TX, C, NC, NCH>()) {
             f(std::integral_constant<int, NC>{});
             return true;
         }
@@ -709,39 +712,41 @@ void mmv_launch_hint(dim3 grid, int nt, int wpb, hipStream_t stream, const bf16n
     hipLaunchKernelGGL((k_w64_mmv<TX, C, NC, 1, HINT>), grid, dim3(nt), w64_shm(wpb), stream, w, p, upw);
 }
 // instances of k_w64_mmv that a launch can reach: not those of several columns of 2048 or more that fill the registers
-template <typename TX, int C, int NC> constexpr bool in_registers() { return NC == 1 || C < 4 || !wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2, C); }
-template <typename TX, int C, int NC>
-void mmv_launch(dim3 grid, int nt, int wpb, hipStream_t stream, const bf16n_weight & w, const cols & p, int upw) {
-    if constexpr (in_registers<TX, C, NC>()) {
-        if (p.plane_once != p.stream_once) { // (launch_w64_mmv sets both alike; the run-time form stays for other callers)
-            mmv_launch_hint<TX, C, NC, -1>(grid, nt, wpb, stream, w, p, upw);
-        } else if (p.plane_once) {
-            mmv_launch_hint<TX, C, NC, 1>(grid, nt, wpb, stream, w, p, upw);
-        } else {
-            mmv_launch_hint<TX, C, NC, 0>(grid, nt, wpb, stream, w, p, upw);
-        }
+template <typename TX, int C, int NC> constexpr bool in_registers() {
+    return NC <= max_group<TX, C>() && (NC == 1 || C < 4 || !wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2, C));
+}
+// columns that share one decode in either kernel (k_w64_mmv_lds: eight; four FP32 columns of 4096, 64 KiB)
+template <typename TX, int C> constexpr int group_cols() { return C < 4 ? max_group<TX, C>() : C == 8 && sizeof(TX) == 4 ? 4 : 8; }
+// every column count that launch_w64_mmv forms has an instance whatever the units per wavefront are
+template <typename TX, int C, int NC = 1> constexpr bool all_counts_have_instances() {
+    if constexpr (NC > group_cols<TX, C>()) {
+        return true;
+    } else {
+        return (in_registers<TX, C, NC>() || has_lds<TX, C, NC, 1>()) && all_counts_have_instances<TX, C, NC + 1>();
     }
 }
+static_assert(all_counts_have_instances<bf16_t, 1>() && all_counts_have_instances<bf16_t, 2>() && all_counts_have_instances<bf16_t, 4>() &&
+              all_counts_have_instances<bf16_t, 8>() && all_counts_have_instances<float, 1>() && all_counts_have_instances<float, 2>() &&
+              all_counts_have_instances<float, 4>() && all_counts_have_instances<float, 8>(), "a column count without a kernel");
 
-template <typename TX, int C>
+template <typename TX, int C, int NC = 1>
 void mmv_nc(int nc, dim3 grid, int nt, int wpb, hipStream_t stream, const bf16n_weight & w, const cols & p, int upw) {
-    constexpr int G = max_group<TX, C>();
-    if (nc == 1) {
-        mmv_launch<TX, C, 1>(grid, nt, wpb, stream, w, p, upw);
-    } else if (nc == 2) {
-        if constexpr (G >= 2) mmv_launch<TX, C, 2>(grid, nt, wpb, stream, w, p, upw);
-    } else if (nc == 3) {
-        if constexpr (G >= 3) mmv_launch<TX, C, 3>(grid, nt, wpb, stream, w, p, upw);
-    } else if (nc == 4) {
-        if constexpr (G >= 4) mmv_launch<TX, C, 4>(grid, nt, wpb, stream, w, p, upw);
-    } else if (nc == 5) {
-        if constexpr (G >= 8) mmv_launch<TX, C, 5>(grid, nt, wpb, stream, w, p, upw);
-    } else if (nc == 6) {
-        if constexpr (G >= 8) mmv_launch<TX, C, 6>(grid, nt, wpb, stream, w, p, upw);
-    } else if (nc == 7) {
-        if constexpr (G >= 8) mmv_launch<TX, C, 7>(grid, nt, wpb, stream, w, p, upw);
+    if constexpr (NC > 8) {
+        throw std::logic_error("bf16n: no wave64 product of that many columns");
     } else {
-        if constexpr (G >= 8) mmv_launch<TX, C, 8>(grid, nt, wpb, stream, w, p, upw);
+        if constexpr (in_registers<TX, C, NC>()) {
+            if (nc == NC) {
+                if (p.plane_once != p.stream_once) { // (launch_w64_mmv sets both alike; the run-time form stays for other callers)
+                    mmv_launch_hint<TX, C, NC, -1>(grid, nt, wpb, stream, w, p, upw);
+                } else if (p.plane_once) {
+                    mmv_launch_hint<TX, C, NC, 1>(grid, nt, wpb, stream, w, p, upw);
+                } else {
+                    mmv_launch_hint<TX, C, NC, 0>(grid, nt, wpb, stream, w, p, upw);
+                }
+                return;
+            }
+        }
+        mmv_nc<TX, C, NC + 1>(nc, grid, nt, wpb, stream, w, p, upw);
     }
 }
 
@@ -757,12 +762,12 @@ void mmv_c(int C, int nc, dim3 grid, int nt, int wpb, hipStream_t stream, const 
 
 template <typename TX>
 int group_for(int C) {
-    return C == 1 ? max_group<TX, 1>() : C == 2 ? max_group<TX, 2>() : C == 4 ? max_group<TX, 4>() : max_group<TX, 8>();
+    return C == 1 ? group_cols<TX, 1>() : C == 2 ? group_cols<TX, 2>() : C == 4 ? group_cols<TX, 4>() : group_cols<TX, 8>();
 }
 
 template <typename TX, int C, int NC>
 void set_attr() {
-    if constexpr (NC <= max_group<TX, C>() && in_registers<TX, C, NC>()) {
+    if constexpr (in_registers<TX, C, NC>()) {
         (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(16));
         if constexpr (two_chains<TX, C, NC>()) {
             (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(32));
@@ -809,9 +814,8 @@ bool w64_mmv_supported(const bf16n_weight & w, bool) {
 void launch_w64_mmv(const bf16n_weight & w, const cols & p, int ncols, bool x_bf16, bool multi_col, int cus, hipStream_t stream) {
     const int C = (int) (w.K / CHUNK);
     const int64_t units = p.nrows / w.R;
-    // dense batches: groups of columns share one decode (max_group)
-    const int in_lds = C == 4 || (C == 8 && x_bf16) ? 8 : C == 8 ? 4 : 0; // (k_w64_mmv_lds; FP32 columns of 4096: 64 KiB at four)
-    const int group_max = !multi_col || p.ids ? 1 : in_lds ? in_lds : x_bf16 ? group_for<bf16_t>(C) : group_for<float>(C);
+    // dense batches: groups of columns share one decode (group_cols)
+    const int group_max = !multi_col || p.ids ? 1 : x_bf16 ? group_for<bf16_t>(C) : group_for<float>(C);
     for (int c0 = 0; c0 < (group_max == 1 ? 1 : ncols); c0 += group_max) {
         const int nc = group_max == 1 ? 1 : (ncols - c0 < group_max ? ncols - c0 : group_max);
         const int ny = group_max == 1 ? ncols : 1;
