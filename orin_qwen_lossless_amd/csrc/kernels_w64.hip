@@ -15,6 +15,7 @@
 // FP32 (v_dot2_f32_bf16 for BF16 activations, v_fma_f32 for FP32 ones) and reduced across the wave once per row.
 #include "dev_common.h"
 #include "dev_w64.h"
+#include "launch_dims.h"
 #include "launchers.h"
 
 #include <stdexcept>
@@ -659,7 +660,8 @@ template <typename TX, int C, int NC, int NCH> constexpr bool lds_columns() {
     return NCH == 2 ? C >= 4 && !two_chains<TX, C, NC>() : wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2, C);
 }
 template <typename TX, int C, int NC, int NCH> constexpr size_t lds_shm(int wpb) { return xl_bytes<TX, C, NC>() + (size_t) wpb * NCH * WAVE_LDS_WORDS * 4; }
-// wavefronts per block: eight, two blocks to a CU, where two copies of the activations fit beside the rings
+// wavefronts per block of a launch that fills the device: eight, two blocks to a CU, where two copies of the activations fit
+// beside the rings (smaller launches: spread_waves)
 template <typename TX, int C, int NC, int NCH> constexpr int lds_wpb() { return 2 * (lds_shm<TX, C, NC, NCH>(8) + LUT_WORDS * 4) <= LDS_BYTES ? 8 : 16; }
 template <typename TX, int C, int NC, int NCH> constexpr bool has_lds() { return lds_columns<TX, C, NC, NCH>() && lds_shm<TX, C, NC, NCH>(16) + LUT_WORDS * 4 <= LDS_BYTES; }
 // f(NC as a type) for the instance of nc columns; false: there is none
@@ -675,23 +677,24 @@ template <typename TX, int C, int NCH, int NC = 1, typename F> bool with_lds(int
     }
     return false;
 }
-template <typename TX, int C, int NCH> bool mmv_lds_launch(int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
+template <typename TX, int C, int NCH> bool mmv_lds_launch(int nc, int waves, int upw, int cus, hipStream_t stream, const bf16n_weight & w, const cols & p) {
     return with_lds<TX, C, NCH>(nc, [&](auto n) {
-        constexpr int NC = decltype(n)::value, wpb = lds_wpb<TX, C, NC, NCH>();
+        constexpr int NC = decltype(n)::value;
+        const int wpb = spread_waves(waves, cus, lds_wpb<TX, C, NC, NCH>());
         const dim3 grid((unsigned) ((waves + wpb - 1) / wpb));
         note_kernel("k_w64_mmv_lds", tx_name<TX>(), 4, C, NC, NCH, (int) p.plane_once);
         if (p.plane_once) hipLaunchKernelGGL((k_w64_mmv_lds<TX, C, NC, NCH, 1>), grid, dim3(wpb * 64), (lds_shm<TX, C, NC, NCH>(wpb)), stream, w, p, upw);
         else              hipLaunchKernelGGL((k_w64_mmv_lds<TX, C, NC, NCH, 0>), grid, dim3(wpb * 64), (lds_shm<TX, C, NC, NCH>(wpb)), stream, w, p, upw);
     });
 }
-template <typename TX, int NCH> bool mmv_lds(int C, int nc, int waves, int upw, hipStream_t stream, const bf16n_weight & w, const cols & p) {
-    return C == 4 ? mmv_lds_launch<TX, 4, NCH>(nc, waves, upw, stream, w, p) : C == 8 && mmv_lds_launch<TX, 8, NCH>(nc, waves, upw, stream, w, p);
+template <typename TX, int NCH> bool mmv_lds(int C, int nc, int waves, int upw, int cus, hipStream_t stream, const bf16n_weight & w, const cols & p) {
+    return C == 4 ? mmv_lds_launch<TX, 4, NCH>(nc, waves, upw, cus, stream, w, p) : C == 8 && mmv_lds_launch<TX, 8, NCH>(nc, waves, upw, cus, stream, w, p);
 }
 template <typename TX, int C, int NCH> void set_attr_lds() {
     for (int nc = 1; nc <= 8; nc++) {
         with_lds<TX, C, NCH>(nc, [](auto n) {
             constexpr int NC = decltype(n)::value;
-            const int shm = (int) lds_shm<TX, C, NC, NCH>(lds_wpb<TX, C, NC, NCH>());
+            const int shm = (int) lds_shm<TX, C, NC, NCH>(16); // (spread_waves gives up to sixteen)
             (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<TX, C, NC, NCH, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
             (void) hipFuncSetAttribute((const void *) k_w64_mmv_lds<TX, C, NC, NCH, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
         });
@@ -836,8 +839,8 @@ void launch_w64_mmv(const bf16n_weight & w, const cols & p, int ncols, bool x_bf
             w64_dims(units, ny, cus, wpb, blocks, upw);
             const int waves = (int) ((units + upw - 1) / upw);
             // (K = 4096: the rings of seven or eight columns leave room for one chain per wavefront)
-            if (x_bf16 ? (upw >= 2 && mmv_lds<bf16_t, 2>(C, nc, waves, upw, stream, w, q)) || mmv_lds<bf16_t, 1>(C, nc, waves, upw, stream, w, q)
-                       : (upw >= 2 && mmv_lds<float, 2>(C, nc, waves, upw, stream, w, q)) || mmv_lds<float, 1>(C, nc, waves, upw, stream, w, q)) {
+            if (x_bf16 ? (upw >= 2 && mmv_lds<bf16_t, 2>(C, nc, waves, upw, cus, stream, w, q)) || mmv_lds<bf16_t, 1>(C, nc, waves, upw, cus, stream, w, q)
+                       : (upw >= 2 && mmv_lds<float, 2>(C, nc, waves, upw, cus, stream, w, q)) || mmv_lds<float, 1>(C, nc, waves, upw, cus, stream, w, q)) {
                 continue;
             }
         }
