@@ -11,9 +11,11 @@ from test_gpu_kernels import enc
 pytestmark = pytest.mark.gpu
 
 
-# one unit per wavefront (a single chain), two and a ragged end of three units (two chains, the second ends first)
+# one unit per wavefront (a single chain), two and a ragged end of three units (two chains, the second ends first); units of
+# one loop body (a row) and of several
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("K,R,units", [(2048, 1, 64), (2048, 1, 8199), (4096, 1, 33), (4096, 1, 8199)])
+@pytest.mark.parametrize("K,R,units", [(2048, 1, 64), (2048, 1, 8199), (4096, 1, 33), (4096, 1, 8199),
+                                       (2048, 16, 37), (2048, 4, 4099), (4096, 16, 9), (4096, 2, 4099)])
 def test_columns_in_lds_equal_single_columns(ops, K, R, units, dtype):
     rows = units * R
     w = enc(ops, synth.weights(rows, K, K + units), 3, R, False, True)
