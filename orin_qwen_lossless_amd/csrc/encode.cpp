@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -186,6 +187,7 @@ struct pair_code {
     std::vector<uint8_t> len;   // [65536]
     std::vector<uint16_t> code; // [65536]
     std::vector<uint32_t> lut;  // [4096], entry = e_odd << 23 | e_even << 7 | len
+    uint64_t bits = 0;          // of all the rows' codes
 };
 
 // four adjacent weights in one word: the two pair symbols (exponent of the first | exponent of the second << 8), and the
@@ -262,6 +264,7 @@ bool build_pair_code(const uint16_t * w, int64_t rows, int64_t K, pair_code & pc
         }
         pc.len[s] = (uint8_t) len[s];
         pc.code[s] = (uint16_t) code[s];
+        pc.bits += freq[s] * (uint64_t) len[s];
         const uint32_t ent = ((uint32_t) (s >> 8) << 23) | ((uint32_t) (s & 0xFF) << 7) | (uint32_t) len[s];
         const uint32_t lo = code[s] << (HP_LP - len[s]), hi = (code[s] + 1) << (HP_LP - len[s]);
         std::fill(pc.lut.begin() + lo, pc.lut.begin() + hi, ent);
@@ -586,11 +589,12 @@ bytes encode_hufpair(const uint16_t * w, int64_t rows, int64_t K, int R, bool cm
 // indexed by those 12 bits as they sit in the word (first code bit = index bit 0), i.e. the canonical table with
 // bit-reversed index.  unit_base has units + 1 entries (word index of each unit's first word and the end).
 //
-// One walk over the weights writes the units' words block by block into memory of their own, and when every unit's size
-// is known the blocks are copied into place (sizing the units in a walk of its own took longer than the copy).  The codes
-// of the four weights of a check go into the lane's words as one, and neither a full word nor a refill is a branch: both
-// are taken a third of the time, unpredictably.  With the plane written in the walk that counts the pairs: 16384 x 2048 on
-// eight cores 58.5 -> 32.5 ms; a load of that matrix with upload and verification, on sixteen, 15.0 -> 11.5.
+// One walk over the weights writes the units' words block by block.  A block goes into its place as soon as the blocks
+// before it have their sizes, and its memory is used again, so that the stream is held once (sizing the units in a walk of
+// its own took longer; holding every block to the end took 0.35 byte per weight more host memory).  The codes of the four
+// weights of a check go into the lane's words as one, and neither a full word nor a refill is a branch: both are taken a
+// third of the time, unpredictably.  With the plane written in the walk that counts the pairs: 16384 x 2048 on eight
+// cores 58.5 -> 32.5 ms; a load of that matrix with upload and verification, on sixteen, 15.0 -> 11.5.
 bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, bool cm, uint8_t * plane) {
     pair_code pc;
     if (!build_pair_code(w, rows, K, pc, plane)) {
@@ -609,13 +613,49 @@ bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, boo
             code[sidx] = bitrev(pc.code[sidx], pc.len[sidx]) | (uint32_t) pc.len[sidx] << 16;
         }
     }
+    aux_header h = {};
+    h.magic = MAGIC; h.format = FMT_HUFPAIR; h.K = (uint32_t) K; h.R = (uint32_t) R; h.rows = (uint64_t) rows;
+    h.off_a = HEADER_BYTES;
+    h.off_b = h.off_a + (4u << HP_LP);
+    h.off_d = (h.off_b + ((uint64_t) units + 1) * 4 + 15) & ~15ull;
+    h.off_c = h.off_d;
+    h.n_a = (uint64_t) units; h.flags = FLAG_WAVE64 | (cm ? FLAG_CHUNK_MAJOR : 0);
+    // at most 192 words per unit and a refill per 32 bits of codes (every lane leaves a rest: under two words per lane and
+    // unit too much, never touched); 1024 words of padding: a wave prefetches its stream in 1 KiB blocks and may run up to
+    // three blocks ahead.  Not zeroed as a whole: see below.
+    const uint64_t max_words = 192 * (uint64_t) units + pc.bits / 32;
+    bytes aux(h.off_d + (max_words + 1024) * 4);
+    uint32_t * const stream = (uint32_t *) (aux.data() + h.off_d);
     std::vector<uint64_t> ubase(units + 1, 0);
+    using word_buf = std::vector<uint32_t, uninit_allocator<uint32_t>>;
     constexpr int64_t UNITS = 8; // per block
-    std::vector<std::vector<uint32_t, uninit_allocator<uint32_t>>> words((size_t) ((units + UNITS - 1) / UNITS));
+    std::mutex mu;
+    std::map<int64_t, word_buf> waiting; // encoded blocks behind one that is not
+    int64_t next_block = 0;
+    uint64_t placed = 0;                 // words of the blocks before it
+    // block b of the stream is encoded; `out` comes back empty, with memory of a block that has been copied
+    auto place = [&](int64_t b, word_buf & out) {
+        std::vector<std::pair<uint64_t, word_buf>> ready; // (first word, words)
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            waiting.emplace(b, std::move(out));
+            for (auto it = waiting.begin(); it != waiting.end() && it->first == next_block; it = waiting.erase(it), next_block++) {
+                ready.emplace_back(placed, std::move(it->second));
+                placed += ready.back().second.size();
+            }
+            if (placed > max_words) {
+                invariant("wave64 stream size");
+            }
+        }
+        for (auto & r : ready) {
+            std::memcpy(stream + r.first, r.second.data(), r.second.size() * 4);
+            out = std::move(r.second);
+        }
+        out.clear();
+    };
     // a lane takes at most 24 bits per pair of codes: steps * 4 * 24 bits and the two leading ones, + the zero words behind
     const int64_t maxw = (steps * 4 * 24 + 2 + 31) / 32 + 5;
-    auto encode_block = [&](int64_t u0, int64_t u1, std::vector<uint32_t> & lane_words, std::vector<uint8_t> & order) {
-        auto & out = words[(size_t) (u0 / UNITS)];
+    auto encode_block = [&](int64_t u0, int64_t u1, std::vector<uint32_t> & lane_words, std::vector<uint8_t> & order, word_buf & out) {
         for (int64_t u = u0; u < u1; u++) {
             uint64_t acc[64];
             uint32_t nb[64], P[64];
@@ -667,8 +707,10 @@ bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, boo
     parallel_blocks(units, UNITS, [&](int64_t u0, int64_t u1) {
         std::vector<uint32_t> lane_words((size_t) (64 * maxw));
         std::vector<uint8_t> order((size_t) (steps * 4 * 64 + 1));
+        word_buf out;
         for (int64_t u = u0; u < u1; u += UNITS) { // (one thread gets all units in one call)
-            encode_block(u, std::min(u1, u + UNITS), lane_words, order);
+            encode_block(u, std::min(u1, u + UNITS), lane_words, order, out);
+            place(u / UNITS, out);
         }
     });
     for (int64_t u = 0; u < units; u++) {
@@ -678,17 +720,12 @@ bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, boo
     if (!(n_words + 1024 < (1ull << 32))) {
         invariant("n_words + 1024 < 2^32");
     }
-    aux_header h = {};
-    h.magic = MAGIC; h.format = FMT_HUFPAIR; h.K = (uint32_t) K; h.R = (uint32_t) R; h.rows = (uint64_t) rows;
-    h.off_a = HEADER_BYTES;
-    h.off_b = h.off_a + (4u << HP_LP);
-    h.off_d = (h.off_b + ((uint64_t) units + 1) * 4 + 15) & ~15ull;
-    h.off_c = h.off_d;
-    h.n_a = (uint64_t) units; h.n_b = n_words; h.flags = FLAG_WAVE64 | (cm ? FLAG_CHUNK_MAJOR : 0);
-    // 1024 words of padding: a wave prefetches its stream in 1 KiB blocks and may run up to three blocks ahead
-    // not zeroed as a whole: the copy writes every stream word; zero what it does not write (header padding, the gap
-    // before the stream, the padding behind it)
-    bytes aux(h.off_d + (n_words + 1024) * 4);
+    if (placed != n_words) {
+        invariant("wave64 stream size");
+    }
+    h.n_b = n_words;
+    aux.resize(h.off_d + (n_words + 1024) * 4);
+    // zero what the walk does not write: header padding, the gap before the stream, the padding behind it
     std::memset(aux.data(), 0, h.off_d);
     std::memset(aux.data() + h.off_d + n_words * 4, 0, 1024 * 4);
     std::memcpy(aux.data(), &h, sizeof(h));
@@ -700,12 +737,6 @@ bytes encode_hufpair_w64(const uint16_t * w, int64_t rows, int64_t K, int R, boo
     for (int64_t u = 0; u <= units; u++) {
         unit_base[u] = (uint32_t) ubase[u];
     }
-    uint32_t * stream = (uint32_t *) (aux.data() + h.off_d);
-    parallel_blocks((int64_t) words.size(), 8, [&](int64_t b0, int64_t b1) {
-        for (int64_t b = b0; b < b1; b++) {
-            std::memcpy(stream + ubase[b * UNITS], words[(size_t) b].data(), words[(size_t) b].size() * 4);
-        }
-    });
     return aux;
 }
 
