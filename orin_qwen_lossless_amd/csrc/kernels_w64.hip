@@ -240,7 +240,7 @@ constexpr int x_regs() { return NC * geom<C>::XS * (sizeof(TX) == 2 ? 8 : 16); }
 // eight chunks per row (they spilled at 128); these run in blocks of at most eight wavefronts
 constexpr bool wide_regs(int xr, bool x_bf16, int C) { return xr > 64 || (xr == 64 && (!x_bf16 || C == 8)); }
 
-template <typename TX, int C, int NC, int NCH, int HINT = -1>
+template <typename TX, int C, int NC, int NCH, int HINT>
 __global__ void __launch_bounds__(wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2, C) ? 512 : 1024) k_w64_mmv(const bf16n_weight w, const cols p, int units_per_wave) {
     using G = geom<C>;
     constexpr int K = C * CHUNK;
@@ -275,9 +275,9 @@ __global__ void __launch_bounds__(wide_regs(x_regs<TX, C, NC>(), sizeof(TX) == 2
     }
     chain<G::NB, HINT> ch[2];
     uint32_t * ring = rings + wave * (NCH * WAVE_LDS_WORDS);
-    ch[0].start(ring, q, gu0, nA, u_begin * R, R, K, lane, b0, b1, p.plane_once, p.stream_once);
+    ch[0].start(ring, q, gu0, nA, u_begin * R, R, K, lane, b0, b1);
     if (NCH == 2 && nB > 0) {
-        ch[1].start(ring + WAVE_LDS_WORDS, q, gu0 + nA, nB, (u_begin + nA) * R, R, K, lane, b1, b2, p.plane_once, p.stream_once);
+        ch[1].start(ring + WAVE_LDS_WORDS, q, gu0 + nA, nB, (u_begin + nA) * R, R, K, lane, b1, b2);
     }
     for (int64_t i = 0; i < nA; i++) {
         if (NCH == 2 && i < nB) {
@@ -739,9 +739,7 @@ void mmv_nc(int nc, dim3 grid, int nt, int wpb, hipStream_t stream, const bf16n_
     } else {
         if constexpr (in_registers<TX, C, NC>()) {
             if (nc == NC) {
-                if (p.plane_once != p.stream_once) { // (launch_w64_mmv sets both alike; the run-time form stays for other callers)
-                    mmv_launch_hint<TX, C, NC, -1>(grid, nt, wpb, stream, w, p, upw);
-                } else if (p.plane_once) {
+                if (p.plane_once) { // (launch_w64_mmv sets stream_once alike)
                     mmv_launch_hint<TX, C, NC, 1>(grid, nt, wpb, stream, w, p, upw);
                 } else {
                     mmv_launch_hint<TX, C, NC, 0>(grid, nt, wpb, stream, w, p, upw);
@@ -770,10 +768,12 @@ int group_for(int C) {
 
 template <typename TX, int C, int NC>
 void set_attr() {
-    if constexpr (in_registers<TX, C, NC>()) {
-        (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(16));
+    if constexpr (in_registers<TX, C, NC>()) { // (blocks of up to eight wavefronts: w64_dims)
+        (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 1, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(8));
+        (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 1, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(8));
         if constexpr (two_chains<TX, C, NC>()) {
-            (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(32));
+            (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 2, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(16));
+            (void) hipFuncSetAttribute((const void *) k_w64_mmv<TX, C, NC, 2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) w64_shm(16));
         }
     }
 }
