@@ -274,17 +274,20 @@ int bf16n_mmv(const bf16n_weight * w, const bf16n_mmv_args * a, void * stream, i
     });
 }
 
-// The kernel instance that the calling thread's last product (bf16n_mmv*, bf16n_mm_ids*) chose, as the profiler prints it
+// The kernel instance that the calling thread's last product (bf16n_mmv*, bf16n_mm_ids*, bf16n_add_rmsnorm_mmv) chose, as the profiler prints it
 // ("k_w64_mmv<bf16_t, 4, 1, 2, 1>"); an empty string before the first one or after one on a path that leaves no note.  The pointer stays valid until the thread's next call of this function.
 const char * bf16n_last_kernel(void) {
     const dev::kernel_note & k = dev::g_last_kernel;
     g_kernel_text.clear();
     if (k.name) {
-        g_kernel_text = std::string(k.name) + "<" + (k.tx ? k.tx : "");
-        for (int i = 0; i < k.n_args; i++) {
-            g_kernel_text += (i || k.tx ? ", " : "") + std::to_string(k.arg[i]);
+        g_kernel_text = k.name;
+        if (k.tx || k.n_args) { // (k_norm_nib_mmv is no template)
+            g_kernel_text += std::string("<") + (k.tx ? k.tx : "");
+            for (int i = 0; i < k.n_args; i++) {
+                g_kernel_text += (i || k.tx ? ", " : "") + std::to_string(k.arg[i]);
+            }
+            g_kernel_text += ">";
         }
-        g_kernel_text += ">";
     }
     return g_kernel_text.c_str();
 }

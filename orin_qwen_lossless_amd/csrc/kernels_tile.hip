@@ -2019,18 +2019,20 @@ int64_t nib_mm_ids_units_bound(int n_experts, int64_t n_pairs, int pass_tokens) 
 template <int NT>
 void nb_launch(const bf16n_weight & w, const bf16n_weight * up, const mm_args & a, int cus, hipStream_t stream) {
     const size_t shm = NT == 1 ? NF_SHM : nb_shm<NT>();
-    const dim3 grid((unsigned) (cus * std::max(1, (int) (160 * 1024 / shm))));
+    const dim3 grid((unsigned) (cus * std::max(1, (int) (LDS_BYTES / shm))));
     if constexpr (NT == 1) {
         // a stack of 2^27 weights outlasts the caches between two launches: its lines stay out of the way of the activations
         const bool once = w.rows * w.K >= ((int64_t) 1 << 27);
         auto go = [&](auto glu, const bf16n_weight & w1) {
             constexpr bool G = decltype(glu)::value;
+            note_kernel("k_nib_mm_few", G ? "true" : "false", 1, once);
             if (once) hipLaunchKernelGGL((k_nib_mm_few<G, true>), grid, dim3(NB_WAVES * 64), shm, stream, w, w1, a);
             else      hipLaunchKernelGGL((k_nib_mm_few<G, false>), grid, dim3(NB_WAVES * 64), shm, stream, w, w1, a);
         };
         if (up) go(std::true_type{}, *up);
         else    go(std::false_type{}, w);
     } else {
+        note_kernel("k_nib_mm_ids", up ? "true" : "false", 1, NT);
         if (up) hipLaunchKernelGGL((k_nib_mm_ids<true, NT>), grid, dim3(NB_WAVES * 64), shm, stream, w, *up, a);
         else    hipLaunchKernelGGL((k_nib_mm_ids<false, NT>), grid, dim3(NB_WAVES * 64), shm, stream, w, w, a);
     }

@@ -140,6 +140,35 @@ def test_which_token_counts_take_the_batched_kernels(ops):
         assert got == list(range(1, last_gemv + 1)), (fmt, R, got)
 
 
+def test_which_kernel_takes_how_many_pairs_per_expert(ops):
+    """k_nib_mm_few up to 28 routed pairs per expert on average, passes of 64 tokens up to 40, of 128 beyond; the
+    non-temporal hint from 2^27 weights on.  One product on each side of every line: the same bits (a token's sums do not
+    depend on the pass), and the last expert's last rows against FP64."""
+    E, N, K, topk = 16, 64, 512, 4
+    w = synth.weights_torch(E * N, K, 81, "cuda")
+    gate = nib(ops, w)
+    lines = {28: ("k_nib_mm_few<%s, 0>", 112), 29: ("k_nib_mm_ids<%s, 2>", 113), 40: ("k_nib_mm_ids<%s, 2>", 160), 41: ("k_nib_mm_ids<%s, 4>", 161)}
+    T_max = 161
+    x = synth.activations_torch(T_max, K, 82, "cuda")
+    ids = ((torch.arange(T_max, device="cuda", dtype=torch.int32)[:, None] * topk + torch.arange(topk, device="cuda", dtype=torch.int32)[None, :]) % E).contiguous()
+    ref = {}
+    for name, T in lines.values():
+        for up, glu in ((None, "false"), (gate, "true")):
+            y = ops.moe_mm_ids(x[:T], ids[:T], gate, E, up=up, out_dtype=torch.float32)
+            assert ops.last_kernel() == name % glu, T
+            if glu in ref:
+                assert torch.equal(y[:112], ref[glu]), T
+            else:
+                ref[glu] = y
+    t = int(torch.nonzero(ids[:112, topk - 1] == E - 1)[-1])
+    want = w[(E - 1) * N:].double() @ x[t].double()
+    bound = w[(E - 1) * N:].double().abs() @ x[t].double().abs()
+    assert torch.all((ref["false"][t, topk - 1].double() - want).abs() <= 1e-5 * bound)
+    big = nib(ops, synth.weights_torch(256 * 512, 1024, 83, "cuda"))
+    ops.moe_mm_ids(synth.activations_torch(2, 1024, 84, "cuda"), ids[:2], big, 256)
+    assert ops.last_kernel() == "k_nib_mm_few<false, 1>"
+
+
 def test_a_call_whose_unit_list_would_not_fit_is_refused(ops):
     """The batched kernel lists (expert, pass) units in LDS, 2048 at most: a call with more (experts + routed pairs / 128
     with the longest passes) is refused on the host instead of leaving the last experts uncomputed; the largest call

@@ -20,6 +20,7 @@ def test_router_that_forms_its_own_input(ops, rows, T, addends, gamma):
     xs = [torch.randn((T, 2048), generator=g, device="cuda").to(torch.bfloat16) for _ in range(addends)] + [None] * (3 - addends)
     gm = torch.randn(2048, generator=g, device="cuda").to(torch.bfloat16) if gamma else None
     y, s, p = ops.add_rmsnorm_mmv(xs[0], w, xs[1], xs[2], gamma=gm)
+    assert ops.last_kernel() == "k_norm_nib_mmv"
     y2, s2 = ops.add_rmsnorm(xs[0], xs[1], xs[2], gamma=gm, want_sum=True)
     assert torch.equal(y, y2) and torch.equal(s, s2)
     assert torch.equal(p, ops.mmv(y2, w, multi_col=False))
