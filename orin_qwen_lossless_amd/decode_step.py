@@ -68,7 +68,7 @@ def layer_bytes(nbytes: dict, tokens: int, expected: bool = False) -> int:
 
 def launches_per_layer(ops, tokens: int, gemv_path: bool) -> int:
     """Kernel launches of one layer of Bf16nStep: qkv, o, (glue,) router, (top-k,) gate / up, down, glue."""
-    glue = 0 if tokens <= ops.NORM_MMV_TOKENS else 1
+    glue = 0 if E * tokens <= ops.NORM_MMV_RESULTS else 1
     if gemv_path:
         return glue + (6 if getattr(ops, "TOPK_IN_EXPERT_GEMV", False) else 7)
     return glue + (7 if tokens <= ops.TOPK_ROUTE_ONE_LAUNCH_TOKENS else 8)
@@ -100,7 +100,7 @@ class Bf16nStep:
             hidden = ops.mmv_glu2_topk(x2, w["gate"], w["up"], logits, TOPK, N_MID, self.routing)
             return ops.mmv(hidden, w["down"], ids, K_MODEL), wts, ids
         if batched:
-            wts, ids, routes = ops.router_topk_routes(logits, TOPK, EA, out=self.routing)  # one launch up to 16 tokens
+            wts, ids, routes = ops.router_topk_routes(logits, TOPK, EA, out=self.routing)  # one launch up to 12 tokens
         else:
             wts, ids = ops.router_topk(logits, TOPK, out=self.routing)
         return ops.moe_experts_rows(x2, w["gate"], w["up"], w["down"], ids, EA, routes), wts, ids

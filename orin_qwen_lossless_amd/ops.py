@@ -624,14 +624,18 @@ def add_rmsnorm(a: torch.Tensor, b: torch.Tensor | None = None, c: torch.Tensor 
     return (y, ysum) if want_sum else y
 
 
-# tokens up to which add_rmsnorm_mmv (every block forms its token's row) beats the two launches
-NORM_MMV_TOKENS = 16
+# results (matrix rows x tokens) up to which add_rmsnorm_mmv beats the two launches: every block forms its token's row for two
+# rows of the matrix, so 4096 results are eight blocks of four wavefronts per CU, one round; beyond it the rows are formed
+# again in a second one.  us, one launch / two (in a graph): 256 rows at 1 / 16 / 24 tokens 3.3 / 6.7 / 8.1 against 5.5 / 7.4 / 7.9;
+# 64 rows at 64 / 128 7.0 / 11.7 against 7.7 / 9.0; 512 at 8 / 16 6.5 / 9.7 against 7.0 / 8.4; 1024 at 4 / 8 6.0 / 9.2 against
+# 7.3 / 7.5; 2048 at 2 / 4 6.0 / 9.5 against 6.9 / 7.2; 4096 at 1 / 2 6.2 / 9.4 against 7.2 / 7.0
+NORM_MMV_RESULTS = 4096
 
 
 def add_rmsnorm_mmv_supported(w: Weight, n_tok: int, *inputs: torch.Tensor) -> bool:
     """Whether add_rmsnorm_mmv takes this matrix and these inputs (their 16-byte alignment, which add_rmsnorm does without)
     and is the faster way for n_tok tokens."""
-    return (w.meta.format == FMT_NIBBLE and w.meta.K == 2048 and w.meta.rows <= 1024 and 0 < n_tok <= NORM_MMV_TOKENS
+    return (w.meta.format == FMT_NIBBLE and w.meta.K == 2048 and n_tok > 0 and w.meta.rows * n_tok <= NORM_MMV_RESULTS
             and all(t.data_ptr() % 16 == 0 for t in inputs))
 
 

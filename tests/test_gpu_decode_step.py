@@ -124,5 +124,5 @@ def test_step_on_hidden_states_that_are_not_16_byte_aligned(ops, sets40, T, monk
     h.copy_(synth.activations_torch(T, D.K_MODEL, 5200, "cuda"))
     assert h.is_contiguous() and h.data_ptr() % 16
     got = step(h)
-    monkeypatch.setattr(ops, "NORM_MMV_TOKENS", 0)  # the two launches
+    monkeypatch.setattr(ops, "NORM_MMV_RESULTS", 0)  # the two launches
     assert torch.equal(got, step(h))
