@@ -109,18 +109,21 @@ class Weight:
 
 # A small product is bound by the host's call (512 x 2048, one token: 14.9 us with torch's Python-level device guard and
 # stream objects and a view in and out, 9.3 without; the kernel takes 3.2), so the calls below stay off both when the
-# tensor's device is the current one anyway.
+# tensor's device is the current one anyway.  The two functions are private to torch (torch.cuda.current_device and the code
+# that torch.compile generates call them); where a release lacks them the public ones stand in.
 _HERE = contextlib.nullcontext()
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _on(device: torch.device):
     """A guard that makes `device` current."""
-    return _HERE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+    return _HERE if _current_device() == device.index else torch.cuda.device(device)
 
 
 def _stream() -> int:
     """The current stream of the current device."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return _raw_stream(_current_device())
 
 
 def _cweight(w: Weight) -> _lib.Weight:

@@ -17,6 +17,25 @@ def bf16(bits: np.ndarray) -> torch.Tensor:
     return torch.from_numpy(np.ascontiguousarray(bits).view(np.int16)).view(torch.bfloat16)
 
 
+def test_device_and_stream_without_torchs_private_functions():
+    """A torch without the two private functions: the public ones give the current device and its stream."""
+    import os
+    import subprocess
+    import sys
+
+    code = """
+import torch, types
+del torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+torch.cuda.current_device = lambda: 3
+torch.cuda.current_stream = lambda index: types.SimpleNamespace(cuda_stream=70 + index)
+from orin_qwen_lossless_amd import ops
+assert ops._stream() == 73
+assert ops._on(torch.device("cuda", 3)) is ops._HERE and ops._on(torch.device("cuda", 2)) is not ops._HERE
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([sys.executable, "-c", code], cwd=root, check=True, timeout=120)
+
+
 def test_schemas_match_the_reference_extension():
     want = {
         "encode": "bf16n::encode(Tensor w, int format, int R, bool chunk_major, bool frag_order=False) -> (Tensor, Tensor)",
