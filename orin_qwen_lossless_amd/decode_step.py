@@ -71,7 +71,7 @@ def launches_per_layer(ops, tokens: int, gemv_path: bool) -> int:
     glue = 0 if E * tokens <= ops.NORM_MMV_RESULTS else 1
     if gemv_path:
         return glue + (6 if getattr(ops, "TOPK_IN_EXPERT_GEMV", False) else 7)
-    return glue + (7 if tokens <= ops.TOPK_ROUTE_ONE_LAUNCH_TOKENS else 8)
+    return glue + (7 if tokens <= ops.topk_route_one_launch_tokens(E, TOPK, TOPK + 1) else 8)
 
 
 def routing_buffers(n_tok: int, device) -> tuple[torch.Tensor, torch.Tensor]:

@@ -698,22 +698,31 @@ def router_topk(logits: torch.Tensor, k: int, renorm: bool = True, out: tuple[to
     return wts, ids
 
 
-# router_topk_routes: tokens up to which one block that selects and sorts beats the two launches (its one CU runs a
-# wavefront per token: 6.8 / 7.8 / 8.9 / 9.7 / 10.1 us at 4 / 8 / 12 / 14 / 16 tokens against 9.2 to 9.4 for the two in a graph)
-TOPK_ROUTE_ONE_LAUNCH_TOKENS = 12
+# router_topk_routes: tokens up to which one block that selects and sorts is taken instead of two launches, whatever the sizes
+# (its one CU runs a wavefront per token; k of 256, us one launch / two in a graph: k = 8 at 4 / 8 tokens 6.4 / 7.4 against 7.7 / 7.8,
+# k = 32 at 8 18.7 against 19.3)
+TOPK_ROUTE_ONE_LAUNCH_TOKENS = 8
+
+
+def topk_route_one_launch_tokens(n_experts: int, k: int, n_slots: int) -> int:
+    """Tokens up to which router_topk_routes is one launch: 12 where the selection is short (four logits per lane, at most
+    nine picks) and the other way's list kernel has more than its eight slots: 8 of 256 with nine slots at 9 / 12 / 14
+    tokens takes 8.5 / 8.7 / 9.7 us against 9.3 / 9.2 / 9.3.  With eight slots (8.2 / 8.5 against 7.8 at 9 / 12), more experts (512: 15.1 / 15.7
+    against 12.0) or more picks (16: 12.6 / 13.1 against 12.2) the two launches are ahead from nine tokens on."""
+    return max(TOPK_ROUTE_ONE_LAUNCH_TOKENS, 12 if n_experts <= 256 and k <= 9 and 8 < n_slots <= 24 else 0)
 
 
 def router_topk_routes(logits: torch.Tensor, k: int, n_listed: int, renorm: bool = True,
                        out: tuple[torch.Tensor, torch.Tensor] | None = None):
     """router_topk followed by mm_ids_route(ids, n_listed, False) over every column of the id rows: (weights, ids,
-    (ids_src1, ids_dst, bounds)).  One launch (bf16n_router_topk_route) up to TOPK_ROUTE_ONE_LAUNCH_TOKENS tokens, two
-    beyond."""
+    (ids_src1, ids_dst, bounds)).  One launch (bf16n_router_topk_route) up to topk_route_one_launch_tokens(...) tokens,
+    two beyond."""
     if out is not None and not (out[1].dim() == 2 and out[1].shape[1] >= k):
         raise ValueError("bf16n.router_topk_routes: out must be (f32, int32) [tokens, m >= k] tensors")
     T = logits.shape[0] if logits.dim() == 2 else 0
     n_slots = out[1].shape[1] if out is not None else k
     L = _lib.lib()
-    if T == 0 or T > TOPK_ROUTE_ONE_LAUNCH_TOKENS or not L.bf16n_router_topk_route_fits(T, n_slots, n_listed):
+    if T == 0 or T > topk_route_one_launch_tokens(logits.shape[1], k, n_slots) or not L.bf16n_router_topk_route_fits(T, n_slots, n_listed):
         wts, ids = router_topk(logits, k, renorm, out)
         return wts, ids, mm_ids_route(ids, n_listed, False)
     if not (logits.is_cuda and logits.dtype == torch.float32 and logits.stride(1) == 1):

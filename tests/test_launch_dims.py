@@ -38,3 +38,12 @@ def test_where_the_router_forms_its_own_input(rows, last):
     if rows == decode_step.E:  # what a step reports is what it launches
         per_layer = [decode_step.launches_per_layer(ops, T, False) for T in (12, 13, 16, 17)]
         assert per_layer == [7, 8, 8, 9]
+
+
+@pytest.mark.parametrize("n_experts,k,n_slots,last", [(256, 8, 9, 12), (64, 2, 10, 12), (256, 8, 8, 8), (257, 8, 9, 8), (512, 8, 9, 8),
+                                                      (256, 10, 11, 8), (64, 4, 4, 8), (256, 9, 9, 12), (256, 1, 25, 8)])
+def test_where_selection_and_lists_are_one_launch(n_experts, k, n_slots, last):
+    """Nine to twelve tokens only where one launch was measured to be ahead."""
+    from orin_qwen_lossless_amd import ops
+
+    assert ops.topk_route_one_launch_tokens(n_experts, k, n_slots) == last
