@@ -1421,7 +1421,10 @@ __global__ void __launch_bounds__(NB_WAVES * 64) k_nib_mm_ids(const bf16n_weight
 // meet all banks.  An operand is 32 rows: of the matrix, or sixteen of gate and the same sixteen of up, which end in the
 // same lanes.  A step is 128 columns: a line of plane bytes per row, and every second step a line of code bytes (taken 64
 // bytes at a time they came from HBM twice: fetched 1.25 times the weights' bytes, now 1.04).  Loads are one step (two steps) ahead in
-// registers, over the end of an item too: 4 KiB per wavefront, sixteen wavefronts per CU.  77 tokens, fused gate / up and down:
+// registers, over the end of an item too: 4 KiB per wavefront, sixteen wavefronts per CU.  (Behind its last item a wavefront
+// asks for that item's first lines once more, 8 KiB that nothing uses: 33.6 MB of a launch that fills the device, from HBM
+// where the hint keeps them out of the caches.  77 tokens: 765 MB fetched for 733 of gate / up, 412 for 367 of down; a
+// descriptor of zero bytes would drop these loads.)  77 tokens, fused gate / up and down:
 // 182 + 106 us with lanes that load their own rows, 138 + 79 here (5.4 TB/s of weights).  48 experts of 512 x 1536, 150 tokens,
 // whole call: 92 and 59.  In passes of 64 tokens this form measures as much as k_nib_mm_ids, in passes of 128 a third more
 // (2048 tokens 588 against 433 us): an operand of activations serves one row group here and two there.
