@@ -507,7 +507,9 @@ __global__ void __launch_bounds__(NT) k_nib_mmv(const bf16n_weight w, const bf16
 // the token's row itself (12 KB at most, while its weights are on their way) and takes its two rows of the matrix from
 // there, and the first block stores the row.  The bits are those of k_add_rmsnorm8 and k_nib_mmv<bf16_t, 0, 1>.  256 rows,
 // one token: 3.9 us against 3.7 + 3.0 and the gap between two launches (three layers of the decode step 158 -> 150 us,
-// half a microsecond a layer of it by the faster selection); 16 tokens, two layers: 330 -> 325.
+// half a microsecond a layer of it by the faster selection); 16 tokens, two layers: 330 and 325, which is what runs differ by.
+// More than 4096 results (rows x tokens) form the rows again in a second round of blocks: the two launches then (the
+// operator layer's NORM_MMV_RESULTS has the figures).
 __global__ void __launch_bounds__(NT) k_norm_nib_mmv(const bf16n_weight w, const add_norm_args p, float * __restrict__ y, int64_t y_tok) {
     constexpr int C = NORM8_N / CHUNK, RPB = HALVES / C;
     static_assert(NT == NORM8_THREADS, "a thread per eight elements of the row");
