@@ -434,9 +434,17 @@ __device__ __forceinline__ float nib_escapes(const nib_ptrs & w, uint32_t e0, ui
 // pair, every load of a pair issued at once, the C chunk sums of a row combined through LDS in chunk order.
 // NC: columns per decode (dense batches: a (row, chunk) is decoded once for NC token columns, each of which gets the
 // bits of its single-column launch); columns past the last repeat it and are not stored.
-template <typename TX, int GLU, int NC>
+// RW: (row, chunk) pairs per half-wave and turn.  A launch is a few latencies of memory, so the more of its bytes are asked
+// for before the first wait the better, until a block's decode is longer than what it waits for.  The barrier keeps the
+// loads of all pairs ahead of the first decode: left alone the compiler waits for one pair before it asks for the next
+// (a gate / up pair of 512 x 2048 for two slots: 6.8 us, 5.3 with it, 5.2 with RW = 1).  us with RW = 1 / 2 (4 is behind 2 nearly everywhere):
+//   dense, one BF16 column: 2048 x 2048 3.55 / 3.35, 5120 x 2048 6.0 / 5.5, 2048 x 4096 5.3 / 5.1, 16384 x 512 5.0 / 4.7
+//   FP32, three / eight columns: 5120 x 2048 10.2 / 16.8 -> 8.2 / 12.9, 2048 x 4096 9.3 / 15.8 -> 8.0 / 12.7
+//   257 experts' down (2048 x 512), 1 / 4 / 12 tokens of nine slots: 6.8 / 18.1 / 47 -> 5.7 / 14.5 / 35.3; gate / up 8.8 / 24.8 / 65 -> 9.2 / 23.6 / 59
+template <typename TX, int GLU, int NC, int RW>
 __global__ void __launch_bounds__(NT) k_nib_mmv(const bf16n_weight w, const bf16n_weight w_up, const cols p, const int ncols) {
-    __shared__ float part[2][NC][HALVES];
+    constexpr int M = GLU ? 2 : 1;
+    __shared__ float part[RW][M][NC][HALVES];
     const int K = (int) w.K, C = K / CHUNK; // 1 .. 8
     col_view cv[NC];
 #pragma unroll
@@ -444,59 +452,93 @@ __global__ void __launch_bounds__(NT) k_nib_mmv(const bf16n_weight w, const bf16
         const int col = (int) blockIdx.y * NC + j;
         cv[j] = col_setup(p, col < ncols ? col : ncols - 1);
     }
-    const nib_ptrs g = nibp(w, 0);
-    const nib_ptrs u = GLU == 1 ? nibp(w, p.nrows) : nibp(w_up, 0);
+    const nib_ptrs q[2] = {nibp(w, 0), GLU == 1 ? nibp(w, p.nrows) : nibp(w_up, 0)};
     const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5;
-    const int rpb = HALVES / C; // rows per block: C half-waves per row (C = 3, 5, 6, 7 leave some half-waves idle)
+    const int rpb = HALVES / C; // rows per block and turn: C half-waves per row (C = 3, 5, 6, 7 leave some half-waves idle)
     const int lr = half / C, c = half % C;
-    for (int64_t base = (int64_t) blockIdx.x * rpb; base < p.nrows; base += (int64_t) gridDim.x * rpb) {
-        const bool live = lr < rpb && base + lr < p.nrows;
-        const int64_t r = live ? base + lr : 0;
-        const int64_t gr = cv[0].rbase + r; // dense batches share the rows; with expert ids NC is 1
-        uint32_t wg[8], wu[8];
-        const uint2 eg = make_uint2(g.esc_off[gr], g.esc_off[gr + 1]);
-        const uint2 eu = GLU ? make_uint2(u.esc_off[gr], u.esc_off[gr + 1]) : make_uint2(0, 0);
-        nib_load_chunk(g, gr, C, c, *(const uint4 *) (g.table + gr * 16), l32, wg);
-        if (GLU) {
-            nib_load_chunk(u, gr, C, c, *(const uint4 *) (u.table + gr * 16), l32, wu);
+    for (int64_t base = (int64_t) blockIdx.x * (rpb * RW); base < p.nrows; base += (int64_t) gridDim.x * (rpb * RW)) {
+        uint4 sm[RW][M], T[RW][M];
+        uint2 cd[RW][M], esc[RW][M];
+#pragma unroll
+        for (int t = 0; t < RW; t++) {
+            const int64_t r = base + t * rpb + lr, gr = cv[0].rbase + (lr < rpb && r < p.nrows ? r : 0); // dense batches share the rows; with expert ids NC is 1
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                sm[t][m] = *((const uint4 *) (q[m].plane + gr * K + c * CHUNK) + l32);
+                cd[t][m] = *((const uint2 *) (q[m].codes + gr * (K / 2) + c * (CHUNK / 2)) + l32);
+                T[t][m] = *(const uint4 *) (q[m].table + gr * 16);
+                esc[t][m] = make_uint2(q[m].esc_off[gr], q[m].esc_off[gr + 1]);
+            }
+        }
+        uint32_t xp[8];
+        float xv[16];
+        auto load_x = [&](int j) {
+            if constexpr (sizeof(TX) == 2) {
+                x_pairs16(cv[j].x, c * CHUNK + 4 * l32, xp);
+            } else {
+                x_chunk16<TX>(cv[j].x, c * CHUNK + 4 * l32, xv);
+            }
+        };
+        if constexpr (NC == 1) {
+            load_x(0);
+        }
+        if constexpr (RW > 1) {
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        uint32_t wp[RW][M][8];
+#pragma unroll
+        for (int t = 0; t < RW; t++) {
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                nib_chunk(sm[t][m], cd[t][m], T[t][m], wp[t][m]);
+            }
         }
 #pragma unroll
         for (int j = 0; j < NC; j++) {
-            float v, vu = 0.f;
-            if constexpr (sizeof(TX) == 2) {
-                uint32_t xp[8];
-                x_pairs16(cv[j].x, c * CHUNK + 4 * l32, xp);
-                v = nib_dot_pairs(wg, xp);
-                if (GLU) {
-                    vu = nib_dot_pairs(wu, xp);
-                }
-            } else {
-                float xv[16];
-                x_chunk16<TX>(cv[j].x, c * CHUNK + 4 * l32, xv);
-                v = nib_dot(wg, xv);
-                if (GLU) {
-                    vu = nib_dot(wu, xv);
+            float v[RW][M];
+            if constexpr (NC > 1) {
+                load_x(j);
+            }
+#pragma unroll
+            for (int t = 0; t < RW; t++) {
+#pragma unroll
+                for (int m = 0; m < M; m++) {
+                    if constexpr (sizeof(TX) == 2) {
+                        v[t][m] = nib_dot_pairs(wp[t][m], xp);
+                    } else {
+                        v[t][m] = nib_dot(wp[t][m], xv);
+                    }
                 }
             }
             if (c == 0) {
-                v += nib_escapes<TX>(g, eg.x, eg.y, cv[j].x, l32);
-                if (GLU) {
-                    vu += nib_escapes<TX>(u, eu.x, eu.y, cv[j].x, l32);
+#pragma unroll
+                for (int t = 0; t < RW; t++) {
+#pragma unroll
+                    for (int m = 0; m < M; m++) {
+                        v[t][m] += nib_escapes<TX>(q[m], esc[t][m].x, esc[t][m].y, cv[j].x, l32);
+                    }
                 }
             }
             if (l32 == 31) {
-                part[0][j][half] = v;
-                part[1][j][half] = vu;
+#pragma unroll
+                for (int t = 0; t < RW; t++) {
+#pragma unroll
+                    for (int m = 0; m < M; m++) {
+                        part[t][m][j][half] = v[t][m];
+                    }
+                }
             }
         }
         __syncthreads();
-        if (live && c == 0 && l32 < NC && (int) blockIdx.y * NC + l32 < ncols) {
-            float s = part[0][l32][half], su = part[1][l32][half];
+        const int t = l32 / NC, j = l32 % NC; // one lane per (turn, column) of the row's first half-wave
+        const int64_t r = base + t * rpb + lr;
+        if (c == 0 && lr < rpb && t < RW && r < p.nrows && (int) blockIdx.y * NC + j < ncols) {
+            float s = part[t][0][j][half], su = part[t][M - 1][j][half];
             for (int i = 1; i < C; i++) {
-                s += part[0][l32][half + i];
-                su += part[1][l32][half + i];
+                s += part[t][0][j][half + i];
+                su += part[t][M - 1][j][half + i];
             }
-            store_y(cv[0].y + l32 * p.y_tok, p.y_bf16, r, GLU ? su * silu(s) : s); // l32 > 0 only in dense batches
+            store_y(cv[0].y + j * p.y_tok, p.y_bf16, r, GLU ? su * silu(s) : s); // j > 0 only in dense batches
         }
         __syncthreads();
     }
@@ -758,8 +800,11 @@ __global__ void __launch_bounds__(NM_WAVES * 64) k_nib_mm16(const bf16n_weight w
     }
 }
 
-// exact rows of a NIBBLE matrix: FP32 or BF16, to out + i * stride (bytes); row index from ids (gather) or row0 + i
-template <bool BF>
+// exact rows of a NIBBLE matrix: FP32 or BF16, to out + i * stride (bytes); row index from ids (gather) or row0 + i.
+// AHEAD: chunks whose bytes are asked for together, the row's first four at most: a half-wave's row is otherwise one latency
+// of memory per chunk.  The barrier keeps them so.  us, one chunk at a time / this: dequant of 2048 x 2048 6.0 / 5.2, 2048 x 4096
+// 11.3 / 9.7, 3000 x 1536 5.6 / 5.3, 5120 x 2048 8.7 / 8.6 (37 MB read and written); 513 rows of 5120 x 2048 4.0 / 3.6, of 2048 x 4096 7.9 / 6.9
+template <bool BF, int AHEAD>
 __global__ void __launch_bounds__(NT) k_nib_rows(const bf16n_weight w, const char * __restrict__ ids, int64_t ids_s0, int64_t n,
                                                  int64_t row0, char * __restrict__ dst, int64_t dst_s1) {
     const nib_ptrs q = nibp(w, 0);
@@ -770,9 +815,7 @@ __global__ void __launch_bounds__(NT) k_nib_rows(const bf16n_weight w, const cha
         char * o = dst + i * dst_s1;
         const uint4 T = nib_rotated(*(const uint4 *) (q.table + gr * 16));
         const uint32_t e0 = q.esc_off[gr], e1 = q.esc_off[gr + 1];
-        for (int c = 0; c < C; c++) {
-            const uint4 sm = *((const uint4 *) (q.plane + gr * K + c * CHUNK) + l32);
-            const uint2 cd = *((const uint2 *) (q.codes + gr * (K / 2) + c * 256) + l32);
+        auto store = [&](int c, const uint4 sm, const uint2 cd) {
             uint32_t wp[8];
             nib_chunk<true>(sm, cd, T, wp);
             // the row's escapes go into the registers of the lane that holds their column: every element is stored once
@@ -798,6 +841,23 @@ __global__ void __launch_bounds__(NT) k_nib_rows(const bf16n_weight w, const cha
                 } else {
                     *(float4 *) (o + 4 * col) = make_float4(bf16_bits_to_f32(wp[2 * j] & 0xFFFFu), __uint_as_float(wp[2 * j] & 0xFFFF0000u),
                                                             bf16_bits_to_f32(wp[2 * j + 1] & 0xFFFFu), __uint_as_float(wp[2 * j + 1] & 0xFFFF0000u));
+                }
+            }
+        };
+        for (int c0 = 0; c0 < C; c0 += AHEAD) {
+            uint4 sm[AHEAD];
+            uint2 cd[AHEAD];
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) { // (past the end the last chunk again, unused)
+                const int c = c0 + i < C ? c0 + i : C - 1;
+                sm[i] = *((const uint4 *) (q.plane + gr * K + c * CHUNK) + l32);
+                cd[i] = *((const uint2 *) (q.codes + gr * (K / 2) + c * 256) + l32);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) {
+                if (c0 + i < C) {
+                    store(c0 + i, sm[i], cd[i]);
                 }
             }
         }
@@ -926,13 +986,20 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
         const bool fills = blocks1 >= 4 * (int64_t) cus; // one column's blocks keep every CU busy by themselves
         const int nc = p.ids ? 1 : fills ? (ncols >= 3 ? 4 : ncols == 2 ? 2 : 1) : ncols >= 16 ? 4 : ncols >= 8 ? 2 : 1;
         const int ngroups = (ncols + nc - 1) / nc;
-        const dim3 grid(grid_for((p.nrows + rpb - 1) / rpb * HALVES, ngroups, cus), ngroups);
-        note_kernel("k_nib_mmv", x_bf16 ? "bf16_t" : "float", 2, glu, nc);
-#define NIBC(TX, G, N) hipLaunchKernelGGL((k_nib_mmv<TX, G, N>), grid, dim3(NT), 0, stream, w, wu, p, ncols)
-#define NIB(TX, G) do { if (nc == 4) NIBC(TX, G, 4); else if (nc == 2) NIBC(TX, G, 2); else NIBC(TX, G, 1); } while (0)
+        // two (row, chunk) pairs per half-wave from three blocks per CU on, gate and up (twice the loads to a pair) from
+        // sixteen: 256 x 2048, eight FP32 columns (two per CU) 3.3 us with one pair, 3.6 with two, 512 x 2048, three columns 3.4 and 3.3;
+        // gate / up of 512 x 2048, nine slots (nine per CU) 8.8 and 9.2, of 1024 x 1536 (eighteen) 13.0 and 11.7
+        const int rw = blocks1 * ngroups >= (glu ? 16 : 3) * (int64_t) cus ? 2 : 1;
+        const int64_t per = (int64_t) rpb * rw;
+        const dim3 grid(grid_for((p.nrows + per - 1) / per * HALVES, ngroups, cus), ngroups);
+        note_kernel("k_nib_mmv", x_bf16 ? "bf16_t" : "float", 3, glu, nc, rw);
+#define NIBC(TX, G, N, R) hipLaunchKernelGGL((k_nib_mmv<TX, G, N, R>), grid, dim3(NT), 0, stream, w, wu, p, ncols)
+#define NIBR(TX, G, N) do { if (rw == 2) NIBC(TX, G, N, 2); else NIBC(TX, G, N, 1); } while (0)
+#define NIB(TX, G) do { if (nc == 4) NIBR(TX, G, 4); else if (nc == 2) NIBR(TX, G, 2); else NIBR(TX, G, 1); } while (0)
         if (x_bf16) { if (glu == 0) NIB(bf16_t, 0); else if (glu == 1) NIB(bf16_t, 1); else NIB(bf16_t, 2); }
         else        { if (glu == 0) NIB(float, 0);  else if (glu == 1) NIB(float, 1);  else NIB(float, 2); }
 #undef NIB
+#undef NIBR
 #undef NIBC
         return;
     }
@@ -966,14 +1033,23 @@ void launch_norm_nib_mmv(const bf16n_weight & w, const add_norm_args & a, float 
     hipLaunchKernelGGL(k_norm_nib_mmv, dim3((unsigned) ((w.rows + RPB - 1) / RPB), n_tok), dim3(NT), 0, stream, w, a, y, y_tok);
 }
 
+// (rows of one or two chunks: one at a time; 16384 x 512 measured 7.1 us so and 7.3 with four ahead, 8192 x 1024 6.6, with two 7.3, with four 6.9)
+static void launch_nib_rows(const bf16n_weight & w, const char * ids, int64_t ids_s0, int64_t n, int64_t row0, char * dst, bool dst_bf16,
+                            int64_t dst_s1, dim3 grid, hipStream_t stream) {
+#define ROWS(BF, A) hipLaunchKernelGGL((k_nib_rows<BF, A>), grid, dim3(NT), 0, stream, w, ids, ids_s0, n, row0, dst, dst_s1)
+#define ROWSA(BF) do { if (w.K <= 2 * CHUNK) ROWS(BF, 1); else ROWS(BF, 4); } while (0)
+    if (dst_bf16) ROWSA(true); else ROWSA(false);
+#undef ROWSA
+#undef ROWS
+}
+
 void launch_compat_dequant(const bf16n_weight & w, int64_t row0, int64_t nrows, uint16_t * out, int cus, hipStream_t stream) {
     const int64_t work = w.format == FMT_NIBBLE ? nrows : nrows / w.R;
     const int waves = w.format == FMT_NIBBLE ? NT / 64 : huf_waves(work, 1, cus, w.R * (int) (w.K / CHUNK));
     const int64_t blocks = (work + 2 * waves - 1) / (2 * waves);
     const dim3 grid((unsigned) (blocks < (int64_t) cus * 16 ? blocks : (int64_t) cus * 16));
     if (w.format == FMT_NIBBLE) {
-        hipLaunchKernelGGL((k_nib_rows<true>), grid, dim3(NT), 0, stream, w, (const char *) nullptr, (int64_t) 0, nrows, row0,
-                           (char *) out, (int64_t) w.K * 2);
+        launch_nib_rows(w, nullptr, 0, nrows, row0, (char *) out, true, (int64_t) w.K * 2, grid, stream);
     } else if (w.format == FMT_HUFPAIR) {
         hipLaunchKernelGGL((k_huf_dequant<FMT_HUFPAIR>), grid, dim3(waves * 64), 0, stream, w, row0, nrows, out);
     } else {
@@ -985,8 +1061,7 @@ void launch_compat_get_rows(const bf16n_weight & w, const void * ids, int64_t id
                             int64_t dst_s1, int64_t row0, hipStream_t stream) {
     const dim3 grid((unsigned) ((n + HALVES - 1) / HALVES));
     if (w.format == FMT_NIBBLE) {
-        if (dst_bf16) hipLaunchKernelGGL((k_nib_rows<true>), grid, dim3(NT), 0, stream, w, (const char *) ids, ids_s0, n, row0, (char *) dst, dst_s1);
-        else          hipLaunchKernelGGL((k_nib_rows<false>), grid, dim3(NT), 0, stream, w, (const char *) ids, ids_s0, n, row0, (char *) dst, dst_s1);
+        launch_nib_rows(w, (const char *) ids, ids_s0, n, row0, (char *) dst, dst_bf16, dst_s1, grid, stream);
     } else {
         if (dst_bf16) hipLaunchKernelGGL((k_hp_get_rows<true>), grid, dim3(NT), 0, stream, w, (const char *) ids, ids_s0, n, row0, (char *) dst, dst_s1);
         else          hipLaunchKernelGGL((k_hp_get_rows<false>), grid, dim3(NT), 0, stream, w, (const char *) ids, ids_s0, n, row0, (char *) dst, dst_s1);
