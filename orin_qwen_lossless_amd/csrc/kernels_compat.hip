@@ -4,6 +4,7 @@
 // A wave64 carries two units (HUFPAIR / HUFFMAN) or two rows (NIBBLE): lanes 0..31 the even one, lanes 32..63 the odd
 // one; each half reads its 512-byte plane chunk with one 16-byte load per lane, four chunks ahead.  Lane streams pass
 // through rings in LDS (lane_ring), except in products with enough wavefronts to cover each other's misses (huf_direct).
+// Dense products and exact rows of few HUFPAIR units take a block per unit instead (k_hp_split).
 // These kernels take any K, R, layout, expert ids and FP32 or BF16 activations; the wave64 layout (kernels_w64.hip),
 // which has twice the chains per unit, is the fast path.
 #include "dev_common.h"
@@ -21,6 +22,7 @@ namespace {
 constexpr int NT = 256;          // threads per block
 constexpr int NIB_MM_MIN_COLS = 5; // dense NIBBLE batches of BF16 columns go through the matrix cores from this many on at the earliest
 constexpr int HALVES = NT / 32;  // units (rows) per block
+constexpr int LUT_PAIRS = 1 << HP_LP;
 
 // One lane's MSB-first bit stream, read through a ring of 16 words in LDS.  What bounds these kernels is the chain of
 // one unit (two dependent table lookups per two codes, all lanes of a half-wave in step), so nothing else may be waited
@@ -380,6 +382,235 @@ __device__ __forceinline__ void nib_load_chunk(const nib_ptrs & w, int64_t gr, i
     const uint4 sm = *((const uint4 *) (w.plane + gr * K + c * CHUNK) + l32);
     const uint2 cd = *((const uint2 *) (w.codes + gr * (K / 2) + c * 256) + l32);
     nib_chunk(sm, cd, T, wp);
+}
+
+// ---------------------------------------------------------------- HUFPAIR units, a lane's stream in segments
+//
+// With one half-wave per unit (above) a matrix of few units is the chain of one lane: R K / 64 pair codes one after the other
+// on a device that is otherwise idle (8192 x 2048, R = 16: 512 units, two per CU).  Here a block takes a unit and S threads a
+// lane's stream, each a segment of its bits.  Where the first code of a segment begins is not stored, but a prefix code falls
+// into step by itself after a few codes: every thread decodes from its segment's first bit and notes where the first code
+// past its end begins, then again from where the thread before it ended, until no beginning changes any more.  The first
+// segment's is known, so all are then exact: after two rounds nearly always, after S at worst (codes of one length never fall
+// into step; of normal weights' codes 3 in 100 starts take more than 16, 1 in 1000 more than 32: the first round begins half a
+// segment early, 48 codes, because one thread out of step costs its block another round).
+// The number of codes in the segments before it gives a thread its place, and a last round writes the exponents to LDS in the
+// order of the plane.  The products are those of unit_dot, a row per half-wave, added in the same order: the same bits.
+// Two rounds and a half of a sixteenth of the chain instead of the chain, for as many lookups per code: for launches that wait for
+// the chain (hp_split_cols).  8192 x 2048, one column: 42.4 -> 26.6 us (34 with a third round that wrote the exponents: the
+// codes of the second stay in registers until their place is known).
+constexpr int SPLIT_PAIRS = 32;                  // pair codes per segment at most
+constexpr int SPLIT_PAD = 4;                     // words in front of and behind the staged streams
+constexpr int SPLIT_KEEP = 24;                   // twice as many of a segment's codes stay in registers
+constexpr int SPLIT_AHEAD = 4;                   // plane chunks of a row asked for before its streams are decoded
+// words of a unit's streams at most: twelve bits a pair code, the last word of each lane begun
+__host__ __device__ constexpr uint32_t split_words(int pairs) { return (uint32_t) (HP_LP * pairs + 32); }
+constexpr size_t split_shm(int pairs, int threads) {
+    return ((size_t) LUT_PAIRS + split_words(pairs) + 2 * SPLIT_PAD + 16 * (size_t) pairs + 2 * (size_t) threads + (size_t) threads / 32 + 1) * 4;
+}
+
+// A position in the words at st.  n: minus the bit position; its low five bits are what the funnel shift takes (the next 32
+// bits are in w0:w1, w0 used up where they are zero), and a word boundary is passed where bit 5 changes (24 bits at a time
+// at most).  nw: the word after w1.  Words past the staged ones are read and not used: the padding, then what follows in LDS.
+struct seg_bits {
+    const uint32_t * st;
+    uint32_t w0, w1, nw, n;
+    __device__ __forceinline__ uint32_t ahead() const { // the word after w1
+        return *(const uint32_t *) ((const char *) st + 4 - (((int32_t) n >> 3) & ~3));
+    }
+    __device__ __forceinline__ seg_bits(const uint32_t * st_, uint32_t pos) : st(st_), n(0u - pos) {
+        const uint32_t j = (pos + 31) >> 5;
+        w0 = st[(int) j - 1]; // (in front of the first word: unused)
+        w1 = st[j];
+        nw = ahead();
+    }
+    // the next pair code, and the one after it if it begins before bit `nstop` (as n); returns how many.  e: the entries' sum has the
+    // length of both in its low five bits; an entry of unused codes, met out of step only, was given a length when staged
+    __device__ __forceinline__ bool two(const uint32_t * lut, uint32_t nstop, uint32_t & e0, uint32_t & e1) {
+        const uint32_t W = __builtin_amdgcn_alignbit(w0, w1, n);
+        e0 = lut[W >> (32 - HP_LP)];
+        e1 = lut[(W << (e0 & 31u)) >> (32 - HP_LP)];
+        const bool both = (int32_t) (n - (e0 & 31u)) > (int32_t) nstop;
+        const uint32_t to = n - ((e0 + (both ? e1 : 0u)) & 31u);
+        const bool m = ((to ^ n) & 32u) != 0;
+        n = to;
+        w0 = m ? w1 : w0;
+        w1 = m ? nw : w1;
+        nw = ahead();
+        return both;
+    }
+};
+
+// DEQ: the exact BF16 bits of the rows to out, no products
+template <typename TX, bool DEQ>
+__global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const cols p, int ncols, uint16_t * __restrict__ out) {
+    extern __shared__ __align__(16) unsigned char shm_raw[];
+    const int K = (int) w.K, C = K / CHUNK, R = w.R, pairs = R * C * 8, S = (int) blockDim.x >> 5;
+    const uint32_t cap = split_words(pairs);
+    uint32_t * lut = (uint32_t *) shm_raw;
+    uint32_t * st = lut + LUT_PAIRS + SPLIT_PAD;
+    uint16_t * ex = (uint16_t *) (st + cap + SPLIT_PAD); // [chunk][lane][8 pairs], an exponent per byte
+    uint32_t * ends = (uint32_t *) (ex + 32 * pairs), * counts = ends + blockDim.x, * again = counts + blockDim.x; // [round]
+    const hp_ptrs q = hpp(w);
+    const int tid = threadIdx.x, l32 = tid & 31, seg = tid >> 5;
+    const bool cm = (w.flags & FLAG_CHUNK_MAJOR) != 0;
+    for (int i = tid; i < LUT_PAIRS / 4; i += (int) blockDim.x) {
+        uint4 v = ((const uint4 *) q.lut)[i];
+        v.x += (v.x & 31u) == 0; v.y += (v.y & 31u) == 0; v.z += (v.z & 31u) == 0; v.w += (v.w & 31u) == 0;
+        ((uint4 *) lut)[i] = v;
+    }
+    const int64_t units = p.nrows / R, all_units = w.rows / R;
+    for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
+        const int64_t gu = p.row0 / R + u;
+        const uint4 * plane = (const uint4 *) (w.plane + gu * R * (int64_t) K) + l32;
+        auto chunk_at = [&](int rr, int c) { return cm ? c * R + rr : rr * C + c; }; // in stream order
+        const uint32_t base = q.ubase[gu], end = gu + 1 < all_units ? q.ubase[gu + 1] : (uint32_t) ((const aux_header *) w.aux)->n_b;
+        const uint32_t words = end - base < cap ? end - base : cap;
+        uint32_t from = q.lrel[gu * 32 + l32], to = l32 < 31 ? q.lrel[gu * 32 + l32 + 1] : words;
+        from = from < words ? from : words;
+        to = to < from ? from : to < words ? to : words;
+        uint4 ahead[SPLIT_AHEAD];
+#pragma unroll
+        for (int i = 0; i < SPLIT_AHEAD; i++) {
+            ahead[i] = plane[chunk_at(seg < R ? seg : R - 1, i < C ? i : C - 1) * 32];
+        }
+#pragma unroll 8
+        for (uint32_t i = tid; i < words; i += blockDim.x) {
+            st[i] = q.stream[base + i];
+        }
+        if (tid <= S) {
+            again[tid] = 0;
+        }
+        __syncthreads();
+        const uint32_t first = 32 * from, bits = 32 * (to - from); // (at most 24 K)
+        const uint32_t nstop = 0u - (first + bits * (uint32_t) (seg + 1) / (uint32_t) S);
+        uint32_t start = first + bits * (uint32_t) seg / (uint32_t) S - (seg ? bits / (uint32_t) (2 * S) : 0), n = 0;
+        auto pair = [](uint32_t e) { return (e >> 7 & 0xFFu) | (e >> 15 & 0xFF00u); };
+        uint32_t kept[SPLIT_KEEP] = {}; // the segment's codes, two exponents of a pair each, as far as they fit
+        { // round 0: only where the next segment's first code begins
+            uint32_t e0, e1;
+            seg_bits b(st, start);
+            while ((int32_t) b.n > (int32_t) nstop) {
+                b.two(lut, nstop, e0, e1);
+            }
+            ends[tid] = 0u - b.n;
+        }
+        __syncthreads();
+        for (int round = 0; round <= S; round++) {
+            const uint32_t exact = seg ? ends[tid - 32] : first;
+            const bool moved = exact != start || round == 0;
+            start = exact;
+            if (moved) {
+                again[round] = 1;
+            }
+            __syncthreads();
+            if (again[round] == 0) {
+                break;
+            }
+            if (moved) {
+                seg_bits b(st, start);
+                n = 0;
+#pragma unroll
+                for (int k = 0; k < SPLIT_KEEP; k++) {
+                    if ((int32_t) b.n > (int32_t) nstop) {
+                        uint32_t e0, e1;
+                        n += b.two(lut, nstop, e0, e1) ? 2 : 1;
+                        kept[k] = pair(e0) | pair(e1) << 16;
+                    }
+                }
+                while ((int32_t) b.n > (int32_t) nstop) {
+                    uint32_t e0, e1;
+                    n += b.two(lut, nstop, e0, e1) ? 2 : 1;
+                }
+                ends[tid] = 0u - b.n;
+                counts[tid] = n;
+            }
+            __syncthreads();
+        }
+        uint32_t at = 0;
+        for (int i = 0; i < seg; i++) {
+            at += counts[32 * i + l32];
+        }
+        auto put = [&](uint32_t i, uint32_t e) { ex[((i >> 3) * 32 + (uint32_t) l32) * 8 + (i & 7)] = (uint16_t) e; };
+        n = at + n < (uint32_t) pairs ? n : at < (uint32_t) pairs ? (uint32_t) pairs - at : 0; // (the last word's unused bits)
+#pragma unroll
+        for (int k = 0; k < SPLIT_KEEP; k++) {
+            if (2 * k < (int) n) {
+                put(at + 2 * k, kept[k]);
+                if (2 * k + 1 < (int) n) {
+                    put(at + 2 * k + 1, kept[k] >> 16);
+                }
+            }
+        }
+        if (n > 2 * SPLIT_KEEP || (seg == S - 1 && at + n < (uint32_t) pairs)) { // many short codes: once more, code by code
+            seg_bits b(st, start);
+            const uint32_t to = seg == S - 1 ? (uint32_t) pairs : at + n;
+            while (at < to) {
+                uint32_t e0, e1;
+                const bool both = b.two(lut, 0x80000000u, e0, e1);
+                put(at, pair(e0));
+                if (both && at + 1 < to) {
+                    put(at + 1, pair(e1));
+                }
+                at += 2;
+            }
+        }
+        __syncthreads();
+        for (int rr = seg; rr < R; rr += S) {
+            auto weights = [&](int c, const uint4 sm, uint32_t (&wp)[8]) {
+                const uint4 e = ((const uint4 *) ex)[chunk_at(rr, c) * 32 + l32];
+                const uint32_t ew[4] = {e.x, e.y, e.z, e.w}, smw[4] = {sm.x, sm.y, sm.z, sm.w};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    wp[2 * j] = merge(spread_lo(smw[j]), (ew[j] & 0xFFu) << 7 | (ew[j] & 0xFF00u) << 15);
+                    wp[2 * j + 1] = merge(spread_hi(smw[j]), (ew[j] >> 9 & 0x7F80u) | (ew[j] >> 1 & 0x7F800000u));
+                }
+            };
+            for (int col = 0; col < (DEQ ? 1 : ncols); col++) {
+                float acc = 0.f;
+                for (int c0 = 0; c0 < C; c0 += SPLIT_AHEAD) {
+                    if (c0 != 0 || rr != seg || (col != 0 && C > SPLIT_AHEAD)) {
+#pragma unroll
+                        for (int i = 0; i < SPLIT_AHEAD; i++) {
+                            ahead[i] = plane[chunk_at(rr, c0 + i < C ? c0 + i : C - 1) * 32];
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < SPLIT_AHEAD; i++) {
+                        const int c = c0 + i;
+                        if (c < C) {
+                            uint32_t wp[8];
+                            weights(c, ahead[i], wp);
+                            if constexpr (DEQ) {
+                                uint16_t * dst = out + (u * R + rr) * K + c * CHUNK;
+#pragma unroll
+                                for (int j = 0; j < 4; j++) {
+                                    *(uint2 *) (dst + 128 * j + 4 * l32) = make_uint2(wp[2 * j], wp[2 * j + 1]);
+                                }
+                            } else {
+                                float xv[16];
+                                x_chunk16<TX>(p.x + col * p.x_tok, c * CHUNK + 4 * l32, xv);
+                                float4 x[4];
+#pragma unroll
+                                for (int j = 0; j < 4; j++) {
+                                    x[j] = make_float4(xv[4 * j], xv[4 * j + 1], xv[4 * j + 2], xv[4 * j + 3]);
+                                }
+                                const float d = dot_chunk(wp, x);
+                                acc += cm ? half_wave_sum_dpp(d) : d; // (lane 31 has the sum)
+                            }
+                        }
+                    }
+                }
+                if (!DEQ) {
+                    const float v = cm ? acc : half_wave_sum_dpp(acc);
+                    if (l32 == 31) {
+                        store_y(p.y + col * p.y_tok, p.y_bf16, u * R + rr, v);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // partial dot of a decoded chunk with x.  The four per-position sums are combined as in the reference
@@ -904,7 +1135,46 @@ bool huf_direct(const bf16n_weight & w, int64_t units, int ncols, int cus, size_
     return w.format == FMT_HUFPAIR ? chunks <= 8 && per_cu >= 64 && weights <= (16 << 20) : per_cu >= 16 && (weights <= (16 << 20) || chunks >= 32);
 }
 
+// Columns up to which a launch over `units` units takes k_hp_split (0: none): while the chain of a unit is longer than what its
+// blocks take on the CUs they get.  A CU holds two blocks, one beyond 512 pair codes a lane, and every column adds its products
+// to each of them.  us, one half-wave per unit / this (R = 16 at K = 2048 and 4096, 8 at 3072 and 3584):
+//   one column: 4096 x 2048 40.9 / 17.7, 8192 x 2048 42.4 / 26.6, 12288 x 2048 47.0 / 36.4, 16384 x 2048 45.6 / 46.1; 4096 x 4096 79 / 26,
+//     8192 x 4096 80 / 49, 12288 x 4096 87 / 76, 16384 x 4096 85 / 95; 4096 x 3072 33 / 23, 5000 x 3072 36.4 / 37.3; 6000 x 3584 42 / 36
+//   8192 x 2048 at 4 / 8 columns 43 / 48 and 33 / 44; 8192 x 4096 at 4 80 and 74, at 8 91 and 100; 4096 x 3072 at 4 / 8 34 / 38 and
+//     31 / 43; 8192 x 1024 at 3 / 4 28 / 25 and 25 / 26; 12288 x 4096 at 3 90 and 98; 12288 x 2048 at 8 67 and 60
+//   dequant of 8192 x 2048 38 / 28, 8192 x 4096 70 / 50, 4096 x 3072 30 / 24; 8192 x 1024 22 / 23
+int hp_split_cols(const bf16n_weight & w, int64_t units, int cus) {
+    const int pairs = w.R * (int) (w.K / CHUNK) * 8;
+    if (w.format != FMT_HUFPAIR || pairs < 256 || pairs > 1024 || units > 3 * (int64_t) cus) {
+        return 0;
+    }
+    if (units > 2 * (int64_t) cus) {
+        return pairs == 512 ? 8 : pairs >= 448 ? 1 : 0;
+    }
+    return pairs <= 512 ? (pairs - 128) / 48 : units > cus ? 4 : 8;
+}
+constexpr int SPLIT_DEQUANT_COLS = 3; // what the exact rows cost in its place, in columns
+int split_threads(const bf16n_weight & w) {
+    const int pairs = w.R * (int) (w.K / CHUNK) * 8, segs = (pairs + SPLIT_PAIRS - 1) / SPLIT_PAIRS;
+    return 64 * ((segs + 1) / 2);
+}
+template <typename TX, bool DEQ>
+void launch_hp_split(const bf16n_weight & w, const cols & p, int ncols, uint16_t * out, int cus, hipStream_t stream) {
+    const int threads = split_threads(w);
+    const size_t shm = split_shm(w.R * (int) (w.K / CHUNK) * 8, threads);
+    const int64_t units = p.nrows / w.R, fit = (int64_t) cus * std::max<int64_t>(1, std::min<int64_t>(2048 / threads, (int64_t) (LDS_BYTES / shm)));
+    note_kernel("k_hp_split", tx_name<TX>(), 1, DEQ);
+    hipLaunchKernelGGL((k_hp_split<TX, DEQ>), dim3((unsigned) std::min(units, fit)), dim3(threads), shm, stream, w, p, ncols, out);
+}
+
 } // namespace
+
+void compat_init() {
+    const int shm = (int) split_shm(1024, 1024);
+    (void) hipFuncSetAttribute((const void *) k_hp_split<bf16_t, false>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    (void) hipFuncSetAttribute((const void *) k_hp_split<float, false>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    (void) hipFuncSetAttribute((const void *) k_hp_split<bf16_t, true>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+}
 
 // Steps per wavefront of k_nib_mm16 (a row has K / 128): the fewest for which a block has at most eight wavefronts, or
 // four (fewer, longer wavefronts) when the row groups outnumber the CUs anyway; 0: K does not fit the kernel.
@@ -1005,6 +1275,11 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
     }
     const bool hp = w.format == FMT_HUFPAIR;
     const int64_t work = p.nrows / w.R;
+    if (glu == 0 && !p.ids && ncols <= hp_split_cols(w, work, cus) && ((uintptr_t) p.x & 15) == 0 && (ncols == 1 || p.x_tok % 16 == 0)) {
+        if (x_bf16) launch_hp_split<bf16_t, false>(w, p, ncols, nullptr, cus, stream);
+        else        launch_hp_split<float, false>(w, p, ncols, nullptr, cus, stream);
+        return;
+    }
     const size_t shared = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX));
     const bool direct = !glu && !p.ids && huf_direct(w, work, ncols, cus, shared);
     const int waves = direct ? NT / 64 : huf_waves(work, ncols, cus, w.R * (int) (w.K / CHUNK));
@@ -1050,6 +1325,11 @@ void launch_compat_dequant(const bf16n_weight & w, int64_t row0, int64_t nrows, 
     const dim3 grid((unsigned) (blocks < (int64_t) cus * 16 ? blocks : (int64_t) cus * 16));
     if (w.format == FMT_NIBBLE) {
         launch_nib_rows(w, nullptr, 0, nrows, row0, (char *) out, true, (int64_t) w.K * 2, grid, stream);
+    } else if (hp_split_cols(w, work, cus) >= SPLIT_DEQUANT_COLS) {
+        cols p = {};
+        p.row0 = row0;
+        p.nrows = nrows;
+        launch_hp_split<bf16_t, true>(w, p, 0, out, cus, stream);
     } else if (w.format == FMT_HUFPAIR) {
         hipLaunchKernelGGL((k_huf_dequant<FMT_HUFPAIR>), grid, dim3(waves * 64), 0, stream, w, row0, nrows, out);
     } else {

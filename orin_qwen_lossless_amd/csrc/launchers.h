@@ -21,6 +21,7 @@ inline void note_kernel(const char * name, const char * tx, int n_args, int a0 =
 template <typename TX> constexpr const char * tx_name() { return sizeof(TX) == 2 ? "bf16_t" : "float"; }
 
 // 32-lane layouts (kernels_compat.hip). glu: 0 plain, 1 merged [gate; up] NIBBLE matrix, 2 separate gate / up matrices
+void compat_init();
 bool nib_mm_pays(const bf16n_weight & w, int64_t nrows, int ncols, int cus);
 bool nib_mm16_pays(const bf16n_weight & w, int64_t nrows, int ncols, int cus);
 void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu, const cols & p, int ncols, bool x_bf16,
