@@ -16,6 +16,7 @@ OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libbf16n_hip.so")
 BENCH = os.path.join(HERE, "bf16n_bench")  # stand-alone timing program (csrc/bench_mmv.cpp), linked against the library
 PROBE = os.path.join(HERE, "libbf16n_probe.so")  # read-bandwidth probe (csrc/bench_probe.hip): measurement only, loaded by the benchmarks
+HOST = os.path.join(HERE, "_host.so")  # extension module: the dense product's call from Python (csrc/host_calls.cpp)
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["encode.cpp", "policy.cpp", "capi.cpp", "adapter.cpp", "dense.cpp", "kernels_compat.hip", "kernels_w64.hip", "kernels_moe.hip", "kernels_mm_ids.hip", "kernels_tile.hip"]
@@ -39,10 +40,33 @@ def _compile(src: str, force: bool) -> str:
     return obj
 
 
+def _build_host(force: bool) -> None:
+    src = os.path.join(CSRC, "host_calls.cpp")
+    deps = (src, os.path.join(ROOT, "include", "bf16n_c.h"))
+    if not force and os.path.exists(HOST) and all(os.path.getmtime(HOST) >= os.path.getmtime(d) for d in deps):
+        return
+    import sysconfig
+
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    inc = [os.path.join(ROOT, "include"), os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    r = subprocess.run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + ["-isystem" + i for i in inc] +
+                       [src, "-o", HOST, "-L" + os.path.join(t, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"],
+                       capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stdout + r.stderr)
+        raise RuntimeError("building _host.so failed")
+
+
 def build(force: bool = False) -> str:
     os.makedirs(OBJ, exist_ok=True)
     with ThreadPoolExecutor(max_workers=4) as ex:
+        host = ex.submit(_build_host, force)
         objs = list(ex.map(lambda s: _compile(s, force), SOURCES))
+        host.result()
     if force or not os.path.exists(LIB) or any(os.path.getmtime(o) > os.path.getmtime(LIB) for o in objs):
         r = subprocess.run([HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB] + objs + ["-lpthread", "-ldl"], capture_output=True, text=True)
         if r.returncode != 0:

@@ -1,0 +1,71 @@
+"""The dense product's native call (csrc/host_calls.cpp): it takes the plain case with the result of the Python layer's, and
+answers everything else with None, so that the Python layer's checks and messages hold."""
+from __future__ import annotations
+
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from orin_qwen_lossless_amd import ops, synth
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+class Pass(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _take(x, w, *rest):
+    return (ops._host_mmv or ops._bind_host())(x, w, *rest)
+
+
+def test_nothing_on_the_host_is_taken():
+    meta = ops.Meta(1, 512, 4, 1, False, False, 256, 512, 640, 700)
+    w = ops.Weight(torch.zeros(4 * 512, dtype=torch.uint8), torch.zeros(1024, dtype=torch.uint8), meta)
+    x = torch.zeros(1, 512, dtype=torch.bfloat16)
+    for args in ((x, w, True, True, True, 8), (x, None, True, True, True, 8), (None, w, True, True, True, 8), (x, w), (x, w, 1, 1, 1, "n")):
+        assert _take(*args) is None
+    with pytest.raises(ValueError, match="device"):
+        ops.mmv(x, w)
+
+
+@pytest.mark.gpu
+def test_the_plain_product_and_nothing_else(ops):
+    rows, K = 200, 1024
+    src = torch.from_numpy(synth.weights(rows, K, 3).view("int16")).view(torch.bfloat16)
+    fmt, R, cm, fo, w64 = ops.choose(rows, K)
+    plane, aux, meta = ops.encode(src, fmt, R, cm, fo, w64)
+    w = ops.upload(plane, aux, meta, "cuda")
+    x = synth.weights_torch(9, K, 5, "cuda")
+    for xt in (x, x.float()):
+        for t in (1, 2, 9):
+            for out_bf16 in (False, True):
+                for multi in (False, True):
+                    y = _take(xt[:t], w, out_bf16, multi, False, 65535)
+                    ref = ops._mmv_common(xt[:t], w, None, 0, out_bf16, False, multi)
+                    assert y.dtype == ref.dtype and y.shape == ref.shape and torch.equal(y, ref)
+    wide = torch.zeros(9, K + 8, dtype=torch.bfloat16, device="cuda")
+    wide[:, :K] = x
+    assert torch.equal(_take(wide[:, :K], w, True, True, True, 9), _take(x, w, True, True, True, 9))
+    short = ops.Weight(w.plane[:-K], w.aux, meta)
+    moved = ops.Weight(torch.cat([w.plane, w.plane])[1: rows * K + 1], w.aux, meta)
+    for bad in (x[:, :-8], x[:, ::2], x.half(), x[0], x[:0], x[None], x.cpu(), x.float(), torch.cat([x, x], 1)[:, 1: K + 1], x.to_sparse(),
+                x.as_subclass(Sub), wide[:, 1: K + 1]):
+        assert _take(bad, w, True, True, True, 9) is None
+    assert _take(x, w, True, True, True, 8) is None
+    assert _take(x, short, True, True, True, 9) is None and _take(x, moved, True, True, True, 9) is None
+    with Pass():
+        assert _take(x, w, True, True, True, 9) is None
+    seen = []
+    torch.vmap(lambda v: seen.append(_take(v, w, True, True, True, 9)) or v)(x[None])
+    assert seen == [None]
+    p = torch.nn.Parameter(x.float())
+    assert not _take(p, w, False, True, False, 9).requires_grad
+    # the C ABI's refusals come back as its status
+    fo_meta = ops.Meta(*meta.__dict__.values())
+    object.__setattr__(fo_meta, "frag_order", True)
+    with pytest.raises(ValueError, match="fragment-order"):
+        ops.mmv(x, ops.Weight(w.plane, w.aux, fo_meta))
