@@ -108,7 +108,7 @@ class Weight:
 
 
 # A small product is bound by the host's call (512 x 2048, one token: 14.9 us with torch's Python-level device guard and
-# stream objects and a view in and out, 9.3 without; the kernel takes 3.2; the plain dense product has a native one, _host_mmv), so the calls below stay off both when the
+# stream objects and a view in and out, 9.3 without; the kernel takes 3.2; the plain dense products have a native one, _host), so the calls below stay off both when the
 # tensor's device is the current one anyway.  The two functions are private to torch (torch.cuda.current_device and the code
 # that torch.compile generates call them); where a release lacks them the public ones stand in.
 _HERE = contextlib.nullcontext()
@@ -285,18 +285,20 @@ def roundtrip_equal(w: Weight, src: torch.Tensor, chunk_bytes: int = 64 << 20) -
     return True
 
 
-# the plain dense product's call in native code (csrc/host_calls.cpp), which gives a tensor, a status, or None where the call
-# is not plain and goes through _mmv_common below.  512 x 2048, one token: 9.3 us a call there, 5.0 here (the kernel takes 3)
-_host_mmv = None
+# The plain dense products' calls in native code (csrc/host_calls.cpp), which give a tensor, a status, or None where the call is
+# not plain and goes the general way below.  512 x 2048, one token: 9.3 us a call there, 5.0 here (the kernel takes 3)
+_host_calls = None
 
 
-def _bind_host():
-    global _host_mmv
-    from . import _host  # built with the library (python -m orin_qwen_lossless_amd.build)
+def _host():
+    global _host_calls
+    if _host_calls is None:
+        from . import _host as calls  # built with the library (python -m orin_qwen_lossless_amd.build)
 
-    _host.bind(C.cast(_lib.lib().bf16n_mmv, C.c_void_p).value)
-    _host_mmv = _host.mmv
-    return _host_mmv
+        L = _lib.lib()
+        calls.bind(*(C.cast(f, C.c_void_p).value for f in (L.bf16n_mmv, L.bf16n_gemv_max_tokens, L.bf16n_dequant)))
+        _host_calls = calls
+    return _host_calls
 
 
 def _mmv_common(x: torch.Tensor, w: Weight, ids: torch.Tensor | None, rows_per_matrix: int, out_bf16: bool, glu: bool,
@@ -372,7 +374,7 @@ def mmv(x: torch.Tensor, w: Weight, ids: torch.Tensor | None = None, rows_per_ma
         out_dtype: torch.dtype = torch.float32, multi_col: bool = True) -> torch.Tensor:
     out_bf16 = out_dtype == torch.bfloat16
     if ids is None and rows_per_matrix <= 0:
-        y = (_host_mmv or _bind_host())(x, w, out_bf16, bool(multi_col), False, 65535)
+        y = (_host_calls or _host()).mmv(x, w, out_bf16, bool(multi_col))
         if y is not None:
             return _lib.check(y) if type(y) is int else y
     return _mmv_common(x, w, ids, rows_per_matrix, out_bf16, False, multi_col)
@@ -435,7 +437,7 @@ def linear(x: torch.Tensor, w: Weight, bias: torch.Tensor | None = None) -> torc
     added in FP32 before the one rounding to BF16), more through exact dequant in row chunks + a stock BF16 GEMM
     (core/torch/torch_bindings.cpp:198-239)."""
     if bias is None:
-        y = (_host_mmv or _bind_host())(x, w, True, True, True, GEMV_MAX_TOKENS)
+        y = (_host_calls or _host()).linear(x, w, GEMV_MAX_TOKENS, DEQUANT_CHUNK_BYTES)
         if y is not None:
             return _lib.check(y) if type(y) is int else y
     if x.dtype != torch.bfloat16:

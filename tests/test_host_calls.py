@@ -18,16 +18,18 @@ class Pass(TorchDispatchMode):
         return func(*args, **(kwargs or {}))
 
 
-def _take(x, w, *rest):
-    return (ops._host_mmv or ops._bind_host())(x, w, *rest)
+def _calls():
+    return ops._host_calls or ops._host()
 
 
 def test_nothing_on_the_host_is_taken():
     meta = ops.Meta(1, 512, 4, 1, False, False, 256, 512, 640, 700)
     w = ops.Weight(torch.zeros(4 * 512, dtype=torch.uint8), torch.zeros(1024, dtype=torch.uint8), meta)
     x = torch.zeros(1, 512, dtype=torch.bfloat16)
-    for args in ((x, w, True, True, True, 8), (x, None, True, True, True, 8), (None, w, True, True, True, 8), (x, w), (x, w, 1, 1, 1, "n")):
-        assert _take(*args) is None
+    for args in ((x, w, True, True), (x, None, True, True), (None, w, True, True), (x, w)):
+        assert _calls().mmv(*args) is None
+    for args in ((x, w, 8, 1 << 20), (x, w, "n", 1), (x, w)):
+        assert _calls().linear(*args) is None
     with pytest.raises(ValueError, match="device"):
         ops.mmv(x, w)
 
@@ -44,26 +46,37 @@ def test_the_plain_product_and_nothing_else(ops):
         for t in (1, 2, 9):
             for out_bf16 in (False, True):
                 for multi in (False, True):
-                    y = _take(xt[:t], w, out_bf16, multi, False, 65535)
+                    y = _calls().mmv(xt[:t], w, out_bf16, multi)
                     ref = ops._mmv_common(xt[:t], w, None, 0, out_bf16, False, multi)
                     assert y.dtype == ref.dtype and y.shape == ref.shape and torch.equal(y, ref)
     wide = torch.zeros(9, K + 8, dtype=torch.bfloat16, device="cuda")
     wide[:, :K] = x
-    assert torch.equal(_take(wide[:, :K], w, True, True, True, 9), _take(x, w, True, True, True, 9))
+    assert torch.equal(_calls().mmv(wide[:, :K], w, True, True), _calls().mmv(x, w, True, True))
     short = ops.Weight(w.plane[:-K], w.aux, meta)
     moved = ops.Weight(torch.cat([w.plane, w.plane])[1: rows * K + 1], w.aux, meta)
     for bad in (x[:, :-8], x[:, ::2], x.half(), x[0], x[:0], x[None], x.cpu(), x.float(), torch.cat([x, x], 1)[:, 1: K + 1], x.to_sparse(),
                 x.as_subclass(Sub), wide[:, 1: K + 1]):
-        assert _take(bad, w, True, True, True, 9) is None
-    assert _take(x, w, True, True, True, 8) is None
-    assert _take(x, short, True, True, True, 9) is None and _take(x, moved, True, True, True, 9) is None
+        assert (_calls().mmv(bad, w, True, True) is None or bad.dtype == torch.float32) and _calls().linear(bad, w, 8, 1 << 26) is None
+    for refused in (short, moved):
+        assert _calls().mmv(x, refused, True, True) is None and _calls().linear(x, refused, 8, 1 << 26) is None
     with Pass():
-        assert _take(x, w, True, True, True, 9) is None
+        assert _calls().mmv(x, w, True, True) is None and _calls().linear(x, w, 8, 1 << 26) is None
     seen = []
-    torch.vmap(lambda v: seen.append(_take(v, w, True, True, True, 9)) or v)(x[None])
-    assert seen == [None]
-    p = torch.nn.Parameter(x.float())
-    assert not _take(p, w, False, True, False, 9).requires_grad
+    torch.vmap(lambda v: seen.extend([_calls().mmv(v, w, True, True), _calls().linear(v, w, 8, 1 << 26)]) or v)(x[None])
+    assert seen == [None, None]
+    assert not _calls().mmv(torch.nn.Parameter(x.float()), w, False, True).requires_grad
+    # linear: GEMV columns, columns up to the matrix's own number of them, decoded in one piece (a graph of x's gradient with
+    # it) and, beyond a piece, not at all
+    most = ops.gemv_max_tokens(w)
+    big = synth.weights_torch(most + 1, K, 6, "cuda")
+    for t in (1, 8, 9, most):
+        assert torch.equal(_calls().linear(big[:t], w, 8, 1 << 26), ops._mmv_common(big[:t], w, None, 0, True, False)), t
+    y = _calls().linear(big, w, 8, rows * K * 2)
+    assert torch.equal(y, torch.nn.functional.linear(big, ops.dequant(w)))
+    assert _calls().linear(big, w, 8, rows * K * 2 - 1) is None
+    leaf = big.clone().requires_grad_()
+    ops.linear(leaf, w).sum().backward()
+    assert torch.equal(leaf.grad, torch.ones_like(y) @ ops.dequant(w))
     # the C ABI's refusals come back as its status
     fo_meta = ops.Meta(*meta.__dict__.values())
     object.__setattr__(fo_meta, "frag_order", True)
