@@ -13,6 +13,7 @@
 #include "launchers.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace bf16n {
 namespace dev {
@@ -181,45 +182,93 @@ __device__ __forceinline__ float dot_chunk(const uint32_t (&wp)[8], const float4
     return (a0 + a1) + (a2 + a3);
 }
 
-// One unit of R rows: y[rr] (rr < R) ends up in lane rr of the half-wave.  Row-major streams finish a row every C
-// chunks; chunk-major streams add one partial sum per (chunk, row).
-template <int FORMAT, bool RING>
-__device__ __forceinline__ float unit_dot(const uint8_t * plane, const uint32_t * lut, const uint32_t * sp, uint32_t * ring, int64_t gu, int R,
-                                          int C, bool cm, const float * xs, int l32) {
+// the activations a lane meets in a chunk, from LDS: as FP32, or as the BF16 they came in (several columns)
+template <typename TX> struct x_lds;
+template <> struct x_lds<float> {
+    float4 v[4];
+    __device__ __forceinline__ void load(const float * xs, int col0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            v[j] = *(const float4 *) (xs + col0 + 128 * j);
+        }
+    }
+    __device__ __forceinline__ float4 get(int j) const { return v[j]; }
+    __device__ __forceinline__ static float store(const char * x, int i) { return ((const float *) x)[i]; }
+};
+template <> struct x_lds<bf16_t> {
+    uint2 v[4];
+    __device__ __forceinline__ void load(const uint16_t * xs, int col0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            v[j] = *(const uint2 *) (xs + col0 + 128 * j);
+        }
+    }
+    __device__ __forceinline__ float4 get(int j) const {
+        return make_float4(__uint_as_float(v[j].x << 16), __uint_as_float(v[j].x & 0xFFFF0000u), __uint_as_float(v[j].y << 16), __uint_as_float(v[j].y & 0xFFFF0000u));
+    }
+    __device__ __forceinline__ static uint16_t store(const char * x, int i) { return ((const uint16_t *) x)[i]; }
+};
+
+// One unit of R rows: y[rr] (rr < R) of column n ends up in mine[n] of lane rr of the half-wave.  Row-major streams finish a
+// row every C chunks; chunk-major streams add one partial sum per (chunk, row).  Column n's activations: xs + n * K.
+template <int FORMAT, bool RING, int NC, typename XL, typename XS>
+__device__ __forceinline__ void unit_dot(const uint8_t * plane, const uint32_t * lut, const uint32_t * sp, uint32_t * ring, int64_t gu, int R,
+                                         int C, bool cm, const XS * xs, int l32, float (&mine)[NC]) {
     const bool upper = (threadIdx.x & 32) != 0;
     auto sum = [&](float v) { // over the half-wave, on the VALU (lanes 31 and 63 get the sums)
         const int t = __builtin_bit_cast(int, half_wave_sum_dpp(v));
         const int lo = __builtin_amdgcn_readlane(t, 31), hi = __builtin_amdgcn_readlane(t, 63);
         return __builtin_bit_cast(float, upper ? hi : lo);
     };
-    float mine = 0.f, acc = 0.f;
+    float acc[NC];
+#pragma unroll
+    for (int n = 0; n < NC; n++) {
+        mine[n] = acc[n] = 0.f;
+    }
     int rr = 0, c = 0;
-    float4 x[4]; // the chunk's activations, requested before its chain of lookups (8192 x 2048, one column: 3 us)
+    XL x[NC]; // the chunk's activations, requested before its chain of lookups (8192 x 2048, one column: 3 us)
     for_chunks<FORMAT, RING>(plane + gu * R * (int64_t) C * CHUNK, sp, ring, lut, R * C, l32, [&] {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            x[j] = *(const float4 *) (xs + c * CHUNK + 128 * j + 4 * l32);
+        for (int n = 0; n < NC; n++) {
+            x[n].load(xs + n * C * CHUNK, c * CHUNK + 4 * l32);
         }
         __builtin_amdgcn_sched_barrier(0);
     }, [&](int, const uint32_t (&wp)[8]) {
-        const float d = dot_chunk(wp, x);
+        float d[NC];
+#pragma unroll
+        for (int n = 0; n < NC; n++) {
+            float4 xv[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                xv[j] = x[n].get(j);
+            }
+            d[n] = dot_chunk(wp, xv);
+        }
         if (cm) {
-            const float v = sum(d);
-            mine += l32 == rr ? v : 0.f;
+#pragma unroll
+            for (int n = 0; n < NC; n++) {
+                const float v = sum(d[n]);
+                mine[n] += l32 == rr ? v : 0.f;
+            }
             rr = rr + 1 < R ? rr + 1 : 0;
             c += rr == 0;
         } else {
-            acc += d;
+#pragma unroll
+            for (int n = 0; n < NC; n++) {
+                acc[n] += d[n];
+            }
             c = c + 1 < C ? c + 1 : 0;
             if (c == 0) {
-                const float v = sum(acc);
-                mine = l32 == rr ? v : mine;
-                acc = 0.f;
+#pragma unroll
+                for (int n = 0; n < NC; n++) {
+                    const float v = sum(acc[n]);
+                    mine[n] = l32 == rr ? v : mine[n];
+                    acc[n] = 0.f;
+                }
                 rr++;
             }
         }
     });
-    return mine;
 }
 
 template <int FORMAT>
@@ -233,18 +282,23 @@ __device__ __forceinline__ const uint32_t * lane_stream(const bf16n_weight & w, 
 }
 
 // y = W x (GLU: y = silu(gate x) * up x) for HUFPAIR / HUFFMAN in the 32-lane layouts; one half-wave per unit,
-// blockIdx.y = column.  Shared memory: x as FP32 [K], then one table per matrix, then (RING) a ring per wavefront.
-template <int FORMAT, typename TX, bool GLU, bool RING>
-__global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16n_weight w_up, const cols p) {
+// blockIdx.y = NC columns, which share a decode (NC > 1: dense products; columns past the last repeat it and are not stored).
+// Shared memory: x [NC][K] as FP32 (several BF16 columns: as they are), then one table per matrix, then (RING) a ring per wavefront.
+// What bounds it is the chain of a unit while the device has half-waves to spare, then the lookups; a column more adds 32
+// instructions and four LDS reads to a chunk's 140 and sixteen (huf_columns has the times).
+template <int FORMAT, typename TX, bool GLU, bool RING, int NC = 1>
+__global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16n_weight w_up, const cols p, int ncols) {
     constexpr int LUT_N = FORMAT == FMT_HUFPAIR ? (1 << HP_LP) : (1 << HUF_LMAX);
+    typedef typename std::conditional<NC == 1 || sizeof(TX) == 4, float, uint16_t>::type xs_t;
+    typedef x_lds<typename std::conditional<NC == 1 || sizeof(TX) == 4, float, bf16_t>::type> xl_t;
     extern __shared__ __align__(16) unsigned char shm_raw[];
     const int K = (int) w.K, C = K / CHUNK, R = w.R;
-    float * xs = (float *) shm_raw;
-    uint32_t * lut = (uint32_t *) (xs + K);
+    xs_t * xs = (xs_t *) shm_raw;
+    uint32_t * lut = (uint32_t *) (xs + NC * K);
     uint32_t * lut_up = lut + LUT_N;
     uint32_t * ring = lut + (GLU ? 2 : 1) * LUT_N + (threadIdx.x >> 6) * (LR_BYTES / 4) + (threadIdx.x & 63);
-    const int nt = (int) blockDim.x;
-    const col_view cv = col_setup(p, blockIdx.y);
+    const int nt = (int) blockDim.x, col0 = (int) blockIdx.y * NC;
+    const col_view cv = col_setup(p, col0);
     // (many loads in flight: the smallest blocks are one wavefront)
 #pragma unroll 16
     for (int i = threadIdx.x; i < LUT_N; i += nt) {
@@ -256,9 +310,17 @@ __global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16
             lut_up[i] = ((const uint32_t *) (w_up.aux + w_up.off_a))[i];
         }
     }
+#pragma unroll
+    for (int n = 0; n < NC; n++) {
+        const char * x = cv.x + (col0 + n < ncols ? n : ncols - 1 - col0) * p.x_tok;
 #pragma unroll 8
-    for (int i = threadIdx.x; i < K; i += nt) {
-        xs[i] = x_at<TX>(cv.x, i);
+        for (int i = threadIdx.x; i < K; i += nt) {
+            if constexpr (NC == 1) {
+                xs[i] = x_at<TX>(cv.x, i);
+            } else {
+                xs[n * K + i] = xl_t::store(x, i);
+            }
+        }
     }
     __syncthreads();
     const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5, halves = nt >> 5;
@@ -268,13 +330,20 @@ __global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16
         // (both halves of a wavefront stay together: a missing last unit is decoded twice and stored once)
         const int64_t u = u0 + (half & 1) < units ? u0 + (half & 1) : u0;
         const int64_t gu = cv.rbase / R + u;
-        float v = unit_dot<FORMAT, RING>(w.plane, lut, lane_stream<FORMAT>(w, gu, l32), ring, gu, R, C, cm, xs, l32);
-        if (GLU) {
-            const float uv = unit_dot<FORMAT, RING>(w_up.plane, lut_up, lane_stream<FORMAT>(w_up, gu, l32), ring, gu, R, C, false, xs, l32);
-            v = uv * silu(v);
+        float v[NC];
+        unit_dot<FORMAT, RING, NC, xl_t>(w.plane, lut, lane_stream<FORMAT>(w, gu, l32), ring, gu, R, C, cm, xs, l32, v);
+        if constexpr (GLU) {
+            float uv[NC];
+            unit_dot<FORMAT, RING, NC, xl_t>(w_up.plane, lut_up, lane_stream<FORMAT>(w_up, gu, l32), ring, gu, R, C, false, xs, l32, uv);
+            v[0] = uv[0] * silu(v[0]);
         }
         if (l32 < R && u == u0 + (half & 1)) {
-            store_y(cv.y, p.y_bf16, u * R + l32, v);
+#pragma unroll
+            for (int n = 0; n < NC; n++) {
+                if (NC == 1 || col0 + n < ncols) {
+                    store_y(cv.y + n * p.y_tok, p.y_bf16, u * R + l32, v[n]);
+                }
+            }
         }
     }
 }
@@ -1113,25 +1182,35 @@ int huf_waves(int64_t units, int ncols, int cus, int chunks) {
     return waves;
 }
 
-// Dense products whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers per
-// wavefront, so that 16 of them (12 at K = 4096) fit a CU instead of 20 (16), and a lane that has not moved on loads its
-// block again; with that many wavefronts there the misses of one are covered by the others.  Without against with rings:
-//  * Several columns whose wavefronts fit the CUs at once this way and not with rings: 32768 x 2048, R = 16, five columns
-//    109 us against 126 (four: 102 against 90; six: 195 against 129); 2048 x 4096, R = 4, sixteen 43 against 51; 8192 x 1024,
-//    R = 4, five 16.7 against 19.8.
-//  * HUFPAIR in short units that the caches hold, from 64 wavefronts per CU on: 16384 x 512, R = 1, eight columns 27
-//    against 40 us (32768 x 2048, four chunks: 202 against 174).
-//  * HUFFMAN, which loads a block per eight codes where HUFPAIR has one per sixteen, from 16 wavefronts per CU on unless
-//    the matrix comes from memory in short units: 8192 x 1024, R = 4, eight columns 31 against 34 us; 32768 x 1024,
-//    R = 16, sixteen 211 against 267; 32768 x 4096, R = 4, one 142 against 208; but R = 4 at 32768 x 1024, eight chunks,
-//    sixteen 242 against 223.
-bool huf_direct(const bf16n_weight & w, int64_t units, int ncols, int cus, size_t shared) {
-    const int ring = (int) std::min<size_t>(4, LDS_BYTES / (shared + 4 * LR_BYTES)), direct = std::min(5, (int) ((LDS_BYTES - 1) / shared));
-    const int64_t per_cu = units * ncols / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
+// Columns that share one decode in dense products.  Each column in a launch of its own units decodes the matrix again, which
+// costs nothing while the device has half-waves to spare (a unit's chain is longer than what they do beside it), and everything
+// beyond: from sixteen half-waves per CU on two columns share one, from eight groups of four per CU on four.  us, each column by
+// itself / two / four of BF16 (HUFPAIR but the last):
+//   two columns: 16384 x 2048, R = 16 (1024 units) 44 / 52 / 65, 32768 x 2048 51 / 53 / 66, 16656 x 3584, R = 8 (2082) 68 / 57 / 72,
+//     42264 x 3072, R = 8 146 / 89 / 105, 59473 x 2560, R = 1 127 / 79 / 93
+//   four: 16384 x 2048 49 / 52 / 66, 24608 x 1024, R = 16 (1538) 60 / 38 / 40, 32768 x 2048 85 / 63 / 67, 42264 x 3072 254 / 153 / 107,
+//     218800 x 512, R = 1 225 / 142 / 90, 7624 x 1536, R = 4 (1906) 22.5 / 19.1 / 19.1, and three there 19.0 / 19.4 / 18.8
+//   eight: 10336 x 3584, R = 16 (646) 130 / 105 / 113, 16384 x 2048 77 / 62 / 66, 24608 x 1024 109 / 64 / 49, 42264 x 3072 496 / 257 / 181,
+//     59473 x 2560 405 / 257 / 172, 16384 x 3072, R = 8, HUFFMAN 231 / 111 / 86
+// Blocks of eight wavefronts instead of four: 5 to 25 % behind but for long rows of short units.
+int huf_columns(const bf16n_weight & w, int64_t units, int ncols, int cus) {
     const int chunks = w.R * (int) (w.K / CHUNK);
-    if (ncols > 1 && units * ncols > (int64_t) 8 * ring * cus && units * ncols <= (int64_t) 8 * direct * cus) {
-        return true;
+    if (ncols > 2 && units * ((ncols + 3) / 4) > 8 * (int64_t) cus) {
+        return 4;
     }
+    return ncols > 1 && units * ncols > 16 * (int64_t) cus && (ncols != 3 || chunks >= 16) ? 2 : 1;
+}
+
+// Dense products of one column whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers
+// per wavefront, so that 16 of them (12 at K = 4096) fit a CU instead of 20 (16), and a lane that has not moved on loads its
+// block again; with many wavefronts the misses of one are covered by the others.  Without against with rings:
+//  * HUFPAIR in short units that the caches hold, from 64 wavefronts per CU on (32768 x 2048, four chunks, eight columns one by one:
+//    202 against 174 us).
+//  * HUFFMAN, which loads a block per eight codes where HUFPAIR has one per sixteen, from 16 wavefronts per CU on unless
+//    the matrix comes from memory in short units: 32768 x 4096, R = 4 142 against 208 us.
+bool huf_direct(const bf16n_weight & w, int64_t units, int cus) {
+    const int64_t per_cu = units / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
+    const int chunks = w.R * (int) (w.K / CHUNK);
     return w.format == FMT_HUFPAIR ? chunks <= 8 && per_cu >= 64 && weights <= (16 << 20) : per_cu >= 16 && (weights <= (16 << 20) || chunks >= 32);
 }
 
@@ -1170,6 +1249,10 @@ void launch_hp_split(const bf16n_weight & w, const cols & p, int ncols, uint16_t
 } // namespace
 
 void compat_init() {
+#define HUFA(F, TX, N) (void) hipFuncSetAttribute((const void *) k_huf_mmv<F, TX, false, true, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) LDS_BYTES)
+    HUFA(FMT_HUFPAIR, bf16_t, 2); HUFA(FMT_HUFPAIR, bf16_t, 4); HUFA(FMT_HUFPAIR, float, 2); HUFA(FMT_HUFPAIR, float, 4);
+    HUFA(FMT_HUFFMAN, bf16_t, 2); HUFA(FMT_HUFFMAN, bf16_t, 4); HUFA(FMT_HUFFMAN, float, 2); HUFA(FMT_HUFFMAN, float, 4);
+#undef HUFA
     const int shm = (int) split_shm(1024, 1024);
     (void) hipFuncSetAttribute((const void *) k_hp_split<bf16_t, false>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
     (void) hipFuncSetAttribute((const void *) k_hp_split<float, false>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
@@ -1281,11 +1364,28 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
         return;
     }
     const size_t shared = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX));
-    const bool direct = !glu && !p.ids && huf_direct(w, work, ncols, cus, shared);
+    const int nc = glu || p.ids ? 1 : huf_columns(w, work, ncols, cus);
+    if (nc > 1) {
+        const int waves = NT / 64, groups = (ncols + nc - 1) / nc;
+        const size_t shm = (size_t) nc * w.K * (x_bf16 ? 2 : 4) + (hp ? (4u << HP_LP) : (4u << HUF_LMAX)) + (size_t) waves * LR_BYTES;
+        const int64_t blocks = std::min<int64_t>((work + 2 * waves - 1) / (2 * waves), (int64_t) cus * (int64_t) (LDS_BYTES / shm));
+        const dim3 grid((unsigned) blocks, (unsigned) groups); // (a block stages its table and columns once)
+#define HUFN(F, TX, N) hipLaunchKernelGGL((k_huf_mmv<F, TX, false, true, N>), grid, dim3(waves * 64), shm, stream, w, wu, p, ncols)
+#define HUFNX(F, TX) do { if (nc == 4) HUFN(F, TX, 4); else HUFN(F, TX, 2); } while (0)
+        if (hp) {
+            if (x_bf16) HUFNX(FMT_HUFPAIR, bf16_t); else HUFNX(FMT_HUFPAIR, float);
+        } else {
+            if (x_bf16) HUFNX(FMT_HUFFMAN, bf16_t); else HUFNX(FMT_HUFFMAN, float);
+        }
+#undef HUFNX
+#undef HUFN
+        return;
+    }
+    const bool direct = !glu && !p.ids && ncols == 1 && huf_direct(w, work, cus);
     const int waves = direct ? NT / 64 : huf_waves(work, ncols, cus, w.R * (int) (w.K / CHUNK));
     const size_t shm = shared + (direct ? 0 : (size_t) waves * LR_BYTES);
     const dim3 grid(grid_for(work, ncols, cus, 2 * waves), ncols);
-#define HUF(F, TX, G, RING) hipLaunchKernelGGL((k_huf_mmv<F, TX, G, RING>), grid, dim3(waves * 64), shm, stream, w, wu, p)
+#define HUF(F, TX, G, RING) hipLaunchKernelGGL((k_huf_mmv<F, TX, G, RING>), grid, dim3(waves * 64), shm, stream, w, wu, p, ncols)
 #define HUFX(F, TX) do { if (glu) HUF(F, TX, true, true); else if (direct) HUF(F, TX, false, false); else HUF(F, TX, false, true); } while (0)
     if (hp) {
         if (x_bf16) HUFX(FMT_HUFPAIR, bf16_t); else HUFX(FMT_HUFPAIR, float);
