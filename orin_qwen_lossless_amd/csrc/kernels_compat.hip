@@ -534,7 +534,7 @@ __global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const c
         const uint4 * plane = (const uint4 *) (w.plane + gu * R * (int64_t) K) + l32;
         auto chunk_at = [&](int rr, int c) { return cm ? c * R + rr : rr * C + c; }; // in stream order
         const uint32_t base = q.ubase[gu], end = gu + 1 < all_units ? q.ubase[gu + 1] : (uint32_t) ((const aux_header *) w.aux)->n_b;
-        const uint32_t words = end - base < cap ? end - base : cap;
+        const uint32_t words = end <= base ? 0 : end - base < cap ? end - base : cap; // (none for a base past the stream's end)
         uint32_t from = q.lrel[gu * 32 + l32], to = l32 < 31 ? q.lrel[gu * 32 + l32 + 1] : words;
         from = from < words ? from : words;
         to = to < from ? from : to < words ? to : words;
@@ -1242,7 +1242,9 @@ void launch_hp_split(const bf16n_weight & w, const cols & p, int ncols, uint16_t
     const int threads = split_threads(w);
     const size_t shm = split_shm(w.R * (int) (w.K / CHUNK) * 8, threads);
     const int64_t units = p.nrows / w.R, fit = (int64_t) cus * std::max<int64_t>(1, std::min<int64_t>(2048 / threads, (int64_t) (LDS_BYTES / shm)));
-    note_kernel("k_hp_split", tx_name<TX>(), 1, DEQ);
+    if (!DEQ) { // (the note is of products)
+        note_kernel("k_hp_split", tx_name<TX>(), 1, 0);
+    }
     hipLaunchKernelGGL((k_hp_split<TX, DEQ>), dim3((unsigned) std::min(units, fit)), dim3(threads), shm, stream, w, p, ncols, out);
 }
 
