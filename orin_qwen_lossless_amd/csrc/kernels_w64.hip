@@ -66,66 +66,6 @@ template <> struct xchunk<float> {
     }
 };
 
-// ---------------------------------------------------------------- sums over the lanes, several columns at once
-//
-// A DPP add writes only the lanes of its bank mask, so the first two levels of the reductions of four values come out in
-// one register, value i in quad i of every row of 16, for six adds where four separate reductions take eight; the two
-// levels inside a quad are then two adds instead of eight, and the permlane swaps of the last two levels carry the values
-// of two chains and of columns 4 to 7 along.  Four columns of two chains: 21 instructions against 48, eight: 38 against 96.
-// 248320 x 2048, us with a reduction and a store per column / with this: 3 / 4 / 6 / 8 BF16 columns 125 / 136 / 157 / 182 ->
-// 120 / 129 / 148 / 165, 3 / 4 / 8 FP32 142 / 157 / 240 -> 136 / 146 / 227; 131072 x 4096, 4 / 8 BF16 131 / 199 -> 128 / 193.
-// (The products on v_mfma_f32_4x4x4_16b_bf16 instead, a lane's own on the diagonal of its block: an instruction costs the
-// time of the two dot products that it replaces, and the sums of eight columns of two chains then take 64 registers.)
-// In asm because the compiler splits a masked add into two instructions; it does not see the writes in there, so the
-// wait states between a VALU write and a DPP read (two) or a permlane swap are spelled out.
-#define BF16N_ADD(D, S, CTRL, BANKS) "v_add_f32_dpp " D ", " S ", " S " " CTRL " row_mask:0xf bank_mask:" BANKS "\n\t"
-#define BF16N_QUAD "s_nop 1\n\t" BF16N_ADD("%0", "%0", "quad_perm:[1,0,3,2]", "0xf") "s_nop 1\n\t" BF16N_ADD("%0", "%0", "quad_perm:[2,3,0,1]", "0xf") "s_nop 3"
-// the sums over each row of 16 of N <= 4 values: value i in quad i
-template <int N> __device__ __forceinline__ float row_sums(const float * a) {
-    float t, u;
-    if constexpr (N == 1) {
-        asm("s_nop 1\n\t" BF16N_ADD("%1", "%2", "row_half_mirror", "0xf") "s_nop 1\n\t" BF16N_ADD("%0", "%1", "row_ror:8", "0xf") BF16N_QUAD
-            : "=&v"(t), "=&v"(u) : "v"(a[0]));
-    } else if constexpr (N == 2) {
-        asm("s_nop 1\n\t" BF16N_ADD("%1", "%2", "row_half_mirror", "0x5") BF16N_ADD("%1", "%3", "row_half_mirror", "0xa")
-            "s_nop 1\n\t" BF16N_ADD("%0", "%1", "row_ror:8", "0xf") BF16N_QUAD : "=&v"(t), "=&v"(u) : "v"(a[0]), "v"(a[1]));
-    } else if constexpr (N == 3) {
-        float v;
-        asm("s_nop 1\n\t" BF16N_ADD("%1", "%3", "row_half_mirror", "0x5") BF16N_ADD("%1", "%4", "row_half_mirror", "0xa")
-            BF16N_ADD("%2", "%5", "row_half_mirror", "0xf")
-            "s_nop 1\n\t" BF16N_ADD("%0", "%1", "row_ror:8", "0x3") BF16N_ADD("%0", "%2", "row_ror:8", "0xc") BF16N_QUAD
-            : "=&v"(t), "=&v"(u), "=&v"(v) : "v"(a[0]), "v"(a[1]), "v"(a[2]));
-    } else {
-        float v;
-        asm("s_nop 1\n\t" BF16N_ADD("%1", "%3", "row_half_mirror", "0x5") BF16N_ADD("%1", "%4", "row_half_mirror", "0xa")
-            BF16N_ADD("%2", "%5", "row_half_mirror", "0x5") BF16N_ADD("%2", "%6", "row_half_mirror", "0xa")
-            "s_nop 1\n\t" BF16N_ADD("%0", "%1", "row_ror:8", "0x3") BF16N_ADD("%0", "%2", "row_ror:8", "0xc") BF16N_QUAD
-            : "=&v"(t), "=&v"(u), "=&v"(v) : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
-    }
-    return t;
-}
-#undef BF16N_QUAD
-#undef BF16N_ADD
-// rows 0 and 2 of 16 lanes: a's sums over rows 0, 1 and 2, 3; rows 1 and 3: b's
-__device__ __forceinline__ float add_rows(float a, float b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-// lanes 0..31: a's sums over both halves; lanes 32..63: b's
-__device__ __forceinline__ float add_halves(float a, float b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-// one value's sum over the wavefront with the same pairs of summands at every level; valid in lane 63
-__device__ __forceinline__ float wave_sum_cols(float v) {
-    v = dpp_add<0x141, 0xf>(v); // row_half_mirror
-    v = dpp_add<0x128, 0xf>(v); // row_ror:8
-    v = dpp_add<0xB1, 0xf>(v);  // quad_perm [1,0,3,2]
-    v = dpp_add<0x4E, 0xf>(v);  // quad_perm [2,3,0,1]
-    v = dpp_add<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
-    return dpp_add<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
-}
-
 // ---------------------------------------------------------------- GEMV
 //
 // C = K / 512 in {1, 2, 4, 8}.  The loop body covers NB steps (2, or 4 for C = 8) so that the plane registers of a step
