@@ -9,7 +9,9 @@ from __future__ import annotations
 
 import contextlib
 import ctypes as C
+import importlib
 import struct
+import warnings
 from dataclasses import dataclass
 
 import numpy as np
@@ -286,17 +288,30 @@ def roundtrip_equal(w: Weight, src: torch.Tensor, chunk_bytes: int = 64 << 20) -
 
 
 # The plain dense products' calls in native code (csrc/host_calls.cpp), which give a tensor, a status, or None where the call is
-# not plain and goes the general way below.  512 x 2048, one token: 9.3 us a call there, 5.0 here (the kernel takes 3)
+# not plain and goes the general way below.  512 x 2048, one token: 9.3 us a call there, 5.0 here (the kernel takes 3).  Where the
+# extension module is not there or does not load, every call goes the general way: the same kernels, the slower call.
 _host_calls = None
+
+
+class _NoNativeCalls:
+    @staticmethod
+    def mmv(*_):
+        return None
+
+    linear = mmv
 
 
 def _host():
     global _host_calls
     if _host_calls is None:
-        from . import _host as calls  # built with the library (python -m orin_qwen_lossless_amd.build)
-
         L = _lib.lib()
-        calls.bind(*(C.cast(f, C.c_void_p).value for f in (L.bf16n_mmv, L.bf16n_gemv_max_tokens, L.bf16n_dequant)))
+        try:
+            calls = importlib.import_module("._host", __package__)
+            calls.bind(*(C.cast(f, C.c_void_p).value for f in (L.bf16n_mmv, L.bf16n_gemv_max_tokens, L.bf16n_dequant)))
+        except ImportError as e:
+            warnings.warn(f"bf16n: dense products are called without their native part ({e}): a call takes about 4 us longer; "
+                          "build it with `python -m orin_qwen_lossless_amd.build`", RuntimeWarning, stacklevel=3)
+            calls = _NoNativeCalls
         _host_calls = calls
     return _host_calls
 

@@ -2,6 +2,9 @@
 answers everything else with None, so that the Python layer's checks and messages hold."""
 from __future__ import annotations
 
+import sys
+import warnings
+
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -32,6 +35,20 @@ def test_nothing_on_the_host_is_taken():
         assert _calls().linear(*args) is None
     with pytest.raises(ValueError, match="device"):
         ops.mmv(x, w)
+
+
+def test_without_the_extension_module_calls_go_the_general_way(monkeypatch):
+    monkeypatch.setattr(ops, "_host_calls", None)
+    monkeypatch.setitem(sys.modules, "orin_qwen_lossless_amd._host", None)  # an import that fails
+    meta = ops.Meta(1, 512, 4, 1, False, False, 256, 512, 640, 700)
+    w = ops.Weight(torch.zeros(4 * 512, dtype=torch.uint8), torch.zeros(1024, dtype=torch.uint8), meta)
+    x = torch.zeros(1, 512, dtype=torch.bfloat16)
+    with pytest.warns(RuntimeWarning, match="build it with"), pytest.raises(ValueError, match="device"):
+        ops.mmv(x, w)
+    for call in (ops.mmv, ops.linear):                   # (said once)
+        with warnings.catch_warnings(), pytest.raises(ValueError, match="device"):
+            warnings.simplefilter("error")
+            call(x, w)
 
 
 @pytest.mark.gpu
