@@ -7,6 +7,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -16,7 +17,8 @@ OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libbf16n_hip.so")
 BENCH = os.path.join(HERE, "bf16n_bench")  # stand-alone timing program (csrc/bench_mmv.cpp), linked against the library
 PROBE = os.path.join(HERE, "libbf16n_probe.so")  # read-bandwidth probe (csrc/bench_probe.hip): measurement only, loaded by the benchmarks
-HOST = os.path.join(HERE, "_host.so")  # extension module: the dense product's call from Python (csrc/host_calls.cpp)
+# extension module: the dense product's call from Python (csrc/host_calls.cpp); the suffix keeps it from other Pythons
+HOST = os.path.join(HERE, "_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["encode.cpp", "policy.cpp", "capi.cpp", "adapter.cpp", "dense.cpp", "kernels_compat.hip", "kernels_w64.hip", "kernels_moe.hip", "kernels_mm_ids.hip", "kernels_tile.hip"]
@@ -40,25 +42,34 @@ def _compile(src: str, force: bool) -> str:
     return obj
 
 
-def _build_host(force: bool) -> None:
-    src = os.path.join(CSRC, "host_calls.cpp")
-    deps = (src, os.path.join(ROOT, "include", "bf16n_c.h"))
-    if not force and os.path.exists(HOST) and all(os.path.getmtime(HOST) >= os.path.getmtime(d) for d in deps):
-        return
-    import sysconfig
+def torch_release() -> str:
+    """What the extension module is built for, and runs with only: it inlines the internals of torch's tensors."""
+    import torch
 
+    return f"{torch.__version__} {torch.version.git_version}"
+
+
+def _build_host(force: bool) -> None:
+    src, stamp = os.path.join(CSRC, "host_calls.cpp"), os.path.join(OBJ, "_host.torch")
+    deps = (src, os.path.join(ROOT, "include", "bf16n_c.h"))
+    if not force and os.path.exists(HOST) and os.path.exists(stamp) and all(os.path.getmtime(HOST) >= os.path.getmtime(d) for d in deps):
+        with open(stamp) as f:
+            if f.read() == torch_release():
+                return
     import torch
 
     t = os.path.dirname(torch.__file__)
     inc = [os.path.join(ROOT, "include"), os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
            "/opt/rocm/include", sysconfig.get_paths()["include"]]
     r = subprocess.run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-                        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + ["-isystem" + i for i in inc] +
+                        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DBUILT_FOR="{torch_release()}"'] + ["-isystem" + i for i in inc] +
                        [src, "-o", HOST, "-L" + os.path.join(t, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"],
                        capture_output=True, text=True)
     if r.returncode != 0:
         sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("building _host.so failed")
+        raise RuntimeError(f"building {os.path.basename(HOST)} failed")
+    with open(stamp, "w") as f:
+        f.write(torch_release())
 
 
 def build(force: bool = False) -> str:

@@ -216,5 +216,11 @@ PyMODINIT_FUNC PyInit__host(void) {
             return nullptr;
         }
     }
-    return PyModule_Create(&g_module);
+    // the release of torch whose internals are inlined above; the Python layer uses the module with no other
+    PyObject * m = PyModule_Create(&g_module);
+    if (m && PyModule_AddStringConstant(m, "built_for", BUILT_FOR) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

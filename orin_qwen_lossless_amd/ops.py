@@ -18,6 +18,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from .build import torch_release
 
 FMT_NIBBLE, FMT_HUFFMAN, FMT_HUFPAIR = 1, 2, 3
 FORMAT_NAMES = {FMT_NIBBLE: "nibble", FMT_HUFFMAN: "huffman", FMT_HUFPAIR: "hufpair"}
@@ -289,7 +290,8 @@ def roundtrip_equal(w: Weight, src: torch.Tensor, chunk_bytes: int = 64 << 20) -
 
 # The plain dense products' calls in native code (csrc/host_calls.cpp), which give a tensor, a status, or None where the call is
 # not plain and goes the general way below.  512 x 2048, one token: 9.3 us a call there, 5.0 here (the kernel takes 3).  Where the
-# extension module is not there or does not load, every call goes the general way: the same kernels, the slower call.
+# extension module is not there, does not load or was built for another torch, every call goes the general way: the same
+# kernels, the slower call.
 _host_calls = None
 
 
@@ -307,6 +309,8 @@ def _host():
         L = _lib.lib()
         try:
             calls = importlib.import_module("._host", __package__)
+            if getattr(calls, "built_for", None) != torch_release():
+                raise ImportError("it was built for another release of torch")
             calls.bind(*(C.cast(f, C.c_void_p).value for f in (L.bf16n_mmv, L.bf16n_gemv_max_tokens, L.bf16n_dequant)))
         except ImportError as e:
             warnings.warn(f"bf16n: dense products are called without their native part ({e}): a call takes about 4 us longer; "

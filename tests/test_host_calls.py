@@ -3,13 +3,14 @@ answers everything else with None, so that the Python layer's checks and message
 from __future__ import annotations
 
 import sys
+import types
 import warnings
 
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from orin_qwen_lossless_amd import ops, synth
+from orin_qwen_lossless_amd import build, ops, synth
 
 
 class Sub(torch.Tensor):
@@ -49,6 +50,27 @@ def test_without_the_extension_module_calls_go_the_general_way(monkeypatch):
         with warnings.catch_warnings(), pytest.raises(ValueError, match="device"):
             warnings.simplefilter("error")
             call(x, w)
+
+
+def test_a_module_built_for_another_torch_is_not_used_and_is_built_again(monkeypatch):
+    assert _calls().built_for == build.torch_release()
+    stale = types.ModuleType("_host")
+    stale.built_for = "1.0 0"
+    stale.bind = stale.mmv = stale.linear = lambda *_: pytest.fail("called")
+    monkeypatch.setattr(ops, "_host_calls", None)
+    for module in (stale, types.SimpleNamespace(bind=stale.bind)):  # (before there was a release in it)
+        monkeypatch.setitem(sys.modules, "orin_qwen_lossless_amd._host", module)
+        ops._host_calls = None
+        with pytest.warns(RuntimeWarning, match="another release of torch"):
+            assert ops._host().mmv(None, None, True, True) is None
+    started = []
+    monkeypatch.setattr(build.subprocess, "run", lambda cmd, **_: started.append(cmd) or types.SimpleNamespace(returncode=1, stdout="", stderr=""))
+    build._build_host(False)
+    assert not started                                   # up to date
+    monkeypatch.setattr(build, "torch_release", lambda: "1.0 0")
+    with pytest.raises(RuntimeError, match="building"):
+        build._build_host(False)
+    assert started
 
 
 @pytest.mark.gpu
