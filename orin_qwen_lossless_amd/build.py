@@ -1,4 +1,5 @@
-"""Builds libbf16n_hip.so (host encoder/policy + C ABI + HIP kernels for gfx950) in-tree with hipcc.
+"""Builds libbf16n_hip.so (host encoder/policy + C ABI + HIP kernels for gfx950) in-tree with hipcc, and with g++ the
+extension module of the Python layer's native calls where torch is there to build it for; the rest needs no torch.
 
 python -m orin_qwen_lossless_amd.build            # compile what changed
 The library sits next to this file so that it travels with the source tree; nothing is installed."""
@@ -50,14 +51,19 @@ def torch_release() -> str:
 
 
 def _build_host(force: bool) -> None:
+    try:
+        import torch
+    except ImportError:
+        torch = None
+    if torch is None or not torch.version.hip:
+        sys.stderr.write(f"{os.path.basename(HOST)} is not built: it needs torch for ROCm (only the Python layer uses it, and does without)\n")
+        return
     src, stamp = os.path.join(CSRC, "host_calls.cpp"), os.path.join(OBJ, "_host.torch")
     deps = (src, os.path.join(ROOT, "include", "bf16n_c.h"))
     if not force and os.path.exists(HOST) and os.path.exists(stamp) and all(os.path.getmtime(HOST) >= os.path.getmtime(d) for d in deps):
         with open(stamp) as f:
             if f.read() == torch_release():
                 return
-    import torch
-
     t = os.path.dirname(torch.__file__)
     inc = [os.path.join(ROOT, "include"), os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
            "/opt/rocm/include", sysconfig.get_paths()["include"]]
@@ -77,7 +83,6 @@ def build(force: bool = False) -> str:
     with ThreadPoolExecutor(max_workers=4) as ex:
         host = ex.submit(_build_host, force)
         objs = list(ex.map(lambda s: _compile(s, force), SOURCES))
-        host.result()
     if force or not os.path.exists(LIB) or any(os.path.getmtime(o) > os.path.getmtime(LIB) for o in objs):
         r = subprocess.run([HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB] + objs + ["-lpthread", "-ldl"], capture_output=True, text=True)
         if r.returncode != 0:
@@ -96,6 +101,7 @@ def build(force: bool = False) -> str:
         if r.returncode != 0:
             sys.stderr.write(r.stdout + r.stderr)
             raise RuntimeError("building bf16n_bench failed")
+    host.result()  # (a failure here leaves the library and what links it built)
     return LIB
 
 
