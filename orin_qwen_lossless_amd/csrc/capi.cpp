@@ -34,7 +34,7 @@ std::once_flag g_once;
 // Routing lists of bf16n_moe_mm_ids_static: device memory that belongs to the library, so that the call allocates
 // nothing.  Every GPU holds its own copy of the array for the life of the process (about 516 KiB).  In host code the
 // array's name is not a device address; the address on a device comes from hipGetSymbolAddress with that device
-// current, once per device (route_lists_of_current_device), and only that pointer is handed to kernels.
+// current, once per device (ensure_init), and only that pointer is handed to kernels.
 constexpr int STATIC_MAX_PAIRS = 1 << 16;   // routed (token, slot) pairs per call: 8192 tokens of top-8
 constexpr int STATIC_MAX_EXPERTS = 1024;
 struct route_lists {
@@ -45,8 +45,10 @@ struct route_lists {
 static __device__ __align__(256) unsigned char scratch[sizeof(route_lists)];
 
 constexpr int MAX_DEVICES = 64;
-route_lists * g_route_lists[MAX_DEVICES] = {};
-std::mutex g_route_lists_mutex;
+struct per_device {
+    std::once_flag once;
+    route_lists * lists = nullptr;
+} g_devices[MAX_DEVICES];
 
 void require(bool cond, const char * msg) {
     if (!cond) {
@@ -60,33 +62,30 @@ void hip_check(hipError_t e, const char * what) {
     }
 }
 
-route_lists * route_lists_of_current_device() {
+// What a launch needs of its device, at the first call with that device current: the kernels' shared-memory limits (a kernel
+// beyond 64 KiB may be refused on a device where its limit was not raised) and the address of the routing lists.  The counts
+// of CUs and LDS bytes are those of the first device.
+per_device & ensure_init() {
     int dev = 0;
     hip_check(hipGetDevice(&dev), "hipGetDevice");
     if (dev < 0 || dev >= MAX_DEVICES) {
         throw std::runtime_error("bf16n: device ordinal beyond the library's per-device tables");
     }
-    std::lock_guard<std::mutex> lock(g_route_lists_mutex);
-    if (!g_route_lists[dev]) {
-        void * p = nullptr;
-        hip_check(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)), "hipGetSymbolAddress (routing lists)");
-        g_route_lists[dev] = static_cast<route_lists *>(p);
-    }
-    return g_route_lists[dev];
-}
-
-void ensure_init() {
-    std::call_once(g_once, [] {
-        int dev = 0;
-        hip_check(hipGetDevice(&dev), "hipGetDevice");
+    std::call_once(g_once, [&] {
         hip_check(hipDeviceGetAttribute(&g_cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
         hip_check(hipDeviceGetAttribute(&g_lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev), "hipDeviceGetAttribute");
+    });
+    per_device & d = g_devices[dev];
+    std::call_once(d.once, [&] {
         dev::compat_init();
         dev::w64_init();
         dev::mm_ids_init();
         dev::tile_init();
+        void * p = nullptr;
+        hip_check(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)), "hipGetSymbolAddress (routing lists)");
+        d.lists = static_cast<route_lists *>(p);
     });
-    (void) route_lists_of_current_device(); // per device; after the first call on a device this is a table lookup
+    return d;
 }
 
 template <typename F>
@@ -560,7 +559,7 @@ int bf16n_moe_mm_ids_static(const bf16n_weight * w, const bf16n_weight * up, con
         require((int64_t) n_tok * ids_row_stride < INT32_MAX, "routing ids too large for 32-bit indexing");
         require(((uintptr_t) x_bf16 & 15) == 0 && x_row % 8 == 0, "activations must be 16-byte aligned with 16-byte row strides");
         require(((uintptr_t) dst & 15) == 0 && dst_col % 4 == 0, "dst must be 16-byte aligned with a column stride that is a multiple of 4");
-        route_lists * r = route_lists_of_current_device();
+        route_lists * r = ensure_init().lists;
         const int nch = per_slot ? n_used : 1; // activations per (token, slot), as the down product takes them, or per token
         // every list entry and every bound the product reads is rewritten by the routing kernel: nothing to clear
         dev::launch_route(ids, ids_i64 != 0, ids_row_stride, r->src1, r->dst, r->bounds, n_experts, n_tok, n_used, nch, nch,

@@ -32,6 +32,16 @@ def test_cpp_headers_compile_and_run(tmp_path):
     assert got["views"] == "8 1"
 
 
+def test_every_device_gets_its_limits(tmp_path):
+    """Kernels beyond 64 KiB of shared memory need their limit raised on the device they run on, not on the first one only."""
+    exe = str(tmp_path / "two_devices")
+    subprocess.run([shutil.which("g++"), "-std=c++17", "-I" + os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "cpp", "two_devices.cpp"),
+                    "-o", exe, "-L" + LIBDIR, "-lbf16n_hip", "-Wl,-rpath," + LIBDIR, "-L/opt/rocm/lib", "-Wl,-rpath-link,/opt/rocm/lib"],
+                   check=True, capture_output=True, timeout=300)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout.split()
+    assert int(out[0]) > 0 and out[1:] == ["1", out[0], "1", "1"], out
+
+
 @pytest.mark.gpu
 def test_cpp_api_on_the_device(tmp_path):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
