@@ -51,7 +51,7 @@ template <int FORMAT> struct lane_ring {
     }
     __device__ __forceinline__ uint32_t word(uint32_t i) const { return ring[(i & (LR_WORDS - 1)) * 64]; }
     __device__ __forceinline__ void begin(const uint32_t * sp, uint32_t * ring_) {
-        src = (const uint4 *) ((uintptr_t) sp & ~(uintptr_t) 15);
+        src = (const uint4 *) (sp - ((uintptr_t) sp >> 2 & 3)); // (as a number it would lose its address space)
         ring = ring_;
         uint4 b[LOOK + 1];
 #pragma unroll
@@ -170,6 +170,14 @@ __device__ __forceinline__ float x_at(const char * x, int i);
 template <> __device__ __forceinline__ float x_at<float>(const char * x, int i) { return ((const float *) x)[i]; }
 template <> __device__ __forceinline__ float x_at<bf16_t>(const char * x, int i) { return bf16_bits_to_f32(((const uint16_t *) x)[i]); }
 
+template <typename TX>
+__device__ __forceinline__ float4 x_four(const char * x, int i);
+template <> __device__ __forceinline__ float4 x_four<float>(const char * x, int i) { return ((const float4 *) x)[i]; }
+template <> __device__ __forceinline__ float4 x_four<bf16_t>(const char * x, int i) {
+    const uint2 v = ((const uint2 *) x)[i];
+    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u));
+}
+
 __device__ __forceinline__ float dot_chunk(const uint32_t (&wp)[8], const float4 (&x)[4]) {
     float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
@@ -182,7 +190,7 @@ __device__ __forceinline__ float dot_chunk(const uint32_t (&wp)[8], const float4
     return (a0 + a1) + (a2 + a3);
 }
 
-// the activations a lane meets in a chunk, from LDS: as FP32, or as the BF16 they came in (several columns)
+// the activations a lane meets in a chunk, from LDS (or from where they came): as FP32, or as BF16 (several columns)
 template <typename TX> struct x_lds;
 template <> struct x_lds<float> {
     float4 v[4];
@@ -203,9 +211,7 @@ template <> struct x_lds<bf16_t> {
             v[j] = *(const uint2 *) (xs + col0 + 128 * j);
         }
     }
-    __device__ __forceinline__ float4 get(int j) const {
-        return make_float4(__uint_as_float(v[j].x << 16), __uint_as_float(v[j].x & 0xFFFF0000u), __uint_as_float(v[j].y << 16), __uint_as_float(v[j].y & 0xFFFF0000u));
-    }
+    __device__ __forceinline__ float4 get(int j) const { return x_four<bf16_t>((const char *) v, j); }
     __device__ __forceinline__ static uint16_t store(const char * x, int i) { return ((const uint16_t *) x)[i]; }
 };
 
@@ -348,6 +354,28 @@ __global__ void __launch_bounds__(NT) k_huf_mmv(const bf16n_weight w, const bf16
     }
 }
 
+// exact BF16 bits of unit gu, the u-th of the rows at out, by one half-wave
+template <int FORMAT>
+__device__ __forceinline__ void unit_rows(const bf16n_weight & w, const uint32_t * lut, uint32_t * ring, int64_t gu, int64_t u, int l32, uint16_t * __restrict__ out) {
+    const int K = (int) w.K, C = K / CHUNK, R = w.R;
+    const bool cm = (w.flags & FLAG_CHUNK_MAJOR) != 0;
+    int rr = 0, c = 0;
+    for_chunks<FORMAT>(w.plane + gu * R * (int64_t) K, lane_stream<FORMAT>(w, gu, l32), ring, lut, R * C, l32, [] {}, [&](int, const uint32_t (&wp)[8]) {
+        uint16_t * dst = out + (u * R + rr) * K + c * CHUNK;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            *(uint2 *) (dst + 128 * j + 4 * l32) = make_uint2(wp[2 * j], wp[2 * j + 1]);
+        }
+        if (cm) {
+            rr = rr + 1 < R ? rr + 1 : 0;
+            c += rr == 0;
+        } else {
+            c = c + 1 < C ? c + 1 : 0;
+            rr += c == 0;
+        }
+    });
+}
+
 // exact BF16 bits of rows [row0, row0 + nrows) (whole units), row-major; one half-wave per unit
 template <int FORMAT>
 __global__ void __launch_bounds__(NT) k_huf_dequant(const bf16n_weight w, int64_t row0, int64_t nrows, uint16_t * __restrict__ out) {
@@ -360,27 +388,10 @@ __global__ void __launch_bounds__(NT) k_huf_dequant(const bf16n_weight w, int64_
         lut[i] = ((const uint32_t *) (w.aux + w.off_a))[i];
     }
     __syncthreads();
-    const int K = (int) w.K, C = K / CHUNK, R = w.R;
-    const bool cm = (w.flags & FLAG_CHUNK_MAJOR) != 0;
-    const int l32 = threadIdx.x & 31, half = threadIdx.x >> 5, halves = nt >> 5;
+    const int R = w.R, l32 = threadIdx.x & 31, half = threadIdx.x >> 5, halves = nt >> 5;
     uint32_t * ring = rings + (threadIdx.x >> 6) * (LR_BYTES / 4) + (threadIdx.x & 63);
     for (int64_t u = (int64_t) blockIdx.x * halves + half; u < nrows / R; u += (int64_t) gridDim.x * halves) {
-        const int64_t gu = row0 / R + u;
-        int rr = 0, c = 0;
-        for_chunks<FORMAT>(w.plane + gu * R * (int64_t) K, lane_stream<FORMAT>(w, gu, l32), ring, lut, R * C, l32, [] {}, [&](int, const uint32_t (&wp)[8]) {
-            uint16_t * dst = out + (u * R + rr) * K + c * CHUNK;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                *(uint2 *) (dst + 128 * j + 4 * l32) = make_uint2(wp[2 * j], wp[2 * j + 1]);
-            }
-            if (cm) {
-                rr = rr + 1 < R ? rr + 1 : 0;
-                c += rr == 0;
-            } else {
-                c = c + 1 < C ? c + 1 : 0;
-                rr += c == 0;
-            }
-        });
+        unit_rows<FORMAT>(w, lut, ring, row0 / R + u, u, l32, out);
     }
 }
 
@@ -465,6 +476,11 @@ __device__ __forceinline__ void nib_load_chunk(const nib_ptrs & w, int64_t gr, i
 // segment early, 48 codes, because one thread out of step costs its block another round).
 // The number of codes in the segments before it gives a thread its place, and a last round writes the exponents to LDS in the
 // order of the plane.  The products are those of unit_dot, a row per half-wave, added in the same order: the same bits.
+// Codes whose lengths are nearly all multiples of one number keep a wrong phase for long: such tables are told by their lengths
+// (falls_into_step), and their units go to one half-wave each in here too (split_whole).  In a run of one code, rows of zeros for
+// instance, no thread falls into step: every second round the threads past the first one that still moves take their phase from
+// the code that begins there, if the next three are the same (14 of 16 rows of 4096, one unit of 64: 136 us with a round per
+// segment, 52 so, 80 in k_huf_mmv; the threads before it are exact, and it gains one a round, so S rounds are enough).
 // Two rounds and a half of a sixteenth of the chain instead of the chain, for as many lookups per code: for launches that wait for
 // the chain (hp_split_cols).  8192 x 2048, one column: 42.4 -> 26.6 us (34 with a third round that wrote the exponents: the
 // codes of the second stay in registers until their place is known).
@@ -475,7 +491,7 @@ constexpr int SPLIT_AHEAD = 4;                   // plane chunks of a row asked 
 // words of a unit's streams at most: twelve bits a pair code, the last word of each lane begun
 __host__ __device__ constexpr uint32_t split_words(int pairs) { return (uint32_t) (HP_LP * pairs + 32); }
 constexpr size_t split_shm(int pairs, int threads) {
-    return ((size_t) LUT_PAIRS + split_words(pairs) + 2 * SPLIT_PAD + 16 * (size_t) pairs + 2 * (size_t) threads + (size_t) threads / 32 + 1) * 4;
+    return ((size_t) LUT_PAIRS + split_words(pairs) + 2 * SPLIT_PAD + 16 * (size_t) pairs + 2 * (size_t) threads + 32 + (size_t) threads / 32 + 1) * 4;
 }
 
 // A position in the words at st.  n: minus the bit position; its low five bits are what the funnel shift takes (the next 32
@@ -510,32 +526,111 @@ struct seg_bits {
     }
 };
 
+// Whether a decoder that begins anywhere falls into step with this table's codes soon enough.  Its phase modulo g moves only at
+// codes whose length is no multiple of g: with a share s of multiples one of 2 (1 - s) codes moves one of the two, and one in
+// g - 1 moves ends in step, after (g - 1) / (2 (1 - s)) codes on average.  The share is that of 64 samples of the table, which
+// stands in the order of its codes: as many of a length as its codes are met.  Codes all of one length are told by the first
+// and the last: segments begin at multiples of it, all in step, and only the LDS bank at which every lane's stream then begins costs.
+__device__ __forceinline__ bool falls_into_step(uint32_t entry, uint32_t inv_codes, bool equal) { // lane i: entry 64 i + 32, lanes 0 and 63: the first, the last
+    const uint32_t len = entry & 31u;
+    bool does = true;
+#pragma unroll
+    for (int g : {2, 3, 4, 5, 6, 7, 11}) { // (8 to 10 and 12 are multiples of these)
+        does &= (uint32_t) __builtin_popcountll(__ballot(len != 0 && len % (uint32_t) g == 0)) <= 64 - (((uint32_t) (g - 1) * inv_codes + 255) >> 8);
+    }
+    const uint32_t first = __builtin_amdgcn_readlane(len, 0), last = __builtin_amdgcn_readlane(len, 63);
+    return first == last ? equal : does;
+}
+
+// units: the launch's first, all of the matrix, the launch's; the device's CUs; 8192 over the codes that a wrong phase may last
+struct split_units { int64_t first, all; int count, cus; uint32_t inv_codes; };
+
+// The units of a launch by one half-wave each, two units of a column to a wavefront, in `words` words of LDS at lds: the
+// activations of the block's column and a ring per wavefront (5120 words at K = 4096 with one, of 7700 at least).
+template <typename TX, bool DEQ>
+__device__ __forceinline__ void split_whole(const bf16n_weight & w, const cols & p, int ncols, uint16_t * __restrict__ out, const split_units & su,
+                                            const uint32_t * lut, uint32_t * lds, int words) {
+    const int K = (int) w.K, lane = threadIdx.x & 63, l32 = lane & 31, wave = threadIdx.x >> 6, all = blockDim.x >> 6;
+    const int n = DEQ ? 1 : ncols, per_col = (su.count + 1) / 2; // wavefronts a column
+    // one block of a CU while its wavefronts have a SIMD each (512 units, four columns: 41.1 us, on two blocks 46.7)
+    const int blocks = per_col * n <= 4 * su.cus && (int) gridDim.x > su.cus ? su.cus : (int) gridDim.x;
+    int mine = (per_col * n + blocks - 1) / blocks; // wavefronts of a block, all of one column
+    while ((per_col + mine - 1) / mine * n > blocks && mine < per_col) {
+        mine++;
+    }
+    const int col_blocks = (per_col + mine - 1) / mine, fit = (words - (DEQ ? 0 : K)) / (LR_BYTES / 4), waves = fit < all ? fit : all;
+    for (int b = (int) blockIdx.x; b < col_blocks * n; b += (int) gridDim.x) { // (once but for more columns than blocks)
+        const int col = b / col_blocks, j0 = b % col_blocks * mine, j1 = j0 + mine < per_col ? j0 + mine : per_col;
+        float * xs = (float *) lds;
+        __syncthreads();
+        if constexpr (!DEQ) {
+            for (int i = threadIdx.x; i < K / 4; i += (int) blockDim.x) {
+                ((float4 *) xs)[i] = x_four<TX>(p.x + col * p.x_tok, i);
+            }
+            __syncthreads();
+        }
+        uint32_t * ring = lds + (DEQ ? 0 : K) + wave * (LR_BYTES / 4) + lane;
+        for (int j = wave < waves ? j0 + wave : j1; j < j1; j += waves) {
+            const int u = 2 * j + (lane >> 5) < su.count ? 2 * j + (lane >> 5) : 2 * j;
+            if constexpr (DEQ) {
+                unit_rows<FMT_HUFPAIR>(w, lut, ring, su.first + u, u, l32, out);
+            } else {
+                float v[1];
+                unit_dot<FMT_HUFPAIR, true, 1, x_lds<float>>(w.plane, lut, lane_stream<FMT_HUFPAIR>(w, su.first + u, l32), ring, su.first + u, w.R, K / CHUNK,
+                                                             (w.flags & FLAG_CHUNK_MAJOR) != 0, xs, l32, v);
+                if (l32 < w.R && u == 2 * j + (lane >> 5)) { // (a missing second unit is the first again, which is stored once)
+                    store_y(p.y + col * p.y_tok, p.y_bf16, (int64_t) u * w.R + l32, v[0]);
+                }
+            }
+        }
+    }
+}
+
 // DEQ: the exact BF16 bits of the rows to out, no products
 template <typename TX, bool DEQ>
-__global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const cols p, int ncols, uint16_t * __restrict__ out) {
+__global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const cols p, int ncols, uint16_t * __restrict__ out, const split_units su) {
     extern __shared__ __align__(16) unsigned char shm_raw[];
     const int K = (int) w.K, C = K / CHUNK, R = w.R, pairs = R * C * 8, S = (int) blockDim.x >> 5;
     const uint32_t cap = split_words(pairs);
     uint32_t * lut = (uint32_t *) shm_raw;
     uint32_t * st = lut + LUT_PAIRS + SPLIT_PAD;
     uint16_t * ex = (uint16_t *) (st + cap + SPLIT_PAD); // [chunk][lane][8 pairs], an exponent per byte
-    uint32_t * ends = (uint32_t *) (ex + 32 * pairs), * counts = ends + blockDim.x, * again = counts + blockDim.x; // [round]
+    uint32_t * ends = (uint32_t *) (ex + 32 * pairs), * counts = ends + blockDim.x;
+    uint32_t * front = counts + blockDim.x, * again = front + 32, * in_step = lut + LUT_PAIRS; // [lane], [round], in front of the streams
     const hp_ptrs q = hpp(w);
     const int tid = threadIdx.x, l32 = tid & 31, seg = tid >> 5;
     const bool cm = (w.flags & FLAG_CHUNK_MAJOR) != 0;
+    // what the first unit's loads and the branch wait for is asked for ahead of the table
+    const uint32_t sample = q.lut[tid % 64 == 0 ? 0 : tid % 64 == 63 ? LUT_PAIRS - 1 : tid % 64 * (LUT_PAIRS / 64) + LUT_PAIRS / 128];
+    uint32_t base, end, from, to;
+    auto head = [&](int u) {
+        const int64_t gu = su.first + u;
+        base = q.ubase[gu];
+        end = gu + 1 < su.all ? q.ubase[gu + 1] : (uint32_t) ((const aux_header *) w.aux)->n_b;
+        from = q.lrel[gu * 32 + l32];
+        to = q.lrel[gu * 32 + (l32 < 31 ? l32 + 1 : l32)];
+    };
+    head((int) blockIdx.x < su.count ? (int) blockIdx.x : 0);
     for (int i = tid; i < LUT_PAIRS / 4; i += (int) blockDim.x) {
         uint4 v = ((const uint4 *) q.lut)[i];
         v.x += (v.x & 31u) == 0; v.y += (v.y & 31u) == 0; v.z += (v.z & 31u) == 0; v.w += (v.w & 31u) == 0;
         ((uint4 *) lut)[i] = v;
     }
-    const int64_t units = p.nrows / R, all_units = w.rows / R;
-    for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
-        const int64_t gu = p.row0 / R + u;
+    if (tid < 64) {
+        const bool does = falls_into_step(sample, su.inv_codes, su.count <= (int) gridDim.x);
+        if (tid == 0) {
+            *in_step = does;
+        }
+    }
+    for (int u = (int) blockIdx.x; u == (int) blockIdx.x || u < su.count; u += (int) gridDim.x) { // (split_whole has work for a block without a unit)
+        if (u != (int) blockIdx.x) {
+            head(u);
+        }
+        const int64_t gu = su.first + (u < su.count ? u : 0);
         const uint4 * plane = (const uint4 *) (w.plane + gu * R * (int64_t) K) + l32;
         auto chunk_at = [&](int rr, int c) { return cm ? c * R + rr : rr * C + c; }; // in stream order
-        const uint32_t base = q.ubase[gu], end = gu + 1 < all_units ? q.ubase[gu + 1] : (uint32_t) ((const aux_header *) w.aux)->n_b;
         const uint32_t words = end <= base ? 0 : end - base < cap ? end - base : cap; // (none for a base past the stream's end)
-        uint32_t from = q.lrel[gu * 32 + l32], to = l32 < 31 ? q.lrel[gu * 32 + l32 + 1] : words;
+        to = l32 < 31 ? to : words;
         from = from < words ? from : words;
         to = to < from ? from : to < words ? to : words;
         uint4 ahead[SPLIT_AHEAD];
@@ -543,14 +638,32 @@ __global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const c
         for (int i = 0; i < SPLIT_AHEAD; i++) {
             ahead[i] = plane[chunk_at(seg < R ? seg : R - 1, i < C ? i : C - 1) * 32];
         }
-#pragma unroll 8
-        for (uint32_t i = tid; i < words; i += blockDim.x) {
-            st[i] = q.stream[base + i];
+        for (uint32_t i0 = tid; i0 < words; i0 += 8 * blockDim.x) {
+            uint32_t v[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k++) { // (asked for together; past the end the last one again, unused)
+                const uint32_t i = i0 + k * blockDim.x;
+                v[k] = q.stream[base + (i < words ? i : words - 1)];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k++) {
+                const uint32_t i = i0 + k * blockDim.x;
+                if (i < words) {
+                    st[i] = v[k];
+                }
+            }
         }
         if (tid <= S) {
             again[tid] = 0;
         }
         __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(*in_step) == 0) {
+            split_whole<TX, DEQ>(w, p, ncols, out, su, lut, lut + LUT_PAIRS, (int) (again - lut) - LUT_PAIRS);
+            return;
+        }
+        if (u >= su.count) {
+            return;
+        }
         const uint32_t first = 32 * from, bits = 32 * (to - from); // (at most 24 K)
         const uint32_t nstop = 0u - (first + bits * (uint32_t) (seg + 1) / (uint32_t) S);
         uint32_t start = first + bits * (uint32_t) seg / (uint32_t) S - (seg ? bits / (uint32_t) (2 * S) : 0), n = 0;
@@ -567,14 +680,32 @@ __global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const c
         __syncthreads();
         for (int round = 0; round <= S; round++) {
             const uint32_t exact = seg ? ends[tid - 32] : first;
-            const bool moved = exact != start || round == 0;
+            bool moved = exact != start || round == 0;
             start = exact;
             if (moved) {
                 again[round] = 1;
+                if (round % 2 == 0) {
+                    atomicMin(&front[l32], (uint32_t) seg);
+                }
+            }
+            if (round % 2 != 0 && seg == 0) {
+                front[l32] = (uint32_t) S;
             }
             __syncthreads();
             if (again[round] == 0) {
                 break;
+            }
+            if (round != 0 && round % 2 == 0 && front[l32] < (uint32_t) seg) {
+                const uint32_t begins = ends[32 * front[l32] - 32 + l32], mine = first + bits * (uint32_t) seg / (uint32_t) S;
+                uint32_t e0, e1, e2, e3;
+                seg_bits b(st, begins);
+                b.two(lut, 0x80000000u, e0, e1);
+                b.two(lut, 0x80000000u, e2, e3);
+                if (e0 == e1 && e1 == e2 && e2 == e3) { // a run
+                    const uint32_t len = e0 & 31u;
+                    start = mine > begins ? begins + (mine - begins + len - 1) / len * len : begins;
+                    moved = true;
+                }
             }
             if (moved) {
                 seg_bits b(st, start);
@@ -651,7 +782,7 @@ __global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const c
                             uint32_t wp[8];
                             weights(c, ahead[i], wp);
                             if constexpr (DEQ) {
-                                uint16_t * dst = out + (u * R + rr) * K + c * CHUNK;
+                                uint16_t * dst = out + ((int64_t) u * R + rr) * K + c * CHUNK;
 #pragma unroll
                                 for (int j = 0; j < 4; j++) {
                                     *(uint2 *) (dst + 128 * j + 4 * l32) = make_uint2(wp[2 * j], wp[2 * j + 1]);
@@ -673,7 +804,7 @@ __global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const c
                 if (!DEQ) {
                     const float v = cm ? acc : half_wave_sum_dpp(acc);
                     if (l32 == 31) {
-                        store_y(p.y + col * p.y_tok, p.y_bf16, u * R + rr, v);
+                        store_y(p.y + col * p.y_tok, p.y_bf16, (int64_t) u * R + rr, v);
                     }
                 }
             }
@@ -1237,15 +1368,24 @@ int split_threads(const bf16n_weight & w) {
     const int pairs = w.R * (int) (w.K / CHUNK) * 8, segs = (pairs + SPLIT_PAIRS - 1) / SPLIT_PAIRS;
     return 64 * ((segs + 1) / 2);
 }
+// Codes that a wrong phase may last on average before the units go to a half-wave each (falls_into_step): a round more costs
+// a sixteenth of the chain on a CU that has one unit, more beside others, and beyond two the gain is small.  One column, in
+// segments / by half-waves against a chain each (k_huf_mmv), at 1 / 2 / 3 units of 16 x 2048 per CU: codes of three bits
+// with one in eight of four (8) 0.57 / 0.76 / 0.93, of five bits with one in eight of four and six (16) 0.72 / 0.80 / 1.17, of seven
+// so (24) 0.92 / 1.27 / 1.55, 94 % of four bits (24) 0.65 to 1.10 / 0.84 to 1.13 / 1.04 to 1.87, 95 % and all but a few of six
+// (50 and more) 1.21 and 1.34 / 1.33 and 1.52 / 1.96 and 2.11; by half-waves in here 0.98 to 1.07 throughout
+uint32_t split_codes(int64_t units, int cus) { return units <= cus ? 30 : units <= 2 * (int64_t) cus ? 20 : 7; }
 template <typename TX, bool DEQ>
 void launch_hp_split(const bf16n_weight & w, const cols & p, int ncols, uint16_t * out, int cus, hipStream_t stream) {
     const int threads = split_threads(w);
     const size_t shm = split_shm(w.R * (int) (w.K / CHUNK) * 8, threads);
     const int64_t units = p.nrows / w.R, fit = (int64_t) cus * std::max<int64_t>(1, std::min<int64_t>(2048 / threads, (int64_t) (LDS_BYTES / shm)));
+    const int64_t blocks = std::max(units, (units + 1) / 2 * ncols); // (split_whole: a block per two units of a column)
     if (!DEQ) { // (the note is of products)
         note_kernel("k_hp_split", tx_name<TX>(), 1, 0);
     }
-    hipLaunchKernelGGL((k_hp_split<TX, DEQ>), dim3((unsigned) std::min(units, fit)), dim3(threads), shm, stream, w, p, ncols, out);
+    hipLaunchKernelGGL((k_hp_split<TX, DEQ>), dim3((unsigned) std::min(blocks, fit)), dim3(threads), shm, stream, w, p, ncols, out,
+                       split_units{p.row0 / w.R, w.rows / w.R, (int) units, cus, 8192u / split_codes(units, cus)});
 }
 
 } // namespace

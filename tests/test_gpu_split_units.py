@@ -1,6 +1,9 @@
 """k_hp_split (HUFPAIR units whose lanes' streams are decoded in segments): the bits of the kernel with one half-wave per
-unit, which takes the batches of more columns, for streams that fall into step, that never do, and of very short codes."""
+unit, which takes the batches of more columns, for streams that fall into step, that never or hardly do (whole tables, or runs of one
+code in a unit), and of very short codes; the streams that do not cost no more than that kernel's chain."""
 from __future__ import annotations
+
+import statistics
 
 import numpy as np
 import pytest
@@ -21,6 +24,15 @@ def _matrix(kind: str, rows: int, K: int) -> np.ndarray:
         return np.where(rng.random(wb.shape) < 0.03, 0x4081, 0x3F81).astype(np.uint16)
     if kind == "flat":         # 4096 pairs, equally frequent: codes of twelve bits throughout, which never fall into step
         return ((wb & 0x807F) | (rng.integers(64, 128, wb.shape) << 7)).astype(np.uint16)
+    if kind == "equal":        # sixteen pairs, equally frequent
+        return ((wb & 0x807F) | (rng.integers(100, 104, wb.shape) << 7)).astype(np.uint16)
+    if kind == "rare":         # 64 pairs of six bits, and one weight in two thousand of another exponent: out of step for hundreds of codes
+        e = np.where(rng.random(wb.shape) < 0.0005, rng.integers(90, 92, wb.shape), rng.integers(100, 108, wb.shape))
+        return ((wb & 0x807F) | (e << 7)).astype(np.uint16)
+    if kind == "run":          # rows of zeros in the middle of a unit, in another two runs of one code each
+        wb[rows // 2 + 1: rows // 2 + 15] = 0
+        wb[2:6] = 0
+        wb[9:14] = 0x3F00
     return wb
 
 
@@ -29,7 +41,10 @@ def _matrix(kind: str, rows: int, K: int) -> np.ndarray:
     ("normal", 1, 2048, 16, False), ("normal", 300, 2048, 16, True), ("normal", 513, 2048, 16, False), ("normal", 5, 4096, 16, True),
     ("normal", 257, 4096, 16, False), ("normal", 33, 1024, 16, True), ("normal", 7, 2048, 8, False), ("normal", 9, 3072, 8, True),
     ("normal", 9, 2560, 8, False), ("one", 3, 2048, 16, False), ("short", 3, 2048, 16, False), ("short", 2, 4096, 16, True),
-    ("flat", 3, 2048, 16, False), ("flat", 2, 4096, 16, False), ("flat", 2, 2048, 8, True)])
+    ("flat", 3, 2048, 16, False), ("flat", 2, 4096, 16, False), ("flat", 2, 2048, 8, True),
+    ("equal", 1, 2048, 16, False), ("equal", 2, 4096, 4, False), ("equal", 515, 2048, 16, False), ("rare", 7, 2048, 16, True),
+    ("rare", 7, 4096, 8, False), ("rare", 301, 4096, 16, False), ("rare", 33, 3072, 8, True), ("rare", 513, 2048, 16, False),
+    ("run", 9, 2048, 16, False), ("run", 3, 4096, 16, False), ("run", 300, 2048, 16, True), ("run", 5, 1024, 16, False), ("run", 4, 3072, 8, False)])
 def test_split_units_have_the_bits_of_whole_ones(ops, kind, units, K, R, cm):
     rows = units * R
     wb = _matrix(kind, rows, K)
@@ -49,3 +64,32 @@ def test_split_units_have_the_bits_of_whole_ones(ops, kind, units, K, R, cm):
     if units > 2:                                              # a range of units that ends before the matrix, and the last one
         assert np.array_equal(bits(ops.dequant(w, R, R)), wb[R:2 * R])
         assert np.array_equal(bits(ops.dequant(w, rows - R, R)), wb[-R:])
+
+
+def _us(f) -> float:
+    """Median time of a call among thirty, in microseconds."""
+    times = []
+    f()
+    for _ in range(7):
+        t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        t0.record()
+        for _ in range(30):
+            f()
+        t1.record()
+        t1.synchronize()
+        times.append(t0.elapsed_time(t1) * 1000 / 30)
+    return statistics.median(times)
+
+
+# 64 units: nine columns are nine chains side by side on an otherwise idle device, k_huf_mmv's time.  Measured here / there, us:
+# rare 40 / 43 (59 with a round per segment), run 52 / 81 (136)
+@pytest.mark.parametrize("kind,K", [("rare", 2048), ("run", 4096)])
+def test_streams_out_of_step_take_no_longer_than_a_chain(ops, kind, K):
+    w = enc(ops, _matrix(kind, 64 * 16, K), HP, 16, False, False)
+    x = tbf16(synth.activations(9, K, 7))
+    split = _us(lambda: ops.mmv(x[:1], w))
+    assert ops.last_kernel().startswith("k_hp_split<")
+    chain = _us(lambda: ops.mmv(x, w))
+    assert not ops.last_kernel().startswith("k_hp_split<")
+    print(f"{kind}: {split:.1f} us, chain {chain:.1f}")
+    assert split <= 1.2 * chain, (split, chain)
