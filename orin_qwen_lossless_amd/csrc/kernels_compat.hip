@@ -1346,22 +1346,26 @@ bool huf_direct(const bf16n_weight & w, int64_t units, int cus) {
 }
 
 // Columns up to which a launch over `units` units takes k_hp_split (0: none): while the chain of a unit is longer than what its
-// blocks take on the CUs they get.  A CU holds two blocks, one beyond 512 pair codes a lane, and every column adds its products
-// to each of them.  us, one half-wave per unit / this (R = 16 at K = 2048 and 4096, 8 at 3072 and 3584):
-//   one column: 4096 x 2048 40.9 / 17.7, 8192 x 2048 42.4 / 26.6, 12288 x 2048 47.0 / 36.4, 16384 x 2048 45.6 / 46.1; 4096 x 4096 79 / 26,
-//     8192 x 4096 80 / 49, 12288 x 4096 87 / 76, 16384 x 4096 85 / 95; 4096 x 3072 33 / 23, 5000 x 3072 36.4 / 37.3; 6000 x 3584 42 / 36
-//   8192 x 2048 at 4 / 8 columns 43 / 48 and 33 / 44; 8192 x 4096 at 4 80 and 74, at 8 91 and 100; 4096 x 3072 at 4 / 8 34 / 38 and
-//     31 / 43; 8192 x 1024 at 3 / 4 28 / 25 and 25 / 26; 12288 x 4096 at 3 90 and 98; 12288 x 2048 at 8 67 and 60
-//   dequant of 8192 x 2048 38 / 28, 8192 x 4096 70 / 50, 4096 x 3072 30 / 24; 8192 x 1024 22 / 23
-int hp_split_cols(const bf16n_weight & w, int64_t units, int cus) {
-    const int pairs = w.R * (int) (w.K / CHUNK) * 8;
+// blocks take on the CUs they get.  A CU holds two blocks up to 512 pair codes a lane, one beyond.  Every column adds its products
+// to a block, and where a row has more chunks than its first wavefront keeps it reads the plane again (`rows`: exact rows, which
+// read it once).  Times as multiples of k_huf_mmv's, BF16 columns:
+//   up to two units per CU, one / 2 / 4 / 6 / 8 columns: 8192 x 2048, R = 16 0.64 / 0.64 / 0.78 / 0.78 / 0.87, 4096 x 2048 0.46 / 0.50 /
+//     0.55 / 0.58 / 0.73; 4096 x 4096, R = 8 0.58 / 0.64 / 0.86 / 0.89 / 1.02; 4096 x 3584, R = 8 0.69 / 0.72 / 0.93 / 0.95 / 1.09; 4096 x 3072,
+//     R = 8 0.71 / 0.76 / 0.96 / 0.98 / 1.12; 8192 x 1024 0.84 / 0.87 / 1.07 / 1.09 / 1.22; 8192 x 4096 0.68 / 0.72 / 0.96 / 1.05 / 1.28
+//   three, in two passes of two blocks: 12288 x 2048 0.82 / 0.84 / 0.95 / 0.77 / 0.82 (640 units, six: 1.05); 6144 x 4096, R = 8 0.83 / 0.94 /
+//     1.14 / 1.00 / 1.09; 6144 x 3584 0.92 / 0.99; 6144 x 3072 1.00 / 1.07; or in three passes of one, a column: 12288 x 2560 1.06,
+//     12288 x 3072 0.96, 12288 x 3584 0.96, 12288 x 4096 0.94
+//   dequant at two units per CU 0.78 / 0.70 / 0.80 / 0.82 / 0.93 / 0.79 in the first line's order, at three 0.93, 0.93, 1.02, 1.11
+int hp_split_cols(const bf16n_weight & w, int64_t units, int cus, bool rows = false) {
+    const int C = (int) (w.K / CHUNK), pairs = w.R * C * 8;
+    const bool kept = rows || C <= SPLIT_AHEAD;
     if (w.format != FMT_HUFPAIR || pairs < 256 || pairs > 1024 || units > 3 * (int64_t) cus) {
         return 0;
     }
     if (units > 2 * (int64_t) cus) {
-        return pairs == 512 ? 8 : pairs >= 448 ? 1 : 0;
+        return pairs == 512 ? kept ? 8 : 2 : pairs == 448 || pairs >= 768 ? 1 : 0;
     }
-    return pairs <= 512 ? (pairs - 128) / 48 : units > cus ? 4 : 8;
+    return pairs <= 512 ? std::min((pairs - 128) / 48, kept ? 8 : 6) : units > cus ? 4 : 8;
 }
 constexpr int SPLIT_DEQUANT_COLS = 3; // what the exact rows cost in its place, in columns
 int split_threads(const bf16n_weight & w) {
@@ -1567,7 +1571,7 @@ void launch_compat_dequant(const bf16n_weight & w, int64_t row0, int64_t nrows, 
     const dim3 grid((unsigned) (blocks < (int64_t) cus * 16 ? blocks : (int64_t) cus * 16));
     if (w.format == FMT_NIBBLE) {
         launch_nib_rows(w, nullptr, 0, nrows, row0, (char *) out, true, (int64_t) w.K * 2, grid, stream);
-    } else if (hp_split_cols(w, work, cus) >= SPLIT_DEQUANT_COLS) {
+    } else if (hp_split_cols(w, work, cus, true) >= SPLIT_DEQUANT_COLS) {
         cols p = {};
         p.row0 = row0;
         p.nrows = nrows;
