@@ -1313,6 +1313,11 @@ int huf_waves(int64_t units, int ncols, int cus, int chunks) {
     return waves;
 }
 
+// LDS of a block of k_huf_mmv with several columns
+size_t huf_shared(const bf16n_weight & w, int nc, bool x_bf16) {
+    return (size_t) nc * w.K * (x_bf16 ? 2 : 4) + (w.format == FMT_HUFPAIR ? 4u << HP_LP : 4u << HUF_LMAX) + (size_t) (NT / 64) * LR_BYTES;
+}
+
 // Columns that share one decode in dense products.  Each column in a launch of its own units decodes the matrix again, which
 // costs nothing while the device has half-waves to spare (a unit's chain is longer than what they do beside it), and everything
 // beyond: from sixteen half-waves per CU on two columns share one, from eight groups of four per CU on four.  us, each column by
@@ -1323,25 +1328,40 @@ int huf_waves(int64_t units, int ncols, int cus, int chunks) {
 //     218800 x 512, R = 1 225 / 142 / 90, 7624 x 1536, R = 4 (1906) 22.5 / 19.1 / 19.1, and three there 19.0 / 19.4 / 18.8
 //   eight: 10336 x 3584, R = 16 (646) 130 / 105 / 113, 16384 x 2048 77 / 62 / 66, 24608 x 1024 109 / 64 / 49, 42264 x 3072 496 / 257 / 181,
 //     59473 x 2560 405 / 257 / 172, 16384 x 3072, R = 8, HUFFMAN 231 / 111 / 86
+// A last group of four may hold one column: pairs then, and single columns, while their blocks are no more than the CUs hold anyway
+// (two of pairs, three where units are short).  1030 units of 4 x 1024, five columns 11.6 / 11.9 / 15.1, of 1 x 512 5.2 / 5.5 / 6.5; 1400, seven
+// 5.7 (6.7 by fours); but 2060 units, eight 8.5 / 7.2.
+// Four FP32 columns of 3584 and more leave a CU one block, so that the second waits for the first: pairs, but for HUFFMAN's longer units
+// once their pairs wait too.  1030 units of 1 x 4096, five columns 11.7 / 10.9 / 20.7, of 16 x 4096 160 / 101 / 193; HUFFMAN 1400 of
+// 1 x 4096, five 20.0 / 16.8 / 26.7, 800 of 4 x 4096, twelve 126 / 59 / 81, 3000, eight 485 / 163 / 121.
 // Blocks of eight wavefronts instead of four: 5 to 25 % behind but for long rows of short units.
-int huf_columns(const bf16n_weight & w, int64_t units, int ncols, int cus) {
+int huf_columns(const bf16n_weight & w, int64_t units, int ncols, bool x_bf16, int cus) {
     const int chunks = w.R * (int) (w.K / CHUNK);
-    if (ncols > 2 && units * ((ncols + 3) / 4) > 8 * (int64_t) cus) {
-        return 4;
+    const int64_t pairs = units * ((ncols + 1) / 2), fours = units * ((ncols + 3) / 4), full = 8 * (int64_t) cus; // half-waves; of a block per CU
+    int nc = ncols > 2 && fours > full ? 4 : ncols > 1 && units * ncols > 2 * full && (ncols != 3 || chunks >= 16) ? 2 : 1;
+    const bool alone = 2 * huf_shared(w, 4, x_bf16) > LDS_BYTES;
+    if (nc == 4 && (pairs <= (chunks <= 4 ? 3 : 2) * full || (alone && (w.format == FMT_HUFPAIR || chunks <= 8 || pairs <= 3 * full)))) {
+        nc = 2;
     }
-    return ncols > 1 && units * ncols > 16 * (int64_t) cus && (ncols != 3 || chunks >= 16) ? 2 : 1;
+    return nc == 2 && units * ncols <= 2 * full ? 1 : nc;
 }
 
-// Dense products of one column whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers
+// Dense products whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers
 // per wavefront, so that 16 of them (12 at K = 4096) fit a CU instead of 20 (16), and a lane that has not moved on loads its
-// block again; with many wavefronts the misses of one are covered by the others.  Without against with rings:
+// block again; with many wavefronts the misses of one are covered by the others.  Without against with rings, one column:
 //  * HUFPAIR in short units that the caches hold, from 64 wavefronts per CU on (32768 x 2048, four chunks, eight columns one by one:
 //    202 against 174 us).
 //  * HUFFMAN, which loads a block per eight codes where HUFPAIR has one per sixteen, from 16 wavefronts per CU on unless
 //    the matrix comes from memory in short units: 32768 x 4096, R = 4 142 against 208 us.
-bool huf_direct(const bf16n_weight & w, int64_t units, int cus) {
-    const int64_t per_cu = units / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
+// Several columns, one by one without rings against the fours that would share a decode: units of one chunk that the caches hold, from 48
+// wavefronts per CU on, where a quarter of the fours' columns or more would be missing: 9000 x 512, five 11.8 against 15.0, six 13.5 and
+// 15.0, nine 18.5 and 20.8 (seven 15.7 and 15.0); HUFFMAN 14.1 and 16.9, 16.0 and 16.9, 22 and 23.8.
+bool huf_direct(const bf16n_weight & w, int64_t units, int ncols, int nc, int cus) {
+    const int64_t per_cu = units * ncols / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
     const int chunks = w.R * (int) (w.K / CHUNK);
+    if (ncols > 1) {
+        return nc == 4 && chunks == 1 && per_cu >= 48 && weights <= (16 << 20) && ncols > 4 && ncols <= 3 * ((ncols + 3) / 4);
+    }
     return w.format == FMT_HUFPAIR ? chunks <= 8 && per_cu >= 64 && weights <= (16 << 20) : per_cu >= 16 && (weights <= (16 << 20) || chunks >= 32);
 }
 
@@ -1510,12 +1530,15 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
         return;
     }
     const size_t shared = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX));
-    const int nc = glu || p.ids ? 1 : huf_columns(w, work, ncols, cus);
-    if (nc > 1) {
+    const char * instance = hp ? x_bf16 ? "3, bf16_t" : "3, float" : x_bf16 ? "2, bf16_t" : "2, float";
+    const int nc = glu || p.ids ? 1 : huf_columns(w, work, ncols, x_bf16, cus);
+    const bool direct = !glu && !p.ids && huf_direct(w, work, ncols, nc, cus);
+    if (nc > 1 && !direct) {
         const int waves = NT / 64, groups = (ncols + nc - 1) / nc;
-        const size_t shm = (size_t) nc * w.K * (x_bf16 ? 2 : 4) + (hp ? (4u << HP_LP) : (4u << HUF_LMAX)) + (size_t) waves * LR_BYTES;
+        const size_t shm = huf_shared(w, nc, x_bf16);
         const int64_t blocks = std::min<int64_t>((work + 2 * waves - 1) / (2 * waves), (int64_t) cus * (int64_t) (LDS_BYTES / shm));
         const dim3 grid((unsigned) blocks, (unsigned) groups); // (a block stages its table and columns once)
+        note_kernel("k_huf_mmv", instance, 3, 0, 1, nc);
 #define HUFN(F, TX, N) hipLaunchKernelGGL((k_huf_mmv<F, TX, false, true, N>), grid, dim3(waves * 64), shm, stream, w, wu, p, ncols)
 #define HUFNX(F, TX) do { if (nc == 4) HUFN(F, TX, 4); else HUFN(F, TX, 2); } while (0)
         if (hp) {
@@ -1527,7 +1550,7 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
 #undef HUFN
         return;
     }
-    const bool direct = !glu && !p.ids && ncols == 1 && huf_direct(w, work, cus);
+    note_kernel("k_huf_mmv", instance, 3, glu != 0, !direct, 1);
     const int waves = direct ? NT / 64 : huf_waves(work, ncols, cus, w.R * (int) (w.K / CHUNK));
     const size_t shm = shared + (direct ? 0 : (size_t) waves * LR_BYTES);
     const dim3 grid(grid_for(work, ncols, cus, 2 * waves), ncols);

@@ -11,6 +11,9 @@ from test_gpu_kernels import HP, HUF, enc, tbf16
 pytestmark = pytest.mark.gpu
 
 
+reached: set[str] = set()
+
+
 # units around 8 and 16 per CU (a column by itself, two, four) and beyond; the most columns of LDS (K = 4096)
 @pytest.mark.parametrize("fmt,K,R,units,cm", [(HP, 512, 1, 1025, False), (HP, 512, 1, 2049, False), (HP, 1024, 4, 2051, True), (HP, 1536, 2, 1031, False),
                                               (HP, 2048, 8, 525, False), (HP, 4096, 1, 2051, False), (HP, 2048, 8, 1030, True),
@@ -21,9 +24,36 @@ def test_columns_that_share_a_decode(ops, fmt, K, R, units, cm):
     x = tbf16(synth.activations(11, K, 7))
     for xt in (x, x.float()):
         one = torch.cat([ops.mmv(xt[t:t + 1], w) for t in range(11)])
+        assert ops.last_kernel().endswith(", 1>")
         for t in (2, 3, 4, 5, 7, 8, 11):
             assert torch.equal(ops.mmv(xt[:t], w), one[:t]), t
+            reached.add(ops.last_kernel().split("<")[1][0] + ops.last_kernel()[-5:])
         assert torch.equal(ops.mmv(xt[:7], w, out_dtype=torch.bfloat16), one[:7].to(torch.bfloat16))
+    if (fmt, K, units) == (HUF, 4096, 2051):                   # (the last case) every instance but the one of columns without rings
+        assert reached >= {f"{f}1, {n}>" for f in (HP, HUF) for n in (1, 2, 4)}, reached
     wide = torch.zeros((5, K + 64), dtype=x.dtype, device="cuda")
     wide[:, :K] = x[:5]
     assert torch.equal(ops.mmv(wide[:, :K], w), ops.mmv(x[:5], w))
+
+
+# the lines between the instances on 256 CUs: RING and NC for each count of columns.  A last group of four with a column or two missing,
+# four FP32 columns of 4096 (a block per CU), one chunk a unit (columns one by one without rings)
+@pytest.mark.parametrize("fmt,K,R,units,f32,want", [
+    (HP, 1024, 4, 1030, False, {2: "1, 1", 4: "1, 2", 5: "1, 2", 7: "1, 4", 8: "1, 4"}),
+    (HP, 512, 1, 1030, False, {3: "1, 1", 5: "1, 2", 9: "1, 2", 12: "1, 4"}),
+    (HP, 4096, 1, 1030, True, {3: "1, 1", 5: "1, 2", 8: "1, 2", 16: "1, 2"}),
+    (HP, 4096, 1, 1030, False, {5: "1, 2", 8: "1, 4"}),
+    (HUF, 4096, 1, 1400, True, {5: "1, 2", 12: "1, 2"}),
+    (HUF, 4096, 4, 800, True, {9: "1, 2", 16: "1, 4"}),
+    (HP, 512, 1, 9000, True, {2: "1, 2", 4: "1, 4", 5: "0, 1", 6: "0, 1", 7: "1, 4", 9: "0, 1"}),
+    (HUF, 512, 1, 9000, False, {5: "0, 1", 8: "1, 4"})])
+def test_the_instance_for_a_count_of_columns(ops, fmt, K, R, units, f32, want):
+    if ops.cu_count() != 256:
+        pytest.skip("the counts are those of 256 CUs")
+    w = enc(ops, synth.weights(R * units, K, R * units + K), fmt, R, False, False)
+    x = tbf16(synth.activations(16, K, 7))
+    x = x.float() if f32 else x
+    one = torch.cat([ops.mmv(x[t:t + 1], w) for t in range(16)])
+    for t, instance in want.items():
+        assert torch.equal(ops.mmv(x[:t], w), one[:t]), t
+        assert ops.last_kernel() == f"k_huf_mmv<{fmt}, {'float' if f32 else 'bf16_t'}, 0, {instance}>", t
