@@ -872,8 +872,10 @@ __device__ __forceinline__ float nib_escapes(const nib_ptrs & w, uint32_t e0, ui
 //   dense, one BF16 column: 2048 x 2048 3.55 / 3.35, 5120 x 2048 6.0 / 5.5, 2048 x 4096 5.3 / 5.1, 16384 x 512 5.0 / 4.7
 //   FP32, three / eight columns: 5120 x 2048 10.2 / 16.8 -> 8.2 / 12.9, 2048 x 4096 9.3 / 15.8 -> 8.0 / 12.7
 //   257 experts' down (2048 x 512), 1 / 4 / 12 tokens of nine slots: 6.8 / 18.1 / 47 -> 5.7 / 14.5 / 35.3; gate / up 8.8 / 24.8 / 65 -> 9.2 / 23.6 / 59
+// One column and one pair: eight wavefronts to a SIMD, 64 registers; with the 65 that gate and up of FP32 take if left alone eight
+// blocks do not fit a CU (512 x 2048, eight slots 8.3 us for 7.7).
 template <typename TX, int GLU, int NC, int RW>
-__global__ void __launch_bounds__(NT) k_nib_mmv(const bf16n_weight w, const bf16n_weight w_up, const cols p, const int ncols) {
+__global__ void __launch_bounds__(NT, NC == 1 && RW == 1 ? 8 : 0) k_nib_mmv(const bf16n_weight w, const bf16n_weight w_up, const cols p, const int ncols) {
     constexpr int M = GLU ? 2 : 1;
     __shared__ float part[RW][M][NC][HALVES];
     const int K = (int) w.K, C = K / CHUNK; // 1 .. 8
