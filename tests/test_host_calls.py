@@ -32,7 +32,7 @@ def test_nothing_on_the_host_is_taken():
     x = torch.zeros(1, 512, dtype=torch.bfloat16)
     for args in ((x, w, True, True), (x, None, True, True), (None, w, True, True), (x, w)):
         assert _calls().mmv(*args) is None
-    for args in ((x, w, 8, 1 << 20), (x, w, "n", 1), (x, w)):
+    for args in ((x, w, 8, 1 << 20), (x, w)):
         assert _calls().linear(*args) is None
     with pytest.raises(ValueError, match="device"):
         ops.mmv(x, w)
@@ -93,9 +93,15 @@ def test_the_plain_product_and_nothing_else(ops):
     assert torch.equal(_calls().mmv(wide[:, :K], w, True, True), _calls().mmv(x, w, True, True))
     short = ops.Weight(w.plane[:-K], w.aux, meta)
     moved = ops.Weight(torch.cat([w.plane, w.plane])[1: rows * K + 1], w.aux, meta)
-    for bad in (x[:, :-8], x[:, ::2], x.half(), x[0], x[:0], x[None], x.cpu(), x.float(), torch.cat([x, x], 1)[:, 1: K + 1], x.to_sparse(),
+    for bad in (x[:, :-8], x[:, ::2], x.half(), x[0], x[:0], x[None], x.cpu(), torch.cat([x, x], 1)[:, 1: K + 1], x.to_sparse(),
                 x.as_subclass(Sub), wide[:, 1: K + 1]):
-        assert (_calls().mmv(bad, w, True, True) is None or bad.dtype == torch.float32) and _calls().linear(bad, w, 8, 1 << 26) is None
+        assert _calls().mmv(bad, w, True, True) is None and _calls().linear(bad, w, 8, 1 << 26) is None
+    assert _calls().mmv(x.float(), w, True, True) is not None and _calls().linear(x.float(), w, 8, 1 << 26) is None
+    # numbers that are none, or none of these (an error that was left set would come up in the call after it)
+    for gemv_tokens, chunk_bytes in (("n", 1 << 26), (8, None), (-1, 1 << 26), (8, -1), (1 << 70, 1 << 26), (8, 1 << 70), (8.5, 1 << 26)):
+        assert _calls().linear(x, w, gemv_tokens, chunk_bytes) is None
+        assert torch.equal(_calls().linear(x, w, 8, 1 << 26), ops.linear(x, w))
+    assert _calls().mmv(x, w, True) is None and _calls().linear(x, w, 8) is None
     for refused in (short, moved):
         assert _calls().mmv(x, refused, True, True) is None and _calls().linear(x, refused, 8, 1 << 26) is None
     with Pass():
