@@ -3,13 +3,14 @@ unit, which takes the batches of more columns, for streams that fall into step, 
 code in a unit), and of very short codes; the streams that do not cost no more than that kernel's chain."""
 from __future__ import annotations
 
+import ctypes as C
 import statistics
 
 import numpy as np
 import pytest
 import torch
 
-from orin_qwen_lossless_amd import synth
+from orin_qwen_lossless_amd import _lib, synth
 from test_gpu_kernels import HP, bits, enc, tbf16
 
 pytestmark = pytest.mark.gpu
@@ -64,6 +65,27 @@ def test_split_units_have_the_bits_of_whole_ones(ops, kind, units, K, R, cm):
     if units > 2:                                              # a range of units that ends before the matrix, and the last one
         assert np.array_equal(bits(ops.dequant(w, R, R)), wb[R:2 * R])
         assert np.array_equal(bits(ops.dequant(w, rows - R, R)), wb[-R:])
+
+
+def test_strided_and_misaligned_columns(ops):
+    """Token strides of whole 16 bytes are taken; the C ABI's others, and columns that begin elsewhere, go to a half-wave per unit."""
+    K, R, rows = 2048, 16, 80
+    w = enc(ops, _matrix("normal", rows, K), HP, R, False, False)
+    x = tbf16(synth.activations(5, K, 7))
+    for xt in (x, x.float()):
+        one = ops.mmv(xt, w)
+        wide = torch.zeros((5, K + 24), dtype=xt.dtype, device="cuda")
+        wide[:, 8: 8 + K] = xt
+        assert torch.equal(ops.mmv(wide[:, 8: 8 + K], w), one) and ops.last_kernel().startswith("k_hp_split<")
+        for shift, pad in ((0, 1), (1, 0), (1, 7)):
+            flat = torch.zeros(shift + 5 * (K + pad), dtype=xt.dtype, device="cuda")
+            view = flat[shift:].view(5, K + pad)[:, :K]
+            view.copy_(xt)
+            y = torch.full_like(one, 7.0)
+            a = _lib.MmvArgs(view.data_ptr(), y.data_ptr(), None, view.stride(0) * view.element_size(), rows * 4, 0, 0, 0, 0, rows, 0, rows, 5, 1, 1,
+                             xt.dtype == torch.bfloat16, False)
+            _lib.check(_lib.lib().bf16n_mmv(C.byref(ops._cweight(w)), C.byref(a), torch.cuda.current_stream().cuda_stream, 1))
+            assert ops.last_kernel().startswith("k_huf_mmv<") and torch.equal(y, one), (shift, pad)
 
 
 # beyond two units per CU: rows whose planes stay in registers, rows whose planes are read again for every column, and a launch
