@@ -479,8 +479,10 @@ __device__ __forceinline__ void nib_load_chunk(const nib_ptrs & w, int64_t gr, i
 // Codes whose lengths are nearly all multiples of one number keep a wrong phase for long: such tables are told by their lengths
 // (falls_into_step), and their units go to one half-wave each in here too (split_whole).  In a run of one code, rows of zeros for
 // instance, no thread falls into step: every second round the threads past the first one that still moves take their phase from
-// the code that begins there, if the next three are the same (14 of 16 rows of 4096, one unit of 64: 136 us with a round per
-// segment, 52 so, 80 in k_huf_mmv; the threads before it are exact, and it gains one a round, so S rounds are enough).
+// the code that begins there, if the next three are the same and four like it stand where they would begin (14 of 16 rows of
+// 4096, one unit of 64: 136 us with a round per segment, 39 so, 80 in k_huf_mmv; without the look at their own place the threads
+// past the run were put out of step as well: 51, and a row of zeros here and there 34.6 for 28.7; the threads before it are exact,
+// and it gains one a round, so S rounds are enough).
 // Two rounds and a half of a sixteenth of the chain instead of the chain, for as many lookups per code: for launches that wait for
 // the chain (hp_split_cols).  8192 x 2048, one column: 42.4 -> 26.6 us (34 with a third round that wrote the exponents: the
 // codes of the second stay in registers until their place is known).
@@ -702,9 +704,14 @@ __global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const c
                 b.two(lut, 0x80000000u, e0, e1);
                 b.two(lut, 0x80000000u, e2, e3);
                 if (e0 == e1 && e1 == e2 && e2 == e3) { // a run
-                    const uint32_t len = e0 & 31u;
-                    start = mine > begins ? begins + (mine - begins + len - 1) / len * len : begins;
-                    moved = true;
+                    const uint32_t run = e0, len = run & 31u, at = mine > begins ? begins + (mine - begins + len - 1) / len * len : begins;
+                    seg_bits here(st, at);
+                    here.two(lut, 0x80000000u, e0, e1);
+                    here.two(lut, 0x80000000u, e2, e3);
+                    if (at != start && e0 == run && e1 == run && e2 == run && e3 == run) { // (it may have ended)
+                        start = at;
+                        moved = true;
+                    }
                 }
             }
             if (moved) {
