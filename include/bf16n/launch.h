@@ -58,7 +58,7 @@ inline bf16n_mmv_args c_args(const mmv_args & a) {
 }
 } // namespace detail
 
-// once per process before any launch and before graph capture
+// once per device that is used, before graph capture
 inline void init() { detail::check(bf16n_init()); }
 inline int sm_count() { int n = 0; detail::check(bf16n_cu_count(&n)); return n; } // compute units of the device
 inline int cu_count() { return sm_count(); }

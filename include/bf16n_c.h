@@ -75,7 +75,7 @@ typedef struct bf16n_mmv_args {
 } bf16n_mmv_args;
 
 /* ---- launchers: core/include/bf16n/launch.h:46-83, core/src/launch.cu ------------------------------------------------ */
-int bf16n_init(void);                 /* init(), launch.h:47, launch.cu:270-306: once per process, before graph capture */
+int bf16n_init(void);                 /* init(), launch.h:47, launch.cu:270-306: once per device that is used, before graph capture */
 int bf16n_cu_count(int * out);        /* sm_count(), launch.h:48 */
 int bf16n_mmv(const bf16n_weight * w, const bf16n_mmv_args * a, void * stream, int multi_col); /* mmv, launch.h:52, launch.cu:313-325 */
 /* (multi_col, launch.h:52: columns of a dense batch may share decodes.  0: every column has the bits of its own

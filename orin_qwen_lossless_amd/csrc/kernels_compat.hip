@@ -28,9 +28,9 @@ constexpr int LUT_PAIRS = 1 << HP_LP;
 // One lane's MSB-first bit stream, read through a ring of 16 words in LDS.  What bounds these kernels is the chain of
 // one unit (two dependent table lookups per two codes, all lanes of a half-wave in step), so nothing else may be waited
 // for in it: 64 lanes read 64 cache lines, and with the next word loaded where it is needed nearly every pair of codes
-// waited for some lane's cache miss (one column of 8192 x 2048, R = 16: 77.7 us then, 42.3 now, about 15 of them by the
-// ring, the rest by plane chunks ahead, small blocks and sums on the VALU; 65536 x 4096: 266 and 162; dequant of the first
-// 88 and 49).  Here a lane loads whole 16-byte blocks, one per four code pairs (96 bits at most, less than a block), LOOK blocks beyond the one it reads, and stores
+// waited for some lane's cache miss (one column of 8192 x 2048, R = 16, a chain each: 77.7 us then, 39.6 now, about 15 of the
+// difference by the ring, the rest by plane chunks ahead, small blocks, sums on the VALU and loads that the compiler knows to be
+// global; 65536 x 4096: 266 and 143; dequant of the first 88 and 34).  Here a lane loads whole 16-byte blocks, one per four code pairs (96 bits at most, less than a block), LOOK blocks beyond the one it reads, and stores
 // what it loaded DEEP rounds ago; the same block again while it has not moved on.  The stream buffers end with padding
 // words (32 of HUFPAIR, 16 of HUFFMAN): the last lane reads at most 17 (13) words past its end.
 constexpr int LR_WORDS = 16;                     // ring words per lane
@@ -484,7 +484,7 @@ __device__ __forceinline__ void nib_load_chunk(const nib_ptrs & w, int64_t gr, i
 // past the run were put out of step as well: 51, and a row of zeros here and there 34.6 for 28.7; the threads before it are exact,
 // and it gains one a round, so S rounds are enough).
 // Two rounds and a half of a sixteenth of the chain instead of the chain, for as many lookups per code: for launches that wait for
-// the chain (hp_split_cols).  8192 x 2048, one column: 42.4 -> 26.6 us (34 with a third round that wrote the exponents: the
+// the chain (hp_split_cols).  8192 x 2048, one column: 39.6 -> 24.7 us (7 more with a third round that wrote the exponents: the
 // codes of the second stay in registers until their place is known).
 constexpr int SPLIT_PAIRS = 32;                  // pair codes per segment at most
 constexpr int SPLIT_PAD = 4;                     // words in front of and behind the staged streams
@@ -666,7 +666,7 @@ __global__ void __launch_bounds__(1024) k_hp_split(const bf16n_weight w, const c
         if (u >= su.count) {
             return;
         }
-        const uint32_t first = 32 * from, bits = 32 * (to - from); // (at most 24 K)
+        const uint32_t first = 32 * from, bits = 32 * (to - from); // (12 a pair code and the last word's rest: 12.3 K at most)
         const uint32_t nstop = 0u - (first + bits * (uint32_t) (seg + 1) / (uint32_t) S);
         uint32_t start = first + bits * (uint32_t) seg / (uint32_t) S - (seg ? bits / (uint32_t) (2 * S) : 0), n = 0;
         auto pair = [](uint32_t e) { return (e >> 7 & 0xFFu) | (e >> 15 & 0xFF00u); };
@@ -1331,18 +1331,18 @@ size_t huf_shared(const bf16n_weight & w, int nc, bool x_bf16) {
 // costs nothing while the device has half-waves to spare (a unit's chain is longer than what they do beside it), and everything
 // beyond: from sixteen half-waves per CU on two columns share one, from eight groups of four per CU on four.  us, each column by
 // itself / two / four of BF16 (HUFPAIR but the last):
-//   two columns: 16384 x 2048, R = 16 (1024 units) 44 / 52 / 65, 32768 x 2048 51 / 53 / 66, 16656 x 3584, R = 8 (2082) 68 / 57 / 72,
-//     42264 x 3072, R = 8 146 / 89 / 105, 59473 x 2560, R = 1 127 / 79 / 93
-//   four: 16384 x 2048 49 / 52 / 66, 24608 x 1024, R = 16 (1538) 60 / 38 / 40, 32768 x 2048 85 / 63 / 67, 42264 x 3072 254 / 153 / 107,
-//     218800 x 512, R = 1 225 / 142 / 90, 7624 x 1536, R = 4 (1906) 22.5 / 19.1 / 19.1, and three there 19.0 / 19.4 / 18.8
-//   eight: 10336 x 3584, R = 16 (646) 130 / 105 / 113, 16384 x 2048 77 / 62 / 66, 24608 x 1024 109 / 64 / 49, 42264 x 3072 496 / 257 / 181,
-//     59473 x 2560 405 / 257 / 172, 16384 x 3072, R = 8, HUFFMAN 231 / 111 / 86
+//   two columns: 16384 x 2048, R = 16 (1024 units) 41 / 49 / 61, 32768 x 2048 49 / 49 / 62, 16656 x 3584, R = 8 (2082) 70 / 53 / 67,
+//     42264 x 3072, R = 8 127 / 82 / 96, 59473 x 2560, R = 1 108 / 68 / 86
+//   four: 16384 x 2048 49 / 49 / 61, 24608 x 1024, R = 16 (1538) 58 / 35 / 38, 32768 x 2048 96 / 60 / 61, 42264 x 3072 235 / 139 / 98,
+//     218800 x 512, R = 1 216 / 123 / 84, 7624 x 1536, R = 4 (1906) 20.2 / 17.6 / 17.6, and three there 17.4 / 18.0 / 17.8
+//   eight: 10336 x 3584, R = 16 (646) 137 / 99 / 106, 16384 x 2048 80 / 59 / 61, 24608 x 1024 98 / 66 / 47, 42264 x 3072 441 / 238 / 173,
+//     59473 x 2560 378 / 235 / 161, 16384 x 3072, R = 8, HUFFMAN 209 / 111 / 84
 // A last group of four may hold one column: pairs then, and single columns, while their blocks are no more than the CUs hold anyway
-// (two of pairs, three where units are short).  1030 units of 4 x 1024, five columns 11.6 / 11.9 / 15.1, of 1 x 512 5.2 / 5.5 / 6.5; 1400, seven
-// 5.7 (6.7 by fours); but 2060 units, eight 8.5 / 7.2.
+// (two of pairs, three where units are short).  1030 units of 4 x 1024, five columns 12.1 / 12.3 / 15.3, of 1 x 512 5.1 / 5.4 / 6.2; 1400, seven
+// 7.4 / 6.0 / 6.7; but 2060 units, eight 10.5 / 8.8 / 7.3.
 // Four FP32 columns of 3584 and more leave a CU one block, so that the second waits for the first: pairs, but for HUFFMAN's longer units
-// once their pairs wait too.  1030 units of 1 x 4096, five columns 11.7 / 10.9 / 20.7, of 16 x 4096 160 / 101 / 193; HUFFMAN 1400 of
-// 1 x 4096, five 20.0 / 16.8 / 26.7, 800 of 4 x 4096, twelve 126 / 59 / 81, 3000, eight 485 / 163 / 121.
+// once their pairs wait too.  1030 units of 1 x 4096, five columns 11.8 / 11.2 / 20.7, of 16 x 4096 158 / 101 / 192; HUFFMAN 1400 of
+// 1 x 4096, five 20.6 / 17.7 / 26.9, 800 of 4 x 4096, twelve 125 / 59 / 80, 3000, eight 475 / 164 / 121.
 // Blocks of eight wavefronts instead of four: 5 to 25 % behind but for long rows of short units.
 int huf_columns(const bf16n_weight & w, int64_t units, int ncols, bool x_bf16, int cus) {
     const int chunks = w.R * (int) (w.K / CHUNK);
@@ -1357,14 +1357,14 @@ int huf_columns(const bf16n_weight & w, int64_t units, int ncols, bool x_bf16, i
 
 // Dense products whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers
 // per wavefront, so that 16 of them (12 at K = 4096) fit a CU instead of 20 (16), and a lane that has not moved on loads its
-// block again; with many wavefronts the misses of one are covered by the others.  Without against with rings, one column:
-//  * HUFPAIR in short units that the caches hold, from 64 wavefronts per CU on (32768 x 2048, four chunks, eight columns one by one:
-//    202 against 174 us).
+// block again; with many wavefronts the misses of one are covered by the others.  us without against with rings, one column:
+//  * HUFPAIR in short units that the caches hold, from 64 wavefronts per CU on: 32768 x 512 11.7 against 14.2 (from memory, 32768 x 2048,
+//    R = 1, 30.6 and 28.2).  The line is on the careful side: 16384 x 512 has 7.9 and 9.7.
 //  * HUFFMAN, which loads a block per eight codes where HUFPAIR has one per sixteen, from 16 wavefronts per CU on unless
-//    the matrix comes from memory in short units: 32768 x 4096, R = 4 142 against 208 us.
+//    the matrix comes from memory in short units: 8192 x 512 5.6 against 6.1, 32768 x 4096, R = 4 139 and 199 (16384 x 2048, R = 4 32.3 and 24.7).
 // Several columns, one by one without rings against the fours that would share a decode: units of one chunk that the caches hold, from 48
-// wavefronts per CU on, where a quarter of the fours' columns or more would be missing: 9000 x 512, five 11.8 against 15.0, six 13.5 and
-// 15.0, nine 18.5 and 20.8 (seven 15.7 and 15.0); HUFFMAN 14.1 and 16.9, 16.0 and 16.9, 22 and 23.8.
+// wavefronts per CU on, where a quarter of the fours' columns or more would be missing: 9000 x 512, five 12.4 against 15.5, six 13.6 and
+// 15.1, nine 18.4 and 20.7 (seven 15.4 and 15.0); HUFFMAN 14.0 and 16.8, 15.8 and 16.8, 21.9 and 23.7.
 bool huf_direct(const bf16n_weight & w, int64_t units, int ncols, int nc, int cus) {
     const int64_t per_cu = units * ncols / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
     const int chunks = w.R * (int) (w.K / CHUNK);

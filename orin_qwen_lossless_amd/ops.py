@@ -3,7 +3,8 @@ Python operator module (engines/vllm/vllm_bf16n/ops.py) so that code and tests w
 encode / upload / dequant / roundtrip_equal / mmv / mmv_glu / linear / get_rows / embedding / moe_mm_ids /
 moe_combine / swiglu / moe_experts, plus router_topk and choose.
 
-torch is used for device memory and streams only; every product runs in libbf16n_hip.so.  Weights are passed
+torch is used for device memory, streams and the stock BF16 product that `linear` puts behind the exact dequant of many
+tokens (as the reference does); everything else runs in libbf16n_hip.so.  Weights are passed
 explicitly as plane + aux uint8 tensors with metadata parsed once from the aux header on the host."""
 from __future__ import annotations
 
@@ -171,7 +172,7 @@ def _check_ids(ids: torch.Tensor) -> None:
 
 
 def init() -> None:
-    """Device attributes and kernel shared-memory limits; once per process, before any launch / graph capture."""
+    """Device attributes and kernel shared-memory limits of the current device; once for each that is used, before any launch / graph capture."""
     _lib.check(_lib.lib().bf16n_init())
 
 
