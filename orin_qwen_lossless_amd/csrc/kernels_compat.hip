@@ -1381,6 +1381,7 @@ bool huf_direct(const bf16n_weight & w, int64_t units, int ncols, int nc, int cu
 //   up to two units per CU, one / 2 / 4 / 6 / 8 columns: 8192 x 2048, R = 16 0.64 / 0.64 / 0.78 / 0.78 / 0.87, 4096 x 2048 0.46 / 0.50 /
 //     0.55 / 0.58 / 0.73; 4096 x 4096, R = 8 0.58 / 0.64 / 0.86 / 0.89 / 1.02; 4096 x 3584, R = 8 0.69 / 0.72 / 0.93 / 0.95 / 1.09; 4096 x 3072,
 //     R = 8 0.71 / 0.76 / 0.96 / 0.98 / 1.12; 8192 x 1024 0.84 / 0.87 / 1.07 / 1.09 / 1.22; 8192 x 4096 0.68 / 0.72 / 0.96 / 1.05 / 1.28
+//   up to one, where the plane read again finds the CU idle: 1912 x 4096, R = 8, 7 / 8 FP32 columns 0.65 / 0.69, BF16 0.79 / 0.86
 //   three, in two passes of two blocks: 12288 x 2048 0.82 / 0.84 / 0.95 / 0.77 / 0.82 (640 units, six: 1.05); 6144 x 4096, R = 8 0.83 / 0.94 /
 //     1.14 / 1.00 / 1.09; 6144 x 3584 0.92 / 0.99; 6144 x 3072 1.00 / 1.07; or in three passes of one, a column: 12288 x 2560 1.06,
 //     12288 x 3072 0.96, 12288 x 3584 0.96, 12288 x 4096 0.94
@@ -1394,7 +1395,7 @@ int hp_split_cols(const bf16n_weight & w, int64_t units, int cus, bool rows = fa
     if (units > 2 * (int64_t) cus) {
         return pairs == 512 ? kept ? 8 : 2 : pairs == 448 || pairs >= 768 ? 1 : 0;
     }
-    return pairs <= 512 ? std::min((pairs - 128) / 48, kept ? 8 : 6) : units > cus ? 4 : 8;
+    return pairs <= 512 ? std::min((pairs - 128) / 48, kept || units <= cus ? 8 : 6) : units > cus ? 4 : 8;
 }
 constexpr int SPLIT_DEQUANT_COLS = 3; // what the exact rows cost in its place, in columns
 int split_threads(const bf16n_weight & w) {

@@ -44,7 +44,7 @@ def _matrix(kind: str, rows: int, K: int) -> np.ndarray:
 @pytest.mark.parametrize("kind,units,K,R,cm", [
     ("normal", 1, 2048, 16, False), ("normal", 300, 2048, 16, True), ("normal", 513, 2048, 16, False), ("normal", 5, 4096, 16, True),
     ("normal", 257, 4096, 16, False), ("normal", 33, 1024, 16, True), ("normal", 7, 2048, 8, False), ("normal", 9, 3072, 8, True),
-    ("normal", 9, 2560, 8, False), ("one", 3, 2048, 16, False), ("short", 3, 2048, 16, False), ("short", 2, 4096, 16, True),
+    ("normal", 9, 2560, 8, False), ("normal", 239, 4096, 8, False), ("normal", 257, 4096, 8, True), ("one", 3, 2048, 16, False), ("short", 3, 2048, 16, False), ("short", 2, 4096, 16, True),
     ("flat", 3, 2048, 16, False), ("flat", 2, 4096, 16, False), ("flat", 2, 2048, 8, True),
     ("equal", 1, 2048, 16, False), ("equal", 2, 4096, 4, False), ("equal", 515, 2048, 16, False), ("rare", 7, 2048, 16, True),
     ("rare", 7, 4096, 8, False), ("rare", 301, 4096, 16, False), ("rare", 33, 3072, 8, True), ("rare", 513, 2048, 16, False),
@@ -56,7 +56,7 @@ def test_split_units_have_the_bits_of_whole_ones(ops, kind, units, K, R, cm):
     w = enc(ops, wb, HP, R, cm, False)
     assert w.meta.format == HP and w.meta.chunk_major == cm
     xb = tbf16(synth.activations(9, K, 7))
-    limit = min(8 if K <= 2048 else 6, (R * K // 64 - 128) // 48) if R * K // 64 <= 512 else 4
+    limit = min(8 if K <= 2048 or units <= ops.cu_count() else 6, (R * K // 64 - 128) // 48) if R * K // 64 <= 512 else 4
     for x in (xb, xb.float()):
         whole = ops.mmv(x, w)
         assert ops.last_kernel().startswith("k_huf_mmv<3, ")
