@@ -1327,50 +1327,63 @@ size_t huf_shared(const bf16n_weight & w, int nc, bool x_bf16) {
     return (size_t) nc * w.K * (x_bf16 ? 2 : 4) + (w.format == FMT_HUFPAIR ? 4u << HP_LP : 4u << HUF_LMAX) + (size_t) (NT / 64) * LR_BYTES;
 }
 
+// What a chunk of a unit costs with nc columns to a decode, in 10 ns, by the blocks that a CU has at once (fitted to 8000 launches of
+// 64 to 9000 units of one to 128 chunks, two to sixteen columns; 6 to 8 % rms): mostly the chain of lookups, a column and the second
+// block beside the first a sixth to a quarter of it each.  Three and four FP32 columns have registers for three blocks.
+constexpr uint16_t HUF_CHUNK[2][2][3][4] = { // [HUFFMAN, HUFPAIR][FP32, BF16][nc - 2][blocks - 1]
+    {{{101, 123, 172, 199}, {111, 136, 180, 0}, {121, 149, 200, 0}}, {{104, 130, 181, 234}, {118, 146, 200, 258}, {130, 163, 225, 288}}},
+    {{{64, 80, 105, 125}, {73, 90, 120, 0}, {84, 103, 131, 0}}, {{69, 88, 119, 144}, {82, 102, 142, 166}, {94, 121, 159, 197}}}};
+int64_t huf_time(const bf16n_weight & w, int64_t units, int ncols, int nc, bool x_bf16, int cus) {
+    const uint16_t (&t)[4] = HUF_CHUNK[w.format == FMT_HUFPAIR][x_bf16][nc - 2];
+    const int64_t fit = std::min<int64_t>((int64_t) (LDS_BYTES / huf_shared(w, nc, x_bf16)), x_bf16 || nc == 2 ? 4 : 3); // blocks of a CU at once
+    const int64_t blocks = (units + HALVES - 1) / HALVES * ((ncols + nc - 1) / nc), rounds = blocks / (fit * cus), last = (blocks % (fit * cus) + cus - 1) / cus;
+    return rounds * t[fit - 1] + (last ? t[last - 1] : 0);
+}
+
 // Columns that share one decode in dense products.  Each column in a launch of its own units decodes the matrix again, which
 // costs nothing while the device has half-waves to spare (a unit's chain is longer than what they do beside it), and everything
-// beyond: from sixteen half-waves per CU on two columns share one, from eight groups of four per CU on four.  us, each column by
-// itself / two / four of BF16 (HUFPAIR but the last):
-//   two columns: 16384 x 2048, R = 16 (1024 units) 41 / 49 / 61, 32768 x 2048 49 / 49 / 62, 16656 x 3584, R = 8 (2082) 70 / 53 / 67,
-//     42264 x 3072, R = 8 127 / 82 / 96, 59473 x 2560, R = 1 108 / 68 / 86
-//   four: 16384 x 2048 49 / 49 / 61, 24608 x 1024, R = 16 (1538) 58 / 35 / 38, 32768 x 2048 96 / 60 / 61, 42264 x 3072 235 / 139 / 98,
-//     218800 x 512, R = 1 216 / 123 / 84, 7624 x 1536, R = 4 (1906) 20.2 / 17.6 / 17.6, and three there 17.4 / 18.0 / 17.8
-//   eight: 10336 x 3584, R = 16 (646) 137 / 99 / 106, 16384 x 2048 80 / 59 / 61, 24608 x 1024 98 / 66 / 47, 42264 x 3072 441 / 238 / 173,
-//     59473 x 2560 378 / 235 / 161, 16384 x 3072, R = 8, HUFFMAN 209 / 111 / 84
-// A last group of four may hold one column: pairs then, and single columns, while their blocks are no more than the CUs hold anyway
-// (two of pairs, three where units are short).  1030 units of 4 x 1024, five columns 12.1 / 12.3 / 15.3, of 1 x 512 5.1 / 5.4 / 6.2; 1400, seven
-// 7.4 / 6.0 / 6.7; but 2060 units, eight 10.5 / 8.8 / 7.3.
-// Four FP32 columns of 3584 and more leave a CU one block, so that the second waits for the first: pairs, but for HUFFMAN's longer units
-// once their pairs wait too.  1030 units of 1 x 4096, five columns 11.8 / 11.2 / 20.7, of 16 x 4096 158 / 101 / 192; HUFFMAN 1400 of
-// 1 x 4096, five 20.6 / 17.7 / 26.9, 800 of 4 x 4096, twelve 125 / 59 / 80, 3000, eight 475 / 164 / 121.
+// beyond: from fifteen half-waves per CU on two or three columns share one (from sixteen in units of at most 32 chunks, 24 of at
+// most four), from eight groups of four per CU on four.  us, each column by itself / two / three / four, BF16 and HUFPAIR but where named:
+//   two columns: 16384 x 2048, R = 16 (1024 units) 41 / 49, 32768 x 2048 49 / 49, 16656 x 3584, R = 8 (2082) 70 / 53, 42264 x 3072,
+//     R = 8 127 / 82, 59473 x 2560, R = 1 108 / 68
+//   three: 10920 x 3072, R = 8 (1365 units, 16 half-waves per CU) 53.3 / 48.2 / 46.0, FP32 54.2 / 44.2 / 41.6
+//   four: 24608 x 1024, R = 16 (1538) 58 / 35 / - / 38, 32768 x 2048 96 / 60 / - / 61, 42264 x 3072 235 / 139 / - / 98, 218800 x 512, R = 1
+//     216 / 123 / - / 84
+//   eight: 10336 x 3584, R = 16 (646) 137 / 99 / - / 106, 24608 x 1024 98 / 66 / - / 47, 42264 x 3072 441 / 238 / - / 173, 16384 x 3072, R = 8,
+//     HUFFMAN 209 / 111 / - / 84
+// Another count than these lines give where huf_time has it 6 % ahead: three, where a group of four would lack a column or more or leave a
+// CU one block of FP32, and pairs where their blocks fit the CUs at once: FP32, six columns, 1365 units of 8 x 3072 97 / 74 / 48 / 53; nine,
+// 848 of 1 x 3584 16.2 / 17.9 / 12.6 / 22.6, 1368 of 1 x 1536 12.4 / 12.2 / 9.4 / 15.0; BF16, nine, 5057 of 1 x 1536 31.7 / 31.2 / 27.1 / 31.2;
+// HUFFMAN, four FP32, 2152 of 1 x 4096 26 / 17.6 / 26 / 24.
 // Blocks of eight wavefronts instead of four: 5 to 25 % behind but for long rows of short units.
 int huf_columns(const bf16n_weight & w, int64_t units, int ncols, bool x_bf16, int cus) {
     const int chunks = w.R * (int) (w.K / CHUNK);
-    const int64_t pairs = units * ((ncols + 1) / 2), fours = units * ((ncols + 3) / 4), full = 8 * (int64_t) cus; // half-waves; of a block per CU
-    int nc = ncols > 2 && fours > full ? 4 : ncols > 1 && units * ncols > 2 * full && (ncols != 3 || chunks >= 16) ? 2 : 1;
-    const bool alone = 2 * huf_shared(w, 4, x_bf16) > LDS_BYTES;
-    if (nc == 4 && (pairs <= (chunks <= 4 ? 3 : 2) * full || (alone && (w.format == FMT_HUFPAIR || chunks <= 8 || pairs <= 3 * full)))) {
-        nc = 2;
+    if (ncols == 1 || units * ncols <= (chunks <= 4 ? 24 : chunks <= 32 ? 16 : 15) * (int64_t) cus) {
+        return 1;
     }
-    return nc == 2 && units * ncols <= 2 * full ? 1 : nc;
+    const int line = ncols > 2 && units * ((ncols + 3) / 4) > HALVES * (int64_t) cus ? 4 : ncols == 3 ? 3 : 2;
+    int best = line;
+    int64_t time = huf_time(w, units, ncols, line, x_bf16, cus) * 94;
+    for (int nc = 2; nc <= std::min(4, ncols); nc++) {
+        const int64_t t = huf_time(w, units, ncols, nc, x_bf16, cus) * 100;
+        if (nc != line && t < time) {
+            best = nc;
+            time = t;
+        }
+    }
+    return best;
 }
 
-// Dense products whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers
+// Dense products of one column whose lanes read their streams without the rings.  A ring costs 4 KiB of LDS and thirty registers
 // per wavefront, so that 16 of them (12 at K = 4096) fit a CU instead of 20 (16), and a lane that has not moved on loads its
-// block again; with many wavefronts the misses of one are covered by the others.  us without against with rings, one column:
+// block again; with many wavefronts the misses of one are covered by the others.  us without against with rings:
 //  * HUFPAIR in short units that the caches hold, from 64 wavefronts per CU on: 32768 x 512 11.7 against 14.2 (from memory, 32768 x 2048,
 //    R = 1, 30.6 and 28.2).  The line is on the careful side: 16384 x 512 has 7.9 and 9.7.
 //  * HUFFMAN, which loads a block per eight codes where HUFPAIR has one per sixteen, from 16 wavefronts per CU on unless
 //    the matrix comes from memory in short units: 8192 x 512 5.6 against 6.1, 32768 x 4096, R = 4 139 and 199 (16384 x 2048, R = 4 32.3 and 24.7).
-// Several columns, one by one without rings against the fours that would share a decode: units of one chunk that the caches hold, from 48
-// wavefronts per CU on, where a quarter of the fours' columns or more would be missing: 9000 x 512, five 12.4 against 15.5, six 13.6 and
-// 15.1, nine 18.4 and 20.7 (seven 15.4 and 15.0); HUFFMAN 14.0 and 16.8, 15.8 and 16.8, 21.9 and 23.7.
-bool huf_direct(const bf16n_weight & w, int64_t units, int ncols, int nc, int cus) {
-    const int64_t per_cu = units * ncols / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
+bool huf_direct(const bf16n_weight & w, int64_t units, int cus) {
+    const int64_t per_cu = units / (2 * cus), weights = units * w.R * w.K; // wavefronts of the launch per CU
     const int chunks = w.R * (int) (w.K / CHUNK);
-    if (ncols > 1) {
-        return nc == 4 && chunks == 1 && per_cu >= 48 && weights <= (16 << 20) && ncols > 4 && ncols <= 3 * ((ncols + 3) / 4);
-    }
     return w.format == FMT_HUFPAIR ? chunks <= 8 && per_cu >= 64 && weights <= (16 << 20) : per_cu >= 16 && (weights <= (16 << 20) || chunks >= 32);
 }
 
@@ -1426,8 +1439,9 @@ void launch_hp_split(const bf16n_weight & w, const cols & p, int ncols, uint16_t
 
 void compat_init() {
 #define HUFA(F, TX, N) (void) hipFuncSetAttribute((const void *) k_huf_mmv<F, TX, false, true, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) LDS_BYTES)
-    HUFA(FMT_HUFPAIR, bf16_t, 2); HUFA(FMT_HUFPAIR, bf16_t, 4); HUFA(FMT_HUFPAIR, float, 2); HUFA(FMT_HUFPAIR, float, 4);
-    HUFA(FMT_HUFFMAN, bf16_t, 2); HUFA(FMT_HUFFMAN, bf16_t, 4); HUFA(FMT_HUFFMAN, float, 2); HUFA(FMT_HUFFMAN, float, 4);
+#define HUFAN(F, TX) HUFA(F, TX, 2); HUFA(F, TX, 3); HUFA(F, TX, 4)
+    HUFAN(FMT_HUFPAIR, bf16_t); HUFAN(FMT_HUFPAIR, float); HUFAN(FMT_HUFFMAN, bf16_t); HUFAN(FMT_HUFFMAN, float);
+#undef HUFAN
 #undef HUFA
     const int shm = (int) split_shm(1024, 1024);
     (void) hipFuncSetAttribute((const void *) k_hp_split<bf16_t, false>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
@@ -1542,15 +1556,14 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
     const size_t shared = (size_t) w.K * 4 + (size_t) (glu ? 2 : 1) * (hp ? (4u << HP_LP) : (4u << HUF_LMAX));
     const char * instance = hp ? x_bf16 ? "3, bf16_t" : "3, float" : x_bf16 ? "2, bf16_t" : "2, float";
     const int nc = glu || p.ids ? 1 : huf_columns(w, work, ncols, x_bf16, cus);
-    const bool direct = !glu && !p.ids && huf_direct(w, work, ncols, nc, cus);
-    if (nc > 1 && !direct) {
+    if (nc > 1) {
         const int waves = NT / 64, groups = (ncols + nc - 1) / nc;
         const size_t shm = huf_shared(w, nc, x_bf16);
         const int64_t blocks = std::min<int64_t>((work + 2 * waves - 1) / (2 * waves), (int64_t) cus * (int64_t) (LDS_BYTES / shm));
         const dim3 grid((unsigned) blocks, (unsigned) groups); // (a block stages its table and columns once)
         note_kernel("k_huf_mmv", instance, 3, 0, 1, nc);
 #define HUFN(F, TX, N) hipLaunchKernelGGL((k_huf_mmv<F, TX, false, true, N>), grid, dim3(waves * 64), shm, stream, w, wu, p, ncols)
-#define HUFNX(F, TX) do { if (nc == 4) HUFN(F, TX, 4); else HUFN(F, TX, 2); } while (0)
+#define HUFNX(F, TX) do { if (nc == 4) HUFN(F, TX, 4); else if (nc == 3) HUFN(F, TX, 3); else HUFN(F, TX, 2); } while (0)
         if (hp) {
             if (x_bf16) HUFNX(FMT_HUFPAIR, bf16_t); else HUFNX(FMT_HUFPAIR, float);
         } else {
@@ -1560,6 +1573,7 @@ void launch_compat_mmv(const bf16n_weight & w, const bf16n_weight * up, int glu,
 #undef HUFN
         return;
     }
+    const bool direct = !glu && !p.ids && ncols == 1 && huf_direct(w, work, cus);
     note_kernel("k_huf_mmv", instance, 3, glu != 0, !direct, 1);
     const int waves = direct ? NT / 64 : huf_waves(work, ncols, cus, w.R * (int) (w.K / CHUNK));
     const size_t shm = shared + (direct ? 0 : (size_t) waves * LR_BYTES);
